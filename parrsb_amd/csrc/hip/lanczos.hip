@@ -57,35 +57,88 @@ struct lz_args {
   const int *act_tiles;  // if set: blockIdx.x -> tile (compacted active list)
   const int *act_segs;   // if set: blockIdx.x -> segment, for k_lz_fin
   int pstride;           // partial is slot-major: slot k of tile t at k * pstride + t
+  struct lz_it *st0;     // if set: FIN_SETUP1 fills the state the fused iterations start from
 };
 
+// What a tile's workgroup needs to know, in one record of 64 bytes: one
+// load instead of a chain of them (list entry -> tile -> segment table,
+// halo table).  The running list of the fused iterations holds copies.
+struct __attribute__((aligned(16))) lz_desc {
+  int s, row0, row1, pstart;
+  int n, first, count, nhalo;
+  int64_t halo_off;
+  int ti, pad0;
+  int pad[4];
+};
+
+// Scalar state of a segment between two launches of the fused iterations.
+struct lz_it {
+  double rtz1, rtz2, beta, pap, pap_old, meanp, alpha, rtol;
+  int it, mi;  // iteration whose apply ran last; the pass's length
+};
+// field by field: a struct copy went through LDS
+__device__ inline void it_load(lz_it &x, const lz_it *__restrict__ p) {
+  x.rtz1 = p->rtz1, x.rtz2 = p->rtz2, x.beta = p->beta, x.pap = p->pap, x.pap_old = p->pap_old;
+  x.meanp = p->meanp, x.alpha = p->alpha, x.rtol = p->rtol, x.it = p->it, x.mi = p->mi;
+}
+__device__ inline void it_store(lz_it *__restrict__ p, const lz_it &x) {
+  p->rtz1 = x.rtz1, p->rtz2 = x.rtz2, p->beta = x.beta, p->pap = x.pap, p->pap_old = x.pap_old;
+  p->meanp = x.meanp, p->alpha = x.alpha, p->rtol = x.rtol, p->it = x.it, p->mi = x.mi;
+}
+
 #define SC(s, j) a.sc[(size_t)(s) * LZ_NSC + (j)]
+
+// Every product that meets a sum on the iterations' path is an explicit
+// fused multiply-add, and the sums themselves contract nothing: left to the
+// compiler, which products were fused depended on the code around them, and
+// two kernels doing the same sum differed in the last bit.
+__device__ inline float fmat(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ inline double fmat(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
 template <typename T>
 struct acc_t;
 template <>
 struct acc_t<double> {
   double v = 0.0;
-  __device__ inline void dot(double x, double y) { v += x * y; }
-  __device__ inline void add(double x) { v += x; }
+  __device__ inline void dot(double x, double y) { v = fmat(x, y, v); }
+  // the product rounded before it is added
+  __device__ inline void dot2(double x, double y) {
+#pragma clang fp contract(off)
+    v = v + x * y;
+  }
+  __device__ inline void add(double x) {
+#pragma clang fp contract(off)
+    v = v + x;
+  }
   __device__ inline double value() const { return v; }
 };
 template <>
 struct acc_t<float> {
   float s = 0.f, c = 0.f;
+  // s + xy rounded once; c takes that sum's error and the product's
   __device__ inline void dot(float x, float y) {
-    float p = x * y;
-    float ep = __builtin_fmaf(x, y, -p);  // exact product error
-    float t, et;
-    two_sum(s, p, t, et);
+#pragma clang fp contract(off)
+    const float ep = fmat(x, y, -(x * y));
+    const float t = fmat(x, y, s), bb = t - s;
+    const float et = (s - (t - bb)) + fmat(x, y, -bb);
     s = t;
-    c += ep + et;
+    c = c + (ep + et);
+  }
+  // the product rounded before it is added
+  __device__ inline void dot2(float x, float y) {
+#pragma clang fp contract(off)
+    const float p = x * y, ep = fmat(x, y, -p);
+    const float t = s + p, bb = t - s;
+    const float et = (s - (t - bb)) + (p - bb);
+    s = t;
+    c = c + (ep + et);
   }
   __device__ inline void add(float x) {
-    float t, et;
-    two_sum(s, x, t, et);
+#pragma clang fp contract(off)
+    const float t = s + x, bb = t - s;
+    const float et = (s - (t - bb)) + (x - bb);
     s = t;
-    c += et;
+    c = c + et;
   }
   __device__ inline double value() const { return (double)s + (double)c; }
 };
@@ -135,7 +188,7 @@ __device__ inline bool tile_of(const lz_args &a, int want_status, tile_t &t, int
 template <int NV>
 __device__ inline void publish(const lz_args &a, const tile_t &t, double (&v)[NV]) {
   __shared__ double red[(RSB_BLOCK / RSB_WAVE) * (NV > 4 ? NV : 4)];
-  block_sum<NV>(v, red);
+  block_sum<NV, RSB_BLOCK / RSB_WAVE>(v, red);
   if (threadIdx.x == 0)
     for (int k = 0; k < NV; k++) a.partial[(size_t)k * a.pstride + t.ti] = v[k];
 }
@@ -227,7 +280,7 @@ __device__ inline T rval(const T *__restrict__ r, const T *__restrict__ wp, uint
 template <typename T, bool FIRST, bool FOLD>
 __device__ inline T qval(const T *__restrict__ p, const T *__restrict__ r,
                          const T *__restrict__ wp, uint32_t c, T beta, T m, T alpha) {
-  return FIRST ? r[c] : beta * (p[c] - m) + rval<T, FOLD>(r, wp, c, alpha);
+  return FIRST ? r[c] : fmat(beta, p[c] - m, rval<T, FOLD>(r, wp, c, alpha));
 }
 
 template <typename T, bool FIRST, bool FOLD>
@@ -245,11 +298,12 @@ __device__ inline T lap_row_q(const uint32_t *__restrict__ e, int wd, T qi,
     for (int u = 0; u < 8; u++)
       v[u] = qval<T, FIRST, FOLD>(p, r, wp, q[u] & 0x0fffffffu, beta, m, alpha);
 #pragma unroll
-    for (int u = 0; u < 8; u++) sum += (T)(q[u] >> 28) * (qi - v[u]);
+    for (int u = 0; u < 8; u++) sum = fmat((T)(q[u] >> 28), qi - v[u], sum);
   }
   for (; j < wd; j++) {
     uint32_t q = __builtin_nontemporal_load(e + (size_t)j * RSB_WAVE);
-    sum += (T)(q >> 28) * (qi - qval<T, FIRST, FOLD>(p, r, wp, q & 0x0fffffffu, beta, m, alpha));
+    sum = fmat((T)(q >> 28), qi - qval<T, FIRST, FOLD>(p, r, wp, q & 0x0fffffffu, beta, m, alpha),
+               sum);
   }
   return sum;
 }
@@ -283,7 +337,7 @@ __device__ inline void lz_apply_rows(const lz_args &a, const tile_t &t, const T 
     const T ri = rval<T, UPD>(r, fd.wp, (uint32_t)row, fd.alpha);
     T qi = (T)0, wi = (T)0;
     if (real) {
-      qi = FIRST ? ri : beta * (pold[row] - m) + ri;
+      qi = FIRST ? ri : fmat(beta, pold[row] - m, ri);
       const int sl = row >> 6;
       wi = lap_row_q<T, FIRST, UPD>(ell + slice_off[sl] + (row & 63), slice_w[sl], qi, pold, r,
                                     fd.wp, beta, m, fd.alpha);
@@ -301,7 +355,14 @@ __device__ inline void lz_apply_rows(const lz_args &a, const tile_t &t, const T 
 // LDS-tiled rows (tiles.hip): q for the tile's rows and its halo is staged
 // in LDS once; every neighbour is then read from LDS through a 16-bit local
 // index, 8 entries per 16-byte load.
+// Where a slice's entries lie in the form the solve reads: its offset, width
+// and (12-bit form) class slots, one 16-byte record instead of three arrays.
+struct __attribute__((aligned(16))) slice_rec {
+  int64_t off;
+  int w, c;
+};
 struct tiled_args {
+  const slice_rec *slice;
   const int64_t *slice_off;
   const int *slice_w;
   const uint32_t *ell;
@@ -311,11 +372,7 @@ struct tiled_args {
   const int64_t *off16;
   const int *w16;
   const uint16_t *e16;
-  // the 12-bit form (tiles.hip), or e12 == nullptr
-  const int64_t *off12;
-  const int *w12;
-  const uint32_t *e12;
-  const int *c12;
+  const uint32_t *e12;  // the 12-bit form (tiles.hip), or nullptr
 };
 
 #define TB_LOCAL 4096
@@ -324,12 +381,30 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 template <typename T>
 __device__ inline void acc_entry(uint32_t e, T qi, const T *ql, T &sum) {
-  sum += (T)(e >> 12) * (qi - ql[e & 0xfffu]);
+  sum = fmat((T)(e >> 12), qi - ql[e & 0xfffu], sum);
+}
+
+// The sums a row of the 16-bit form adds.  ODD: the thread's second and
+// fourth row; there the last product of the row (w.q, or w.w with the folded
+// update) is rounded before it is added.  (That is how the rows of this form
+// have been summed since it exists; results stay what they were to the bit.)
+template <bool ODD, typename T, bool FOLD>
+__device__ inline void row_sums16(T qi, T wi, T ri, acc_t<T> &sq, acc_t<T> &swq, acc_t<T> &sw,
+                                  fold_t<T> &fd) {
+  sq.add(qi);
+  if (ODD && !FOLD) swq.dot2(wi, qi);
+  else swq.dot(wi, qi);
+  sw.add(wi);
+  if (FOLD) {
+    fd.rr.dot(ri, ri), fd.rw.dot(ri, wi);
+    if (ODD) fd.ww.dot2(wi, wi);
+    else fd.ww.dot(wi, wi);
+  }
 }
 
 // One row of the tiled apply: its 16-bit entries (groups of 8, then groups
 // of 4 and 2) against the LDS window; writes p', w and the basis entry.
-template <typename T, bool FOLD>
+template <bool ODD, typename T, bool FOLD>
 __device__ inline void apply_row_tiled(int row, const tile_t &t, const tiled_args &ta,
                                        const T *ql, const T *rl, T *__restrict__ pnew,
                                        T *__restrict__ w, int nreal, acc_t<T> &sq,
@@ -368,12 +443,29 @@ __device__ inline void apply_row_tiled(int row, const tile_t &t, const tiled_arg
   pnew[row] = qi;
   w[row] = sum;
   const T ri = FOLD ? rl[li] : (T)0;  // the tile's r is kept in LDS only to fold
-  if (li < nreal) {
-    sq.add(qi);
-    swq.dot(sum, qi);
-    sw.add(sum);
-    if (FOLD) fd.rr.dot(ri, ri), fd.rw.dot(ri, sum), fd.ww.dot(sum, sum);
+  if (li < nreal) row_sums16<ODD, T, FOLD>(qi, sum, ri, sq, swq, sw, fd);
+}
+
+// Where the entries of a thread's (up to four) rows lie: row t.row0 +
+// threadIdx.x + 256 k is in slice (t.row0 >> 6) + wave + 4 k, the same for
+// the whole wave, so these are scalar loads; they are issued before the
+// window is staged (the kernel has stored nothing yet) and are back when the
+// rows want them.
+#define LZ_RPT (RSB_TILE / RSB_BLOCK)
+struct slice_meta {
+  int64_t off[LZ_RPT];
+  int w[LZ_RPT], c[LZ_RPT];  // widths (0: no such rows); class slots (12-bit form)
+};
+__device__ inline slice_meta load_meta(const tile_t &t, const tiled_args &ta) {
+  slice_meta m;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / RSB_WAVE);
+#pragma unroll
+  for (int k = 0; k < LZ_RPT; k++) {
+    const int r = t.row0 + wave * RSB_WAVE + k * RSB_BLOCK;
+    const slice_rec q = ta.slice[min(r, t.row1 - 1) >> 6];
+    m.off[k] = q.off, m.w[k] = r < t.row1 ? q.w : 0, m.c[k] = q.c;
   }
+  return m;
 }
 
 // R rows per thread and step: the entries of all R rows are loaded before
@@ -381,28 +473,35 @@ __device__ inline void apply_row_tiled(int row, const tile_t &t, const tiled_arg
 // whose slice is wider than 32 entries take apply_row_tiled.  Missing groups
 // are zero words (weight 0), which add exact zeros.
 template <typename T, int R, bool FOLD>
-__device__ inline void apply_rows_batched(const tile_t &t, const tiled_args &ta, const T *ql,
-                                          const T *rl, T *__restrict__ pnew, T *__restrict__ w,
-                                          int nreal, acc_t<T> &sq, acc_t<T> &swq, acc_t<T> &sw,
+__device__ inline void apply_rows_batched(const tile_t &t, const tiled_args &ta,
+                                          const slice_meta &sm, const T *ql, const T *rl,
+                                          T *__restrict__ pnew, T *__restrict__ w, int nreal,
+                                          acc_t<T> &sq, acc_t<T> &swq, acc_t<T> &sw,
                                           fold_t<T> &fd) {
-  for (int row0 = t.row0 + threadIdx.x; row0 < t.row1; row0 += R * blockDim.x) {
+#pragma unroll
+  for (int k0 = 0; k0 < LZ_RPT; k0 += R) {
+    const int row0 = t.row0 + threadIdx.x + k0 * RSB_BLOCK;
+    if (row0 >= t.row1) break;
     int rows[R], wd[R];
     const uint16_t *base[R];
     bool wide = false;
 #pragma unroll
     for (int k = 0; k < R; k++) {
-      rows[k] = row0 + k * blockDim.x;
-      const bool has = rows[k] < t.row1;
-      const int sl = (has ? rows[k] : row0) >> 6;
-      base[k] = ta.e16 + ta.off16[sl];
-      wd[k] = has ? ta.w16[sl] : 0;
+      rows[k] = row0 + k * RSB_BLOCK;
+      base[k] = ta.e16 + sm.off[k0 + k];
+      wd[k] = sm.w[k0 + k];
       wide |= wd[k] > 32;
     }
     if (wide) {
 #pragma unroll
       for (int k = 0; k < R; k++)
-        if (rows[k] < t.row1)
-          apply_row_tiled<T, FOLD>(rows[k], t, ta, ql, rl, pnew, w, nreal, sq, swq, sw, fd);
+        if (rows[k] < t.row1) {
+          if (k & 1)
+            apply_row_tiled<true, T, FOLD>(rows[k], t, ta, ql, rl, pnew, w, nreal, sq, swq, sw, fd);
+          else
+            apply_row_tiled<false, T, FOLD>(rows[k], t, ta, ql, rl, pnew, w, nreal, sq, swq, sw,
+                                            fd);
+        }
       continue;
     }
     u32x4 v[R][4];
@@ -450,10 +549,8 @@ __device__ inline void apply_rows_batched(const tile_t &t, const tiled_args &ta,
       w[rows[k]] = sum;
       const T ri = FOLD ? rl[li] : (T)0;
       if (li < nreal) {
-        sq.add(qi);
-        swq.dot(sum, qi);
-        sw.add(sum);
-        if (FOLD) fd.rr.dot(ri, ri), fd.rw.dot(ri, sum), fd.ww.dot(sum, sum);
+        if (k & 1) row_sums16<true, T, FOLD>(qi, sum, ri, sq, swq, sw, fd);
+        else row_sums16<false, T, FOLD>(qi, sum, ri, sq, swq, sw, fd);
       }
     }
   }
@@ -495,22 +592,23 @@ __device__ inline void acc12_words(const unsigned (&wd)[8], int s0, uint64_t m4,
 // word of their blocks and tails loaded before any is summed.  The 64 rows
 // of a wave are one slice, so block and tail counts are uniform in a wave.
 template <typename T, int R, bool FOLD>
-__device__ inline void apply_rows_e12(const tile_t &t, const tiled_args &ta, const T *ql,
-                                      const T *rl, T *__restrict__ pnew, T *__restrict__ w,
-                                      int nreal, acc_t<T> &sq, acc_t<T> &swq, acc_t<T> &sw,
-                                      fold_t<T> &fd) {
-  for (int row0 = t.row0 + threadIdx.x; row0 < t.row1; row0 += R * blockDim.x) {
+__device__ inline void apply_rows_e12(const tile_t &t, const tiled_args &ta, const slice_meta &sm,
+                                      const T *ql, const T *rl, T *__restrict__ pnew,
+                                      T *__restrict__ w, int nreal, acc_t<T> &sq, acc_t<T> &swq,
+                                      acc_t<T> &sw, fold_t<T> &fd) {
+#pragma unroll
+  for (int k0 = 0; k0 < LZ_RPT; k0 += R) {
+    const int row0 = t.row0 + threadIdx.x + k0 * RSB_BLOCK;
+    if (row0 >= t.row1) break;
     int rows[R], nb[R], tw[R], cc[R];
     u32x4 bw[R][2][2], tl[R];
 #pragma unroll
     for (int k = 0; k < R; k++) {
-      rows[k] = row0 + k * blockDim.x;
-      const bool has = rows[k] < t.row1;
-      const int sl = (has ? rows[k] : row0) >> 6, lane = rows[k] & 63;
-      const int info = has ? ta.w12[sl] : 0;
+      rows[k] = row0 + k * RSB_BLOCK;
+      const int lane = rows[k] & 63, info = sm.w[k0 + k];
       nb[k] = info & 0xff, tw[k] = info >> 8;
-      const uint32_t *base = ta.e12 + ta.off12[sl];
-      cc[k] = has ? ta.c12[sl] : 0;
+      const uint32_t *base = ta.e12 + sm.off[k0 + k];
+      cc[k] = sm.c[k0 + k];
 #pragma unroll
       for (int b = 0; b < 2; b++)
 #pragma unroll
@@ -583,7 +681,7 @@ __device__ inline void stage_window(const tile_t &t, const int *__restrict__ hal
   int ibeg = threadIdx.x;
   if constexpr (sizeof(T) == 4) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
-    for (int i = 4 * (int)threadIdx.x; i < nrows; i += 4 * (int)blockDim.x) {
+    for (int i = 4 * (int)threadIdx.x; i < nrows; i += 4 * RSB_BLOCK) {
       f32x4 rv = *(const f32x4 *)(r + t.row0 + i);
       if (UPD) {
         const f32x4 wv = *(const f32x4 *)(wp + t.row0 + i);
@@ -594,8 +692,8 @@ __device__ inline void stage_window(const tile_t &t, const int *__restrict__ hal
       f32x4 q = rv;
       if (!FIRST) {
         const f32x4 pv = *(const f32x4 *)(pold + t.row0 + i);
-        q.x = beta * (pv.x - m) + rv.x, q.y = beta * (pv.y - m) + rv.y;
-        q.z = beta * (pv.z - m) + rv.z, q.w = beta * (pv.w - m) + rv.w;
+        q.x = fmat(beta, pv.x - m, rv.x), q.y = fmat(beta, pv.y - m, rv.y);
+        q.z = fmat(beta, pv.z - m, rv.z), q.w = fmat(beta, pv.w - m, rv.w);
       }
       if (i + 0 >= nreal) q.x = 0.f;
       if (i + 1 >= nreal) q.y = 0.f;
@@ -606,12 +704,12 @@ __device__ inline void stage_window(const tile_t &t, const int *__restrict__ hal
     }
     ibeg = nrows + threadIdx.x;
   }
-  for (int i0 = ibeg; i0 < tot; i0 += SU * blockDim.x) {
+  for (int i0 = ibeg; i0 < tot; i0 += SU * RSB_BLOCK) {
     int gr[SU];
     T rg[SU], po[SU], wg[SU];
 #pragma unroll
     for (int k = 0; k < SU; k++) {
-      const int idx = i0 + k * blockDim.x;
+      const int idx = i0 + k * RSB_BLOCK;
       gr[k] = idx < nrows ? t.row0 + idx : (idx < tot ? halo[idx - nrows] : t.row0);
     }
 #pragma unroll
@@ -625,9 +723,9 @@ __device__ inline void stage_window(const tile_t &t, const int *__restrict__ hal
       for (int k = 0; k < SU; k++) rg[k] = rsub(rg[k], alpha, wg[k]);
 #pragma unroll
     for (int k = 0; k < SU; k++) {
-      const int idx = i0 + k * blockDim.x;
+      const int idx = i0 + k * RSB_BLOCK;
       if (idx >= tot) break;
-      T q = FIRST ? rg[k] : beta * (po[k] - m) + rg[k];
+      T q = FIRST ? rg[k] : fmat(beta, po[k] - m, rg[k]);
       if (idx < nrows) {
         if (KEEP_R) rl[idx] = rg[k];
         if (UPD && rn) rn[gr[k]] = rg[k];  // r_it to its basis slot
@@ -653,14 +751,15 @@ __device__ inline void lz_apply_tiled(const lz_args &a, const tile_t &t, const t
   // 256^3 box took 279 us against 269); the FP64 kernel drops it and runs
   // four workgroups per CU instead of three (0.217 -> 0.209 ms per launch)
   constexpr bool KEEP_R = FOLD || sizeof(T) == 4;
+  const slice_meta sm = load_meta(t, ta);
   stage_window<T, FIRST, KEEP_R, FOLD>(t, ta.halo + ta.halo_off[t.ti], nh, ql, rl, r, pold, beta,
                                        m, fd.wp, fd.alpha, fd.rn);
   // two rows per thread and step (measured 15% faster than one at a time
   // on the 256^3 workload: more loads in flight per lane)
   if (ta.e12)
-    apply_rows_e12<T, 2, FOLD>(t, ta, ql, rl, pnew, w, nreal, sq, swq, sw, fd);
+    apply_rows_e12<T, 2, FOLD>(t, ta, sm, ql, rl, pnew, w, nreal, sq, swq, sw, fd);
   else
-    apply_rows_batched<T, 2, FOLD>(t, ta, ql, rl, pnew, w, nreal, sq, swq, sw, fd);
+    apply_rows_batched<T, 2, FOLD>(t, ta, sm, ql, rl, pnew, w, nreal, sq, swq, sw, fd);
 }
 
 // The residuals of a pass live in the basis, unscaled: r_it in slot it
@@ -1516,29 +1615,44 @@ __device__ inline int fin_status(int op) {
   }
 }
 
-// Totals of partial slots k0 .. k0 + nv - 1 (nv <= 3) of a segment: 8 tiles
-// per thread in flight (large segments have up to 16k tiles), a fixed order
-// of summation (each slot's partials are contiguous).  Thread 0 holds them.
-template <int NV>
-__device__ inline void fin_sums(const lz_args &a, int first, int count, int k0,
-                                double (&tot)[NV], double *red) {
+// Totals of NV partial slots (slot k at partial + k * stride) of a segment:
+// U tiles per thread in flight (large segments have up to 16k tiles), a
+// fixed order of summation (thread t adds tiles t, t + blockDim.x, ... in
+// turn, then the block's tree).  Thread 0 holds them.
+template <int NV, int U, int NT>
+__device__ inline void fin_sums(const double *__restrict__ partial, int stride, int first,
+                                int count, double (&tot)[NV], double *red) {
 #pragma unroll
   for (int k = 0; k < NV; k++) tot[k] = 0.0;
-  for (int i0 = threadIdx.x; i0 < count; i0 += 8 * blockDim.x) {
-    double v[NV][8];
+  for (int i0 = 0; i0 < count; i0 += U * NT) {
+    double v[NV][U];
 #pragma unroll
-    for (int k = 0; k < NV; k++)
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * NT + (int)threadIdx.x;
+      const double *p = partial + first + min(i, count - 1);
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int i = i0 + u * blockDim.x;
-        v[k][u] = i < count ? a.partial[(size_t)(k0 + k) * a.pstride + first + i] : 0.0;
+      for (int k = 0; k < NV; k++) {
+        const double x = p[(size_t)k * stride];
+        v[k][u] = i < count ? x : 0.0;
       }
+    }
 #pragma unroll
-    for (int u = 0; u < 8; u++)
+    for (int u = 0; u < U; u++)
 #pragma unroll
       for (int k = 0; k < NV; k++) tot[k] += v[k][u];
   }
-  block_sum<NV>(tot, red);
+  block_sum<NV, NT / RSB_WAVE>(tot, red);
+}
+
+// |r - af w|^2 from the folded apply's sums r.r, r.w, w.w, af = alpha as the
+// next launch rounds it: FP64 sums of exact FP32 products, from this
+// iteration's stored r and w, so the value does not drift over the
+// iterations; it differs from the sum of squares of the rounded new r by at
+// most 2^-23 relative.
+__device__ inline double fold_rtr(double alpha, double rr, double rw, double ww) {
+  const double af = (double)(float)alpha;
+  const double rtr = fmat(af * af, ww, fmat(-2.0 * af, rw, rr));
+  return rtr > 0.0 ? rtr : 0.0;
 }
 
 // The stop test and the next coefficients after the residual update of
@@ -1552,7 +1666,7 @@ __device__ inline void rupdate_step(const lz_args &a, int s, double rtr) {
   if (it == 0) {
     Td[0] = pap / rtz1;
   } else {
-    Td[it] = (beta * beta * pap_old + pap) / rtz1;
+    Td[it] = fmat(beta * beta, pap_old, pap) / rtz1;
     Tu[it - 1] = -beta * pap_old / sqrt(rtz2 * rtz1);
   }
   SC(s, SC_RTR) = rtr;
@@ -1585,14 +1699,14 @@ __global__ void __launch_bounds__(NT) k_lz_fin(lz_args a, int op) {
   // one pass over the slots the phase wrote (all of them in flight together)
   double tot[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   if (op == FIN_APPLYR) {
-    fin_sums<6>(a, first, count, 0, tot, red);
+    fin_sums<6, 8, NT>(a.partial, a.pstride, first, count, tot, red);
   } else if (op == FIN_APPLY) {
     double t3[3];
-    fin_sums<3>(a, first, count, 0, t3, red);
+    fin_sums<3, 8, NT>(a.partial, a.pstride, first, count, t3, red);
     tot[0] = t3[0], tot[1] = t3[1], tot[2] = t3[2];
   } else {
     double t1[1];
-    fin_sums<1>(a, first, count, 0, t1, red);
+    fin_sums<1, 8, NT>(a.partial, a.pstride, first, count, t1, red);
     tot[0] = t1[0];
   }
   if (threadIdx.x != 0) return;
@@ -1629,6 +1743,7 @@ __global__ void __launch_bounds__(NT) k_lz_fin(lz_args a, int op) {
       SC(s, SC_BETA) = 0.0;
       SC(s, SC_PAP) = 0.0;
       SC(s, SC_MEANP) = 0.0;
+      if (a.st0) a.st0[s] = lz_it{rtr, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, rn * a.tol, -1, a.miter[s]};
       a.iter[s] = 0;
       a.status[s] = LZ_RUNNING;
       atomicAdd(&a.running[0], 1);
@@ -1636,7 +1751,7 @@ __global__ void __launch_bounds__(NT) k_lz_fin(lz_args a, int op) {
     }
     case FIN_APPLY: {  // mean of p, pap = w.(p - mean), alpha (fiedler.c:470-478)
       double mq = tot[0] / n;
-      double pap = tot[1] - mq * tot[2];
+      double pap = fmat(-mq, tot[2], tot[1]);
       SC(s, SC_MEANP) = mq;
       SC(s, SC_PAPOLD) = SC(s, SC_PAP);
       SC(s, SC_PAP) = pap;
@@ -1646,19 +1761,13 @@ __global__ void __launch_bounds__(NT) k_lz_fin(lz_args a, int op) {
     case FIN_RUPDATE: rupdate_step(a, s, tot[0]); break;  // tot: r.r
     case FIN_APPLYR: {  // FIN_APPLY, then the update's r.r from the sums r.r, r.w, w.w
       double mq = tot[0] / n;
-      double pap = tot[1] - mq * tot[2];
+      double pap = fmat(-mq, tot[2], tot[1]);
       SC(s, SC_MEANP) = mq;
       SC(s, SC_PAPOLD) = SC(s, SC_PAP);
       SC(s, SC_PAP) = pap;
       const double alpha = SC(s, SC_RTZ1) / pap;
       SC(s, SC_ALPHA) = alpha;
-      // |r - af w|^2 with af = alpha as the next launch rounds it: the FP64
-      // sums of exact FP32 products, from this iteration's stored r and w,
-      // so the value does not drift over the iterations; it differs from
-      // the sum of squares of the rounded new r by at most 2^-23 relative
-      const double af = (double)(float)alpha;
-      double rtr = tot[3] - 2.0 * af * tot[4] + af * af * tot[5];
-      if (!(rtr > 0.0)) rtr = 0.0;
+      const double rtr = fold_rtr(alpha, tot[3], tot[4], tot[5]);
       SC(s, SC_NFOLD) += 1.0;
       rupdate_step(a, s, rtr);
       break;
@@ -1702,13 +1811,389 @@ __global__ void __launch_bounds__(NT) k_lz_fin(lz_args a, int op) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Fused iterations: the finishing step of each reduction is done by the
+// launch that needs its result.  Every workgroup of a segment sums the
+// segment's partials (the order of k_lz_fin<RSB_BLOCK>, so every workgroup
+// gets the same bits) and forms the scalars itself; the workgroup of the
+// segment's first tile also records them.  An iteration is then one launch
+// with the folded update and two without, instead of two and four, and the
+// sums overlap the loads of the window, which do not need them.  Launches
+// read one copy of the partials and of the segment state and write the
+// other, so no workgroup reads what another of the same launch writes
+// (status apart: a segment that stops is recorded there by its first tile,
+// and every other workgroup of it leaves either way).
+// These launches are bound by their chain of dependent loads: one record per
+// tile and one per slice instead of walking five tables, and the sums in the
+// shadow of the window, took 250 tiles of quads (FP32, folded) from 11.8 +
+// 5.4 us (apply, finishing launch) to 10.3 us an iteration, 184 tiles of
+// hexes in FP64 from 13.5 + 4.0 + 2 x 3.75 to 11.6 + 4.1 us.
+struct lz_fuse {
+  const lz_desc *list;  // tiles of the launch, split over the XCDs as in list_index
+  int nlist, per, it;   // per: grid / LZ_XCDS
+        // it: iteration of the pass (the same for every running segment)
+  const lz_it *st_in;
+  lz_it *st_out;
+  const double *pa_in;  // partials of the launch before; those of this one go to lz_args.partial
+};
+#define LZ_FUSE_TILES 1024  // most tiles of a segment (see run_lanczos)
+
+// Scalars after the apply's sums: mean of p, pap, alpha (FIN_APPLY).
+__device__ inline void step_apply(lz_it &x, double n, double sq, double swq, double sw) {
+  const double mq = sq / n;
+  const double pap = fmat(-mq, sw, swq);
+  x.meanp = mq;
+  x.pap_old = x.pap;
+  x.pap = pap;
+  x.alpha = x.rtz1 / pap;
+}
+// The stop test and next coefficients after r.r of iteration x.it
+// (rupdate_step on the state record); lead: this workgroup records them.
+// Returns false when the pass is over.
+__device__ inline bool step_update(const lz_args &a, int s, lz_it &x, double rtr, bool lead,
+                                   bool fold) {
+  const int it = x.it;
+  const double rnorm = sqrt(rtr);
+  const bool stop = rnorm < x.rtol || it + 1 == x.mi;
+  if (lead) {
+    double *Td = a.T + (size_t)s * 2 * a.miter_max, *Tu = Td + a.miter_max;
+    if (it == 0) {
+      Td[0] = x.pap / x.rtz1;
+    } else {
+      Td[it] = fmat(x.beta * x.beta, x.pap_old, x.pap) / x.rtz1;
+      Tu[it - 1] = -x.beta * x.pap_old / sqrt(x.rtz2 * x.rtz1);
+    }
+    a.rn[(size_t)s * (a.miter_max + 1) + it + 1] = 1.0 / rnorm;
+    if (stop) {
+      SC(s, SC_RTR) = rtr;
+      SC(s, SC_RNORM) = rnorm;
+      SC(s, SC_RNI) = 1.0 / rnorm;
+      SC(s, SC_RTZ1) = x.rtz1, SC(s, SC_RTZ2) = x.rtz2, SC(s, SC_BETA) = x.beta;
+      SC(s, SC_PAP) = x.pap, SC(s, SC_PAPOLD) = x.pap_old;
+      SC(s, SC_MEANP) = x.meanp, SC(s, SC_ALPHA) = x.alpha;
+      if (fold) SC(s, SC_NFOLD) += it + 1;
+      a.iter[s] = it;
+      a.k[s] = it + 1;
+      a.status[s] = LZ_PASSDONE;
+      atomicSub(&a.running[0], 1);
+    }
+  }
+  if (stop) return false;
+  const double rtz1 = x.rtz1;
+  x.rtz2 = rtz1;
+  x.rtz1 = rtr;
+  x.beta = rtr / rtz1;
+  return true;
+}
+
+struct lz_bc {
+  double beta, m, alpha;
+  int go;
+};
+// The finishing step in front of an apply: sums of the launch before, the
+// scalars of the next iteration (broadcast through LDS), their record.
+// Returns false where the segment's pass is over.
+template <bool FOLD>
+__device__ inline bool fuse_next(const lz_args &a, const lz_fuse &fu, const lz_desc &d, int status,
+                                 double *red, lz_bc *bc) {
+  constexpr int NV = FOLD ? 6 : 1;
+  double tot[NV];
+  lz_it x;
+  it_load(x, fu.st_in + d.s);
+  fin_sums<NV, FOLD ? 2 : 4, RSB_BLOCK>(fu.pa_in, a.pstride, d.first, d.count, tot, red);
+  if (threadIdx.x == 0) {
+    const bool run = status == LZ_RUNNING, lead = run && d.ti == d.first;
+    double rtr = tot[0];
+    if constexpr (FOLD) {
+      step_apply(x, (double)d.n, tot[0], tot[1], tot[2]);
+      rtr = fold_rtr(x.alpha, tot[3], tot[4], tot[5]);
+    }
+    const bool go = step_update(a, d.s, x, rtr, lead, FOLD) && run;
+    if (go && lead) {
+      x.it++;
+      it_store(fu.st_out + d.s, x);
+    }
+    bc->beta = x.beta, bc->m = x.meanp, bc->alpha = x.alpha, bc->go = go;
+  }
+  __syncthreads();
+  return bc->go != 0;
+}
+
+__device__ inline tile_t tile_from(const lz_desc &d) {
+  tile_t t;
+  t.ti = d.ti, t.s = d.s, t.row0 = d.row0, t.row1 = d.row1;
+  t.pstart = d.pstart, t.n = d.n, t.first = d.first, t.count = d.count;
+  return t;
+}
+
+// The window's loads: the thread's own rows and its first halo rows, in
+// registers while the sums are formed.  Own rows: four in one access (FP32:
+// 4 tid .. + 3), or two pairs (FP64: 2 tid, 2 tid + 512).
+template <typename T, bool UPD>
+struct window_regs {
+  static constexpr int SU = 4;
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+  static constexpr int V = 16 / sizeof(T), NV = LZ_RPT / V;  // rows per access, accesses
+  vec r[NV], p[NV], w[NV];
+  int gr[SU];
+  T rg[SU], po[SU], wg[SU];
+  __device__ inline void load(const tile_t &t, const int *__restrict__ halo, int nh,
+                              const T *__restrict__ rr, const T *__restrict__ pold,
+                              const T *__restrict__ wp) {
+    const int nrows = t.row1 - t.row0;
+#pragma unroll
+    for (int k = 0; k < SU; k++) {
+      const int i = (int)threadIdx.x + k * RSB_BLOCK;
+      gr[k] = i < nh ? halo[i] : t.row0;
+    }
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const int i = V * ((int)threadIdx.x + k * RSB_BLOCK);
+      const int o = t.row0 + (i < nrows ? i : 0);
+      r[k] = *(const vec *)(rr + o);
+      p[k] = *(const vec *)(pold + o);
+      if (UPD) w[k] = *(const vec *)(wp + o);
+    }
+#pragma unroll
+    for (int k = 0; k < SU; k++) {
+      rg[k] = rr[gr[k]];
+      po[k] = pold[gr[k]];
+      wg[k] = UPD ? wp[gr[k]] : (T)0;
+    }
+  }
+  // q = beta (p - m) + r into the window, r of the tile's rows beside it
+  // (UPD: r = r - alpha w first, also written to its basis slot rn)
+  template <bool KEEP_R>
+  __device__ inline void fill(const tile_t &t, const int *__restrict__ halo, int nh, T *ql, T *rl,
+                              const T *__restrict__ rr, const T *__restrict__ pold,
+                              const T *__restrict__ wp, T beta, T m, T alpha,
+                              T *__restrict__ rn) {
+    const int nrows = t.row1 - t.row0;
+    const int nreal = min(nrows, t.pstart + t.n - t.row0);
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const int i = V * ((int)threadIdx.x + k * RSB_BLOCK);
+      if (i >= nrows) continue;
+      vec x = r[k], q;
+#pragma unroll
+      for (int j = 0; j < V; j++) {
+        if (UPD) x[j] = rsub(x[j], alpha, w[k][j]);
+        q[j] = fmat(beta, p[k][j] - m, x[j]);
+        if (i + j >= nreal) q[j] = (T)0;
+      }
+      if (UPD) *(vec *)(rn + t.row0 + i) = x;
+      *(vec *)(ql + i) = q;
+      if (KEEP_R) *(vec *)(rl + i) = x;
+    }
+#pragma unroll
+    for (int k = 0; k < SU; k++) {
+      const int i = (int)threadIdx.x + k * RSB_BLOCK;
+      if (i >= nh) break;
+      const T x = UPD ? rsub(rg[k], alpha, wg[k]) : rg[k];
+      ql[nrows + i] = fmat(beta, po[k] - m, x);
+    }
+    for (int i0 = (int)threadIdx.x + SU * RSB_BLOCK; i0 < nh; i0 += SU * RSB_BLOCK) {
+#pragma unroll
+      for (int k = 0; k < SU; k++) {
+        const int i = i0 + k * RSB_BLOCK;
+        gr[k] = i < nh ? halo[i] : t.row0;
+      }
+#pragma unroll
+      for (int k = 0; k < SU; k++) {
+        rg[k] = rr[gr[k]];
+        po[k] = pold[gr[k]];
+        wg[k] = UPD ? wp[gr[k]] : (T)0;
+      }
+#pragma unroll
+      for (int k = 0; k < SU; k++) {
+        const int i = i0 + k * RSB_BLOCK;
+        if (i >= nh) break;
+        const T x = UPD ? rsub(rg[k], alpha, wg[k]) : rg[k];
+        ql[nrows + i] = fmat(beta, po[k] - m, x);
+      }
+    }
+    __syncthreads();
+  }
+};
+
+template <typename T, bool FOLD>
+__global__ void __launch_bounds__(RSB_BLOCK) k_lz_apply_f(lz_args a, lz_fuse fu,
+                                                          const T *__restrict__ pold,
+                                                          T *__restrict__ pnew, T *__restrict__ w,
+                                                          T *__restrict__ basis, int64_t mpad,
+                                                          tiled_args ta,
+                                                          const T *__restrict__ wprev) {
+  __shared__ __attribute__((aligned(16))) T ql[TB_LOCAL];
+  // as in lz_apply_tiled
+  constexpr bool KEEP_R = FOLD || sizeof(T) == 4;
+  __shared__ __attribute__((aligned(16))) T rl[KEEP_R ? RSB_TILE : 4];
+  __shared__ double red[(RSB_BLOCK / RSB_WAVE) * 6];
+  __shared__ lz_bc bc;
+  const int li = (int)(blockIdx.x % LZ_XCDS) * fu.per + (int)(blockIdx.x / LZ_XCDS);
+  if (li >= fu.nlist) return;
+  const lz_desc d = fu.list[li];
+  // tested with the sums, when the window's loads are on their way (a test
+  // here would put a round trip in front of them; they stay in bounds for a
+  // segment that has stopped)
+  const int status = a.status[d.s];
+  const tile_t t = tile_from(d);
+  const int it = fu.it, nh = d.nhalo;
+  T *cur = basis + (size_t)it * mpad;
+  const slice_meta sm = load_meta(t, ta);
+  acc_t<T> sq, swq, sw;
+  fold_t<T> fd;
+  fd.wp = wprev, fd.rn = it == 0 ? nullptr : cur, fd.alpha = (T)0;
+  const int nreal = min(t.row1 - t.row0, t.pstart + t.n - t.row0);
+  const int *halo = ta.halo + d.halo_off;
+  if (it == 0) {
+    if (status != LZ_RUNNING) return;
+    if (threadIdx.x == 0 && d.ti == d.first) {
+      lz_it x;
+      it_load(x, fu.st_in + d.s);
+      x.it = 0;
+      it_store(fu.st_out + d.s, x);
+    }
+    if (nh >= 0)
+      stage_window<T, true, KEEP_R, FOLD>(t, halo, nh, ql, rl, cur, pold, (T)0, (T)0);
+    else
+      lz_apply_rows<T, true, FOLD>(a, t, cur, pold, pnew, w, (T)0, (T)0, ta.slice_off, ta.slice_w,
+                                   ta.ell, sq, swq, sw, fd);
+  } else {
+    // r_it, or r_{it-1} to update
+    const T *__restrict__ r = FOLD ? cur - mpad : cur;
+    if (nh >= 0) {
+      window_regs<T, FOLD> wr;
+      wr.load(t, halo, nh, r, pold, wprev);
+      if (!fuse_next<FOLD>(a, fu, d, status, red, &bc)) return;
+      wr.template fill<KEEP_R>(t, halo, nh, ql, rl, r, pold, wprev, (T)bc.beta, (T)bc.m,
+                             (T)bc.alpha, cur);
+    } else {
+      if (!fuse_next<FOLD>(a, fu, d, status, red, &bc)) return;
+      fd.alpha = (T)bc.alpha;
+      lz_apply_rows<T, false, FOLD>(a, t, r, pold, pnew, w, (T)bc.beta, (T)bc.m, ta.slice_off,
+                                    ta.slice_w, ta.ell, sq, swq, sw, fd);
+    }
+  }
+  if (nh >= 0) {
+    if (ta.e12)
+      apply_rows_e12<T, 2, FOLD>(t, ta, sm, ql, rl, pnew, w, nreal, sq, swq, sw, fd);
+    else
+      apply_rows_batched<T, 2, FOLD>(t, ta, sm, ql, rl, pnew, w, nreal, sq, swq, sw, fd);
+  }
+  if (FOLD) {
+    double v[6] = {sq.value(), swq.value(), sw.value(),
+                   fd.rr.value(), fd.rw.value(), fd.ww.value()};
+    publish<6>(a, t, v);
+  } else {
+    double v[3] = {sq.value(), swq.value(), sw.value()};
+    publish<3>(a, t, v);
+  }
+}
+
+// The update r_{it+1} = r_it - alpha w of the fused iterations, with the
+// apply's finishing step in front (k_lz_rupdate otherwise).
+template <typename T>
+__global__ void __launch_bounds__(RSB_BLOCK) k_lz_rupdate_f(lz_args a, lz_fuse fu,
+                                                            T *__restrict__ basis, int64_t mpad,
+                                                            const T *__restrict__ w) {
+  __shared__ double red[(RSB_BLOCK / RSB_WAVE) * 3];
+  __shared__ double balpha;
+  const int li = (int)(blockIdx.x % LZ_XCDS) * fu.per + (int)(blockIdx.x / LZ_XCDS);
+  if (li >= fu.nlist) return;
+  const lz_desc d = fu.list[li];
+  const int status = a.status[d.s];
+  const tile_t t = tile_from(d);
+  const T *__restrict__ r = basis + (size_t)fu.it * mpad;
+  T *__restrict__ rn = basis + (size_t)(fu.it + 1) * mpad;
+  const int nrows = t.row1 - t.row0;
+  // the rows of a thread, in the order their squares are summed: four
+  // consecutive ones (FP32, one access), or every 256th (FP64)
+  constexpr int V = sizeof(T) == 4 ? LZ_RPT : 1, R = LZ_RPT / V;
+  typedef T vec __attribute__((ext_vector_type(V)));
+  vec rv[R], wv[R];
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    const int i = V * ((int)threadIdx.x + k * RSB_BLOCK);
+    const int o = t.row0 + (i < nrows ? i : 0);
+    rv[k] = *(const vec *)(r + o);
+    wv[k] = *(const vec *)(w + o);
+  }
+  lz_it x;
+  it_load(x, fu.st_in + d.s);
+  double tot[3];
+  fin_sums<3, 4, RSB_BLOCK>(fu.pa_in, a.pstride, d.first, d.count, tot, red);
+  if (status != LZ_RUNNING) return;
+  if (threadIdx.x == 0) {
+    step_apply(x, (double)d.n, tot[0], tot[1], tot[2]);
+    if (d.ti == d.first) it_store(fu.st_out + d.s, x);
+    balpha = x.alpha;
+  }
+  __syncthreads();
+  const T alpha = (T)balpha;
+  acc_t<T> acc;
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    const int i = V * ((int)threadIdx.x + k * RSB_BLOCK);
+    if (i >= nrows) continue;
+    vec y;
+#pragma unroll
+    for (int j = 0; j < V; j++) y[j] = rsub(rv[k][j], alpha, wv[k][j]);
+    *(vec *)(rn + t.row0 + i) = y;
+#pragma unroll
+    for (int j = 0; j < V; j++) acc.dot(y[j], y[j]);
+  }
+  double v[1] = {acc.value()};
+  publish<1>(a, t, v);
+}
+
+// The finishing step after the last iteration of a pass.
+template <bool FOLD>
+__global__ void __launch_bounds__(RSB_BLOCK) k_lz_last(lz_args a, lz_fuse fu,
+                                                       const int *__restrict__ segs) {
+  __shared__ double red[(RSB_BLOCK / RSB_WAVE) * 6];
+  __shared__ lz_bc bc;
+  lz_desc d;
+  d.s = segs[blockIdx.x];
+  const int status = a.status[d.s];
+  if (status != LZ_RUNNING) return;
+  d.first = d.ti = a.seg_tiles[2 * d.s], d.count = a.seg_tiles[2 * d.s + 1];
+  d.n = a.seg[a.nseg + d.s];
+  fuse_next<FOLD>(a, fu, d, status, red, &bc);
+}
+
+__global__ void k_lz_slices(int64_t nslices, const int64_t *__restrict__ off,
+                            const int *__restrict__ w, const int *__restrict__ c,
+                            slice_rec *__restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nslices) out[i] = slice_rec{off[i], w[i], c ? c[i] : 0};
+}
+
+__global__ void k_lz_desc(lz_args a, int ntiles, const int *__restrict__ nhalo,
+                          const int64_t *__restrict__ halo_off, lz_desc *__restrict__ out) {
+  const int ti = blockIdx.x * blockDim.x + threadIdx.x;
+  if (ti >= ntiles) return;
+  lz_desc d;
+  d.s = a.tile[3 * ti], d.row0 = a.tile[3 * ti + 1], d.row1 = a.tile[3 * ti + 2];
+  d.pstart = a.seg[4 * a.nseg + d.s], d.n = a.seg[a.nseg + d.s];
+  d.first = a.seg_tiles[2 * d.s], d.count = a.seg_tiles[2 * d.s + 1];
+  d.nhalo = nhalo[ti], d.halo_off = halo_off[ti], d.ti = ti;
+  d.pad0 = 0;
+  for (int k = 0; k < 4; k++) d.pad[k] = 0;
+  out[ti] = d;
+}
+
 // Lists of the tiles and segments in a given state (order irrelevant: every
 // tile writes its partial at its own index and k_lz_fin sums them in tile
 // order).
 __global__ void k_lz_compact(lz_args a, int ntiles, int want, int *__restrict__ tiles,
-                             int *__restrict__ segs, int *__restrict__ counts) {
+                             int *__restrict__ segs, int *__restrict__ counts,
+                             const lz_desc *__restrict__ desc, lz_desc *__restrict__ list) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < ntiles && a.status[a.tile[3 * i]] == want) tiles[atomicAdd(&counts[0], 1)] = i;
+  if (i < ntiles && a.status[a.tile[3 * i]] == want) {
+    const int k = atomicAdd(&counts[0], 1);
+    tiles[k] = i;
+    if (list) list[k] = desc[i];
+  }
   if (i < a.nseg && a.status[i] == want) segs[atomicAdd(&counts[1], 1)] = i;
 }
 
@@ -1796,11 +2281,12 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   }
   if (ntiles > g->lz_tile_cap) {
     if (L.partial) RSB_TRY(rsb_dev_free(L.partial));
-    RSB_TRY(rsb_dev_malloc((void **)&L.partial, sizeof(double) * 6 * std::max(ntiles, 1)));
+    RSB_TRY(rsb_dev_malloc((void **)&L.partial, sizeof(double) * 12 * std::max(ntiles, 1)));
     g->lz_tile_cap = ntiles;
   }
   if (!L.running) RSB_TRY(rsb_dev_malloc((void **)&L.running, sizeof(int) * 2));
   lz_args a;
+  a.st0 = nullptr;
   a.act_tiles = nullptr, a.act_segs = nullptr;
   a.seg = g->d_seg, a.tile = g->d_tile, a.seg_tiles = g->d_seg_tiles, a.row_elem = g->d_row_elem;
   a.nseg = nseg;
@@ -1832,10 +2318,33 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   RSB_TRY(RSB_SCRATCH(act, sizeof(int) * ((size_t)ntiles + nseg + 2)));
   int *act_t = act, *act_s = act + ntiles, *act_n = act + ntiles + nseg;
   int nact[2] = {ntiles, nseg};
+  // segments of at most LZ_FUSE_TILES tiles take the fused iterations: every
+  // workgroup sums its segment's partials by itself
+  int max_seg_tiles = 0;
+  for (int q = 0; q < nseg; q++) max_seg_tiles = std::max(max_seg_tiles, g->h_seg_tiles[2 * q + 1]);
+  const char *gv = getenv("PARRSB_AMD_LZ_GRAPH");
+  const bool use_graph = !g->prof_spmv && gv && atoi(gv) == 1;
+  // the vertex form serves the FP32 path (vectors of T = float)
+  const bool vform = g->vt_ok && sizeof(T) == 4;
+  const char *fuv = getenv("PARRSB_AMD_LZ_FUSE_TILES");
+  const int fuse_tiles = fuv ? std::min(atoi(fuv), LZ_FUSE_TILES) : LZ_FUSE_TILES;
+  const bool fuse = !vform && !use_graph && max_seg_tiles <= fuse_tiles;
+  lz_desc *desc = nullptr, *act_d = nullptr;
+  lz_it *stt = nullptr;
+  if (fuse && ntiles > 0) {
+    RSB_TRY(RSB_SCRATCH(desc, sizeof(lz_desc) * 2 * (size_t)ntiles));
+    act_d = desc + ntiles;
+    RSB_TRY(RSB_SCRATCH(stt, sizeof(lz_it) * 2 * (size_t)nseg));
+    a.st0 = stt + nseg;  // the copy the first launch of a pass reads
+    k_lz_desc<<<nblocks(ntiles, 256), 256, 0, st>>>(a, ntiles, g->d_tnhalo, g->d_thalo_off, desc);
+    RSB_LAUNCH_CHECK();
+  }
+  double *const PA[2] = {L.partial, L.partial + (size_t)6 * std::max(g->lz_tile_cap, 1)};
   auto compact = [&](int want) -> int {
     RSB_TRY(hipMemsetAsync(act_n, 0, sizeof(int) * 2, st));
     k_lz_compact<<<nblocks(std::max(ntiles, nseg), 256), 256, 0, st>>>(a, ntiles, want, act_t,
-                                                                        act_s, act_n);
+                                                                        act_s, act_n, desc,
+                                                                        act_d);
     RSB_LAUNCH_CHECK();
     RSB_TRY(hipMemcpyAsync(nact, act_n, sizeof(int) * 2, hipMemcpyDeviceToHost, st));
     RSB_TRY(hipStreamSynchronize(st));
@@ -1848,14 +2357,19 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   // 0.253 against 0.233 ms per launch on the 256^3 box (FP32: 0.163 against
   // 0.177), the class sums in doubles costing more than the bytes they save.
   const bool use12 = g->e12_ok && (sizeof(T) == 4 || g->e12_f64);
-  tiled_args ta{g->d_slice_off, g->d_slice_w, g->d_ell,  g->d_tnhalo,
-                g->d_thalo_off, g->d_halo,    g->d_off16, g->d_w16,
-                g->d_e16,       g->d_off12,   g->d_w12,   use12 ? g->d_e12 : nullptr,
-                g->d_c12};
+  slice_rec *srec = nullptr;
+  RSB_TRY(RSB_SCRATCH(srec, sizeof(slice_rec) * (size_t)std::max<int64_t>(g->nslices, 1)));
+  if (ntiles > 0) {
+    k_lz_slices<<<nblocks(g->nslices, 256), 256, 0, st>>>(
+        g->nslices, use12 ? g->d_off12 : g->d_off16, use12 ? g->d_w12 : g->d_w16,
+        use12 ? g->d_c12 : nullptr, srec);
+    RSB_LAUNCH_CHECK();
+  }
+  tiled_args ta{srec,           g->d_slice_off, g->d_slice_w, g->d_ell, g->d_tnhalo,
+                g->d_thalo_off, g->d_halo,      g->d_off16,   g->d_w16, g->d_e16,
+                use12 ? g->d_e12 : nullptr};
   vtile_args va{g->d_vt_n,  g->d_vt_loff,    g->d_vt_list, g->d_vt_rowv,
                 g->d_tnhalo, g->d_thalo_off, g->d_halo,    g->nv};
-  // the vertex form serves the FP32 path (vectors of T = float)
-  const bool vform = g->vt_ok && sizeof(T) == 4;
   // FP32 with the neighbour entries: a pass that starts with at most
   // fold_tiles running tiles folds the r-update into the next apply
   // (k_lz_apply<float, true>, FIN_APPLYR: two launches per iteration instead
@@ -1868,10 +2382,29 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   T *const W[2] = {w, (T *)g->d_w2};
   // one iteration (it: the pass iteration, where every running segment is):
   // the apply launch, then the finishing step(s) and the r-update
+  // fused launches: which copies of the state and partials they read; they
+  // write the other (without the fold: the apply writes copy 0)
+  auto fused = [&](int it, int rd, lz_args &af) {
+    af = ai;
+    af.partial = PA[rd ^ 1];
+    return lz_fuse{act_d, nact[0], (nact[0] + LZ_XCDS - 1) / LZ_XCDS, it, stt + (size_t)rd * nseg, stt + (size_t)(rd ^ 1) * nseg,
+                   PA[rd]};
+  };
   auto apply_launch = [&](int it) {
     T *pold = (it & 1) ? p2 : p, *pnew = (it & 1) ? p : p2;
     const unsigned grid = xgrid(nact[0]);
-    if (fold)
+    if (fuse) {
+      lz_args af;
+      if (fold) {
+        const lz_fuse fu = fused(it, (it + 1) & 1, af);
+        k_lz_apply_f<T, true><<<grid, RSB_BLOCK, 0, st>>>(af, fu, pold, pnew, W[it & 1], basis,
+                                                          mpad, ta, W[(it + 1) & 1]);
+      } else {
+        const lz_fuse fu = fused(it, 1, af);
+        k_lz_apply_f<T, false><<<grid, RSB_BLOCK, 0, st>>>(af, fu, pold, pnew, w, basis, mpad, ta,
+                                                           nullptr);
+      }
+    } else if (fold)
       k_lz_apply<T, true><<<grid, RSB_BLOCK, 0, st>>>(ai, pold, pnew, W[it & 1], basis, mpad, ta,
                                                       nact[0], W[(it + 1) & 1]);
     else if (vform)
@@ -1883,15 +2416,18 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
                                                        nact[0], nullptr);
   };
   // the iteration sums: wide workgroups where the segments are big
-  int max_seg_tiles = 0;
-  for (int q = 0; q < nseg; q++) max_seg_tiles = std::max(max_seg_tiles, g->h_seg_tiles[2 * q + 1]);
   const bool wide_fin = max_seg_tiles > LZ_FIN_WIDE;
   auto fin_launch = [&](int op) {
     if (wide_fin) k_lz_fin<2 * RSB_BLOCK><<<nact[1], 2 * RSB_BLOCK, 0, st>>>(ai, op);
     else k_lz_fin<RSB_BLOCK><<<nact[1], RSB_BLOCK, 0, st>>>(ai, op);
   };
-  auto after_apply = [&]() {
-    if (fold) {
+  auto after_apply = [&](int it) {
+    if (fuse) {
+      if (fold) return;
+      lz_args af;
+      const lz_fuse fu = fused(it, 0, af);
+      k_lz_rupdate_f<T><<<xgrid(nact[0]), RSB_BLOCK, 0, st>>>(af, fu, basis, mpad, w);
+    } else if (fold) {
       fin_launch(FIN_APPLYR);
     } else {
       fin_launch(FIN_APPLY);
@@ -1939,8 +2475,6 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
       fold = nact[0] <= fold_tiles;
       RSB_TRY(hipEventRecord(g->lz_ev0, st));
       int it, nrec = 0;
-      const char *gv = getenv("PARRSB_AMD_LZ_GRAPH");
-      const bool use_graph = !g->prof_spmv && gv && atoi(gv) == 1;
       hipGraphExec_t gexec = nullptr;
       int gn[2] = {-1, -1};
       if (g->prof_spmv && (int)g->spmv_ev.size() < 2 * miter_max) {
@@ -1965,7 +2499,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
             // (it is a multiple of 8: the chunk's buffer parities are q's)
             for (int q = 0; q < 8; q++) {
               apply_launch(q);
-              after_apply();
+              after_apply(q);
             }
             RSB_TRY(hipStreamEndCapture(st, &gr));
             if (gexec) RSB_TRY(hipGraphExecDestroy(gexec));
@@ -1993,7 +2527,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
           RSB_TRY(hipEventRecord(g->spmv_ev[2 * nrec + 1], st));
           nrec++;
         }
-        after_apply();
+        after_apply(it);
         RSB_LAUNCH_CHECK();
         g->lz_launches++;
         if (it == next_c && it + 1 < miter_max) {
@@ -2004,6 +2538,14 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
           step = nact[1] == before ? std::min(2 * step, 32) : 8;
           next_c = it + step;
         }
+      }
+      if (fuse && nact[1] > 0) {
+        // the sums of the last iteration
+        lz_args af;
+        const lz_fuse fu = fused(miter_max, fold ? (miter_max + 1) & 1 : 1, af);
+        if (fold) k_lz_last<true><<<nact[1], RSB_BLOCK, 0, st>>>(af, fu, act_s);
+        else k_lz_last<false><<<nact[1], RSB_BLOCK, 0, st>>>(af, fu, act_s);
+        RSB_LAUNCH_CHECK();
       }
       RSB_TRY(hipEventRecord(g->lz_ev1, st));
       RSB_TRY(hipMemsetAsync(L.running + 1, 0, sizeof(int), st));

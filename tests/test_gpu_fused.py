@@ -1,0 +1,55 @@
+"""Fused Lanczos iterations against the separate finishing launches: the same
+sums in the same order, so every result has the same bits."""
+import numpy as np
+import pytest
+
+from parrsb_amd import meshgen as M
+
+pytestmark = pytest.mark.gpu
+
+
+def _solve(vtx, xyz, nv, bounds, prec):
+    """Fiedler solve of the segments [bounds[i], bounds[i+1]) of the input
+    order, two virtual ranks each."""
+    import parrsb_amd as pa
+    b = np.asarray(bounds)
+    nseg = b.size - 1
+    with pa.Device() as d:
+        d.set_mesh(vtx, xyz, nv)
+        d.set_segments(b[:-1], np.diff(b), np.full(nseg, 2), 2 * np.arange(nseg))
+        d.prepartition(1)
+        d.level_laplacian()
+        out = d.fiedler(nseg, precision=prec, max_passes=6)
+        return out, d.fiedler_values()
+
+
+CASES = {
+    # a pass shorter than rsb_max_iter, one row past a tile, a whole number
+    # of tiles, and many segments that stop at different iterations
+    "tiny": lambda: (M.box_hex(3, 2, 2), [0, 12]),
+    "tile_plus_one": lambda: (M.box_hex(41, 25, 1), [0, 1025]),
+    "tiles": lambda: (M.box_hex(32, 16, 16, jitter=0.1), [0, 8192]),
+    "uneven": lambda: (M.warped_box_hex(24, seed=3), [0, 2, 67, 1091, 1092, 6000, 13824]),
+    "quads": lambda: (M.holed_quads(150, 140, seed=4, rmax=9.0), None),
+}
+
+
+@pytest.mark.parametrize("tiles", ["lds", "global"])
+@pytest.mark.parametrize("prec,fold", [(64, "0"), (32, "0"), (32, "4096")])
+@pytest.mark.parametrize("name", list(CASES))
+def test_fused_iterations_equal_separate_launches(name, prec, fold, tiles, monkeypatch):
+    print("fused", name, prec, fold, tiles, flush=True)
+    (vtx, xyz, nv), bounds = CASES[name]()
+    n = vtx.shape[0]
+    bounds = bounds or [0, n // 3, n // 3 + 1200, n]
+    monkeypatch.setenv("PARRSB_AMD_LZ_FOLD_TILES", fold)
+    if tiles == "global":
+        monkeypatch.setenv("PARRSB_AMD_NO_TILES", "1")
+    res = {}
+    for fuse in ("1024", "0"):
+        monkeypatch.setenv("PARRSB_AMD_LZ_FUSE_TILES", fuse)
+        res[fuse] = _solve(vtx, xyz, nv, bounds, prec)
+    (of, ff), (ou, fu) = res["1024"], res["0"]
+    for k in ("niter", "npass", "lambda", "rnorm", "resid"):
+        assert np.array_equal(of[k], ou[k], equal_nan=True), k
+    assert np.array_equal(ff, fu)
