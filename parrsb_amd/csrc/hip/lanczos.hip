@@ -1042,113 +1042,210 @@ __device__ inline double lane_get(double v, int i) {
   return __longlong_as_double(
       (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned long long)(unsigned)lo));
 }
-struct lanes2 {
-  double a, b;  // entries lane and lane + 64
-  __device__ inline double get(int i) const { return i < RSB_WAVE ? lane_get(a, i) : lane_get(b, i - RSB_WAVE); }
+// W words per lane: entries lane (and lane + 64 if W == 2).  Vectors of at
+// most 64 entries take W == 1, which leaves no branch in a read or a write.
+template <int W>
+struct lanes_t {
+  double a, b;
+  __device__ inline double get(int i) const {
+    if (W == 1) return lane_get(a, i);
+    return i < RSB_WAVE ? lane_get(a, i) : lane_get(b, i - RSB_WAVE);
+  }
   __device__ inline void set(int i, double x, int lane) {
-    if (i < RSB_WAVE) {
-      if (lane == i) a = x;
-    } else if (lane == i - RSB_WAVE) {
-      b = x;
-    }
+    if (W == 1 || i < RSB_WAVE) a = lane == i ? x : a;
+    else b = lane == i - RSB_WAVE ? x : b;
+  }
+  __device__ inline void load(const double *v, int n, int lane) {
+    a = lane < n ? v[lane] : 0.0;
+    b = W == 2 && lane + RSB_WAVE < n ? v[lane + RSB_WAVE] : 0.0;
+  }
+  __device__ inline void store(double *v, int n, int lane) const {
+    if (lane < n) v[lane] = a;
+    if (W == 2 && lane + RSB_WAVE < n) v[lane + RSB_WAVE] = b;
   }
 };
 
-__device__ void tqli_wave(int n, double *d, double *e, double *z, double *y, double *lam_out) {
-  const int lane = threadIdx.x;
-  for (int i = lane; i < n * n; i += RSB_WAVE) z[i] = 0.0;
+// a / b for |a|, |b| in [2^-400, 2^400]: the operations of the compiler's own
+// divide (a reciprocal estimate, two Newton steps, the quotient corrected by
+// its exact remainder) without the scaling and special cases it wraps around
+// them, so the result is the same correctly rounded quotient.
+__device__ inline double div_plain(double a, double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = fmat(y, fmat(-b, y, 1.0), y);
+  y = fmat(y, fmat(-b, y, 1.0), y);
+  const double q = a * y;
+  return fmat(fmat(-b, q, a), y, q);
+}
+__device__ inline bool in_plain_range(double a) {
+  const int ex = (__double2hiint(a) >> 20) & 0x7ff;
+  return ex > 1023 - 400 && ex < 1023 + 400;
+}
+// r = sqrt(x) and 1 / r, both correctly rounded, for x in [1, 2]: Goldschmidt
+// steps from the reciprocal square root estimate (the compiler's, without its
+// scaling), then the refined estimate of 1 / sqrt(x) corrected twice against
+// r: after the first correction it is within an ulp of 1 / r, and a second
+// one is then correctly rounded unless r's significand is all ones
+// (Markstein, IBM J. Res. Dev. 34, 1990), which r <= sqrt(2) rules out.
+__device__ inline void sqrt_rcp_plain(double x, double &r, double &ri) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = fmat(-h, g, 0.5);
+  g = fmat(g, e, g);
+  h = fmat(h, e, h);
+  g = fmat(fmat(-g, g, x), h, g);
+  g = fmat(fmat(-g, g, x), h, g);
+  double z = 2.0 * h;
+  z = fmat(z, fmat(-g, z, 1.0), z);
+  r = g;
+  ri = fmat(z, fmat(-g, z, 1.0), z);
+}
+
+// Two wavefronts: the first runs the serial recurrence, whose every step is a
+// divide, a square root and a reciprocal one after another, and leaves each
+// sweep's rotations in LDS; the second applies them to the eigenvector
+// matrix while the first is in its next sweep (one barrier a sweep).  With
+// the rotations in the recurrence's own instruction stream, their LDS round
+// trips lengthened every step, and branches cost as much again: 1.00 ms per call
+// for a pass of 50, now 0.49 (what is left is the latency of ~31 dependent FP64
+// operations a step; unrolling it changed nothing).
+// z: column i of the matrix at z + i * zp, zp = n rounded up to 64.
+struct tqli_shared {
+  double cs[2][2][128];  // c and s of a sweep's steps, by buffer
+  int l[2], m[2];        // its range; m < 0: no more sweeps
+  int failed;
+};
+__device__ inline int tqli_pitch(int n) { return (n + RSB_WAVE - 1) / RSB_WAVE * RSB_WAVE; }
+
+template <int W>
+__device__ void tqli_wave(int n, double *d, double *e, double *z, double *y, double *lam_out,
+                          tqli_shared *sh) {
+  const int lane = threadIdx.x % RSB_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / RSB_WAVE);
+  const int zp = tqli_pitch(n);
+  for (int i = threadIdx.x; i < n * zp; i += 2 * RSB_WAVE) z[i] = i / zp == i % zp ? 1.0 : 0.0;
   __syncthreads();
-  for (int i = lane; i < n; i += RSB_WAVE) z[i * n + i] = 1.0;
-  lanes2 D, E;
-  D.a = lane < n ? d[lane] : 0.0;
-  D.b = lane + RSB_WAVE < n ? d[lane + RSB_WAVE] : 0.0;
-  E.a = lane < n ? e[lane] : 0.0;
-  E.b = lane + RSB_WAVE < n ? e[lane + RSB_WAVE] : 0.0;
-  __syncthreads();
-  int failed = 0;
-  for (int l = 0; l < n && !failed; l++) {
-    int sweeps = 0, m;
-    while (true) {
-      // d[m + 1] next to d[m]: lane 63's neighbour is entry 64
-      double dn_a = __shfl_down(D.a, 1, RSB_WAVE);
-      const double d64 = lane_get(D.b, 0);
-      if (lane == RSB_WAVE - 1) dn_a = d64;
-      const double dn_b = __shfl_down(D.b, 1, RSB_WAVE);
-      const int ma = lane, mb = lane + RSB_WAVE;
-      const bool ta = ma >= l && ma < n - 1 && fabs(E.a) / (fabs(D.a) + fabs(dn_a)) < 1e-12;
-      const bool tb = mb >= l && mb < n - 1 && fabs(E.b) / (fabs(D.b) + fabs(dn_b)) < 1e-12;
-      const unsigned long long ba = __ballot(ta), bb = __ballot(tb);
-      m = ba ? __ffsll((long long)ba) - 1 : bb ? RSB_WAVE + __ffsll((long long)bb) - 1 : n - 1;
-      if (m == l) break;
-      if (sweeps++ == 30) {
-        failed = 1;
-        break;
-      }
-      const double dl = D.get(l), el = E.get(l);
-      double g = (D.get(l + 1) - dl) / (2.0 * el);
-      double r = sqrt(g * g + 1.0);
-      g = D.get(m) - dl + el / (g + sgn_abs(r, g));
-      double s = 1.0, c = 1.0, p = 0.0;
-      for (int i = m - 1; i >= l; i--) {
-        const double ei = E.get(i);
-        double f = s * ei, b = c * ei;
-        double ei1;
-        if (fabs(f) >= fabs(g)) {
-          c = g / f;
-          r = sqrt(c * c + 1.0);
-          ei1 = f * r;
-          s = 1.0 / r;
-          c = c * s;
-        } else {
-          s = f / g;
-          r = sqrt(s * s + 1.0);
-          ei1 = g * r;
-          c = 1.0 / r;
-          s = s * c;
+  lanes_t<W> D, E;
+  if (wave == 1) {
+    for (int buf = 0;; buf ^= 1) {
+      __syncthreads();
+      const int l = sh->l[buf], m = sh->m[buf];
+      if (m < 0) break;
+      const double *C = sh->cs[buf][0], *S = sh->cs[buf][1];
+      for (int k = lane; k < n; k += RSB_WAVE) {
+        // z[k][i + 1] carried from step to step, z[k][i] read one step ahead
+        double zk1 = z[m * zp + k], zk = z[(m - 1) * zp + k];
+        for (int i = m - 1; i >= l; i--) {
+          const double next = i > l ? z[(i - 1) * zp + k] : 0.0;
+          const double c = C[i + 1], s = S[i + 1];
+          z[(i + 1) * zp + k] = s * zk + c * zk1;
+          zk1 = c * zk - s * zk1;
+          zk = next;
         }
-        g = D.get(i + 1) - p;
-        r = (D.get(i) - g) * s + 2.0 * c * b;
-        p = s * r;
-        const double di1 = g + p;
-        g = c * r - b;
-        E.set(i + 1, ei1, lane);
-        D.set(i + 1, di1, lane);
-        for (int k = lane; k < n; k += RSB_WAVE) {
-          double zk1 = z[k * n + i + 1], zk = z[k * n + i];
-          z[k * n + i + 1] = s * zk + c * zk1;
-          z[k * n + i] = c * zk - s * zk1;
-        }
+        z[l * zp + k] = zk1;
       }
-      D.set(l, D.get(l) - p, lane);
-      E.set(l, g, lane);
-      E.set(m, 0.0, lane);
     }
-  }
-  __syncthreads();  // rows of z written by other lanes are read below
-  // eigenvalue of smallest magnitude (first on ties, fiedler.c:538-545)
-  int imin = 0;
-  double emin = fabs(D.get(0));
-  for (int i = 1; i < n; i++) {
-    const double v = fabs(D.get(i));
-    if (v < emin) emin = v, imin = i;
-  }
-  if (failed) {
-    // the reference leaves the rotations untransposed and unnormalised
-    for (int j = lane; j < n; j += RSB_WAVE) y[j] = z[imin * n + j];
   } else {
-    // eigenvector imin = column imin of z, normalised (sum in row order)
-    if (lane == 0) {
-      double nrm = 0.0;
-      for (int i = 0; i < n; i++) nrm += z[i * n + imin] * z[i * n + imin];
-      if (nrm > 0.0) nrm = sqrt(fabs(nrm));
-      e[0] = 1.0 / nrm;
+    D.load(d, n, lane);
+    E.load(e, n, lane);
+    int failed = 0, buf = 0;
+    for (int l = 0; l < n && !failed; l++) {
+      int sweeps = 0, m;
+      while (true) {
+        // d[m + 1] next to d[m]: lane 63's neighbour is entry 64
+        double dn_a = __shfl_down(D.a, 1, RSB_WAVE);
+        double dn_b = 0.0;
+        if (W == 2) {
+          const double d64 = lane_get(D.b, 0);
+          if (lane == RSB_WAVE - 1) dn_a = d64;
+          dn_b = __shfl_down(D.b, 1, RSB_WAVE);
+        }
+        const int ma = lane, mb = lane + RSB_WAVE;
+        const bool ta = ma >= l && ma < n - 1 && fabs(E.a) / (fabs(D.a) + fabs(dn_a)) < 1e-12;
+        const bool tb = W == 2 && mb >= l && mb < n - 1 && fabs(E.b) / (fabs(D.b) + fabs(dn_b)) < 1e-12;
+        const unsigned long long ba = __ballot(ta), bb = __ballot(tb);
+        m = ba ? __ffsll((long long)ba) - 1 : bb ? RSB_WAVE + __ffsll((long long)bb) - 1 : n - 1;
+        if (m == l) break;
+        if (sweeps++ == 30) {
+          failed = 1;
+          break;
+        }
+        lanes_t<W> C, S;  // the step's rotation, in the lane of its e[i + 1]
+        C.a = C.b = S.a = S.b = 0.0;
+        const double dl = D.get(l), el = E.get(l);
+        double g = (D.get(l + 1) - dl) / (2.0 * el);
+        double r = sqrt(g * g + 1.0);
+        double dm = D.get(m);  // d[i + 1] of the step
+        g = dm - dl + el / (g + sgn_abs(r, g));
+        double s = 1.0, c = 1.0, p = 0.0;
+        for (int i = m - 1; i >= l; i--) {
+          const double ei = E.get(i), di = D.get(i);
+          const double f = s * ei, b = c * ei;
+          // the larger of |f|, |g| divides: t = small / large,
+          // r = sqrt(t^2 + 1), 1 / r and t / r are the rotation
+          const bool fg = fabs(f) >= fabs(g);
+          const double big = fg ? f : g, sml = fg ? g : f;
+          double t = div_plain(sml, big), ri;
+          sqrt_rcp_plain(t * t + 1.0, r, ri);
+          if (!(in_plain_range(big) && in_plain_range(sml))) {
+            t = sml / big;
+            r = sqrt(t * t + 1.0);
+            ri = 1.0 / r;
+          }
+          const double ei1 = big * r, tr = t * ri;
+          s = fg ? ri : tr;
+          c = fg ? tr : ri;
+          g = dm - p;
+          dm = di;
+          r = (di - g) * s + 2.0 * c * b;
+          p = s * r;
+          const double di1 = g + p;
+          g = c * r - b;
+          E.set(i + 1, ei1, lane);
+          D.set(i + 1, di1, lane);
+          C.set(i + 1, c, lane);
+          S.set(i + 1, s, lane);
+        }
+        C.store(sh->cs[buf][0], n, lane);
+        S.store(sh->cs[buf][1], n, lane);
+        D.set(l, D.get(l) - p, lane);
+        E.set(l, g, lane);
+        E.set(m, 0.0, lane);
+        if (lane == 0) sh->l[buf] = l, sh->m[buf] = m;
+        __syncthreads();
+        buf ^= 1;
+      }
     }
+    if (lane == 0) sh->m[buf] = -1, sh->failed = failed;
     __syncthreads();
-    double scale = e[0];
-    for (int j = lane; j < n; j += RSB_WAVE) y[j] = z[j * n + imin] * scale;
   }
-  const double lam = D.get(imin);
-  if (lane == 0) *lam_out = lam;
+  // (the last barrier follows the last sweep's rotations)
+  if (wave == 0) {
+    const int failed = sh->failed;
+    // eigenvalue of smallest magnitude (first on ties, fiedler.c:538-545)
+    int imin = 0;
+    double emin = fabs(D.get(0));
+    for (int i = 1; i < n; i++) {
+      const double v = fabs(D.get(i));
+      if (v < emin) emin = v, imin = i;
+    }
+    if (failed) {
+      // the reference leaves the rotations untransposed and unnormalised
+      for (int j = lane; j < n; j += RSB_WAVE) y[j] = z[j * zp + imin];
+    } else {
+      // eigenvector imin = column imin of z, normalised (sum in row order)
+      lanes_t<W> v, q;
+      v.load(z + imin * zp, n, lane);
+      q.a = v.a * v.a, q.b = v.b * v.b;
+      double nrm = 0.0;
+      for (int i = 0; i < n; i++) nrm += q.get(i);
+      if (nrm > 0.0) nrm = sqrt(fabs(nrm));
+      const double scale = 1.0 / nrm;
+      v.a *= scale, v.b *= scale;
+      v.store(y, n, lane);
+    }
+    const double lam = D.get(imin);
+    if (lane == 0) *lam_out = lam;
+  }
   __syncthreads();
 }
 // The same QL steps for passes longer than 128 iterations: d and e in LDS
@@ -1250,8 +1347,23 @@ __device__ void tqli_wave_mem(int n, double *d, double *e, double *z, double *y,
 // the count recurrence with the pivot guard of LAPACK dstebz).  Sign: the
 // component along the first Lanczos vector (the pass's start) is made
 // non-negative.  It agrees with the QL solve to rounding, not bit for bit.
-__device__ inline int sturm_count(int n, const lanes2 &D, const lanes2 &E2, double x,
-                                  double pivmin) {
+// plain: every squared off-diagonal is in div_plain's range and the pivot
+// guard below it.  The count then runs on plain divides without a test in
+// its chain, and again in full if some pivot left the range.
+template <int W>
+__device__ inline int sturm_count(int n, const lanes_t<W> &D, const lanes_t<W> &E2, double x,
+                                  double pivmin, bool plain) {
+  if (plain) {
+    double q = D.get(0) - x;
+    bool ok = in_plain_range(q);
+    int c = q < 0.0;
+    for (int i = 1; i < n; i++) {
+      q = (D.get(i) - x) - div_plain(E2.get(i - 1), q);
+      ok &= in_plain_range(q);
+      c += q < 0.0;
+    }
+    if (__all(ok)) return c;
+  }
   int c = 0;
   double q = D.get(0) - x;
   if (fabs(q) < pivmin) q = -pivmin;
@@ -1265,14 +1377,15 @@ __device__ inline int sturm_count(int n, const lanes2 &D, const lanes2 &E2, doub
 }
 
 // eigenvalue number j (ascending) in [lo, hi]; returns the final interval
-__device__ inline void multisect(int n, const lanes2 &D, const lanes2 &E2, double pivmin, int j,
-                                 double &lo, double &hi) {
+template <int W>
+__device__ inline void multisect(int n, const lanes_t<W> &D, const lanes_t<W> &E2, double pivmin,
+                                 bool plain, int j, double &lo, double &hi) {
   const int lane = threadIdx.x;
   for (int step = 0; step < 16; step++) {
     const double w = hi - lo;
     if (!(w > 2.0 * DBL_EPSILON * fmax(fabs(lo), fabs(hi)) + pivmin)) break;
     const double x = lo + w * (double)(lane + 1) / (double)(RSB_WAVE + 1);
-    const int c = sturm_count(n, D, E2, x, pivmin);
+    const int c = sturm_count<W>(n, D, E2, x, pivmin, plain);
     // lanes whose shift is at or below eigenvalue j: count <= j
     const unsigned long long below = __ballot(c <= j);
     // shifts increase with the lane: the highest such lane is the new lower
@@ -1284,14 +1397,14 @@ __device__ inline void multisect(int n, const lanes2 &D, const lanes2 &E2, doubl
   }
 }
 
+template <int W>
 __device__ void eig_min_wave(int n, const double *d, const double *e, double *y,
-                             double *lam_out, double *work) {
+                             double *lam_out) {
   const int lane = threadIdx.x;
-  lanes2 D, E2;
-  D.a = lane < n ? d[lane] : 0.0;
-  D.b = lane + RSB_WAVE < n ? d[lane + RSB_WAVE] : 0.0;
-  const double ea = lane < n - 1 ? e[lane] : 0.0, eb = lane + RSB_WAVE < n - 1 ? e[lane + RSB_WAVE] : 0.0;
-  E2.a = ea * ea, E2.b = eb * eb;
+  lanes_t<W> D, E, E2;
+  D.load(d, n, lane);
+  E.load(e, n - 1, lane);
+  E2.a = E.a * E.a, E2.b = E.b * E.b;
   // Gershgorin bounds and the pivot guard
   double glo = DBL_MAX, ghi = -DBL_MAX, emax = 0.0, tnorm = 0.0;
   for (int i = lane; i < n; i += RSB_WAVE) {
@@ -1309,64 +1422,82 @@ __device__ void eig_min_wave(int n, const double *d, const double *e, double *y,
   const double pivmin = DBL_MIN * fmax(1.0, emax);
   const double span = fmax(ghi - glo, DBL_MIN);
   glo -= 2.0 * DBL_EPSILON * span, ghi += 2.0 * DBL_EPSILON * span;
+  const bool plain = __all((lane >= n - 1 || in_plain_range(E2.a)) &&
+                           (lane + RSB_WAVE >= n - 1 || in_plain_range(E2.b))) &&
+                     pivmin < 0x1p-400;
   // smallest eigenvalue; if it is negative, compare the eigenvalues either
   // side of 0 by magnitude
   double lo = glo, hi = ghi;
-  multisect(n, D, E2, pivmin, 0, lo, hi);
+  multisect<W>(n, D, E2, pivmin, plain, 0, lo, hi);
   double lam = 0.5 * (lo + hi), shift = lo;
   if (lam < 0.0) {
-    const int k = sturm_count(n, D, E2, 0.0, pivmin);
+    const int k = sturm_count<W>(n, D, E2, 0.0, pivmin, plain);
     double l1 = glo, h1 = ghi;
-    multisect(n, D, E2, pivmin, k - 1, l1, h1);
+    multisect<W>(n, D, E2, pivmin, plain, k - 1, l1, h1);
     lam = 0.5 * (l1 + h1), shift = l1;
     if (k < n) {
       double l2 = glo, h2 = ghi;
-      multisect(n, D, E2, pivmin, k, l2, h2);
+      multisect<W>(n, D, E2, pivmin, plain, k, l2, h2);
       const double lam2 = 0.5 * (l2 + h2);
       if (fabs(lam2) < fabs(lam)) lam = lam2, shift = l2;
     }
   }
-  // inverse iteration (two solves) on lane 0: (T - shift I) = L D L^T, a
-  // pivot below eps * |T|_inf replaced by +-eps * |T|_inf; each solve is
-  // rescaled by its largest entry before normalising
-  if (lane == 0) {
-    double *piv = work, *x = work + n;
-    const double tau = DBL_EPSILON * fmax(tnorm, DBL_MIN);
-    double q = d[0] - shift;
+  // inverse iteration (two solves): (T - shift I) = L D L^T, a pivot below
+  // eps * |T|_inf replaced by +-eps * |T|_inf; each solve is rescaled by its
+  // largest entry before normalising.  Entry i of every vector is in lane
+  // i % 64; only the pivots, the substitutions and the sum of squares are
+  // serial, and those chains read their operands by readlane (on one lane,
+  // with every divide in the chain and every operand from LDS, they were
+  // half of the kernel's 134 us; now 78 us in all).
+  const double tau = DBL_EPSILON * fmax(tnorm, DBL_MIN);
+  lanes_t<W> piv, l, x;
+  piv.a = piv.b = 1.0;
+  double q = D.get(0) - shift;
+  if (fabs(q) < tau) q = q < 0.0 ? -tau : tau;
+  piv.set(0, q, lane);
+  for (int i = 1; i < n; i++) {
+    const double di = D.get(i), e2 = E2.get(i - 1);
+    double t = div_plain(e2, q);
+    if (!(plain && in_plain_range(q))) t = e2 / q;
+    q = (di - shift) - t;
     if (fabs(q) < tau) q = q < 0.0 ? -tau : tau;
-    piv[0] = q;
-    for (int i = 1; i < n; i++) {
-      q = (d[i] - shift) - e[i - 1] * e[i - 1] / q;
-      if (fabs(q) < tau) q = q < 0.0 ? -tau : tau;
-      piv[i] = q;
-    }
-    for (int i = 0; i < n; i++) x[i] = 1.0;
-    for (int it = 0; it < 2; it++) {
-      // L z = x (unit lower, l_i = e_i / piv_i), D w = z, L^T v = w
-      for (int i = 1; i < n; i++) x[i] -= e[i - 1] / piv[i - 1] * x[i - 1];
-      for (int i = 0; i < n; i++) x[i] /= piv[i];
-      for (int i = n - 2; i >= 0; i--) x[i] -= e[i] / piv[i] * x[i + 1];
-      double amax = 0.0;
-      for (int i = 0; i < n; i++) amax = fmax(amax, fabs(x[i]));
-      if (!(amax > 0.0) || amax > DBL_MAX) {
-        for (int i = 0; i < n; i++) x[i] = i == 0 ? 1.0 : 0.0;
-        break;
-      }
-      double nrm = 0.0;
-      for (int i = 0; i < n; i++) {
-        x[i] /= amax;
-        nrm += x[i] * x[i];
-      }
-      nrm = sqrt(nrm);
-      int f = 0;
-      while (f < n - 1 && x[f] == 0.0) f++;
-      const double sc = (x[f] < 0.0 ? -1.0 : 1.0) / nrm;
-      for (int i = 0; i < n; i++) x[i] *= sc;
-    }
-    *lam_out = lam;
+    piv.set(i, q, lane);
   }
-  __syncthreads();
-  for (int j = lane; j < n; j += RSB_WAVE) y[j] = work[n + j];
+  l.a = E.a / piv.a, l.b = E.b / piv.b;  // l_i = e_i / piv_i
+  x.a = x.b = 1.0;
+  for (int it = 0; it < 2; it++) {
+    // L z = x (unit lower), D w = z, L^T v = w
+    double c = x.get(0);
+    for (int i = 1; i < n; i++) {
+      c = fmat(-l.get(i - 1), c, x.get(i));
+      x.set(i, c, lane);
+    }
+    x.a /= piv.a, x.b /= piv.b;
+    c = x.get(n - 1);
+    for (int i = n - 2; i >= 0; i--) {
+      c = fmat(-l.get(i), c, x.get(i));
+      x.set(i, c, lane);
+    }
+    double amax = fmax(lane < n ? fabs(x.a) : 0.0, lane + RSB_WAVE < n ? fabs(x.b) : 0.0);
+    for (int o = RSB_WAVE / 2; o > 0; o >>= 1) amax = fmax(amax, __shfl_xor(amax, o, RSB_WAVE));
+    if (!(amax > 0.0) || amax > DBL_MAX) {
+      x.a = lane == 0 ? 1.0 : 0.0, x.b = 0.0;
+      break;
+    }
+    x.a /= amax, x.b /= amax;
+    double nrm = 0.0;
+    for (int i = 0; i < n; i++) {
+      const double xi = x.get(i);
+      nrm = fmat(xi, xi, nrm);
+    }
+    nrm = sqrt(nrm);
+    int f = 0;
+    while (f < n - 1 && x.get(f) == 0.0) f++;
+    const double sc = (x.get(f) < 0.0 ? -1.0 : 1.0) / nrm;
+    x.a *= sc, x.b *= sc;
+  }
+  if (lane == 0) *lam_out = lam;
+  x.store(y, n, lane);
   __syncthreads();
 }
 
@@ -1375,39 +1506,43 @@ __global__ void __launch_bounds__(RSB_WAVE) k_lz_eigmin(lz_args a) {
   if (a.status[s] != LZ_PASSDONE) return;
   extern __shared__ double lds[];
   const int n = a.k[s], M = a.miter_max;
-  double *d = lds, *e = d + M, *work = e + M;
+  double *d = lds, *e = d + M;
   const double *Td = a.T + (size_t)s * 2 * M, *Tu = Td + M;
   for (int i = threadIdx.x; i < n; i += RSB_WAVE) {
     d[i] = Td[i];
     e[i] = (i < n - 1) ? Tu[i] : 0.0;
   }
   __syncthreads();
-  eig_min_wave(n, d, e, a.y + (size_t)s * M, &SC(s, SC_LAMBDA), work);
+  if (n <= RSB_WAVE) eig_min_wave<1>(n, d, e, a.y + (size_t)s * M, &SC(s, SC_LAMBDA));
+  else eig_min_wave<2>(n, d, e, a.y + (size_t)s * M, &SC(s, SC_LAMBDA));
 }
 
 __global__ void __launch_bounds__(RSB_WAVE) k_eigmin_test(int n, const double *dd,
                                                           const double *ee, double *y,
                                                           double *lam) {
   extern __shared__ double lds[];
-  double *d = lds, *e = d + n, *work = e + n;
+  double *d = lds, *e = d + n;
   for (int i = threadIdx.x; i < n; i += RSB_WAVE) d[i] = dd[i], e[i] = i < n - 1 ? ee[i] : 0.0;
   __syncthreads();
-  eig_min_wave(n, d, e, y, lam, work);
+  if (n <= RSB_WAVE) eig_min_wave<1>(n, d, e, y, lam);
+  else eig_min_wave<2>(n, d, e, y, lam);
 }
 
-__global__ void __launch_bounds__(RSB_WAVE) k_lz_tqli(lz_args a) {
+__global__ void __launch_bounds__(2 * RSB_WAVE) k_lz_tqli(lz_args a) {
   const int s = blockIdx.x;
   if (a.status[s] != LZ_PASSDONE) return;
   extern __shared__ double lds[];
+  __shared__ tqli_shared sh;
   const int n = a.k[s], M = a.miter_max;
   double *d = lds, *e = d + M, *z = e + M;
   const double *Td = a.T + (size_t)s * 2 * M, *Tu = Td + M;
-  for (int i = threadIdx.x; i < n; i += RSB_WAVE) {
+  for (int i = threadIdx.x; i < n; i += 2 * RSB_WAVE) {
     d[i] = Td[i];
     e[i] = (i < n - 1) ? Tu[i] : 0.0;
   }
   __syncthreads();
-  tqli_wave(n, d, e, z, a.y + (size_t)s * M, &SC(s, SC_LAMBDA));
+  if (n <= RSB_WAVE) tqli_wave<1>(n, d, e, z, a.y + (size_t)s * M, &SC(s, SC_LAMBDA), &sh);
+  else tqli_wave<2>(n, d, e, z, a.y + (size_t)s * M, &SC(s, SC_LAMBDA), &sh);
 }
 
 // Passes longer than 128 iterations (both precisions): segments s0 +
@@ -1440,14 +1575,16 @@ __global__ void __launch_bounds__(RSB_WAVE) k_tqli_test_g(int n, const double *d
 }
 
 // Stand-alone tridiagonal solve for the parity tests.
-__global__ void __launch_bounds__(RSB_WAVE) k_tqli_test(int n, const double *dd,
+__global__ void __launch_bounds__(2 * RSB_WAVE) k_tqli_test(int n, const double *dd,
                                                         const double *ee, double *y,
                                                         double *lam) {
   extern __shared__ double lds[];
+  __shared__ tqli_shared sh;
   double *d = lds, *e = d + n, *z = e + n;
-  for (int i = threadIdx.x; i < n; i += RSB_WAVE) d[i] = dd[i], e[i] = i < n - 1 ? ee[i] : 0.0;
+  for (int i = threadIdx.x; i < n; i += 2 * RSB_WAVE) d[i] = dd[i], e[i] = i < n - 1 ? ee[i] : 0.0;
   __syncthreads();
-  tqli_wave(n, d, e, z, y, lam);
+  if (n <= RSB_WAVE) tqli_wave<1>(n, d, e, z, y, lam, &sh);
+  else tqli_wave<2>(n, d, e, z, y, lam, &sh);
 }
 
 // Ritz vector (fiedler.c:547-553): f = sum_j (r_j / |r_j|) y_j, the basis
@@ -2456,7 +2593,8 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   };
   // restarted CG-Lanczos passes of the segments in LZ_SETUP (f holds the
   // normalised start vector; SC_MEANF is 0 for the first pass)
-  const size_t tq_lds = sizeof(double) * (2 * miter_max + miter_max * miter_max);
+  const size_t tq_lds =
+      sizeof(double) * (2 * miter_max + miter_max * ((miter_max + RSB_WAVE - 1) / RSB_WAVE * RSB_WAVE));
   auto passes = [&](int np_max) -> int {
     a.mpass = ai.mpass = np_max;
     // the running lists of a pass: compacted at the end of the pass before
@@ -2561,9 +2699,9 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
           RSB_LAUNCH_CHECK();
         }
       } else if (sizeof(T) == 4) {
-        k_lz_eigmin<<<nseg, RSB_WAVE, sizeof(double) * 4 * miter_max, st>>>(a);
+        k_lz_eigmin<<<nseg, RSB_WAVE, sizeof(double) * 2 * miter_max, st>>>(a);
       } else {
-        k_lz_tqli<<<nseg, RSB_WAVE, tq_lds, st>>>(a);
+        k_lz_tqli<<<nseg, 2 * RSB_WAVE, tq_lds, st>>>(a);
       }
       RSB_LAUNCH_CHECK();
       k_lz_ritz<T><<<ntiles, RSB_BLOCK, 0, st>>>(a, basis, mpad, f);
@@ -2720,14 +2858,14 @@ static int rsb_test_tridiag(const double *d, const double *e, int n, double *y, 
     err = hipMemcpy(de, e, sizeof(double) * (n - 1), hipMemcpyHostToDevice);
   if (err == hipSuccess) {
     if (fast) {
-      k_eigmin_test<<<1, RSB_WAVE, sizeof(double) * 4 * n, 0>>>(n, dd, de, dy, dl);
+      k_eigmin_test<<<1, RSB_WAVE, sizeof(double) * 2 * n, 0>>>(n, dd, de, dy, dl);
     } else if (n > 128) {
       err = rsb_dev_malloc((void **)&dz, sizeof(double) * (size_t)n * n);
       if (err == hipSuccess)
         k_tqli_test_g<<<1, RSB_WAVE, sizeof(double) * 2 * n, 0>>>(n, dd, de, dy, dl, dz);
     } else {
-      size_t lds = sizeof(double) * (2 * n + n * n);
-      k_tqli_test<<<1, RSB_WAVE, lds, 0>>>(n, dd, de, dy, dl);
+      size_t lds = sizeof(double) * (2 * n + n * ((n + RSB_WAVE - 1) / RSB_WAVE * RSB_WAVE));
+      k_tqli_test<<<1, 2 * RSB_WAVE, lds, 0>>>(n, dd, de, dy, dl);
     }
     err = hipGetLastError();
   }

@@ -53,3 +53,30 @@ def test_fused_iterations_equal_separate_launches(name, prec, fold, tiles, monke
     for k in ("niter", "npass", "lambda", "rnorm", "resid"):
         assert np.array_equal(of[k], ou[k], equal_nan=True), k
     assert np.array_equal(ff, fu)
+
+
+@pytest.mark.parametrize("n", [1, 2, 50, 63, 64, 65, 128])
+def test_tridiagonal_solves_over_wide_ranges(n, oracle):
+    """Entries over 300 decades, zero off-diagonals and a zero diagonal leave
+    the plain divide's range: the QL solve keeps the oracle's bits, and the
+    multisection solve's eigenvalue agrees with it to rounding of the largest
+    entry."""
+    import parrsb_amd as pa
+    rng = np.random.default_rng(n)
+    for kind in range(4):
+        if kind == 0:
+            d, e = 10.0 ** rng.uniform(-150, 150, n), 10.0 ** rng.uniform(-150, 150, n - 1)
+        elif kind == 1:
+            d, e = rng.uniform(0.1, 4, n), np.where(rng.random(n - 1) < 0.3, 0.0, 0.5)
+        elif kind == 2:
+            d, e = np.zeros(n), rng.uniform(0.1, 1, n - 1)
+        else:
+            d, e = np.full(n, 2.0), np.full(n - 1, -1.0)
+        print("tridiagonal", n, kind, flush=True)
+        lam, y = pa.test_tqli(d, e)
+        rc, ev, z = oracle.tqli(d, e)
+        k = int(np.argmin(np.abs(ev)))
+        assert lam == ev[k] and np.array_equal(y, z[k]), kind
+        if kind in (1, 3):
+            fast, _ = pa.test_tqli(d, e, fast=True)
+            assert abs(fast - lam) <= 1e-12 * (np.abs(d).max() + 1.0)
