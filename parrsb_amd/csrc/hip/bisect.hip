@@ -434,7 +434,7 @@ extern "C" int rsbgpu_write_part(rsbgpu *g, int *part, int part_is_device) {
   if (!part_is_device) {
     RSB_TRY(hipMemcpyAsync(part, dp, sizeof(int) * nel, hipMemcpyDeviceToHost, g->stream));
     RSB_TRY(hipStreamSynchronize(g->stream));
-    rsb_dev_free(dp);
+    rsb_dev_release(dp);
   } else {
     RSB_TRY(hipStreamSynchronize(g->stream));
   }
@@ -462,7 +462,7 @@ extern "C" int rsbgpu_write_seq(rsbgpu *g, int *seq, int seq_is_device) {
   if (!seq_is_device) {
     RSB_TRY(hipMemcpyAsync(seq, dp, sizeof(int) * nel, hipMemcpyDeviceToHost, g->stream));
     RSB_TRY(hipStreamSynchronize(g->stream));
-    rsb_dev_free(dp);
+    rsb_dev_release(dp);
   } else {
     RSB_TRY(hipStreamSynchronize(g->stream));
   }
@@ -604,7 +604,7 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
     RSB_LAUNCH_CHECK();
     RSB_TRY(hipMemcpyAsync(&hb, bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
     RSB_TRY(hipStreamSynchronize(g->stream));
-    rsb_dev_free(bad);
+    rsb_dev_release(bad);
     if (hb) RSB_FAIL(3, "part ids outside [0, %d)", nparts);
   }
   unsigned long long *acc = nullptr;
@@ -647,6 +647,7 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
   }
   out[0] = (int64_t)ha[0], out[1] = (int64_t)ha[1], out[2] = mx, out[3] = mn, out[4] = tot;
   out[5] = cmx, out[6] = (int64_t)ha[2], out[7] = empty;
-  rsb_dev_free(acc), rsb_dev_free(par), rsb_dev_free(size), rsb_dev_free(key), rsb_dev_free(val);
+  rsb_dev_release(acc), rsb_dev_release(par), rsb_dev_release(size), rsb_dev_release(key),
+      rsb_dev_release(val);
   return 0;
 }

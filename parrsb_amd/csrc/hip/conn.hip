@@ -446,13 +446,15 @@ extern "C" int rsbgpu_conn_mesh(int device, long long *vtx_out, const double *co
   }
 done:
 #undef CON_TRY
-  if (!on_device) {
-    if (dcoord) rsb_dev_free(dcoord);
-    if (dvtx) rsb_dev_free(dvtx);
-  }
-  rsb_dev_free(x), rsb_dev_free(dx), rsb_dev_free(lay), rsb_dev_free(val), rsb_dev_free(segp), rsb_dev_free(flag),
-      rsb_dev_free(excl), rsb_dev_free(key), rsb_dev_free(err), rsb_dev_free(cnt), rsb_dev_free(fill), rsb_dev_free(off),
-      rsb_dev_free(wide), rsb_dev_free(pdev), rsb_dev_free(pfx), rsb_dev_free(pfid), rsb_dev_free(pgone);
+  if (hipStreamSynchronize(st) != hipSuccess && rc == 0) rc = 2;
+  if (on_device) dcoord = nullptr, dvtx = nullptr;  // the caller's
+  for (const void *p :
+       {(const void *)dcoord, (const void *)dvtx, (const void *)x, (const void *)dx,
+        (const void *)lay, (const void *)val, (const void *)segp, (const void *)flag,
+        (const void *)excl, (const void *)key, (const void *)err, (const void *)cnt,
+        (const void *)fill, (const void *)off, (const void *)wide, (const void *)pdev,
+        (const void *)pfid, (const void *)pgone, (const void *)pfx})
+    rsb_dev_release(p);
   if (rc == 2 && msg && msg_len > 0) snprintf(msg, (size_t)msg_len, "device failure in connectivity");
   rsbgpu_close(g);
   return rc;

@@ -2384,20 +2384,22 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   // buffers
   size_t vb = (size_t)mpad * sizeof(T);
   if (vb > g->vec_bytes) {
+    const size_t nb = rsb_grown(g, vb, g->vec_bytes);
     for (void **q : {&g->d_p, &g->d_p2, &g->d_w, &g->d_f, &g->d_w2}) {
-      if (*q) RSB_TRY(rsb_dev_free(*q));
+      RSB_TRY(rsb_retire(g, *q, g->vec_bytes));
       *q = nullptr;
-      RSB_TRY(rsb_dev_malloc(q, vb + 256));
+      RSB_TRY(rsb_dev_malloc(q, nb + 256));
     }
-    g->vec_bytes = vb;
+    g->vec_bytes = nb;
   }
   // the pass's residuals r_0 .. r_miter (the last one written, not used)
   size_t bb = vb * ((size_t)miter_max + 1);
   if (bb > g->basis_bytes) {
-    if (g->d_basis) RSB_TRY(rsb_dev_free(g->d_basis));
+    const size_t nb = rsb_grown(g, bb, g->basis_bytes);
+    RSB_TRY(rsb_retire(g, g->d_basis, g->basis_bytes));
     g->d_basis = nullptr;
-    RSB_TRY(rsb_dev_malloc(&g->d_basis, bb + 256));
-    g->basis_bytes = bb;
+    RSB_TRY(rsb_dev_malloc(&g->d_basis, nb + 256));
+    g->basis_bytes = nb;
   }
   double *xrow = nullptr;
   RSB_TRY(RSB_SCRATCH(xrow, sizeof(double) * (mpad + 1)));
@@ -2405,8 +2407,9 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   if (nseg > g->lz_nseg_cap || miter_max > g->lz_miter_cap) {
     // iter, k, npass, niter and miter are carved from the status block
     for (void *q : {(void *)L.status, (void *)L.sc, (void *)L.T, (void *)L.y, (void *)L.rn})
-      if (q) RSB_TRY(rsb_dev_free(q));
-    int cap = std::max(nseg, 1);
+      RSB_TRY(rsb_retire(g, q, 1));
+    // the segment count doubles every level
+    const int cap = nseg <= 4096 && !g->borrowed ? std::max(64, (g->lz_nseg_cap ? 4 : 1) * nseg) : nseg;
     RSB_TRY(rsb_dev_malloc((void **)&L.status, sizeof(int) * cap * 6));
     L.iter = L.status + cap, L.k = L.status + 2 * cap, L.npass = L.status + 3 * cap;
     L.niter = L.status + 4 * cap;
@@ -2417,9 +2420,10 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
     g->lz_nseg_cap = cap, g->lz_miter_cap = miter_max;
   }
   if (ntiles > g->lz_tile_cap) {
-    if (L.partial) RSB_TRY(rsb_dev_free(L.partial));
-    RSB_TRY(rsb_dev_malloc((void **)&L.partial, sizeof(double) * 12 * std::max(ntiles, 1)));
-    g->lz_tile_cap = ntiles;
+    RSB_TRY(rsb_retire(g, L.partial, 1));
+    const int cap = (int)rsb_grown(g, std::max(ntiles, 1), g->lz_tile_cap);
+    RSB_TRY(rsb_dev_malloc((void **)&L.partial, sizeof(double) * 12 * cap));
+    g->lz_tile_cap = cap;
   }
   if (!L.running) RSB_TRY(rsb_dev_malloc((void **)&L.running, sizeof(int) * 2));
   lz_args a;

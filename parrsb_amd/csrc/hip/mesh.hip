@@ -56,6 +56,13 @@ extern "C" int rsbgpu_open(rsbgpu **out, int device) {
     *out = g;
     return 0;
   }
+  rsb_stream_set ss;
+  if (rsb_pool_take_streams(device, &ss)) {
+    g->stream = ss.stream;
+    g->ev0 = ss.ev[0], g->ev1 = ss.ev[1], g->lz_ev0 = ss.ev[2], g->lz_ev1 = ss.ev[3];
+    *out = g;
+    return 0;
+  }
   if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess ||
       hipEventCreate(&g->lz_ev0) != hipSuccess || hipEventCreate(&g->lz_ev1) != hipSuccess) {
@@ -66,16 +73,18 @@ extern "C" int rsbgpu_open(rsbgpu **out, int device) {
   return 0;
 }
 
-#define FREE(p)                 \
-  do {                          \
-    if (p) rsb_dev_free((void *)p);  \
-    p = nullptr;                \
+#define FREE(p)                       \
+  do {                                \
+    if (drained) rsb_dev_release((void *)p); \
+    else rsb_dev_free((void *)p);     \
+    p = nullptr;                      \
   } while (0)
 
 extern "C" void rsbgpu_close(rsbgpu *g) {
   if (!g) return;
   hipSetDevice(g->device);
-  if (g->stream) hipStreamSynchronize(g->stream);
+  // everything the handle's work used may be handed on once it has finished
+  const bool drained = g->stream && hipStreamSynchronize(g->stream) == hipSuccess;
   rsb_mg_free(g);
   FREE(g->own_vtx);
   FREE(g->own_xyz);
@@ -134,9 +143,13 @@ extern "C" void rsbgpu_close(rsbgpu *g) {
   FREE(g->d_v1);
   FREE(g->d_iscratch);
   for (auto &kv : g->scratch)
-    if (kv.second.first) rsb_dev_free(kv.second.first);
+    FREE(kv.second.first);
   g->scratch.clear();
-  if (!g->borrowed) {
+  for (void *p : g->retired) FREE(p);
+  g->retired.clear();
+  if (!g->borrowed) rsb_pool_tick(g->device);
+  if (!g->borrowed &&
+      !(drained && rsb_pool_give_streams(g->device, {g->stream, {g->ev0, g->ev1, g->lz_ev0, g->lz_ev1}}))) {
     if (g->ev0) hipEventDestroy(g->ev0);
     if (g->ev1) hipEventDestroy(g->ev1);
     if (g->lz_ev0) hipEventDestroy(g->lz_ev0);
@@ -321,7 +334,8 @@ static int build_ranks(rsbgpu *g) {
   int bits = 1;
   while (bits < 32 && (1u << bits) <= maxrank) bits++;
   g->rank_bits = bits;
-  rsb_dev_free(key), rsb_dev_free(val), rsb_dev_free(flag), rsb_dev_free(excl);
+  // (the last axis's copies were waited for, so nothing uses these any more)
+  rsb_dev_release(key), rsb_dev_release(val), rsb_dev_release(flag), rsb_dev_release(excl);
   return 0;
 }
 
@@ -367,8 +381,10 @@ static int build_graph(rsbgpu *g) {
   RSB_LAUNCH_CHECK();
   int nsi = (int)ns;
   RSB_TRY(hipMemcpyAsync(gstart + ng, &nsi, sizeof(int), hipMemcpyHostToDevice, g->stream));
-  rsb_dev_free(key), rsb_dev_free(flag), rsb_dev_free(excl);
-  key = nullptr;
+  if (g->borrowed) {  // the fixed array takes them back now, without a wait
+    rsb_dev_free(key), rsb_dev_free(flag), rsb_dev_free(excl);
+    key = nullptr, flag = nullptr, excl = nullptr;
+  }
   // count, scan, fill
   RSB_TRY(rsb_dev_malloc((void **)&rowlen, sizeof(int64_t) * (n + 1)));
   RSB_TRY(dev_alloc(g, g->d_growptr, (size_t)n + 1));
@@ -398,8 +414,10 @@ static int build_graph(rsbgpu *g) {
   RSB_TRY(hipMemcpyAsync(&ws, vmax, sizeof(ws), hipMemcpyDeviceToHost, g->stream));
   RSB_TRY(hipStreamSynchronize(g->stream));
   g->gwsum = (int64_t)ws;
-  rsb_dev_free(val), rsb_dev_free(slot_group), rsb_dev_free(gstart), rsb_dev_free(rowlen), rsb_dev_free(ovf),
-      rsb_dev_free(vmax);
+  for (const void *p : {(const void *)key, (const void *)flag, (const void *)excl,
+                        (const void *)val, (const void *)slot_group, (const void *)gstart,
+                        (const void *)rowlen, (const void *)ovf, (const void *)vmax})
+    rsb_dev_release(p);
   if (hovf) RSB_FAIL(3, "two elements share more than 15 vertex ids");
   return 0;
 }

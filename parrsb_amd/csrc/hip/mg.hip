@@ -1115,12 +1115,15 @@ struct mg_level_dev {
 struct mg_hier {
   std::vector<mg_level_dev> lv;
   std::vector<std::vector<int>> h_off, h_n;
+  // (rsb_mg_free has waited for the stream)
   ~mg_hier() {
-    for (auto &l : lv) {
-      rsb_dev_free(l.off), rsb_dev_free(l.n), rsb_dev_free(l.rseg), rsb_dev_free(l.rp), rsb_dev_free(l.ci);
-      rsb_dev_free(l.w), rsb_dev_free(l.diag), rsb_dev_free(l.r0), rsb_dev_free(l.sa), rsb_dev_free(l.sb), rsb_dev_free(l.u);
-      rsb_dev_free(l.soff), rsb_dev_free(l.rlen), rsb_dev_free(l.sci), rsb_dev_free(l.sw), rsb_dev_free(l.spk);
-    }
+    for (auto &l : lv)
+      for (const void *p :
+           {(const void *)l.off, (const void *)l.n, (const void *)l.rseg, (const void *)l.rp,
+            (const void *)l.ci, (const void *)l.w, (const void *)l.diag, (const void *)l.r0,
+            (const void *)l.sa, (const void *)l.sb, (const void *)l.u, (const void *)l.soff,
+            (const void *)l.rlen, (const void *)l.sci, (const void *)l.sw, (const void *)l.spk})
+        rsb_dev_release(p);
   }
 };
 
@@ -1135,6 +1138,7 @@ double sigma_cheb(int k, int n, double lmin, double lmax) {
 // The hierarchy of the last rsbgpu_fiedler_mg call stays with the handle
 // (for the parity hook rsbgpu_mg_level_csr) until the next call or close.
 void rsb_mg_free(rsbgpu *g) {
+  if (g->mg && g->stream) (void)hipStreamSynchronize(g->stream);
   delete (mg_hier *)g->mg;
   g->mg = nullptr;
 }
@@ -1173,7 +1177,7 @@ struct mg_scope {
     (void)hipStreamSynchronize(st);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
-    for (void *q : bufs) (void)rsb_dev_free(q);
+    for (void *q : bufs) rsb_dev_release(q);
   }
 };
 

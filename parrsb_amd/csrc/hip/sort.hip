@@ -8,7 +8,8 @@
 
 static int ensure_tmp(rsbgpu *g, size_t bytes) {
   if (bytes <= g->sort_tmp_bytes && g->d_sort_tmp) return 0;
-  if (g->d_sort_tmp) RSB_TRY(rsb_dev_free(g->d_sort_tmp));
+  RSB_TRY(rsb_retire(g, g->d_sort_tmp, g->sort_tmp_bytes));
+  bytes = rsb_grown(g, bytes, g->d_sort_tmp ? g->sort_tmp_bytes : 0);
   g->d_sort_tmp = nullptr;
   RSB_TRY(rsb_dev_malloc(&g->d_sort_tmp, bytes + 256));
   g->sort_tmp_bytes = bytes + 256;
@@ -17,8 +18,8 @@ static int ensure_tmp(rsbgpu *g, size_t bytes) {
 
 static int ensure_kv(rsbgpu *g, size_t n) {
   if (n <= g->sort_cap && g->d_k1) return 0;
-  if (g->d_k1) RSB_TRY(rsb_dev_free(g->d_k1));
-  if (g->d_v1) RSB_TRY(rsb_dev_free(g->d_v1));
+  RSB_TRY(rsb_retire(g, g->d_k1, g->sort_cap * sizeof(uint64_t)));
+  RSB_TRY(rsb_retire(g, g->d_v1, g->sort_cap * sizeof(int)));
   g->d_k1 = nullptr, g->d_v1 = nullptr;
   RSB_TRY(rsb_dev_malloc((void **)&g->d_k1, n * sizeof(uint64_t)));
   RSB_TRY(rsb_dev_malloc((void **)&g->d_v1, n * sizeof(int)));

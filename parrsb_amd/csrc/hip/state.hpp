@@ -23,6 +23,17 @@ template <typename T>
 inline hipError_t rsb_dev_malloc(T **p, size_t bytes) {
   return rsb_dev_malloc((void **)p, bytes);
 }
+// Give back a block that no queued work uses any more: it goes to the pool
+// of idle blocks (rsb_dev_free returns it to the device, waiting for it).
+void rsb_dev_release(const void *p);
+// The stream and events of closed handles, likewise.
+struct rsb_stream_set {
+  hipStream_t stream;
+  hipEvent_t ev[4];
+};
+bool rsb_pool_take_streams(int device, rsb_stream_set *out);
+bool rsb_pool_give_streams(int device, const rsb_stream_set &in);
+void rsb_pool_tick(int device);
 // Inside an allocation-free call on `device`: the stream and the four timing
 // events set up once for that device (returns false otherwise).
 bool rsb_arena_stream(int device, hipStream_t *stream, hipEvent_t *ev);
@@ -167,7 +178,26 @@ struct rsbgpu {
   // per-call scratch buffers, one per call site (file, line), kept across
   // calls while large enough and freed with the handle (rsb_scratch)
   std::map<std::pair<const void *, int>, std::pair<void *, size_t>> scratch;
+  // buffers replaced by larger ones while queued work may still use them,
+  // released when the handle closes
+  std::vector<void *> retired;
 };
+
+// Replaces a buffer: small ones wait for the handle's close instead of making
+// the device wait now (a free does), large ones are freed at once, and so
+// are those of an allocation-free call, whose frees never wait.
+inline hipError_t rsb_retire(rsbgpu *g, void *p, size_t bytes) {
+  if (!p) return hipSuccess;
+  if (g->borrowed || bytes > ((size_t)64 << 20)) return rsb_dev_free(p);
+  g->retired.push_back(p);
+  return hipSuccess;
+}
+// size of a buffer that takes a smaller one's place: the level loop asks for
+// slightly more every level (padding, segment counts); not in the fixed
+// array of an allocation-free call
+inline size_t rsb_grown(const rsbgpu *g, size_t bytes, size_t old) {
+  return old && !g->borrowed ? bytes + bytes / 8 : bytes;
+}
 
 // ---------------------------------------------------------------------------
 // error helpers
@@ -210,13 +240,15 @@ inline hipError_t dev_alloc(rsbgpu *g, T *&p, size_t n) {
   // enough: the level loop re-sizes the same slots every level, and freeing
   // and mapping the multi-GB level matrices again each time cost ~10 ms a
   // level at 16.7M elements (contents are never assumed to be fresh)
-  const size_t bytes = (n ? n : 1) * sizeof(T);
+  size_t bytes = (n ? n : 1) * sizeof(T);
   auto it = g->cap.find((const void *)&p);
-  if (p && it != g->cap.end() && it->second >= bytes) return hipSuccess;
+  const size_t old = p && it != g->cap.end() ? it->second : 0;
+  if (p && old >= bytes) return hipSuccess;
   if (p) {
-    hipError_t e = rsb_dev_free(p);
+    hipError_t e = rsb_retire(g, (void *)p, old);
     if (e != hipSuccess) return e;
     p = nullptr;
+    bytes = rsb_grown(g, bytes, old);
   }
   hipError_t e = rsb_dev_malloc((void **)&p, bytes);
   if (e == hipSuccess) g->cap[(const void *)&p] = bytes;
@@ -235,7 +267,8 @@ inline hipError_t rsb_scratch(rsbgpu *g, const void *file, int line, size_t byte
     return hipSuccess;
   }
   if (s.first) {
-    hipError_t e = rsb_dev_free(s.first);
+    hipError_t e = rsb_retire(g, s.first, s.second);
+    bytes = rsb_grown(g, bytes, s.second);
     s.first = nullptr, s.second = 0;
     if (e != hipSuccess) return e;
   }
