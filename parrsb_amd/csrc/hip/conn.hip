@@ -110,39 +110,101 @@ __global__ void k_con_element_check(int64_t nel, int nv, const int *__restrict__
       if (segp[e * nv + a] == segp[e * nv + b]) atomicOr(err, 1);
 }
 
-// vertex -> elements holding it (CSR over vertex ids)
-__global__ void k_con_vcount(int64_t np, const int *__restrict__ segp, int *__restrict__ cnt) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < np) atomicAdd(&cnt[segp[p]], 1);
+// Where each vertex's points start in the layout (sorted by vertex id);
+// off[nseg] = np.
+__global__ void k_con_starts(int64_t np, int nseg, const int *__restrict__ lay,
+                             const int *__restrict__ segp, int *__restrict__ off) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= np) return;
+  const int v = segp[lay[i]];
+  if (i == 0 || v != segp[lay[i - 1]]) off[v] = (int)i;
+  if (i == np - 1) off[nseg] = (int)np;
 }
 
-__global__ void k_con_vfill(int64_t np, int nv, const int *__restrict__ segp,
-                            const int64_t *__restrict__ off, int *__restrict__ fill,
-                            int *__restrict__ els) {
+// con-check.c:197-260: no element holds exactly 3 of a hex face's 4 corners.
+// One thread per corner of an element e walks the elements at its vertex;
+// the pair (e, el < e) is looked at from its first common corner, where the
+// 64 comparisons of their vertex ids (distinct within an element, which the
+// element check has shown) give the common corners of both, and with them
+// the corners of every face of either that the other holds.  The vertex's
+// elements are read from the layout.  (Counting every face's corners against
+// the lists of its four vertices took 24 ms for 1M hexes: 32 list entries
+// compared with 32 others, each from memory, per face; this takes 0.93 ms.)
+__global__ void __launch_bounds__(256) k_con_face_check(int64_t np, const int *__restrict__ segp,
+                                                        const int *__restrict__ lay,
+                                                        const int *__restrict__ off,
+                                                        int *__restrict__ err) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
-  const int v = segp[p];
-  els[off[v] + atomicAdd(&fill[v], 1)] = (int)(p / nv);
+  const int e = (int)(p >> 3), c = (int)(p & 7);
+  const int4 a0 = *(const int4 *)(segp + 8 * (int64_t)e), a1 = *(const int4 *)(segp + 8 * (int64_t)e + 4);
+  const int va[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+  const int v = segp[p], i1 = off[v + 1];
+  for (int i = off[v]; i < i1; i++) {
+    const int el = lay[i] >> 3;
+    if (el >= e) continue;
+    const int4 b0 = *(const int4 *)(segp + 8 * (int64_t)el), b1 = *(const int4 *)(segp + 8 * (int64_t)el + 4);
+    const int vb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+    unsigned ma = 0, mb = 0;
+#pragma unroll
+    for (int x = 0; x < 8; x++)
+#pragma unroll
+      for (int y = 0; y < 8; y++) {
+        const bool eq = va[x] == vb[y];
+        ma |= eq ? 1u << x : 0u;
+        mb |= eq ? 1u << y : 0u;
+      }
+    if (ma & ((1u << c) - 1u)) continue;  // seen from an earlier corner
+    bool bad = false;
+#pragma unroll
+    for (int f = 0; f < 6; f++) {
+      unsigned m = 0;
+#pragma unroll
+      for (int q = 0; q < 4; q++) m |= 1u << (CON_FACES3D[f][q] - 1);
+      bad |= __popc(ma & m) == 3 || __popc(mb & m) == 3;
+    }
+    if (bad) atomicOr(err, 1);
+  }
 }
 
-// con-check.c:197-260: no element holds exactly 3 of a hex face's 4 corners
-__global__ void k_con_face_check(int64_t nel, const int *__restrict__ segp,
-                                 const int64_t *__restrict__ off, const int *__restrict__ els,
-                                 int *__restrict__ err) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nel * 6) return;
-  const int64_t e = t / 6;
-  const int f = (int)(t % 6);
-  int v[4];
-  for (int c = 0; c < 4; c++) v[c] = segp[e * 8 + CON_FACES3D[f][c] - 1];
-  for (int c = 0; c < 4; c++)
-    for (int64_t l = off[v[c]]; l < off[v[c] + 1]; l++) {
-      const int el = els[l];
-      int m = 0;
-      for (int c2 = 0; c2 < 4; c2++)
-        for (int64_t l2 = off[v[c2]]; l2 < off[v[c2] + 1]; l2++) m += els[l2] == el;
-      if (m == 3) atomicOr(err, 1);
+// Can a later pass still split a segment?  Not where its points' spread
+// along every axis is within the limit of its smallest dx: two points next
+// to each other in any order differ by no more than the spread and their
+// limit is no less (all of it monotone in the rounded operations of
+// k_con_split).  One thread per segment; *more is set where one may split,
+// and workgroups that start after that leave.
+__global__ void k_con_more(int64_t np, int ndim, const int *__restrict__ lay,
+                           const int *__restrict__ segp, const double *__restrict__ x,
+                           const double *__restrict__ dx, double tol2, int *__restrict__ more) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= np || __hip_atomic_load(more, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  int a = lay[i];
+  const int s = segp[a];
+  if (i > 0 && segp[lay[i - 1]] == s) return;
+  double lo[3], hi[3], m = dx[a];
+  for (int d = 0; d < ndim; d++) lo[d] = hi[d] = x[(size_t)d * np + a];
+  for (int64_t j = i + 1; j < np; j++) {
+    if (j - i > 4096) break;  // too long to be one vertex's points: treat as open
+    a = lay[j];
+    if (segp[a] != s) break;
+    m = dx[a] < m ? dx[a] : m;
+    for (int d = 0; d < ndim; d++) {
+      const double v = x[(size_t)d * np + a];
+      lo[d] = v < lo[d] ? v : lo[d], hi[d] = v > hi[d] ? v : hi[d];
     }
+    if (j - i == 4096) m = -1.0;
+  }
+  bool open = !(m >= 0.0);
+  for (int d = 0; d < ndim; d++) {
+    const double df = hi[d] - lo[d];
+    open |= !(df * df <= m * tol2);
+  }
+  if (open) atomicOr(more, 1);
+}
+
+__global__ void k_con_iota(int64_t np, int *__restrict__ lay) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < np) lay[i] = (int)i;
 }
 
 // Periodic faces (con-periodic.c): corners of each record's face, in the
@@ -267,11 +329,6 @@ static int periodic_classes(int nrec, const int *elem, const int *sface, const i
   return 0;
 }
 
-__global__ void k_con_widen(int64_t n, const int *__restrict__ in, int64_t *__restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = in[i];
-}
-
 // vtx_out[nel*nv], coord[nel*nv*ndim]: host or device arrays (on_device).
 // Returns 0, 1 if the element or face check fails, 2 on a device error,
 // 3 on bad input.
@@ -304,8 +361,7 @@ extern "C" int rsbgpu_conn_mesh(int device, long long *vtx_out, const double *co
   hipStream_t st = g->stream;
   double *dcoord = nullptr, *x = nullptr, *dx = nullptr;
   int *lay = nullptr, *val = nullptr, *segp = nullptr, *flag = nullptr, *excl = nullptr,
-      *err = nullptr, *cnt = nullptr, *fill = nullptr;
-  int64_t *off = nullptr, *wide = nullptr;
+      *err = nullptr;
   int *pdev = nullptr, *pfid = nullptr, *pgone = nullptr;
   double *pfx = nullptr;
   uint64_t *key = nullptr;
@@ -330,33 +386,41 @@ extern "C" int rsbgpu_conn_mesh(int device, long long *vtx_out, const double *co
   CON_TRY(rsb_dev_malloc((void **)&val, sizeof(int) * (size_t)np));
   CON_TRY(rsb_dev_malloc((void **)&segp, sizeof(int) * (size_t)np));
   CON_TRY(rsb_dev_malloc((void **)&flag, sizeof(int) * (size_t)np));
-  CON_TRY(rsb_dev_malloc((void **)&excl, sizeof(int) * (size_t)np));
+  CON_TRY(rsb_dev_malloc((void **)&excl, sizeof(int) * ((size_t)np + 1)));
   CON_TRY(rsb_dev_malloc((void **)&key, sizeof(uint64_t) * (size_t)np));
   CON_TRY(rsb_dev_malloc((void **)&err, sizeof(int)));
   {
     const unsigned nb = nblocks(np, 256);
     k_con_points<<<nb, 256, 0, st>>>(dcoord, nel, ndim, nv, x, dx);
     CON_TRY(hipGetLastError());
-    {
-      std::vector<int> iota((size_t)np);
-      for (int64_t i = 0; i < np; i++) iota[i] = (int)i;
-      CON_TRY(hipMemcpyAsync(lay, iota.data(), sizeof(int) * (size_t)np, hipMemcpyHostToDevice, st));
-      CON_TRY(hipMemsetAsync(segp, 0, sizeof(int) * (size_t)np, st));
-      CON_TRY(hipStreamSynchronize(st));
-    }
+    k_con_iota<<<nb, 256, 0, st>>>(np, lay);
+    CON_TRY(hipGetLastError());
+    CON_TRY(hipMemsetAsync(segp, 0, sizeof(int) * (size_t)np, st));
     int nseg = 1;
     const double tol2 = tol * tol;
-    for (int t = 0; t < ndim; t++)
+    for (int t = 0; t < ndim; t++) {
+      if (t > 0) {
+        // another sweep over the axes only if it could split something
+        int more = 0;
+        CON_TRY(hipMemsetAsync(err, 0, sizeof(int), st));
+        k_con_more<<<nb, 256, 0, st>>>(np, ndim, lay, segp, x, dx, tol2, err);
+        CON_TRY(hipGetLastError());
+        CON_TRY(hipMemcpyAsync(&more, err, sizeof(int), hipMemcpyDeviceToHost, st));
+        CON_TRY(hipStreamSynchronize(st));
+        if (!more) break;
+      }
       for (int d = 0; d < ndim; d++) {
         const double *xd = x + (size_t)d * np;
         k_con_axis_keys<<<nb, 256, 0, st>>>(np, lay, xd, key, val);
         CON_TRY(hipGetLastError());
         if (rsb_sort_pairs_u64(g, key, val, np, 0, 64)) { rc = 2; goto done; }
-        k_con_seg_keys<<<nb, 256, 0, st>>>(np, val, segp, (uint32_t *)key);
-        CON_TRY(hipGetLastError());
-        int sb = 1;
-        while ((1ll << sb) < nseg) sb++;
-        if (rsb_sort_pairs_u32(g, (uint32_t *)key, val, np, 0, sb)) { rc = 2; goto done; }
+        if (nseg > 1) {
+          k_con_seg_keys<<<nb, 256, 0, st>>>(np, val, segp, (uint32_t *)key);
+          CON_TRY(hipGetLastError());
+          int sb = 1;
+          while ((1ll << sb) < nseg) sb++;
+          if (rsb_sort_pairs_u32(g, (uint32_t *)key, val, np, 0, sb)) { rc = 2; goto done; }
+        }
         CON_TRY(hipMemcpyAsync(lay, val, sizeof(int) * (size_t)np, hipMemcpyDeviceToDevice, st));
         k_con_split<<<nb, 256, 0, st>>>(np, lay, segp, xd, dx, tol2, flag);
         CON_TRY(hipGetLastError());
@@ -369,6 +433,7 @@ extern "C" int rsbgpu_conn_mesh(int device, long long *vtx_out, const double *co
         CON_TRY(hipStreamSynchronize(st));
         nseg = last[0] + last[1] + 1;
       }
+    }
     // output
     if (on_device) {
       dvtx = vtx_out;
@@ -389,19 +454,9 @@ extern "C" int rsbgpu_conn_mesh(int device, long long *vtx_out, const double *co
     CON_TRY(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, st));
     CON_TRY(hipStreamSynchronize(st));
     if (!herr && ndim == 3) {
-      int *els = val;  // np entries, one per corner
-      CON_TRY(rsb_dev_malloc((void **)&cnt, sizeof(int) * ((size_t)nseg + 1)));
-      CON_TRY(rsb_dev_malloc((void **)&fill, sizeof(int) * ((size_t)nseg + 1)));
-      CON_TRY(rsb_dev_malloc((void **)&off, sizeof(int64_t) * ((size_t)nseg + 1)));
-      CON_TRY(rsb_dev_malloc((void **)&wide, sizeof(int64_t) * ((size_t)nseg + 1)));
-      CON_TRY(hipMemsetAsync(cnt, 0, sizeof(int) * ((size_t)nseg + 1), st));
-      CON_TRY(hipMemsetAsync(fill, 0, sizeof(int) * ((size_t)nseg + 1), st));
-      k_con_vcount<<<nb, 256, 0, st>>>(np, segp, cnt);
-      k_con_widen<<<nblocks(nseg + 1, 256), 256, 0, st>>>(nseg + 1, cnt, wide);
-      CON_TRY(hipGetLastError());
-      if (rsb_exclusive_scan_i64(g, wide, off, nseg + 1)) { rc = 2; goto done; }
-      k_con_vfill<<<nb, 256, 0, st>>>(np, nv, segp, off, fill, els);
-      k_con_face_check<<<nblocks((int64_t)nel * 6, 256), 256, 0, st>>>(nel, segp, off, els, err);
+      int *off = excl;  // the scan's array: a vertex has at least one of the np points
+      k_con_starts<<<nb, 256, 0, st>>>(np, nseg, lay, segp, off);
+      k_con_face_check<<<nb, 256, 0, st>>>(np, segp, lay, off, err);
       CON_TRY(hipGetLastError());
       CON_TRY(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, st));
       CON_TRY(hipStreamSynchronize(st));
@@ -451,8 +506,7 @@ done:
   for (const void *p :
        {(const void *)dcoord, (const void *)dvtx, (const void *)x, (const void *)dx,
         (const void *)lay, (const void *)val, (const void *)segp, (const void *)flag,
-        (const void *)excl, (const void *)key, (const void *)err, (const void *)cnt,
-        (const void *)fill, (const void *)off, (const void *)wide, (const void *)pdev,
+        (const void *)excl, (const void *)key, (const void *)err, (const void *)pdev,
         (const void *)pfid, (const void *)pgone, (const void *)pfx})
     rsb_dev_release(p);
   if (rc == 2 && msg && msg_len > 0) snprintf(msg, (size_t)msg_len, "device failure in connectivity");
