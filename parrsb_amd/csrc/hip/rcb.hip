@@ -12,6 +12,11 @@
 // the current order among them.
 #include <algorithm>
 #include <cfloat>
+#include <cstring>
+#include <climits>
+#include <vector>
+
+#include <rocprim/rocprim.hpp>
 
 #include "state.hpp"
 
@@ -42,6 +47,13 @@ __global__ void k_segof(const int *__restrict__ seg, int nseg, const int *__rest
 extern "C" int rsbgpu_set_segments(rsbgpu *g, int nseg, const int *cstart, const int *n,
                                    const int *p, const int *r0) {
   RSB_TRY(hipSetDevice(g->device));
+  if (g->borrowed) {
+    // an allocation-free call hands the level's scratch back to the fixed
+    // array (no wait: it is reused only after the stream has drained)
+    for (auto &kv : g->scratch)
+      if (kv.second.first) RSB_TRY(rsb_dev_free(kv.second.first));
+    g->scratch.clear();
+  }
   g->nseg = nseg;
   g->h_cstart.assign(cstart, cstart + nseg);
   g->h_n.assign(n, n + nseg);
@@ -225,33 +237,29 @@ __global__ void __launch_bounds__(256) k_node_extent(const int *__restrict__ ord
   }
 }
 
-__global__ void k_node_axis(int K, int ndim, const int *__restrict__ frozen,
-                            const uint64_t *__restrict__ ext, int *__restrict__ axis) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= K) return;
-  if (frozen[k]) {
-    axis[k] = -1;
-    return;
-  }
-  double len[3];
+// Axis of largest extent of node k (ties to the lower axis).
+__device__ inline int node_axis(int K, int k, int ndim, const uint64_t *__restrict__ ext) {
+  double len[3] = {0.0, 0.0, 0.0};
   for (int d = 0; d < ndim; d++)
     len[d] = dkey_inv(ext[(size_t)(2 * d + 1) * K + k]) - dkey_inv(ext[(size_t)(2 * d) * K + k]);
   int a = 0;
   if (len[1] > len[0]) a = 1;
   if (ndim == 3 && len[2] > len[a]) a = 2;
-  axis[k] = a;
+  return a;
 }
 
+// Sort keys (node, rank along the node's axis); 32 bits where they fit.
+template <typename T>
 __global__ void k_rcb_keys(const int *__restrict__ order, const int *__restrict__ nodeof,
-                           const int *__restrict__ axis, const uint32_t *__restrict__ rank,
-                           int nel, int rank_bits, uint64_t *__restrict__ key,
-                           int *__restrict__ val) {
+                           const int *__restrict__ frozen, const uint64_t *__restrict__ ext,
+                           const uint32_t *__restrict__ rank, int nel, int ndim, int K,
+                           int rank_bits, T *__restrict__ key) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nel) return;
-  int node = nodeof[i], e = order[i], a = axis[node];
-  uint64_t r = a < 0 ? 0 : rank[(size_t)a * nel + e];
-  key[i] = ((uint64_t)node << rank_bits) | r;
-  val[i] = e;
+  const int node = nodeof[i];
+  T r = 0;
+  if (!frozen[node]) r = (T)rank[(size_t)node_axis(K, node, ndim, ext) * nel + order[i]];
+  key[i] = ((T)node << rank_bits) | r;
 }
 
 __global__ void k_child_count(int K, const nodes_t nd, int *__restrict__ cnt) {
@@ -300,13 +308,152 @@ __global__ void k_nodeof_next(int nel, const int *__restrict__ first,
   nodeof[i] = first[k] + (i >= split[k] ? 1 : 0);
 }
 
+// Middle of the RCB tree: nodes of up to RCB_MID elements are taken apart by
+// one workgroup each until every part that still splits fits the tail kernel,
+// with the same rules as the global rounds: a block radix sort in LDS of
+// (sub-node, rank) keys is the same stable sort.  A global round of small
+// nodes costs ~10-20 launches whatever its size; on 1M elements the rounds
+// from 8,192 down to 1,024 took ~0.2 ms each, the whole of this kernel 0.1 ms.
+#define RCB_MID 8192
+#define RCB_MID_T 1024
+#define RCB_MID_SUBS 64
+#define RCB_MID_SUB_BITS 6
+#define RCB_TAIL 1024
+
+__global__ void __launch_bounds__(RCB_MID_T) k_rcb_mid(const int *__restrict__ ns, const int *__restrict__ nl,
+                                                       const int *__restrict__ np,
+                                                       const int *__restrict__ frozen, int K,
+                                                       int *__restrict__ order,
+                                                       const double *__restrict__ coord,
+                                                       const uint32_t *__restrict__ rank, int nel,
+                                                       int ndim, int rank_bits) {
+  constexpr int IPT = RCB_MID / RCB_MID_T;
+  typedef rocprim::block_radix_sort<uint32_t, RCB_MID_T, IPT, int> sorter;
+  __shared__ typename sorter::storage_type tmp;
+  __shared__ int s_start[2][RCB_MID_SUBS], s_len[2][RCB_MID_SUBS], s_p[2][RCB_MID_SUBS];
+  __shared__ unsigned long long s_ext[6][RCB_MID_SUBS];
+  __shared__ int s_axis[RCB_MID_SUBS], s_count;
+  const int k = blockIdx.x;
+  const int n = nl[k];
+  if (frozen[k] || n <= RCB_TAIL) return;
+  const int start = ns[k], lane = threadIdx.x & (RSB_WAVE - 1);
+  int el[IPT];
+#pragma unroll
+  for (int q = 0; q < IPT; q++) {
+    const int i = (int)threadIdx.x * IPT + q;
+    el[q] = i < n ? order[start + i] : -1;
+  }
+  if (threadIdx.x == 0) s_start[0][0] = 0, s_len[0][0] = n, s_p[0][0] = np[k], s_count = 1;
+  __syncthreads();
+  for (int g = 0;; g ^= 1) {
+    const int cnt = s_count;
+    bool again = false;
+    for (int t = 0; t < cnt; t++) again |= s_len[g][t] > RCB_TAIL;
+    if (!again) break;
+    for (int t = threadIdx.x; t < cnt; t += RCB_MID_T)
+      for (int d = 0; d < 3; d++) s_ext[2 * d][t] = ~0ull, s_ext[2 * d + 1][t] = 0ull;
+    // sub-node of each item (positions ascend with the item)
+    int sb[IPT];
+    {
+      int t = 0;
+#pragma unroll
+      for (int q = 0; q < IPT; q++) {
+        const int i = (int)threadIdx.x * IPT + q;
+        while (t + 1 < cnt && s_start[g][t + 1] <= i) t++;
+        sb[q] = t;
+      }
+    }
+    __syncthreads();
+    const int wf = __shfl(sb[0], 0, RSB_WAVE), wl = __shfl(sb[IPT - 1], RSB_WAVE - 1, RSB_WAVE);
+    const bool whole = wf == wl;
+    for (int d = 0; d < ndim; d++) {
+      unsigned long long mn = ~0ull, mx = 0ull;
+      int cur = sb[0];
+#pragma unroll
+      for (int q = 0; q < IPT; q++) {
+        if (sb[q] != cur) {
+          if (s_len[g][cur] > RCB_TAIL) {
+            atomicMin(&s_ext[2 * d][cur], mn);
+            atomicMax(&s_ext[2 * d + 1][cur], mx);
+          }
+          cur = sb[q], mn = ~0ull, mx = 0ull;
+        }
+        if (el[q] >= 0) {
+          const unsigned long long v = dkey(coord[(size_t)d * nel + el[q]]);
+          mn = v < mn ? v : mn;
+          mx = v > mx ? v : mx;
+        }
+      }
+      if (whole) {
+        for (int o = RSB_WAVE / 2; o > 0; o >>= 1) {
+          const unsigned long long a = __shfl_xor(mn, o, RSB_WAVE), b = __shfl_xor(mx, o, RSB_WAVE);
+          mn = a < mn ? a : mn;
+          mx = b > mx ? b : mx;
+        }
+        if (lane != 0) continue;
+      }
+      if (s_len[g][cur] > RCB_TAIL) {
+        atomicMin(&s_ext[2 * d][cur], mn);
+        atomicMax(&s_ext[2 * d + 1][cur], mx);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < cnt) {
+      const int t = threadIdx.x;
+      int a = -1;
+      if (s_len[g][t] > RCB_TAIL) {
+        double len[3] = {0.0, 0.0, 0.0};
+        for (int d = 0; d < ndim; d++)
+          len[d] = dkey_inv(s_ext[2 * d + 1][t]) - dkey_inv(s_ext[2 * d][t]);
+        a = 0;
+        if (len[1] > len[0]) a = 1;
+        if (ndim == 3 && len[2] > len[a]) a = 2;
+      }
+      s_axis[t] = a;
+    }
+    __syncthreads();
+    uint32_t key[IPT];
+#pragma unroll
+    for (int q = 0; q < IPT; q++) {
+      const int a = s_axis[sb[q]];
+      key[q] = ~0u;  // past the node's end: stays last
+      if (el[q] >= 0)
+        key[q] = ((uint32_t)sb[q] << rank_bits) | (a < 0 ? 0u : rank[(size_t)a * nel + el[q]]);
+    }
+    int sub_bits = 1;
+    while ((1 << sub_bits) < cnt + 1) sub_bits++;  // (the past-the-end keys stay above)
+    sorter().sort(key, el, tmp, 0, rank_bits + sub_bits);
+    // children of the parts that were sorted
+    if (threadIdx.x == 0) {
+      int c = 0;
+      for (int t = 0; t < cnt; t++) {
+        const int st = s_start[g][t], ln = s_len[g][t], p = s_p[g][t];
+        if (ln > RCB_TAIL) {
+          const int lo = p > 1 ? (int)lower_count_dev(ln, p) : ln / 2;
+          s_start[g ^ 1][c] = st, s_len[g ^ 1][c] = lo, s_p[g ^ 1][c] = p > 1 ? (p + 1) / 2 : 1, c++;
+          s_start[g ^ 1][c] = st + lo, s_len[g ^ 1][c] = ln - lo;
+          s_p[g ^ 1][c] = p > 1 ? p / 2 : 1, c++;
+        } else {
+          s_start[g ^ 1][c] = st, s_len[g ^ 1][c] = ln, s_p[g ^ 1][c] = p, c++;
+        }
+      }
+      s_count = c;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int q = 0; q < IPT; q++) {
+    const int i = (int)threadIdx.x * IPT + q;
+    if (i < n) order[start + i] = el[q];
+  }
+}
+
 // Tail of the RCB tree: once no node holds more than RCB_TAIL elements, one
 // workgroup finishes each node in LDS, depth by depth, with the same rules as
 // the global rounds: per sub-node extents (coordinate min/max), axis of the
 // largest extent (ties to the lower axis), a stable sort along it (bitonic
 // sort of (sub-node, dense rank, position) keys, so ties keep their order),
 // and the split after the lower ranks' share (p > 1) or at n / 2 (p == 1).
-#define RCB_TAIL 1024
 #define RCB_TAIL_T 256
 // depths where no splitting sub-node is larger than this rank by counting
 // instead of the 55-stage bitonic network over the whole node (environment
@@ -578,91 +725,174 @@ static int rcb_depth(int64_t n, int p) {
   return d;
 }
 
+// One generation of nodes on the host: which ranges a round sorts and where
+// it splits them follows from counts alone, so the whole tree is known before
+// any coordinate is looked at and no round has to wait for the device.
+struct host_nodes {
+  std::vector<int> start, len, p, frozen;
+  int size() const { return (int)start.size(); }
+  void push(int s, int n, int q, int f) {
+    start.push_back(s), len.push_back(n), p.push_back(q), frozen.push_back(f);
+  }
+};
+
+// Children of (start, len, p), by the rule of k_children.
+static void split_node(host_nodes &out, int st, int n, int p) {
+  const int nl = p > 1 ? (int)lower_count_dev(n, p) : n / 2;
+  out.push(st, nl, p > 1 ? (p + 1) / 2 : 1, nl <= 1);
+  out.push(st + nl, n - nl, p > 1 ? p / 2 : 1, n - nl <= 1);
+}
+
+// The parts of at most `most` elements that a node is taken apart into.
+static void split_down(host_nodes &out, int st, int n, int p, int most) {
+  if (n <= most) {
+    out.push(st, n, p, n <= 1);
+    return;
+  }
+  host_nodes c;
+  split_node(c, st, n, p);
+  for (int h = 0; h < 2; h++) split_down(out, c.start[h], c.len[h], c.p[h], most);
+}
+
 static int run_rcb(rsbgpu *g) {
   const int nel = g->nel, nseg = g->nseg;
   int rounds = 0;
   for (int s = 0; s < nseg; s++)
     if (g->h_p[s] > 1) rounds = std::max(rounds, rcb_depth(g->h_n[s], g->h_p[s]));
   if (rounds == 0) return 0;
-  // node tables (two generations), sized for the worst case of nel nodes
-  // Every round adds at most one node per non-frozen node (len >= 2), so a
-  // round adds at most nel / 2 nodes; empty children (n < p) keep the count
-  // growing by at most that bound.
-  size_t cap = (size_t)nseg + (size_t)nel * (size_t)std::min(rounds, 4) / 2 + (size_t)nel + 16;
-  int *buf = nullptr;
-  RSB_TRY(RSB_SCRATCH(buf, sizeof(int) * cap * 13 + sizeof(int) * (size_t)nel));
-  nodes_t A{buf, buf + cap, buf + 2 * cap, buf + 3 * cap};
-  nodes_t B{buf + 4 * cap, buf + 5 * cap, buf + 6 * cap, buf + 7 * cap};
-  int *cnt = buf + 8 * cap, *first = buf + 9 * cap, *split = buf + 10 * cap;
-  int *axis = buf + 11 * cap, *nodeof = buf + 13 * cap;
-  uint64_t *ext = nullptr, *key = nullptr;
-  RSB_TRY(RSB_SCRATCH(ext, sizeof(uint64_t) * 6 * cap));
-  RSB_TRY(RSB_SCRATCH(key, sizeof(uint64_t) * ((size_t)nel + 1)));
-  int K = nseg;
-  int *stat = nullptr;
-  RSB_TRY(RSB_SCRATCH(stat, sizeof(int) * 2));
-  // the tail kernel takes over once every splitting node is small and has
-  // no more ranks than elements
+  hipStream_t st = g->stream;
   const char *tv = getenv("PARRSB_AMD_RCB_TAIL");
-  bool tail_ok = !(tv && atoi(tv) == 0);
-  int maxlen = 0, pbig = 0;
+  // the LDS kernels take over once every splitting node is small enough and
+  // has no more ranks than elements (the middle one has 26 bits of a key for
+  // a rank)
+  const bool tail_ok = !(tv && atoi(tv) == 0);
+  const int mid = tail_ok && g->rank_bits + RCB_MID_SUB_BITS <= 32 ? RCB_MID : RCB_TAIL;
+  // generations of the global rounds: node tables, first child and split
+  // position of every node, one upload
+  std::vector<host_nodes> gen(1);
   for (int s = 0; s < nseg; s++)
-    if (g->h_p[s] > 1 && g->h_n[s] > 1) {
-      maxlen = std::max(maxlen, g->h_n[s]);
-      pbig |= g->h_p[s] > g->h_n[s];
-    }
-  k_nodes_from_segments<<<nblocks(nseg, 256), 256, 0, g->stream>>>(g->d_seg, nseg, A);
-  RSB_LAUNCH_CHECK();
-  k_nodeof_init<<<nblocks(nel, 256), 256, 0, g->stream>>>(g->d_seg, nseg, nel, nodeof);
-  RSB_LAUNCH_CHECK();
-  for (int r = 0; r < rounds; r++) {
-    if (tail_ok && maxlen <= RCB_TAIL && !pbig) {
-      const char *rm = getenv("PARRSB_AMD_RCB_RANKMAX");
-      k_rcb_tail<<<K, RCB_TAIL_T, 0, g->stream>>>(A, K, g->d_order, g->d_coord, g->d_rank, nel,
-                                                  g->ndim, rm ? atoi(rm) : RCB_RANKMAX);
-      RSB_LAUNCH_CHECK();
+    gen[0].push(g->h_cstart[s], g->h_n[s], g->h_p[s], g->h_p[s] <= 1 || g->h_n[s] <= 1);
+  std::vector<int> tab;
+  std::vector<size_t> at;  // offset of each generation's six arrays in tab
+  int last = -1;           // generation the LDS kernels start from (-1: never)
+  for (int r = 0;; r++) {
+    const host_nodes &h = gen[r];
+    int maxlen = 0, pbig = 0;
+    for (int k = 0; k < h.size(); k++)
+      if (!h.frozen[k]) maxlen = std::max(maxlen, h.len[k]), pbig |= h.p[k] > h.len[k];
+    at.push_back(tab.size());
+    tab.insert(tab.end(), h.start.begin(), h.start.end());
+    tab.insert(tab.end(), h.len.begin(), h.len.end());
+    tab.insert(tab.end(), h.p.begin(), h.p.end());
+    tab.insert(tab.end(), h.frozen.begin(), h.frozen.end());
+    if (r == rounds || maxlen == 0) break;
+    if (tail_ok && maxlen <= mid && !pbig) {
+      last = r;
       break;
     }
-    k_node_extent_init<<<nblocks(K, 256), 256, 0, g->stream>>>(K, ext);
-    RSB_LAUNCH_CHECK();
-    k_node_extent<<<nblocks(nel, 256 * NE_PER), 256, 0, g->stream>>>(
-        g->d_order, nodeof, A.frozen, g->d_coord, nel, g->ndim, K,
-        (unsigned long long *)ext);
-    RSB_LAUNCH_CHECK();
-    k_node_axis<<<nblocks(K, 256), 256, 0, g->stream>>>(K, g->ndim, A.frozen, ext, axis);
-    RSB_LAUNCH_CHECK();
-    k_rcb_keys<<<nblocks(nel, 256), 256, 0, g->stream>>>(g->d_order, nodeof, axis, g->d_rank,
-                                                         nel, g->rank_bits, key, g->d_order);
-    RSB_LAUNCH_CHECK();
-    int node_bits = 1;
-    while ((1ll << node_bits) < K) node_bits++;
-    int rc = rsb_sort_pairs_u64(g, key, g->d_order, nel, 0, g->rank_bits + node_bits);
-    if (rc) return rc;
-    // children
-    k_child_count<<<nblocks(K, 256), 256, 0, g->stream>>>(K, A, cnt);
-    RSB_LAUNCH_CHECK();
-    rc = rsb_exclusive_scan_i32(g, cnt, first, K);
-    if (rc) return rc;
-    int last[2];
-    RSB_TRY(hipMemcpyAsync(&last[0], first + K - 1, sizeof(int), hipMemcpyDeviceToHost,
-                           g->stream));
-    RSB_TRY(hipMemcpyAsync(&last[1], cnt + K - 1, sizeof(int), hipMemcpyDeviceToHost,
-                           g->stream));
-    RSB_TRY(hipStreamSynchronize(g->stream));
-    int K2 = last[0] + last[1];
-    if ((size_t)K2 > cap) RSB_FAIL(2, "RCB node table overflow (%d > %zu)", K2, cap);
-    RSB_TRY(hipMemsetAsync(stat, 0, sizeof(int) * 2, g->stream));
-    k_children<<<nblocks(K, 256), 256, 0, g->stream>>>(K, A, first, B, split, stat);
-    RSB_LAUNCH_CHECK();
-    int hstat[2];
-    RSB_TRY(hipMemcpyAsync(hstat, stat, sizeof(int) * 2, hipMemcpyDeviceToHost, g->stream));
-    k_nodeof_next<<<nblocks(nel, 256), 256, 0, g->stream>>>(nel, first, split, nodeof);
-    RSB_LAUNCH_CHECK();
-    RSB_TRY(hipStreamSynchronize(g->stream));
-    maxlen = hstat[0], pbig = hstat[1];
-    K = K2;
-    std::swap(A, B);
+    gen.emplace_back();
+    host_nodes &c = gen[r + 1];
+    const host_nodes &p = gen[r];  // (h may have moved)
+    std::vector<int> first, split;
+    for (int k = 0; k < p.size(); k++) {
+      first.push_back(c.size());
+      if (p.frozen[k]) {
+        c.push(p.start[k], p.len[k], p.p[k], 1);
+        split.push_back(INT_MAX);
+      } else {
+        split_node(c, p.start[k], p.len[k], p.p[k]);
+        split.push_back(c.start.back());
+      }
+    }
+    tab.insert(tab.end(), first.begin(), first.end());
+    tab.insert(tab.end(), split.begin(), split.end());
   }
+  const int nround = (int)gen.size() - 1;
+  // the parts the tail kernel finishes
+  host_nodes parts;
+  size_t tail_at = 0;
+  if (last >= 0) {
+    for (int k = 0; k < gen[last].size(); k++)
+      if (!gen[last].frozen[k])
+        split_down(parts, gen[last].start[k], gen[last].len[k], gen[last].p[k], RCB_TAIL);
+    tail_at = tab.size();
+    tab.insert(tab.end(), parts.start.begin(), parts.start.end());
+    tab.insert(tab.end(), parts.len.begin(), parts.len.end());
+    tab.insert(tab.end(), parts.p.begin(), parts.p.end());
+    tab.insert(tab.end(), parts.frozen.begin(), parts.frozen.end());
+  }
+  int *dtab = nullptr;
+  RSB_TRY(RSB_SCRATCH(dtab, sizeof(int) * tab.size()));
+  RSB_TRY(hipMemcpyAsync(dtab, tab.data(), sizeof(int) * tab.size(), hipMemcpyHostToDevice, st));
+  if (nround > 0) {
+    size_t next_total = 0;
+    for (int r = 0; r < nround; r++) next_total += gen[r].size();
+    uint64_t *ext = nullptr, *key = nullptr;
+    int *nodeof = nullptr;
+    RSB_TRY(RSB_SCRATCH(ext, sizeof(uint64_t) * 6 * next_total));
+    RSB_TRY(RSB_SCRATCH(key, sizeof(uint64_t) * ((size_t)nel + 1)));
+    RSB_TRY(RSB_SCRATCH(nodeof, sizeof(int) * (size_t)nel));
+    k_nodeof_init<<<nblocks(nel, 256), 256, 0, st>>>(g->d_seg, nseg, nel, nodeof);
+    RSB_LAUNCH_CHECK();
+    size_t eo = 0;
+    for (int r = 0; r < nround; r++) {
+      const int K = gen[r].size();
+      const int *frozen = dtab + at[r] + 3 * (size_t)K, *first = frozen + K, *split = first + K;
+      uint64_t *ex = ext + 6 * eo;
+      eo += K;
+      k_node_extent_init<<<nblocks(K, 256), 256, 0, st>>>(K, ex);
+      k_node_extent<<<nblocks(nel, 256 * NE_PER), 256, 0, st>>>(
+          g->d_order, nodeof, frozen, g->d_coord, nel, g->ndim, K, (unsigned long long *)ex);
+      RSB_LAUNCH_CHECK();
+      int node_bits = 1;
+      while ((1ll << node_bits) < K) node_bits++;
+      const int bits = g->rank_bits + node_bits;
+      int rc;
+      if (bits <= 32) {
+        k_rcb_keys<uint32_t><<<nblocks(nel, 256), 256, 0, st>>>(
+            g->d_order, nodeof, frozen, ex, g->d_rank, nel, g->ndim, K, g->rank_bits,
+            (uint32_t *)key);
+        RSB_LAUNCH_CHECK();
+        rc = rsb_sort_vals_u32(g, (const uint32_t *)key, g->d_order, g->d_order2, nel, 0, bits);
+      } else {
+        k_rcb_keys<uint64_t><<<nblocks(nel, 256), 256, 0, st>>>(
+            g->d_order, nodeof, frozen, ex, g->d_rank, nel, g->ndim, K, g->rank_bits, key);
+        RSB_LAUNCH_CHECK();
+        rc = rsb_sort_vals_u64(g, key, g->d_order, g->d_order2, nel, 0, bits);
+      }
+      if (rc) return rc;
+      RSB_TRY(hipMemcpyAsync(g->d_order, g->d_order2, sizeof(int) * (size_t)nel,
+                             hipMemcpyDeviceToDevice, st));
+      if (r + 1 < nround) {
+        k_nodeof_next<<<nblocks(nel, 256), 256, 0, st>>>(nel, first, split, nodeof);
+        RSB_LAUNCH_CHECK();
+      }
+    }
+  }
+  if (last >= 0) {
+    const int K = gen[last].size(), KT = parts.size();
+    const int *a = dtab + at[last];
+    if (mid > RCB_TAIL) {
+      bool any = false;
+      for (int k = 0; k < K; k++) any |= !gen[last].frozen[k] && gen[last].len[k] > RCB_TAIL;
+      if (any) {
+        k_rcb_mid<<<K, RCB_MID_T, 0, st>>>(a, a + K, a + 2 * (size_t)K, a + 3 * (size_t)K, K,
+                                           g->d_order, g->d_coord, g->d_rank, nel, g->ndim,
+                                           g->rank_bits);
+        RSB_LAUNCH_CHECK();
+      }
+    }
+    int *t = dtab + tail_at;
+    const char *rm = getenv("PARRSB_AMD_RCB_RANKMAX");
+    if (KT > 0) {
+      k_rcb_tail<<<KT, RCB_TAIL_T, 0, st>>>(
+          nodes_t{t, t + KT, t + 2 * (size_t)KT, t + 3 * (size_t)KT}, KT, g->d_order, g->d_coord,
+          g->d_rank, nel, g->ndim, rm ? atoi(rm) : RCB_RANKMAX);
+      RSB_LAUNCH_CHECK();
+    }
+  }
+  // the table's host copy must outlive its upload
+  RSB_TRY(hipStreamSynchronize(st));
   return 0;
 }
 

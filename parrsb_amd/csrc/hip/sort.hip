@@ -27,17 +27,33 @@ static int ensure_kv(rsbgpu *g, size_t n) {
   return 0;
 }
 
+// Above SORT_MERGE_MAX items the radix sort's single-pass (onesweep) form,
+// below it the merge sort: a merge sort makes a launch per doubling from its
+// block size up.
+#define SORT_MERGE_MAX 65536
+typedef rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
+                                   rocprim::default_config, SORT_MERGE_MAX>
+    sort_cfg;
+
+template <typename K>
+static int sort_into(rsbgpu *g, const K *keys, K *kout, const int *vals, int *vout, int64_t n,
+                     int bb, int eb) {
+  size_t bytes = 0;
+  RSB_TRY(rocprim::radix_sort_pairs<sort_cfg>(nullptr, bytes, keys, kout, vals, vout, (size_t)n,
+                                              bb, eb, g->stream));
+  int rc = ensure_tmp(g, bytes);
+  if (rc) return rc;
+  bytes = g->sort_tmp_bytes;
+  RSB_TRY(rocprim::radix_sort_pairs<sort_cfg>(g->d_sort_tmp, bytes, keys, kout, vals, vout,
+                                              (size_t)n, bb, eb, g->stream));
+  return 0;
+}
+
 int rsb_sort_pairs_u64(rsbgpu *g, uint64_t *keys, int *vals, int64_t n, int bb, int eb) {
   if (n <= 1) return 0;
   int rc = ensure_kv(g, (size_t)n);
   if (rc) return rc;
-  size_t bytes = 0;
-  RSB_TRY(rocprim::radix_sort_pairs(nullptr, bytes, keys, g->d_k1, vals, g->d_v1, (size_t)n,
-                                    bb, eb, g->stream));
-  if ((rc = ensure_tmp(g, bytes))) return rc;
-  bytes = g->sort_tmp_bytes;
-  RSB_TRY(rocprim::radix_sort_pairs(g->d_sort_tmp, bytes, keys, g->d_k1, vals, g->d_v1,
-                                    (size_t)n, bb, eb, g->stream));
+  if ((rc = sort_into(g, keys, g->d_k1, vals, g->d_v1, n, bb, eb))) return rc;
   RSB_TRY(hipMemcpyAsync(keys, g->d_k1, n * sizeof(uint64_t), hipMemcpyDeviceToDevice,
                          g->stream));
   RSB_TRY(hipMemcpyAsync(vals, g->d_v1, n * sizeof(int), hipMemcpyDeviceToDevice, g->stream));
@@ -49,16 +65,26 @@ int rsb_sort_pairs_u32(rsbgpu *g, uint32_t *keys, int *vals, int64_t n, int bb, 
   int rc = ensure_kv(g, (size_t)n);
   if (rc) return rc;
   uint32_t *k1 = (uint32_t *)g->d_k1;
-  size_t bytes = 0;
-  RSB_TRY(rocprim::radix_sort_pairs(nullptr, bytes, keys, k1, vals, g->d_v1, (size_t)n, bb,
-                                    eb, g->stream));
-  if ((rc = ensure_tmp(g, bytes))) return rc;
-  bytes = g->sort_tmp_bytes;
-  RSB_TRY(rocprim::radix_sort_pairs(g->d_sort_tmp, bytes, keys, k1, vals, g->d_v1, (size_t)n,
-                                    bb, eb, g->stream));
+  if ((rc = sort_into(g, keys, k1, vals, g->d_v1, n, bb, eb))) return rc;
   RSB_TRY(hipMemcpyAsync(keys, k1, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, g->stream));
   RSB_TRY(hipMemcpyAsync(vals, g->d_v1, n * sizeof(int), hipMemcpyDeviceToDevice, g->stream));
   return 0;
+}
+
+// Stable sorts of n values by their keys into another array (the keys' array
+// is scratch afterwards): no copies back.
+int rsb_sort_vals_u64(rsbgpu *g, const uint64_t *keys, const int *vals, int *out, int64_t n,
+                      int bb, int eb) {
+  int rc = ensure_kv(g, (size_t)n);
+  if (rc) return rc;
+  return sort_into(g, keys, g->d_k1, vals, out, n, bb, eb);
+}
+
+int rsb_sort_vals_u32(rsbgpu *g, const uint32_t *keys, const int *vals, int *out, int64_t n,
+                      int bb, int eb) {
+  int rc = ensure_kv(g, (size_t)n);
+  if (rc) return rc;
+  return sort_into(g, keys, (uint32_t *)g->d_k1, vals, out, n, bb, eb);
 }
 
 int rsb_exclusive_scan_i64(rsbgpu *g, const int64_t *in, int64_t *out, int64_t n) {
