@@ -1720,10 +1720,18 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_lz_resid(lz_args a, int phase,
     const int sl = row >> 6, lane = row & 63;
     const uint32_t *e = ell + slice_off[sl] + lane;
     const double xi = x[row];
+    const int w = slice_w[sl];
     double sum = 0.0;
-    for (int j = 0; j < slice_w[sl]; j++) {
-      uint32_t q = e[(size_t)j * RSB_WAVE];
-      sum += (double)(q >> 28) * (xi - x[q & 0x0fffffffu]);
+    // eight entries, then their gathers, in flight
+    for (int j0 = 0; j0 < w; j0 += 8) {
+      uint32_t q[8];
+      double xc[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) q[u] = j0 + u < w ? e[(size_t)(j0 + u) * RSB_WAVE] : (uint32_t)row;
+#pragma unroll
+      for (int u = 0; u < 8; u++) xc[u] = x[q[u] & 0x0fffffffu];
+#pragma unroll
+      for (int u = 0; u < 8; u++) sum = fmat((double)(q[u] >> 28), xi - xc[u], sum);
     }
     if (phase == 0) v[0] += sum * xi;
     else {
@@ -2497,7 +2505,12 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   // The FP64 apply reads the 16-bit entries: with the 12-bit form it took
   // 0.253 against 0.233 ms per launch on the 256^3 box (FP32: 0.163 against
   // 0.177), the class sums in doubles costing more than the bytes they save.
-  const bool use12 = g->e12_ok && (sizeof(T) == 4 || g->e12_f64);
+  const bool want12 = sizeof(T) == 4 || g->e12_f64;
+  if (want12) {
+    const int e12rc = rsb_level_e12(g);
+    if (e12rc) return e12rc;
+  }
+  const bool use12 = want12 && g->e12_ok;
   slice_rec *srec = nullptr;
   RSB_TRY(RSB_SCRATCH(srec, sizeof(slice_rec) * (size_t)std::max<int64_t>(g->nslices, 1)));
   if (ntiles > 0) {

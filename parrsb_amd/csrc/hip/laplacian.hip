@@ -39,8 +39,8 @@ __global__ void k_fill_i32(int *__restrict__ a, int64_t n, int v) {
 __global__ void k_level_rowlen(int64_t mpad, const int *__restrict__ row_elem,
                                const int *__restrict__ segof, const int64_t *__restrict__ growptr,
                                const uint32_t *__restrict__ gadj, int *__restrict__ rowlen,
-                               int *__restrict__ slice_w, unsigned long long *__restrict__ nnz,
-                               int64_t *__restrict__ seg_nnz) {
+                               int *__restrict__ slice_w, int64_t *__restrict__ slice_pad,
+                               int *__restrict__ slice_nnz) {
   int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int len = 0;
   if (row < mpad) {
@@ -66,20 +66,29 @@ __global__ void k_level_rowlen(int64_t mpad, const int *__restrict__ row_elem,
     int t = __shfl_xor(m, o, RSB_WAVE);
     m = t > m ? t : m;
   }
-  unsigned long long s = wave_sum((unsigned long long)len);
-  if ((threadIdx.x & (RSB_WAVE - 1)) == 0 && row < mpad) {
-    slice_w[row / RSB_WAVE] = m;
-    atomicAdd(nnz, s);
-    // a segment's rows start 64-aligned, so the first row of a wavefront is
-    // a real row of the wavefront's segment
-    atomicAdd((unsigned long long *)&seg_nnz[segof[row_elem[row]]], s);
+  const int s = wave_sum(len);
+  if ((threadIdx.x & (RSB_WAVE - 1)) == 0 && row <= mpad) {
+    const int64_t sl = row / RSB_WAVE;
+    slice_pad[sl] = (int64_t)m * RSB_WAVE;  // 0 past the last slice
+    if (row < mpad) slice_w[sl] = m, slice_nnz[sl] = s;
   }
 }
 
-__global__ void k_slice_bytes(int64_t nslices, const int *__restrict__ w, int64_t *__restrict__ o) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nslices) o[i] = (int64_t)w[i] * RSB_WAVE;
-  if (i == nslices) o[i] = 0;
+// Entries per segment: a workgroup per segment over its slices.  (Two atomics
+// a slice on one address cost ~0.2 ms a level of 1M rows.)
+__global__ void __launch_bounds__(256) k_seg_nnz(const int *__restrict__ seg, int nseg,
+                                                 const int *__restrict__ slice_nnz,
+                                                 int64_t *__restrict__ seg_nnz) {
+  __shared__ long long red[256 / RSB_WAVE];
+  const int s = blockIdx.x, n = seg[nseg + s], p0 = seg[4 * nseg + s];
+  long long v = 0;
+  if (p0 >= 0)
+    for (int i = p0 / RSB_WAVE + (int)threadIdx.x; i < (p0 + n + RSB_WAVE - 1) / RSB_WAVE; i += 256)
+      v += slice_nnz[i];
+  v = wave_sum(v);
+  if ((threadIdx.x & (RSB_WAVE - 1)) == 0) red[threadIdx.x / RSB_WAVE] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) seg_nnz[s] = red[0] + red[1] + red[2] + red[3];
 }
 
 __global__ void k_level_fill(int64_t mpad, const int *__restrict__ row_elem,
@@ -142,31 +151,27 @@ extern "C" int rsbgpu_level_laplacian(rsbgpu *g) {
   k_row_maps<<<nblocks(nel, 256), 256, 0, g->stream>>>(g->d_order, g->d_segof, g->d_seg, g->nseg,
                                                        nel, g->d_row_elem, g->d_elem_row);
   RSB_LAUNCH_CHECK();
-  unsigned long long *dnnz = nullptr;
-  RSB_TRY(RSB_SCRATCH(dnnz, sizeof(unsigned long long)));
-  RSB_TRY(hipMemsetAsync(dnnz, 0, sizeof(unsigned long long), g->stream));
-  RSB_TRY(dev_alloc(g, g->d_seg_nnz, (size_t)g->nseg));
-  RSB_TRY(hipMemsetAsync(g->d_seg_nnz, 0, sizeof(int64_t) * g->nseg, g->stream));
-  k_level_rowlen<<<nblocks(mpad, 256), 256, 0, g->stream>>>(
-      mpad, g->d_row_elem, g->d_segof, g->d_growptr, g->d_gadj, g->d_rowlen, g->d_slice_w, dnnz,
-      g->d_seg_nnz);
-  RSB_LAUNCH_CHECK();
   int64_t *bytes = nullptr;
+  int *slice_nnz = nullptr;
   RSB_TRY(RSB_SCRATCH(bytes, sizeof(int64_t) * (g->nslices + 1)));
-  k_slice_bytes<<<nblocks(g->nslices + 1, 256), 256, 0, g->stream>>>(g->nslices, g->d_slice_w,
-                                                                     bytes);
+  RSB_TRY(RSB_SCRATCH(slice_nnz, sizeof(int) * (g->nslices + 1)));
+  RSB_TRY(dev_alloc(g, g->d_seg_nnz, (size_t)g->nseg));
+  k_level_rowlen<<<nblocks(mpad + 1, 256), 256, 0, g->stream>>>(
+      mpad, g->d_row_elem, g->d_segof, g->d_growptr, g->d_gadj, g->d_rowlen, g->d_slice_w, bytes,
+      slice_nnz);
+  RSB_LAUNCH_CHECK();
+  k_seg_nnz<<<g->nseg, 256, 0, g->stream>>>(g->d_seg, g->nseg, slice_nnz, g->d_seg_nnz);
   RSB_LAUNCH_CHECK();
   int rc = rsb_exclusive_scan_i64(g, bytes, g->d_slice_off, g->nslices + 1);
   if (rc) return rc;
-  unsigned long long hn = 0;
   RSB_TRY(hipMemcpyAsync(&g->lnnz_pad, g->d_slice_off + g->nslices, sizeof(int64_t),
                          hipMemcpyDeviceToHost, g->stream));
-  RSB_TRY(hipMemcpyAsync(&hn, dnnz, sizeof(hn), hipMemcpyDeviceToHost, g->stream));
   g->h_seg_nnz.assign(g->nseg, 0);
   RSB_TRY(hipMemcpyAsync(g->h_seg_nnz.data(), g->d_seg_nnz, sizeof(int64_t) * g->nseg,
                          hipMemcpyDeviceToHost, g->stream));
   RSB_TRY(hipStreamSynchronize(g->stream));
-  g->lnnz = (int64_t)hn;
+  g->lnnz = 0;
+  for (int64_t v : g->h_seg_nnz) g->lnnz += v;
   RSB_TRY(dev_alloc(g, g->d_ell, (size_t)g->lnnz_pad));
   k_level_fill<<<nblocks(mpad, 256), 256, 0, g->stream>>>(mpad, g->d_row_elem, g->d_segof,
                                                           g->d_elem_row, g->d_growptr,

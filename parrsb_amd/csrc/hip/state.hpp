@@ -88,6 +88,7 @@ struct rsbgpu {
   int64_t *d_growptr = nullptr;
   uint32_t *d_gadj = nullptr; // col | weight << 28
   int64_t gnnz = 0, gwsum = 0;
+  unsigned long long vmax = 0;  // largest vertex id
 
   // level state
   int *d_order = nullptr, *d_order2 = nullptr; // element at compact position
@@ -107,7 +108,7 @@ struct rsbgpu {
   int *d_tnhalo = nullptr, *d_halo = nullptr, *d_w16 = nullptr;
   int64_t *d_thalo_off = nullptr, *d_off16 = nullptr;
   uint16_t *d_e16 = nullptr;
-  int64_t nhalo_total = 0, e16_count = 0;
+  std::vector<int64_t> h_halo_off;
   // the same entries as 12-bit local indices ordered by weight class
   // (tiles.hip): per slice its block count and tail words, its slots per
   // class (n4 | n2 << 8 | n1 << 16, the same for its 64 rows), word offsets
@@ -119,7 +120,8 @@ struct rsbgpu {
   uint32_t *d_e12 = nullptr;
   int *d_c12 = nullptr;
   int e12_ok = 0, e12_f64 = 0;
-  int nwide = 0;
+  int e12_state = 0;  // 0 not wanted, 1 not yet built, 2 looked at (e12_ok)
+  int nwide = 0;  // tiles on the global path (-1: not counted yet)
   // vertex form of the tiles (tiles.hip, rsb_build_vtiles): per tile, the
   // distinct vertex ids of its rows, for each the nv window-local indices of
   // the slots at it (padded); per row its nv local vertex indices
@@ -287,6 +289,7 @@ inline hipError_t rsb_scratch(rsbgpu *g, const void *file, int line, size_t byte
 inline unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 int rsb_build_tiles(rsbgpu *g);   // tiles.hip
+int rsb_level_e12(rsbgpu *g);     // tiles.hip
 int rsb_build_vtiles(rsbgpu *g);  // tiles.hip
 // limits of the vertex form: window rows (tile + halo, the LDS window of the
 // neighbour-entry form) and local vertices
@@ -304,6 +307,8 @@ int rsb_sort_vals_u64(rsbgpu *g, const uint64_t *keys, const int *vals, int *out
                       int begin_bit, int end_bit);
 int rsb_sort_vals_u32(rsbgpu *g, const uint32_t *keys, const int *vals, int *out, int64_t n,
                       int begin_bit, int end_bit);
+int rsb_sort_keys_u32(rsbgpu *g, const uint32_t *keys, uint32_t *out, int64_t n, int end_bit);
+int rsb_sort_keys_u64(rsbgpu *g, const uint64_t *keys, uint64_t *out, int64_t n, int end_bit);
 int rsb_exclusive_scan_i64(rsbgpu *g, const int64_t *in, int64_t *out, int64_t n);
 int rsb_exclusive_scan_i32(rsbgpu *g, const int *in, int *out, int64_t n);
 

@@ -34,6 +34,7 @@
 #include <limits.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "state.hpp"
@@ -67,27 +68,35 @@ __device__ inline int tb_find(const int *keys, int c) {
   return -1;
 }
 
-// Collect the external columns of tile blockIdx.x into the LDS set.
+// Collect the external columns of tile blockIdx.x into the LDS set.  Eight
+// entries of a row are loaded before any is inserted: one at a time, every
+// entry waited for memory, which was most of the tile build (0.37 of 0.47 ms
+// for 1,024 tiles of hexes, in the passes over the entries).
+#define TB_U 8
 __device__ inline bool tb_collect(int *keys, int row0, int row1,
                                   const int64_t *__restrict__ slice_off,
                                   const int *__restrict__ slice_w,
                                   const uint32_t *__restrict__ ell) {
   for (int i = threadIdx.x; i < TB_HASH; i += blockDim.x) keys[i] = -1;
-  __syncthreads();
-  bool ok = true;
-  for (int row = row0 + threadIdx.x; row < row1; row += blockDim.x) {
-    const int sl = row >> 6;
-    const uint32_t *e = ell + slice_off[sl] + (row & 63);
-    for (int j = 0; j < slice_w[sl]; j++) {
-      uint32_t q = e[(size_t)j * RSB_WAVE];
-      int c = (int)(q & 0x0fffffffu);
-      if ((q >> 28) == 0 || (c >= row0 && c < row1)) continue;
-      if (!tb_insert(keys, c)) ok = false;
-    }
-  }
   __shared__ int any_fail;
   if (threadIdx.x == 0) any_fail = 0;
   __syncthreads();
+  bool ok = true;
+  for (int row = row0 + threadIdx.x; row < row1; row += blockDim.x) {
+    const int sl = row >> 6, w = slice_w[sl];
+    const uint32_t *e = ell + slice_off[sl] + (row & 63);
+    for (int j0 = 0; j0 < w; j0 += TB_U) {
+      uint32_t q[TB_U];
+#pragma unroll
+      for (int u = 0; u < TB_U; u++) q[u] = e[(size_t)min(j0 + u, w - 1) * RSB_WAVE];
+#pragma unroll
+      for (int u = 0; u < TB_U; u++) {
+        const int c = (int)(q[u] & 0x0fffffffu);
+        if ((q[u] >> 28) == 0 || (c >= row0 && c < row1)) continue;
+        if (!tb_insert(keys, c)) ok = false;
+      }
+    }
+  }
   if (!ok) atomicOr(&any_fail, 1);
   __syncthreads();
   return any_fail == 0;
@@ -108,23 +117,6 @@ __device__ inline int tb_scan(int v, int *total) {
   *total = s[blockDim.x - 1];
   __syncthreads();
   return incl - v;
-}
-
-// Pass A: number of halo rows per tile (-1 if it does not fit).
-__global__ void __launch_bounds__(RSB_BLOCK) k_tile_count(const int *__restrict__ tile,
-                                                          const int64_t *__restrict__ slice_off,
-                                                          const int *__restrict__ slice_w,
-                                                          const uint32_t *__restrict__ ell,
-                                                          int *__restrict__ nhalo) {
-  __shared__ int keys[TB_HASH];
-  const int t = blockIdx.x, row0 = tile[3 * t + 1], row1 = tile[3 * t + 2];
-  bool ok = tb_collect(keys, row0, row1, slice_off, slice_w, ell);
-  int cnt = 0;
-  const int per = TB_HASH / RSB_BLOCK;
-  for (int k = 0; k < per; k++) cnt += keys[threadIdx.x * per + k] >= 0;
-  int total;
-  tb_scan(cnt, &total);
-  if (threadIdx.x == 0) nhalo[t] = (ok && (row1 - row0) + total <= TB_LOCAL) ? total : -1;
 }
 
 // Position of entry j of lane `lane` in its slice's 16-bit entries: groups
@@ -165,68 +157,83 @@ __device__ inline void lds_bitonic(int *a, int n) {
     }
 }
 
-// Pass B: halo lists and the 16-bit entries.  A tile's halo rows are listed
-// in ascending row order (local index nrows + rank), so the apply's staging
-// gathers them at increasing addresses and neighbouring lanes share cache
-// lines.
-__global__ void __launch_bounds__(RSB_BLOCK) k_tile_fill(
+// Halo lists (nhalo = -1: does not fit) and the 16-bit entries, in one pass:
+// tile t's list has room for every row it can hold (halo_off, from the host),
+// so no count has to come first.  A tile's halo rows are listed in ascending
+// row order (local index nrows + rank), so the apply's staging gathers them
+// at increasing addresses and neighbouring lanes share cache lines.  Entries
+// are written a whole group (16, 8 or 4 bytes a lane) at a time.
+__global__ void __launch_bounds__(RSB_BLOCK) k_tile_build(
     const int *__restrict__ tile, const int64_t *__restrict__ slice_off,
-    const int *__restrict__ slice_w, const uint32_t *__restrict__ ell,
-    const int *__restrict__ nhalo, const int64_t *__restrict__ halo_off,
-    const int64_t *__restrict__ off16, const int *__restrict__ w16, int *__restrict__ halo,
+    const int *__restrict__ slice_w, const uint32_t *__restrict__ ell, int all_wide,
+    const int64_t *__restrict__ halo_off, const int64_t *__restrict__ off16,
+    const int *__restrict__ w16, int *__restrict__ nhalo, int *__restrict__ halo,
     uint16_t *__restrict__ e16) {
   __shared__ int keys[TB_HASH];
   __shared__ short local[TB_HASH];
   __shared__ int srt[TB_LOCAL];
   const int t = blockIdx.x, row0 = tile[3 * t + 1], row1 = tile[3 * t + 2];
   const int nrows = row1 - row0;
-  const bool fits = nhalo[t] >= 0;  // then nrows + halo rows <= TB_LOCAL
+  bool fits = !all_wide && tb_collect(keys, row0, row1, slice_off, slice_w, ell);
+  int total = 0;
   if (fits) {
-    tb_collect(keys, row0, row1, slice_off, slice_w, ell);
     const int per = TB_HASH / RSB_BLOCK;
     int cnt = 0;
-    for (int k = 0; k < per; k++) cnt += keys[threadIdx.x * per + k] >= 0;
-    int total;
+    for (int k = 0; k < per; k++) cnt += keys[threadIdx.x + k * RSB_BLOCK] >= 0;
     int base = tb_scan(cnt, &total);
-    for (int k = 0; k < per; k++) {
-      const int slot = threadIdx.x * per + k;
-      if (keys[slot] >= 0) srt[base++] = keys[slot];
+    fits = nrows + total <= TB_LOCAL;
+    if (fits) {
+      for (int k = 0; k < per; k++) {
+        const int c = keys[threadIdx.x + k * RSB_BLOCK];
+        if (c >= 0) srt[base++] = c;
+      }
+      int n2 = 1;
+      while (n2 < total) n2 <<= 1;
+      for (int i = total + threadIdx.x; i < n2; i += blockDim.x) srt[i] = INT_MAX;
+      __syncthreads();
+      lds_bitonic(srt, n2);
+      for (int i = threadIdx.x; i < total; i += blockDim.x) {
+        const int c = srt[i];
+        local[tb_find(keys, c)] = (short)(nrows + i);
+        halo[halo_off[t] + i] = c;
+      }
+      __syncthreads();
     }
-    int n2 = 1;
-    while (n2 < total) n2 <<= 1;
-    for (int i = total + threadIdx.x; i < n2; i += blockDim.x) srt[i] = INT_MAX;
-    __syncthreads();
-    lds_bitonic(srt, n2);
-    for (int i = threadIdx.x; i < total; i += blockDim.x) {
-      const int c = srt[i];
-      local[tb_find(keys, c)] = (short)(nrows + i);
-      halo[halo_off[t] + i] = c;
-    }
-    __syncthreads();
   }
+  if (threadIdx.x == 0) nhalo[t] = fits ? total : -1;
   for (int row = row0 + threadIdx.x; row < row1; row += blockDim.x) {
     const int sl = row >> 6, lane = row & 63;
     const uint32_t *e = ell + slice_off[sl] + lane;
     uint16_t *o = e16 + off16[sl];
     const int w = slice_w[sl], w8 = w16[sl];
-    const uint16_t self = (uint16_t)(row - row0);
-    for (int j = 0; j < w8; j++) {
-      uint16_t v = self;  // padding: own row, weight 0
-      if (fits && j < w) {
-        uint32_t q = e[(size_t)j * RSB_WAVE];
-        int c = (int)(q & 0x0fffffffu);
-        uint32_t wt = q >> 28;
+    const uint32_t self = (uint32_t)(row - row0);
+    for (int j0 = 0; j0 < w8; j0 += TB_U) {
+      uint32_t q[TB_U], v[TB_U];
+#pragma unroll
+      for (int u = 0; u < TB_U; u++)
+        q[u] = fits && j0 + u < w ? e[(size_t)(j0 + u) * RSB_WAVE] : 0u;
+#pragma unroll
+      for (int u = 0; u < TB_U; u++) {
+        v[u] = self;  // padding: own row, weight 0
+        const uint32_t wt = q[u] >> 28;
         if (wt) {
-          int li = c - row0;
-          if (c < row0 || c >= row1) {
-            int slot = tb_find(keys, c);
-            li = slot >= 0 ? local[slot] : -1;
-          }
-          // every external column was inserted above, so li >= 0
-          if (li >= 0) v = (uint16_t)(li | (wt << 12));
+          const int c = (int)(q[u] & 0x0fffffffu);
+          // every external column was inserted above
+          const int li = c >= row0 && c < row1 ? c - row0 : local[tb_find(keys, c)];
+          v[u] = (uint32_t)li | (wt << 12);
         }
       }
-      o[e16_pos(j, lane, w8)] = v;
+      uint16_t *at = o + (size_t)(j0 >> 3) * 512;
+      const int left = w8 - j0;
+      if (left >= 8) {
+        *(uint4 *)(at + lane * 8) = make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16,
+                                               v[4] | v[5] << 16, v[6] | v[7] << 16);
+      } else {
+        if (left & 4) *(uint2 *)(at + lane * 4) = make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);
+        if (left & 2)
+          *(uint32_t *)(at + (left & 4) * 64 + lane * 2) =
+              left & 4 ? v[4] | v[5] << 16 : v[0] | v[1] << 16;
+      }
     }
   }
 }
@@ -236,41 +243,58 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_tile_fill(
 // region of the slice's size for it, the rest of the region set to the
 // row's own index) into its LDS slots, then packed 21 to a block.
 #define E12_SLOTS (3 * E12_BLK)
+#define E12_GROUPS 6  // groups of 8 that hold E12_MAXW entries
 __global__ void __launch_bounds__(RSB_BLOCK) k_tile_e12(
-    const int *__restrict__ tile, const int *__restrict__ slice_w,
-    const int64_t *__restrict__ off16, const int *__restrict__ w16,
+    const int *__restrict__ tile, const int64_t *__restrict__ off16, const int *__restrict__ w16,
     const uint16_t *__restrict__ e16, const int64_t *__restrict__ off12,
-    const int *__restrict__ w12, const int *__restrict__ c12, uint32_t *__restrict__ e12,
-    int *__restrict__ bad) {
+    const int *__restrict__ w12, const int *__restrict__ c12, uint32_t *__restrict__ e12) {
   __shared__ uint16_t lst[E12_SLOTS * RSB_BLOCK];
   uint16_t *my = lst + threadIdx.x;  // slot k at my[k * RSB_BLOCK]
   const int t = blockIdx.x, row0 = tile[3 * t + 1], row1 = tile[3 * t + 2];
   for (int row = row0 + threadIdx.x; row < row1; row += blockDim.x) {
     const int sl = row >> 6, lane = row & 63;
     const int info = w12[sl], nb = info & 0xff, tw = info >> 8;
-    if (nb > E12_MAXW / E12_BLK) continue;  // too many slots (k_w12 flagged it)
     const uint16_t *o = e16 + off16[sl];
-    const int w = slice_w[sl], w8 = w16[sl], cw = c12[sl];
-    const uint16_t self = (uint16_t)(row - row0);
-    int s0 = 0, over = 0;
+    const int w8 = w16[sl], cw = c12[sl], full = w8 >> 3;
+    const uint32_t self = (uint32_t)(row - row0);
+    // the row's entries (weight 0 past its width), two a word, whole groups
+    // at a time and all loads first
+    uint32_t ent[E12_GROUPS][4];
 #pragma unroll
-    for (int cls = 0; cls < 3; cls++) {
-      const unsigned want = 4u >> cls;
-      const int end = s0 + ((cw >> (8 * cls)) & 0xff);
-      int s = s0;
-      for (int j = 0; j < w; j++) {
-        const uint16_t e = o[e16_pos(j, lane, w8)];
-        if ((unsigned)(e >> 12) != want) continue;
-        if (s < end && s < E12_SLOTS) my[s * RSB_BLOCK] = e & 0xfffu;
-        s++;
+    for (int g = 0; g < E12_GROUPS; g++) {
+      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+      const uint16_t *at = o + (size_t)g * 512;
+      if (g < full) {
+        v = *(const uint4 *)(at + lane * 8);
+      } else if (g == full) {
+        if (w8 & 4) {
+          const uint2 x = *(const uint2 *)(at + lane * 4);
+          v.x = x.x, v.y = x.y;
+        }
+        if (w8 & 2) {
+          const uint32_t x = *(const uint32_t *)(at + (w8 & 4) * 64 + lane * 2);
+          if (w8 & 4) v.z = x;
+          else v.x = x;
+        }
       }
-      over |= s > end;
-      for (; s < end && s < E12_SLOTS; s++) my[s * RSB_BLOCK] = self;
-      s0 = end;
+      ent[g][0] = v.x, ent[g][1] = v.y, ent[g][2] = v.z, ent[g][3] = v.w;
     }
-    if (over) atomicOr(bad, 1);
-    const int upto = (nb + 1) * E12_BLK;  // the tail packs from a whole group of slots
-    for (int k = s0; k < upto && k < E12_SLOTS; k++) my[k * RSB_BLOCK] = self;
+    // each class into its region in entry order, the rest the row itself
+    const int e4 = cw & 0xff, e2 = e4 + ((cw >> 8) & 0xff), e1 = e2 + ((cw >> 16) & 0xff);
+    int s4 = 0, s2 = e4, s1 = e2;
+#pragma unroll
+    for (int g = 0; g < E12_GROUPS; g++)
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const uint32_t e = (ent[g][k >> 1] >> (16 * (k & 1))) & 0xffffu, wt = e >> 12;
+        if (wt == 0) continue;
+        const int at = wt == 4 ? s4++ : wt == 2 ? s2++ : s1++;
+        if (at < E12_SLOTS) my[at * RSB_BLOCK] = (uint16_t)(e & 0xfffu);
+      }
+    for (; s4 < e4; s4++) my[s4 * RSB_BLOCK] = (uint16_t)self;
+    for (; s2 < e2; s2++) my[s2 * RSB_BLOCK] = (uint16_t)self;
+    const int upto = min((nb + 1) * E12_BLK, E12_SLOTS);  // the tail packs whole groups of slots
+    for (; s1 < max(e1, upto) && s1 < E12_SLOTS; s1++) my[s1 * RSB_BLOCK] = (uint16_t)self;
     uint32_t *base = e12 + off12[sl];
     for (int b = 0; b < nb; b++) {
       uint32_t pw[8];
@@ -323,10 +347,16 @@ __global__ void __launch_bounds__(256) k_w12(int64_t nslices, const int64_t *__r
   const uint32_t *e = ell + slice_off[sl] + lane;
   const int w = slice_w[sl];
   int c4 = 0, c2 = 0, c1 = 0, odd = 0;
-  for (int j = 0; j < w; j++) {
-    const unsigned wt = e[(size_t)j * RSB_WAVE] >> 28;
-    c4 += wt == 4, c2 += wt == 2, c1 += wt == 1;
-    odd |= wt != 0 && wt != 1 && wt != 2 && wt != 4;
+  for (int j0 = 0; j0 < w; j0 += TB_U) {
+    uint32_t q[TB_U];
+#pragma unroll
+    for (int u = 0; u < TB_U; u++) q[u] = j0 + u < w ? e[(size_t)(j0 + u) * RSB_WAVE] : 0u;
+#pragma unroll
+    for (int u = 0; u < TB_U; u++) {
+      const unsigned wt = q[u] >> 28;
+      c4 += wt == 4, c2 += wt == 2, c1 += wt == 1;
+      odd |= wt != 0 && wt != 1 && wt != 2 && wt != 4;
+    }
   }
   for (int o = 32; o > 0; o >>= 1) {
     c4 = max(c4, __shfl_xor(c4, o));
@@ -348,96 +378,96 @@ __global__ void __launch_bounds__(256) k_w12(int64_t nslices, const int64_t *__r
 
 __global__ void k_zero_int(int *__restrict__ p) { *p = 0; }
 
-__global__ void k_all_wide(int n, int *__restrict__ nh) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) nh[i] = -1;
-}
-
-__global__ void k_nhalo64(int n, const int *__restrict__ nh, int64_t *__restrict__ o) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) o[i] = nh[i] > 0 ? nh[i] : 0;
-  if (i == n) o[i] = 0;
-}
-
 int rsb_build_tiles(rsbgpu *g) {
   const int nt = g->ntiles;
   const int64_t ns = g->nslices;
+  g->e12_ok = g->e12_state = 0;
+  g->nwide = nt ? -1 : 0;
   if (nt == 0) return 0;
   RSB_TRY(dev_alloc(g, g->d_tnhalo, (size_t)nt + 1));
   RSB_TRY(dev_alloc(g, g->d_thalo_off, (size_t)nt + 1));
   RSB_TRY(dev_alloc(g, g->d_w16, (size_t)ns + 1));
   RSB_TRY(dev_alloc(g, g->d_off16, (size_t)ns + 1));
-  int64_t *tmp = nullptr;
-  RSB_TRY(RSB_SCRATCH(tmp, sizeof(int64_t) * (std::max<int64_t>(ns, nt) + 1)));
-  k_tile_count<<<nt, RSB_BLOCK, 0, g->stream>>>(g->d_tile, g->d_slice_off, g->d_slice_w,
-                                                 g->d_ell, g->d_tnhalo);
-  RSB_LAUNCH_CHECK();
-  const char *off = getenv("PARRSB_AMD_NO_TILES");  // every tile on the global path
-  if (off && atoi(off) == 1) {
-    k_all_wide<<<nblocks(nt, 256), 256, 0, g->stream>>>(nt, g->d_tnhalo);
-    RSB_LAUNCH_CHECK();
+  // room for a tile's halo: what its window takes, and no more rows than the
+  // rest of its segment has
+  g->h_halo_off.resize((size_t)nt + 1);
+  int64_t nh = 0;
+  for (int t = 0; t < nt; t++) {
+    const int s = g->h_tile[3 * t], row0 = g->h_tile[3 * t + 1];
+    const int rows = g->h_tile[3 * t + 2] - row0;
+    const int real = std::min(rows, g->h_n[s] - (row0 - g->h_pstart[s]));
+    g->h_halo_off[t] = nh;
+    nh += std::min(TB_LOCAL - rows, g->h_n[s] - real);
   }
-  k_nhalo64<<<nblocks(nt + 1, 256), 256, 0, g->stream>>>(nt, g->d_tnhalo, tmp);
-  RSB_LAUNCH_CHECK();
-  int rc = rsb_exclusive_scan_i64(g, tmp, g->d_thalo_off, nt + 1);
-  if (rc) return rc;
+  g->h_halo_off[nt] = nh;
+  RSB_TRY(hipMemcpyAsync(g->d_thalo_off, g->h_halo_off.data(), sizeof(int64_t) * ((size_t)nt + 1),
+                         hipMemcpyHostToDevice, g->stream));
+  int64_t *tmp = nullptr;
+  RSB_TRY(RSB_SCRATCH(tmp, sizeof(int64_t) * (ns + 1)));
   k_w16<<<nblocks(ns + 1, 256), 256, 0, g->stream>>>(ns, g->d_slice_w, g->d_w16, tmp);
   RSB_LAUNCH_CHECK();
-  rc = rsb_exclusive_scan_i64(g, tmp, g->d_off16, ns + 1);
+  int rc = rsb_exclusive_scan_i64(g, tmp, g->d_off16, ns + 1);
   if (rc) return rc;
-  int64_t nh = 0, n16 = 0;
-  RSB_TRY(hipMemcpyAsync(&nh, g->d_thalo_off + nt, sizeof(int64_t), hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipMemcpyAsync(&n16, g->d_off16 + ns, sizeof(int64_t), hipMemcpyDeviceToHost,
-                         g->stream));
-  std::vector<int> nhv(nt);
-  RSB_TRY(hipMemcpyAsync(nhv.data(), g->d_tnhalo, sizeof(int) * nt, hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
-  g->nhalo_total = nh;
-  g->e16_count = n16;
-  g->nwide = 0;
-  for (int v : nhv) g->nwide += v < 0;
+  // widths are rounded up to even numbers
   RSB_TRY(dev_alloc(g, g->d_halo, (size_t)nh + 1));
-  RSB_TRY(dev_alloc(g, g->d_e16, (size_t)n16 + 8));
-  // the 12-bit form (unless PARRSB_AMD_E12=0; =2 lets the FP64 solve read
-  // it as well)
-  const char *ev = getenv("PARRSB_AMD_E12");
-  const bool want12 = !(ev && atoi(ev) == 0);
-  g->e12_ok = 0;
-  g->e12_f64 = ev && atoi(ev) == 2;
-  if (want12) {
-    RSB_TRY(dev_alloc(g, g->d_w12, (size_t)ns + 1));
-    RSB_TRY(dev_alloc(g, g->d_c12, (size_t)ns + 1));
-    RSB_TRY(dev_alloc(g, g->d_off12, (size_t)ns + 1));
-    RSB_TRY(dev_alloc(g, g->d_e12_bad, 1));
-    k_zero_int<<<1, 1, 0, g->stream>>>(g->d_e12_bad);
-    k_w12<<<nblocks((ns + 1) * RSB_WAVE, 256), 256, 0, g->stream>>>(
-        ns, g->d_slice_off, g->d_slice_w, g->d_ell, g->d_c12, g->d_w12, tmp, g->d_e12_bad);
-    RSB_LAUNCH_CHECK();
-    rc = rsb_exclusive_scan_i64(g, tmp, g->d_off12, ns + 1);
-    if (rc) return rc;
-    int64_t n12 = 0;
-    RSB_TRY(hipMemcpyAsync(&n12, g->d_off12 + ns, sizeof(int64_t), hipMemcpyDeviceToHost,
-                           g->stream));
-    RSB_TRY(hipStreamSynchronize(g->stream));
-    RSB_TRY(dev_alloc(g, g->d_e12, (size_t)n12 + 8));
-  }
-  k_tile_fill<<<nt, RSB_BLOCK, 0, g->stream>>>(g->d_tile, g->d_slice_off, g->d_slice_w, g->d_ell,
-                                                g->d_tnhalo, g->d_thalo_off, g->d_off16,
-                                                g->d_w16, g->d_halo, g->d_e16);
+  RSB_TRY(dev_alloc(g, g->d_e16, (size_t)(g->lnnz_pad + ns * RSB_WAVE) + 8));
+  const char *off = getenv("PARRSB_AMD_NO_TILES");  // every tile on the global path
+  k_tile_build<<<nt, RSB_BLOCK, 0, g->stream>>>(g->d_tile, g->d_slice_off, g->d_slice_w, g->d_ell,
+                                                 off && atoi(off) == 1, g->d_thalo_off,
+                                                 g->d_off16, g->d_w16, g->d_tnhalo, g->d_halo,
+                                                 g->d_e16);
   RSB_LAUNCH_CHECK();
-  if (want12) {
-    k_tile_e12<<<nt, RSB_BLOCK, 0, g->stream>>>(g->d_tile, g->d_slice_w, g->d_off16, g->d_w16,
-                                                 g->d_e16, g->d_off12, g->d_w12, g->d_c12,
-                                                 g->d_e12, g->d_e12_bad);
-    RSB_LAUNCH_CHECK();
-    int bad = 1;
-    RSB_TRY(hipMemcpyAsync(&bad, g->d_e12_bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-    RSB_TRY(hipStreamSynchronize(g->stream));
-    g->e12_ok = bad == 0;
-  }
+  // the 12-bit form is built where a solve asks for it (rsb_level_e12),
+  // unless PARRSB_AMD_E12=0; =2 lets the FP64 solve read it as well
+  const char *ev = getenv("PARRSB_AMD_E12");
+  g->e12_state = ev && atoi(ev) == 0 ? 0 : 1;
+  g->e12_f64 = ev && atoi(ev) == 2;
+  return 0;
+}
+
+// The level's 12-bit form, built on the first call after its tiles (a level
+// solved in FP64 reads the 16-bit entries and never needs it): sets e12_ok.
+int rsb_level_e12(rsbgpu *g) {
+  if (g->e12_state != 1) return 0;
+  g->e12_state = 2;
+  const int nt = g->ntiles;
+  const int64_t ns = g->nslices;
+  RSB_TRY(dev_alloc(g, g->d_w12, (size_t)ns + 1));
+  RSB_TRY(dev_alloc(g, g->d_c12, (size_t)ns + 1));
+  RSB_TRY(dev_alloc(g, g->d_off12, (size_t)ns + 1));
+  RSB_TRY(dev_alloc(g, g->d_e12_bad, 1));
+  int64_t *tmp = nullptr;
+  RSB_TRY(RSB_SCRATCH(tmp, sizeof(int64_t) * (ns + 1)));
+  k_zero_int<<<1, 1, 0, g->stream>>>(g->d_e12_bad);
+  k_w12<<<nblocks((ns + 1) * RSB_WAVE, 256), 256, 0, g->stream>>>(
+      ns, g->d_slice_off, g->d_slice_w, g->d_ell, g->d_c12, g->d_w12, tmp, g->d_e12_bad);
+  RSB_LAUNCH_CHECK();
+  int rc = rsb_exclusive_scan_i64(g, tmp, g->d_off12, ns + 1);
+  if (rc) return rc;
+  int64_t n12 = 0;
+  int bad = 1;
+  RSB_TRY(hipMemcpyAsync(&n12, g->d_off12 + ns, sizeof(int64_t), hipMemcpyDeviceToHost,
+                         g->stream));
+  RSB_TRY(hipMemcpyAsync(&bad, g->d_e12_bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
   RSB_TRY(hipStreamSynchronize(g->stream));
+  if (bad) return 0;  // a weight other than 1, 2 or 4, or a slice of too many slots
+  RSB_TRY(dev_alloc(g, g->d_e12, (size_t)n12 + 8));
+  k_tile_e12<<<nt, RSB_BLOCK, 0, g->stream>>>(g->d_tile, g->d_off16, g->d_w16, g->d_e16,
+                                               g->d_off12, g->d_w12, g->d_c12, g->d_e12);
+  RSB_LAUNCH_CHECK();
+  g->e12_ok = 1;
+  return 0;
+}
+
+// Tiles on the global path (nhalo < 0), counted when asked for.
+static int level_nwide(rsbgpu *g) {
+  if (g->nwide >= 0) return 0;
+  std::vector<int> nh((size_t)g->ntiles);
+  RSB_TRY(hipMemcpyAsync(nh.data(), g->d_tnhalo, sizeof(int) * nh.size(), hipMemcpyDeviceToHost,
+                         g->stream));
+  RSB_TRY(hipStreamSynchronize(g->stream));
+  g->nwide = 0;
+  for (int v : nh) g->nwide += v < 0;
   return 0;
 }
 
@@ -645,9 +675,9 @@ int rsb_build_vtiles(rsbgpu *g) {
   g->vt_ok = 0;
   // opt-in: PARRSB_AMD_VTILES=1 (FP32 Lanczos only)
   const char *on = getenv("PARRSB_AMD_VTILES");
-  if (nt == 0 || !g->d_vtx || (g->nv != 4 && g->nv != 8) || g->nwide > 0 || !on ||
-      atoi(on) != 1)
-    return 0;
+  if (nt == 0 || !g->d_vtx || (g->nv != 4 && g->nv != 8) || !on || atoi(on) != 1) return 0;
+  if (int rc = level_nwide(g)) return rc;
+  if (g->nwide > 0) return 0;
   RSB_TRY(dev_alloc(g, g->d_vt_n, (size_t)nt + 1));
   RSB_TRY(dev_alloc(g, g->d_vt_loff, (size_t)nt + 1));
   int64_t *nl = nullptr;
@@ -673,6 +703,8 @@ int rsb_build_vtiles(rsbgpu *g) {
 
 extern "C" int rsbgpu_level_form(rsbgpu *g, int *wide_tiles, int *vertex_tiles) {
   RSB_TRY(hipSetDevice(g->device));
+  const int rc = level_nwide(g);
+  if (rc) return rc;
   *wide_tiles = g->nwide;
   *vertex_tiles = 0;
   if (!g->vt_ok || g->ntiles == 0) return 0;
@@ -686,4 +718,7 @@ extern "C" int rsbgpu_level_form(rsbgpu *g, int *wide_tiles, int *vertex_tiles) 
 
 // 1 if the level's tiles carry the 12-bit form (every weight 1, 2 or 4),
 // else 0
-extern "C" int rsbgpu_level_e12(rsbgpu *g) { return g->e12_ok; }
+extern "C" int rsbgpu_level_e12(rsbgpu *g) {
+  if (hipSetDevice(g->device) != hipSuccess || rsb_level_e12(g)) return 0;
+  return g->e12_ok;
+}
