@@ -3,6 +3,9 @@
 #include <algorithm>
 #include <vector>
 
+#include <cstring>
+#include <rocprim/rocprim.hpp>
+
 #include "state.hpp"
 
 // ---------------------------------------------------------------------------
@@ -37,6 +40,40 @@ __global__ void k_permute(const int *__restrict__ perm, const int *__restrict__ 
   fied2[j] = fied[i];
 }
 
+// Segments of up to T * 8 elements: a workgroup sorts one in LDS (the same
+// stable order).  The device-wide sort of 64-bit values makes eight passes
+// over all elements and more for the segments, ~25 launches.
+#define FSORT_IPT 8
+#define FSORT_MAX (1024 * FSORT_IPT)
+template <int T>
+__global__ void __launch_bounds__(T) k_fsort(const double *__restrict__ fied,
+                                             const int *__restrict__ order,
+                                             const int *__restrict__ seg, int nseg,
+                                             int *__restrict__ order2,
+                                             double *__restrict__ fied2) {
+  typedef rocprim::block_radix_sort<uint64_t, T, FSORT_IPT, int> sorter;
+  __shared__ typename sorter::storage_type tmp;
+  const int s = blockIdx.x, cs = seg[s], n = seg[nseg + s];
+  if (seg[2 * nseg + s] <= 1) {
+    for (int i = threadIdx.x; i < n; i += T) order2[cs + i] = order[cs + i], fied2[cs + i] = fied[cs + i];
+    return;
+  }
+  uint64_t key[FSORT_IPT];
+  int val[FSORT_IPT];
+#pragma unroll
+  for (int q = 0; q < FSORT_IPT; q++) {
+    const int i = (int)threadIdx.x * FSORT_IPT + q;
+    key[q] = i < n ? dkey(fied[cs + i]) : ~0ull;
+    val[q] = i;
+  }
+  sorter().sort(key, val, tmp, 0, 64);
+#pragma unroll
+  for (int q = 0; q < FSORT_IPT; q++) {
+    const int i = (int)threadIdx.x * FSORT_IPT + q;
+    if (i < n) order2[cs + i] = order[cs + val[q]], fied2[cs + i] = fied[cs + val[q]];
+  }
+}
+
 extern "C" int rsbgpu_fiedler_sort(rsbgpu *g) {
   RSB_TRY(hipSetDevice(g->device));
   const int nel = g->nel;
@@ -45,6 +82,24 @@ extern "C" int rsbgpu_fiedler_sort(rsbgpu *g) {
   uint64_t *key = nullptr;
   int *perm = nullptr;
   double *fied2 = nullptr;
+  int nmax = 0;
+  for (int s = 0; s < g->nseg; s++)
+    if (g->h_p[s] > 1) nmax = std::max(nmax, g->h_n[s]);
+  if (nmax <= FSORT_MAX) {
+    RSB_TRY(RSB_SCRATCH(fied2, sizeof(double) * (nel + 1)));
+    if (nmax <= 256 * FSORT_IPT)
+      k_fsort<256><<<g->nseg, 256, 0, g->stream>>>(g->d_fied, g->d_order, g->d_seg, g->nseg,
+                                                   g->d_order2, fied2);
+    else
+      k_fsort<1024><<<g->nseg, 1024, 0, g->stream>>>(g->d_fied, g->d_order, g->d_seg, g->nseg,
+                                                     g->d_order2, fied2);
+    RSB_LAUNCH_CHECK();
+    std::swap(g->d_order, g->d_order2);
+    RSB_TRY(hipMemcpyAsync(g->d_fied, fied2, sizeof(double) * nel, hipMemcpyDeviceToDevice,
+                           g->stream));
+    rsb_phase_end(g, PH_SORT);
+    return 0;
+  }
   RSB_TRY(RSB_SCRATCH(key, sizeof(uint64_t) * (nel + 1)));
   RSB_TRY(RSB_SCRATCH(perm, sizeof(int) * (nel + 1)));
   RSB_TRY(RSB_SCRATCH(fied2, sizeof(double) * (nel + 1)));
@@ -113,11 +168,6 @@ __device__ inline void uf_union(int *par, int u, int v) {
     ru = uf_rep(par, old);
     rv = uf_rep(par, rv);
   }
-}
-
-__global__ void k_uf_init(int64_t mpad, int *__restrict__ par) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < mpad) par[i] = (int)i;
 }
 
 // Half of every row (-1 for padding rows), so the edge pass gathers one
@@ -540,25 +590,96 @@ __global__ void k_q_check(int nel, const int *__restrict__ part, int nparts,
   if (e < nel && (part[e] < 0 || part[e] >= nparts)) atomicOr(bad, 1);
 }
 
-__global__ void k_q_edges(int nel, const int64_t *__restrict__ rowptr,
-                          const uint32_t *__restrict__ adj, const int *__restrict__ part,
-                          unsigned long long *__restrict__ cut, int *__restrict__ par,
-                          int *__restrict__ size) {
-  int e = blockIdx.x * blockDim.x + threadIdx.x;
+// Cut edges, part sizes and the components' forest of the elements' own
+// graph, in two passes over its rows: edges within a workgroup's Q_TILE
+// consecutive elements are united in LDS, the others (k_q_cross) in memory,
+// where an edge whose ends already reach one root by plain reads is left
+// alone: such a read may be old, but two elements that once had a common
+// ancestor stay connected.  Sums leave a workgroup as one atomic each (one a
+// wave, on one address, was most of this report's time).
+#define Q_TILE 1024
+__global__ void __launch_bounds__(256) k_q_edges(int nel, const int64_t *__restrict__ rowptr,
+                                                 const uint32_t *__restrict__ adj,
+                                                 const int *__restrict__ part,
+                                                 unsigned long long *__restrict__ cut,
+                                                 int *__restrict__ par, int *__restrict__ size) {
+  __shared__ int lp[Q_TILE], lq[Q_TILE];
+  __shared__ unsigned long long red[2][256 / RSB_WAVE];
+  const int e0 = blockIdx.x * Q_TILE, n = min(Q_TILE, nel - e0), lane = threadIdx.x & (RSB_WAVE - 1);
+  for (int i = threadIdx.x; i < n; i += 256) lp[i] = i, lq[i] = part[e0 + i];
+  __syncthreads();
   unsigned long long w = 0, c = 0;
-  if (e < nel) {
-    int pe = part[e];
-    atomicAdd(&size[pe], 1);
-    for (int64_t k = rowptr[e]; k < rowptr[e + 1]; k++) {
-      int j = (int)(adj[k] & 0x0fffffffu);
-      if (j <= e) continue;
-      if (part[j] != pe) w += adj[k] >> 28, c++;
-      else uf_union(par, j, e);
+  for (int i = threadIdx.x; i < Q_TILE; i += 256) {
+    const bool has = i < n;
+    const int e = e0 + i, pe = has ? lq[i] : -1;
+    if (has) {
+      const int64_t k1 = rowptr[e + 1];
+      for (int64_t k0 = rowptr[e]; k0 < k1; k0 += 8) {
+        uint32_t a[8];
+        int pj[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) a[u] = k0 + u < k1 ? adj[k0 + u] : (uint32_t)e;
+#pragma unroll
+        for (int u = 0; u < 8; u++) pj[u] = part[a[u] & 0x0fffffffu];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          const int j = (int)(a[u] & 0x0fffffffu);
+          if (j <= e) continue;
+          if (pj[u] != pe) w += a[u] >> 28, c++;
+          else if (j < e0 + n) luf_union(lp, i, j - e0);
+        }
+      }
+    }
+    // part sizes: one atomic per part present in the wave
+    unsigned long long left = __ballot(has);
+    while (left) {
+      const int first = __ffsll((long long)left) - 1;
+      const int q = __shfl(pe, first, RSB_WAVE);
+      const unsigned long long same = __ballot(has && pe == q);
+      if (lane == first) atomicAdd(&size[q], __popcll(same));
+      left &= ~same;
     }
   }
   w = wave_sum(w);
   c = wave_sum(c);
-  if ((threadIdx.x & 63) == 0) atomicAdd(&cut[0], w), atomicAdd(&cut[1], c);
+  if (lane == 0) red[0][threadIdx.x / RSB_WAVE] = w, red[1][threadIdx.x / RSB_WAVE] = c;
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    unsigned long long v = 0;
+    for (int q = 0; q < 256 / RSB_WAVE; q++) v += red[threadIdx.x][q];
+    if (v) atomicAdd(&cut[threadIdx.x], v);
+  }
+  for (int i = threadIdx.x; i < n; i += 256) par[e0 + i] = e0 + luf_rep(lp, i);
+}
+
+__device__ inline int q_root(const int *par, int x) {
+  int p = par[x];
+  while (p != x) x = p, p = par[x];
+  return x;
+}
+__global__ void __launch_bounds__(256) k_q_cross(int nel, const int64_t *__restrict__ rowptr,
+                                                 const uint32_t *__restrict__ adj,
+                                                 const int *__restrict__ part, int *par) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= nel) return;
+  const int end = (e / Q_TILE + 1) * Q_TILE, pe = part[e];
+  const int64_t k1 = rowptr[e + 1];
+  for (int64_t k0 = rowptr[e]; k0 < k1; k0 += 8) {
+    uint32_t a[8];
+    int pj[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) a[u] = k0 + u < k1 ? adj[k0 + u] : (uint32_t)e;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int j = (int)(a[u] & 0x0fffffffu);
+      pj[u] = j >= end ? part[j] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int j = (int)(a[u] & 0x0fffffffu);
+      if (pj[u] == pe && q_root(par, j) != q_root(par, e)) uf_union(par, j, e);
+    }
+  }
 }
 
 __global__ void k_q_roots(int nel, const int *__restrict__ part, const int *__restrict__ par,
@@ -567,26 +688,37 @@ __global__ void k_q_roots(int nel, const int *__restrict__ part, const int *__re
   if (e < nel && par[e] == e) atomicAdd(&ncomp[part[e]], 1);
 }
 
+// Keys vertex << shift | part.
+template <typename K>
 __global__ void k_q_vkeys(const long long *__restrict__ vtx, const int *__restrict__ part,
-                          int64_t ns, int nv, uint64_t *__restrict__ key, int *__restrict__ val) {
+                          int64_t ns, int nv, int shift, K *__restrict__ key) {
   int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= ns) return;
-  key[s] = ((uint64_t)vtx[s] << 24) | (uint32_t)part[s / nv];
-  val[s] = 0;
+  key[s] = (K)((K)vtx[s] << shift) | (K)part[s / nv];
 }
 
-__global__ void k_q_volume(const uint64_t *__restrict__ key, int64_t ns,
-                           unsigned long long *__restrict__ vol) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+template <typename K>
+__global__ void __launch_bounds__(256) k_q_volume(const K *__restrict__ key, int64_t ns, int shift,
+                                                  unsigned long long *__restrict__ vol) {
+  __shared__ unsigned long long red[256 / RSB_WAVE];
   unsigned long long v = 0;
-  if (i < ns && (i == 0 || (key[i] >> 24) != (key[i - 1] >> 24)) && (key[i] >> 24) != 0) {
-    unsigned long long k = 0;
-    for (int64_t j = i; j < ns && (key[j] >> 24) == (key[i] >> 24); j++)
-      if (j == i || key[j] != key[j - 1]) k++;
-    v = k * (k - 1);
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < ns; i += (int64_t)gridDim.x * 256) {
+    const K a = key[i], id = a >> shift;
+    if (id == 0 || (i > 0 && (key[i - 1] >> shift) == id)) continue;
+    unsigned long long k = 1;
+    K prev = a;
+    for (int64_t j = i + 1; j < ns; j++) {
+      const K b = key[j];
+      if ((b >> shift) != id) break;
+      k += b != prev;
+      prev = b;
+    }
+    v += k * (k - 1);
   }
   v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) atomicAdd(vol, v);
+  if ((threadIdx.x & (RSB_WAVE - 1)) == 0) red[threadIdx.x / RSB_WAVE] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(vol, red[0] + red[1] + red[2] + red[3]);
 }
 
 extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t *out) {
@@ -615,21 +747,33 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
   ncomp = size + nparts;
   RSB_TRY(hipMemsetAsync(acc, 0, sizeof(unsigned long long) * 4, g->stream));
   RSB_TRY(hipMemsetAsync(size, 0, sizeof(int) * nparts * 2, g->stream));
-  k_uf_init<<<nblocks(nel, 256), 256, 0, g->stream>>>(nel, par);
-  k_q_edges<<<nblocks(nel, 256), 256, 0, g->stream>>>(nel, g->d_growptr, g->d_gadj, d_part, acc,
-                                                      par, size);
+  k_q_edges<<<nblocks(nel, Q_TILE), 256, 0, g->stream>>>(nel, g->d_growptr, g->d_gadj, d_part, acc,
+                                                         par, size);
+  k_q_cross<<<nblocks(nel, 256), 256, 0, g->stream>>>(nel, g->d_growptr, g->d_gadj, d_part, par);
   k_q_roots<<<nblocks(nel, 256), 256, 0, g->stream>>>(nel, d_part, par, ncomp);
   RSB_LAUNCH_CHECK();
   int64_t ns = (int64_t)nel * g->nv;
-  uint64_t *key = nullptr;
-  int *val = nullptr;
+  uint64_t *key = nullptr, *sorted = nullptr;
   RSB_TRY(rsb_dev_malloc((void **)&key, sizeof(uint64_t) * ns));
-  RSB_TRY(rsb_dev_malloc((void **)&val, sizeof(int) * ns));
-  k_q_vkeys<<<nblocks(ns, 256), 256, 0, g->stream>>>(g->d_vtx, d_part, ns, g->nv, key, val);
-  RSB_LAUNCH_CHECK();
-  int rc = rsb_sort_pairs_u64(g, key, val, ns, 0, 64);
-  if (rc) return rc;
-  k_q_volume<<<nblocks(ns, 256), 256, 0, g->stream>>>(key, ns, acc + 2);
+  RSB_TRY(rsb_dev_malloc((void **)&sorted, sizeof(uint64_t) * ns));
+  // as few key bits as the ids and parts take, in 32 bits if they fit
+  int vbits = 1, pbits = 1;
+  while (vbits < 64 && (g->vmax >> vbits) != 0) vbits++;
+  while ((1ll << pbits) < nparts) pbits++;
+  const unsigned vb = (unsigned)std::min<int64_t>(nblocks(ns, 256), 2048);
+  int rc;
+  if (vbits + pbits <= 32) {
+    uint32_t *k4 = (uint32_t *)key, *s4 = (uint32_t *)sorted;
+    k_q_vkeys<<<nblocks(ns, 256), 256, 0, g->stream>>>(g->d_vtx, d_part, ns, g->nv, pbits, k4);
+    RSB_LAUNCH_CHECK();
+    if ((rc = rsb_sort_keys_u32(g, k4, s4, ns, vbits + pbits))) return rc;
+    k_q_volume<<<vb, 256, 0, g->stream>>>(s4, ns, pbits, acc + 2);
+  } else {
+    k_q_vkeys<<<nblocks(ns, 256), 256, 0, g->stream>>>(g->d_vtx, d_part, ns, g->nv, pbits, key);
+    RSB_LAUNCH_CHECK();
+    if ((rc = rsb_sort_keys_u64(g, key, sorted, ns, std::min(64, vbits + pbits)))) return rc;
+    k_q_volume<<<vb, 256, 0, g->stream>>>(sorted, ns, pbits, acc + 2);
+  }
   RSB_LAUNCH_CHECK();
   std::vector<int> hs(2 * (size_t)nparts);
   unsigned long long ha[4];
@@ -648,6 +792,6 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
   out[0] = (int64_t)ha[0], out[1] = (int64_t)ha[1], out[2] = mx, out[3] = mn, out[4] = tot;
   out[5] = cmx, out[6] = (int64_t)ha[2], out[7] = empty;
   rsb_dev_release(acc), rsb_dev_release(par), rsb_dev_release(size), rsb_dev_release(key),
-      rsb_dev_release(val);
+      rsb_dev_release(sorted);
   return 0;
 }

@@ -87,6 +87,26 @@ int rsb_sort_vals_u32(rsbgpu *g, const uint32_t *keys, const int *vals, int *out
   return sort_into(g, keys, (uint32_t *)g->d_k1, vals, out, n, bb, eb);
 }
 
+// Keys alone, into another array.
+template <typename K>
+static int sort_keys(rsbgpu *g, const K *keys, K *out, int64_t n, int eb) {
+  size_t bytes = 0;
+  RSB_TRY(rocprim::radix_sort_keys<sort_cfg>(nullptr, bytes, keys, out, (size_t)n, 0, eb,
+                                             g->stream));
+  int rc = ensure_tmp(g, bytes);
+  if (rc) return rc;
+  bytes = g->sort_tmp_bytes;
+  RSB_TRY(rocprim::radix_sort_keys<sort_cfg>(g->d_sort_tmp, bytes, keys, out, (size_t)n, 0, eb,
+                                             g->stream));
+  return 0;
+}
+int rsb_sort_keys_u32(rsbgpu *g, const uint32_t *keys, uint32_t *out, int64_t n, int eb) {
+  return sort_keys(g, keys, out, n, eb);
+}
+int rsb_sort_keys_u64(rsbgpu *g, const uint64_t *keys, uint64_t *out, int64_t n, int eb) {
+  return sort_keys(g, keys, out, n, eb);
+}
+
 int rsb_exclusive_scan_i64(rsbgpu *g, const int64_t *in, int64_t *out, int64_t n) {
   if (n <= 0) return 0;
   size_t bytes = 0;
