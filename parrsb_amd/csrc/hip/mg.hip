@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_fin(mg_args a, int op, int gat
     MSC(s, MS_RR) = tot[1];
     MSC(s, MS_RTOL) = tot[1] * a.tol * a.tol;
     MSC(s, MS_MEAN) = tot[0] / n;
-    MST(s, MI_PCG) = 1, MST(s, MI_IT) = 0;
+    MST(s, MI_PCG) = 1, MST(s, MI_IT) = 0, MST(s, MI_NC) = 0;
     break;
   }
   case FIN_RZ1: MSC(s, MS_RZ1) = tot[0]; break;
@@ -246,6 +246,7 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_fin(mg_args a, int op, int gat
     const double pw = tot[0];
     MSC(s, MS_ALPHA) = MSC(s, MS_RZ1) / pw;
     MSC(s, MS_PWINV) = 1.0 / sqrt(pw);
+    MST(s, MI_IT) = MST(s, MI_NC);
     break;
   }
   case FIN_CONV: {  // tot: r.r after the update of iteration i
@@ -265,6 +266,7 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_fin(mg_args a, int op, int gat
     const double rzt = MSC(s, MS_RZ1);
     MSC(s, MS_RZ1) = tot[0];
     MSC(s, MS_BETA) = tot[1] / rzt;
+    MST(s, MI_NC) = MST(s, MI_IT) + 1;
     break;
   }
   case FIN_PASSEND: {  // tot: sum of the new start vector (after ortho of y)
@@ -287,22 +289,22 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_fin(mg_args a, int op, int gat
 }
 
 // Totals of the re-orthogonalisation dots W[j].p (j <= i) into the
-// per-segment coefficient array read by k_mg_pcorr; the iteration ends here.
+// per-segment coefficient array read by k_mg_pcorr.  One workgroup per
+// segment and four dots (blockIdx.y): up to 60 dots one after another in one
+// workgroup are 15 rounds of loads and barriers.  The iteration count moves
+// on at the next FIN_ALPHA, when nobody reads it.
 __global__ void __launch_bounds__(RSB_BLOCK) k_mg_coef(mg_args a, double *coef) {
   __shared__ double red[(RSB_BLOCK / RSB_WAVE) * 4];
-  const int s = blockIdx.x;
+  const int s = blockIdx.x, k0 = 4 * (int)blockIdx.y;
   if (!mg_gate(a, s, GATE_PCG)) return;
+  const int nc = MST(s, MI_NC);
+  if (k0 >= nc) return;
   const int first = a.seg_tiles[2 * s], count = a.seg_tiles[2 * s + 1];
-  const int nc = MST(s, MI_IT) + 1;
-  for (int k0 = 0; k0 < nc; k0 += 4) {
-    double tot[4];
-    const int ns = min(4, nc - k0);
-    seg_totals(a, first, count, k0, ns, tot, red);
-    if (threadIdx.x == 0)
-      for (int k = 0; k < ns; k++) coef[(size_t)s * MG_NP + k0 + k] = tot[k];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) MST(s, MI_NC) = nc, MST(s, MI_IT) = nc;
+  double tot[4];
+  const int ns = min(4, nc - k0);
+  seg_totals(a, first, count, k0, ns, tot, red);
+  if (threadIdx.x == 0)
+    for (int k = 0; k < ns; k++) coef[(size_t)s * MG_NP + k0 + k] = tot[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -398,11 +400,13 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_pass1(mg_args a, const double 
   mg_publish<1>(a, t, acc);
 }
 
-// w = L p; partial p.w
+// w = L p; partial p.w.  The first workgroup clears the count of running
+// segments that this iteration's stop test forms two launches later.
 __global__ void __launch_bounds__(RSB_BLOCK) k_mg_apply(mg_args a, int gate, mg_sell L,
                                                        const double *p, double *w) {
   __shared__ double xl[MG_TB_LOCAL];
   mg_tile t;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && gate == GATE_PCG) *a.active = 0;
   if (!mg_tile_of(a, gate, t)) return;
   double acc[1] = {0.0};
   if (mg_stage(L, t, p, xl)) {
@@ -422,11 +426,15 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_apply(mg_args a, int gate, mg_
   mg_publish<1>(a, t, acc);
 }
 
-// W[i] = pwinv w, P[i] = pwinv p, x += alpha p, r -= alpha w; partial r.r
+// W[i] = pwinv w, P[i] = pwinv p, x += alpha p, r -= alpha w; partial r.r.
+// The rows' residuals are in registers here, so the first Jacobi step of the
+// V-cycle that a continuing segment runs next (s = sigma r / D, u = s) is
+// formed too instead of in a launch of its own.
 __global__ void __launch_bounds__(RSB_BLOCK) k_mg_update(mg_args a, int64_t mpad,
                                                         const double *p, const double *w,
                                                         double *x, double *r, double *Wb,
-                                                        double *Pb) {
+                                                        double *Pb, const double *diag,
+                                                        double sigma, double *sv, double *u) {
   mg_tile t;
   if (!mg_tile_of(a, GATE_PCG, t)) return;
   const int i = MST(t.s, MI_IT);
@@ -440,6 +448,9 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_update(mg_args a, int64_t mpad
     const double rv = r[row] - alpha * wv;
     r[row] = rv;
     acc[0] += rv * rv;
+    const double d = diag[row];
+    const double s = d != 0.0 ? sigma * rv / d : 0.0;
+    sv[row] = s, u[row] = s;
   }
   mg_publish<1>(a, t, acc);
 }
@@ -460,28 +471,45 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_zdots(mg_args a, const double 
   mg_publish<2>(a, t, acc);
 }
 
-// p = z + beta p; partials W[j].p for j <= i
+// p = z + beta p; partials W[j].p for j <= i.  Bound by the read of the i + 1
+// earlier vectors; eight of them are summed per pass of the workgroup, so
+// their loads overlap and the two barriers of a block sum are paid once for
+// eight.
 __global__ void __launch_bounds__(RSB_BLOCK) k_mg_pnew(mg_args a, int64_t mpad, const double *z,
                                                       double *p, const double *Wb) {
   mg_tile t;
   if (!mg_tile_of(a, GATE_PCG, t)) return;
   const double beta = MSC(t.s, MS_BETA);
   const int i = MST(t.s, MI_IT);
-  double pv[RSB_TILE / RSB_BLOCK];
-  int k = 0;
-  MG_ROWS(t, row) {
-    const double v = z[row] + beta * p[row];
-    p[row] = v;
-    pv[k++] = v;
+  constexpr int NR = RSB_TILE / RSB_BLOCK, NB = 8;
+  double pv[NR];
+#pragma unroll
+  for (int k = 0; k < NR; k++) {
+    const int row = t.row0 + (int)threadIdx.x + k * RSB_BLOCK;
+    const bool on = row < t.row1 && row - t.pstart < t.n;
+    pv[k] = on ? fma(beta, p[row], z[row]) : 0.0;
+    if (on) p[row] = pv[k];
   }
-  __shared__ double red[(RSB_BLOCK / RSB_WAVE) * 4];
-  for (int j = 0; j <= i; j++) {
-    double acc[1] = {0.0};
-    int q = 0;
-    MG_ROWS(t, row) acc[0] += Wb[(size_t)j * mpad + row] * pv[q++];
-    block_sum<1>(acc, red);
-    if (threadIdx.x == 0) a.partial[(size_t)j * a.ntiles + t.ti] = acc[0];
-    __syncthreads();
+  __shared__ double red[(RSB_BLOCK / RSB_WAVE) * NB];
+  for (int j0 = 0; j0 <= i; j0 += NB) {
+    double acc[NB] = {};
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      const int row = t.row0 + (int)threadIdx.x + k * RSB_BLOCK;
+      const bool on = row < t.row1 && row - t.pstart < t.n;
+      double x[NB];
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+        x[b] = on && j0 + b <= i ? Wb[(size_t)(j0 + b) * mpad + row] : 0.0;
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+        if (on) acc[b] = fma(x[b], pv[k], acc[b]);
+    }
+    block_sum<NB>(acc, red);
+    if (threadIdx.x == 0)
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+        if (j0 + b <= i) a.partial[(size_t)(j0 + b) * a.ntiles + t.ti] = acc[b];
   }
 }
 
@@ -494,19 +522,19 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_pcorr(mg_args a, int64_t mpad,
   const double *c = coef + (size_t)t.s * MG_NP;
   MG_ROWS(t, row) {
     double acc = 0.0;
-    for (int j = 0; j < nc; j++) acc += c[j] * Pb[(size_t)j * mpad + row];
+    for (int j0 = 0; j0 < nc; j0 += 8) {
+      double x[8];
+#pragma unroll
+      for (int b = 0; b < 8; b++) x[b] = j0 + b < nc ? Pb[(size_t)(j0 + b) * mpad + row] : 0.0;
+#pragma unroll
+      for (int b = 0; b < 8; b++)
+        if (j0 + b < nc) acc = fma(c[j0 + b], x[b], acc);
+    }
     p[row] -= acc;
   }
 }
 
 __global__ void k_mg_zero(int *c) { *c = 0; }
-
-// z0 = z (the previous preconditioned residual)
-__global__ void __launch_bounds__(RSB_BLOCK) k_mg_copy(mg_args a, const double *z, double *z0) {
-  mg_tile t;
-  if (!mg_tile_of(a, GATE_PCG, t)) return;
-  MG_ROWS(t, row) z0[row] = z[row];
-}
 
 // fiedler[cstart + i] = x * ni (fiedler.c:606-616)
 __global__ void __launch_bounds__(RSB_BLOCK) k_mg_out(mg_args a, const double *x, double *fied) {
@@ -784,21 +812,14 @@ __global__ void __launch_bounds__(RSB_WAVE) k_gjac_test(int n, const double *Ain
 // ---------------------------------------------------------------------------
 // V-cycle.  Weighted Jacobi step k (multigrid.c:249-268): s = sigma_k r / D
 // (0 where D is 0), u = s on the first step and u += s after, r -= D s - A s.
-// The step's s is formed once per row by the kernel before (k_mg_jac* for
-// the first, the residual kernel of step k - 1 for the others), so the
-// residual kernel reads its neighbours' s and writes the next step's s
-// into the other buffer.
-
-__global__ void __launch_bounds__(RSB_BLOCK) k_mg_jac0(mg_args a, mg_sell L, double sigma,
-                                                      const double *r, double *sv, double *u) {
-  mg_tile t;
-  if (!mg_tile_of(a, GATE_PCG, t)) return;
-  MG_ROWS(t, row) {
-    const double d = L.diag[row];
-    const double v = d != 0.0 ? sigma * r[row] / d : 0.0;
-    sv[row] = v, u[row] = v;
-  }
-}
+// The step's s is formed once per row by the kernel before (k_mg_update or
+// k_mg_down for the first, the residual kernel of step k - 1 for the
+// others), so the residual kernel reads its neighbours' s and writes the
+// next step's s into the other buffer.
+//
+// The levels from the first one whose largest segment has at most
+// MG_LOW_ROWS rows down to the coarsest run in one launch (k_mg_low), those
+// above in one launch per step.
 
 // rout = rin - (D s - A s); then, if sigma_next > 0, the next step's s
 __global__ void __launch_bounds__(RSB_BLOCK) k_mg_res0(mg_args a, mg_sell L, const double *rin,
@@ -830,15 +851,6 @@ struct mg_csr {
   const double *diag;
   const uint32_t *spk;  // if set: packed entries col | weight << 24 (sci, sw unused)
 };
-
-__global__ void __launch_bounds__(RSB_BLOCK) k_mg_jac_c(mg_args a, mg_csr M, double sigma,
-                                                       const double *r, double *sv, double *u) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M.m || !MST(M.rseg[i], MI_PCG)) return;
-  const double d = M.diag[i];
-  const double v = d != 0.0 ? sigma * r[i] / d : 0.0;
-  sv[i] = v, u[i] = v;
-}
 
 __global__ void __launch_bounds__(RSB_BLOCK) k_mg_res_c(mg_args a, mg_csr M, double *r,
                                                        const double *sv, double sigma_next,
@@ -885,14 +897,14 @@ struct mg_lvl {
   const int *off, *n;
 };
 
-// restriction: coarse row c = sum of its children (multigrid.c:271-272)
-__global__ void __launch_bounds__(RSB_BLOCK) k_mg_restrict(mg_args a, int64_t mc,
-                                                          const int *rseg_c, mg_lvl F,
-                                                          mg_lvl Cl, int factor,
-                                                          const double *rf, double *rc) {
+// restriction (coarse row c = sum of its children, multigrid.c:271-272) and
+// the level's first Jacobi step
+__global__ void __launch_bounds__(RSB_BLOCK) k_mg_down(mg_args a, mg_csr M, mg_lvl F, mg_lvl Cl,
+                                                      int factor, const double *rf, double sigma,
+                                                      double *rc, double *sv, double *u) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= mc) return;
-  const int s = rseg_c[c];
+  if (c >= M.m) return;
+  const int s = M.rseg[c];
   if (!MST(s, MI_PCG)) return;
   const int k = (int)(c - Cl.off[s]);
   const int nf = F.n[s], f0 = F.off[s];
@@ -900,6 +912,9 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_restrict(mg_args a, int64_t mc
   double v = 0.0;
   for (int i = i0; i < i1; i++) v += rf[f0 + i];
   rc[c] = v;
+  const double d = M.diag[c];
+  const double x = d != 0.0 ? sigma * v / d : 0.0;
+  sv[c] = x, u[c] = x;
 }
 
 // prolongation, coarse levels: r_f = over * r_c (0 on a one-row level) + u_f
@@ -917,18 +932,255 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_prolong_c(mg_args a, int64_t m
   rf[i] = over * cv + u[i];
 }
 
-// prolongation onto level 0 (tiles), result into z
-__global__ void __launch_bounds__(RSB_BLOCK) k_mg_prolong0(mg_args a, mg_lvl Cl, int factor,
-                                                          double over, const double *rc,
-                                                          const double *u, double *z) {
+// Prolongation onto level 0 (tiles), result into z (the previous one is kept
+// in z0); partial sum of z.  v[depth] holds the result of level depth + 1,
+// v[l] for l < depth the smoothed u of level l + 1: a row's value on each of
+// these levels is formed on the way up by every row below it, the same
+// operations as in one launch per level, and none of them is written.
+#define MG_CHAIN 3
+struct mg_chain {
+  int depth;
+  mg_lvl lv[MG_CHAIN + 1];
+  const double *v[MG_CHAIN + 1];
+};
+__global__ void __launch_bounds__(RSB_BLOCK) k_mg_up0(mg_args a, mg_chain c, int factor,
+                                                     double over, double over0, const double *u,
+                                                     double *z, double *z0) {
   mg_tile t;
   if (!mg_tile_of(a, GATE_PCG, t)) return;
-  const int coff = Cl.off[t.s], cn = Cl.n[t.s];
+  int off[MG_CHAIN + 1], n[MG_CHAIN + 1];
+#pragma unroll
+  for (int l = 0; l <= MG_CHAIN; l++)
+    off[l] = l <= c.depth ? c.lv[l].off[t.s] : 0, n[l] = l <= c.depth ? c.lv[l].n[t.s] : 0;
+  double acc[1] = {0.0};
   MG_ROWS(t, row) {
-    const int k = row - t.pstart;
-    const double cv = cn == 1 ? 0.0 : rc[coff + k / factor];
-    z[row] = over * cv + u[row];
+    int k = row - t.pstart;
+    double v[MG_CHAIN + 1];
+#pragma unroll
+    for (int l = 0; l <= MG_CHAIN; l++) {
+      k /= factor;
+      v[l] = n[l] > 1 ? c.v[l][off[l] + k] : 0.0;
+    }
+    double cv = 0.0;
+#pragma unroll
+    for (int l = MG_CHAIN; l >= 0; l--)
+      if (l <= c.depth) cv = n[l] <= 1 ? 0.0 : l == c.depth ? v[l] : fma(over, cv, v[l]);
+    const double zv = fma(over0, cv, u[row]);
+    z0[row] = z[row];
+    z[row] = zv;
+    acc[0] += zv;
   }
+  mg_publish<1>(a, t, acc);
+}
+
+// The coarse end of the V-cycle, one workgroup per segment: the levels from
+// l0 on, restriction to prolongation, with r, u and s in LDS.  A level of
+// this size has a few hundred nanoseconds of work per step, so one launch per
+// step (six per level, about eleven levels) was launch latency only.  Levels
+// of at most MG_LOW_THREADS rows hold one row per thread, larger ones two;
+// the first entries of each row stay in registers over the three steps.  Levels of at most 64 rows run in one wave without workgroup
+// barriers.  Every row takes the operations of k_mg_down, k_mg_res_c and
+// k_mg_prolong_c in their order, so the results are theirs bit for bit.
+// With the first Jacobi step in k_mg_update / k_mg_down and the way up in
+// k_mg_up0 an iteration on 24,576 hexes takes 28 launches instead of 95:
+// 24 parts of that pipe in 118 ms, 189 before.  MG_LOW_ROWS is what two rows
+// per thread and 98 KB of LDS hold; a level above it fills several CUs.
+#define MG_LOW_THREADS 1024
+#define MG_LOW_ROWS (2 * MG_LOW_THREADS)
+#define MG_LOW_LEVELS 12  // 2048 rows, halved or less per level, while > 1 row
+
+struct mg_low_level {
+  const int *off, *n;
+  const int64_t *soff;
+  const int *rlen, *sci, *sw;
+  const double *diag;
+  const uint32_t *spk;
+};
+struct mg_low {
+  int nlev;    // levels that have a coarser one below
+  int stride;  // rows of the largest segment on the first of them
+  mg_low_level lv[MG_LOW_LEVELS];
+};
+
+template <bool WAVE>
+__device__ inline void mg_low_sync() {
+  if (WAVE) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
+// three Jacobi steps on one level's n rows (rows tid and tid + nt): r comes in
+// registers and goes to R, u goes to U
+template <int NR, bool WAVE>
+__device__ inline void mg_low_smooth(const mg_low_level &L, int off, int n, int nt,
+                                     double (&r)[NR], double sig0, double sig1, double sig2,
+                                     double *R, double *U, double *S0, double *S1) {
+  constexpr int ENT = NR == 1 ? 12 : 6;  // entries of a row kept in registers
+  const int tid = threadIdx.x;
+  double u[NR], d[NR], s[NR];
+  int len[NR], c[NR][ENT], w[NR][ENT];
+  int64_t base[NR];
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    const int k = tid + q * nt;
+    const bool on = k < n;
+    const int i = off + (on ? k : 0);
+    base[q] = L.soff[i / RSB_WAVE] + (i % RSB_WAVE);
+    const int ln = L.rlen[i];
+    const double dv = L.diag[i];
+    len[q] = on ? ln : 0, d[q] = on ? dv : 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    s[q] = d[q] != 0.0 ? sig0 * r[q] / d[q] : 0.0;
+    u[q] = s[q];
+    if (tid + q * nt < n) S0[tid + q * nt] = s[q];
+  }
+  if (L.spk) {
+#pragma unroll
+    for (int q = 0; q < NR; q++)
+#pragma unroll
+      for (int j = 0; j < ENT; j++) {
+        const uint32_t e = j < len[q] ? L.spk[base[q] + (int64_t)j * RSB_WAVE] : (uint32_t)off;
+        c[q][j] = (int)(e & 0xffffffu) - off, w[q][j] = (int)(e >> 24);
+      }
+  } else {
+#pragma unroll
+    for (int q = 0; q < NR; q++)
+#pragma unroll
+      for (int j = 0; j < ENT; j++) {
+        const int64_t k = base[q] + (int64_t)j * RSB_WAVE;
+        c[q][j] = (j < len[q] ? L.sci[k] : off) - off;
+        w[q][j] = j < len[q] ? L.sw[k] : 0;
+      }
+  }
+  mg_low_sync<WAVE>();
+  double *sc = S0, *sn = S1;
+#pragma unroll
+  for (int step = 0; step < 3; step++) {
+    const double sigma = step == 0 ? sig1 : step == 1 ? sig2 : 0.0;
+#pragma unroll
+    for (int q = 0; q < NR; q++) {
+      double as = 0.0;
+      double v[ENT];
+#pragma unroll
+      for (int j = 0; j < ENT; j++) v[j] = sc[c[q][j]];
+#pragma unroll
+      for (int j = 0; j < ENT; j++) {
+        const double x = fma((double)w[q][j], v[j], as);
+        as = j < len[q] ? x : as;
+      }
+      for (int j = ENT; j < len[q]; j++) {
+        const int64_t k = base[q] + (int64_t)j * RSB_WAVE;
+        int ci, wi;
+        if (L.spk) {
+          const uint32_t e = L.spk[k];
+          ci = (int)(e & 0xffffffu), wi = (int)(e >> 24);
+        } else {
+          ci = L.sci[k], wi = L.sw[k];
+        }
+        as = fma((double)wi, sc[ci - off], as);
+      }
+      const double rv = r[q] - fma(d[q], s[q], -as);
+      r[q] = rv;
+      if (step < 2) {
+        s[q] = d[q] != 0.0 ? sigma * rv / d[q] : 0.0;
+        u[q] += s[q];
+        if (tid + q * nt < n) sn[tid + q * nt] = s[q];
+      }
+    }
+    if (step < 2) mg_low_sync<WAVE>();
+    double *x = sc;
+    sc = sn, sn = x;
+  }
+#pragma unroll
+  for (int q = 0; q < NR; q++)
+    if (tid + q * nt < n) R[tid + q * nt] = r[q], U[tid + q * nt] = u[q];
+  mg_low_sync<WAVE>();
+}
+
+// one level down: restriction from the nf rows of rf, then the three steps
+template <int NR, bool WAVE>
+__device__ inline void mg_low_down(const mg_low_level &L, int off, int n, int nt, int factor,
+                                   int nf, const double *rf, double sig0, double sig1,
+                                   double sig2, double *R, double *U, double *S0, double *S1) {
+  double r[NR];
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    const int k = (int)threadIdx.x + q * nt;
+    double v = 0.0;
+    if (k < n)
+      for (int i = k * factor, i1 = min(i + factor, nf); i < i1; i++) v += rf[i];
+    r[q] = v;
+  }
+  mg_low_smooth<NR, WAVE>(L, off, n, nt, r, sig0, sig1, sig2, R, U, S0, S1);
+}
+
+__global__ void __launch_bounds__(MG_LOW_THREADS) k_mg_low(mg_args a, mg_low L, mg_lvl F,
+                                                           int factor, const double *rf,
+                                                           double sig0, double sig1, double sig2,
+                                                           double *rout) {
+  extern __shared__ double lds[];
+  __shared__ int ln[MG_LOW_LEVELS + 1], lo[MG_LOW_LEVELS + 1];
+  const int s = blockIdx.x, nt = blockDim.x;
+  if (!MST(s, MI_PCG)) return;
+  if ((int)threadIdx.x <= MG_LOW_LEVELS) {
+    const bool in = (int)threadIdx.x < L.nlev;
+    ln[threadIdx.x] = in ? L.lv[threadIdx.x].n[s] : 0;
+    lo[threadIdx.x] = in ? L.lv[threadIdx.x].off[s] : 0;
+  }
+  const int nf0 = F.n[s];
+  const double *rf0 = rf + F.off[s];
+  __syncthreads();
+  const int n0 = ln[0];
+  if (n0 <= 1) return;
+  double *S0 = lds, *S1 = lds + n0, *R = lds + 2 * n0, *U = R;
+  int tot = 0, nl = 0, lw = -1;  // levels with rows to smooth; the first that one wave takes
+  while (nl < L.nlev && ln[nl] > 1) {
+    if (lw < 0 && ln[nl] <= RSB_WAVE) lw = nl;
+    tot += ln[nl++];
+  }
+  if (lw < 0) lw = nl;
+  U = R + tot;
+  int pos = 0, l = 0;
+  for (; l < lw; l++) {
+    const int n = ln[l], nf = l ? ln[l - 1] : nf0;
+    const double *src = l ? R + pos - nf : rf0;
+    if (n <= nt)
+      mg_low_down<1, false>(L.lv[l], lo[l], n, nt, factor, nf, src, sig0, sig1, sig2, R + pos,
+                            U + pos, S0, S1);
+    else
+      mg_low_down<2, false>(L.lv[l], lo[l], n, nt, factor, nf, src, sig0, sig1, sig2, R + pos,
+                            U + pos, S0, S1);
+    pos += n;
+  }
+  if (threadIdx.x < RSB_WAVE) {
+    int p = pos;
+    for (; l < nl; l++) {
+      const int n = ln[l], nf = l ? ln[l - 1] : nf0;
+      mg_low_down<1, true>(L.lv[l], lo[l], n, RSB_WAVE, factor, nf, l ? R + p - nf : rf0, sig0,
+                           sig1, sig2, R + p, U + p, S0, S1);
+      p += n;
+    }
+    for (l = nl - 1; l >= lw; l--) {
+      const int n = ln[l], k = threadIdx.x;
+      p -= n;
+      if (k < n) R[p + k] = fma(1.5, l + 1 < nl ? R[p + n + k / factor] : 0.0, U[p + k]);
+      mg_low_sync<true>();
+    }
+  }
+  __syncthreads();
+  for (l = lw - 1; l >= 0; l--) {
+    const int n = ln[l];
+    pos -= n;
+    for (int k = threadIdx.x; k < n; k += nt)
+      R[pos + k] = fma(1.5, l + 1 < nl ? R[pos + n + k / factor] : 0.0, U[pos + k]);
+    __syncthreads();
+  }
+  for (int k = threadIdx.x; k < n0; k += nt) rout[lo[0] + k] = R[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -1429,6 +1681,27 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   const double s1 = sigma_cheb(1, 4, 1.0, 2.0), s2 = sigma_cheb(2, 4, 1.0, 2.0),
                s3 = sigma_cheb(3, 4, 1.0, 2.0);
   const double sig[3] = {s1, s2, s3};
+  // first level that k_mg_low takes, and its LDS: r and u of every level with
+  // rows to smooth, s twice over the first
+  int l0 = 1, low_rows = 0, low_threads = RSB_WAVE;
+  for (;; l0++) {
+    low_rows = 0;
+    for (int s = 0; s < nseg; s++) low_rows = std::max(low_rows, H.h_n[l0][s]);
+    if (low_rows <= MG_LOW_ROWS) break;
+  }
+  mg_low low{};
+  for (int l = l0; l + 1 < nlev; l++) {
+    const mg_level_dev &F = H.lv[l];
+    low.lv[low.nlev++] = mg_low_level{F.off, F.n, F.soff, F.rlen, F.sci, F.sw, F.diag, F.spk};
+  }
+  size_t low_lds = 0;
+  for (int s = 0; s < nseg; s++) {
+    size_t tot = 0;
+    for (int l = l0; l + 1 < nlev; l++) tot += (size_t)H.h_n[l][s];
+    low_lds = std::max(low_lds, sizeof(double) * 2 * (tot + (size_t)H.h_n[l0][s]));
+  }
+  while (low_threads < low_rows && low_threads < MG_LOW_THREADS) low_threads *= 2;
+  low.stride = low_rows;
   // One CG iteration is part_a (w = L p, alpha, the update of x and r, the
   // stop test) and part_b (z = V-cycle(r), beta, the new direction made
   // L-orthogonal to the earlier ones).  The host reads the count of running
@@ -1437,50 +1710,51 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   auto part_a = [&]() -> int {
     k_mg_apply<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_PCG, S, p, w);
     fin(FIN_ALPHA, GATE_PCG, 1);
-    k_mg_update<<<ntiles, RSB_BLOCK, 0, st>>>(a, mpad, p, w, x, r, Wb, Pb);
-    k_mg_zero<<<1, 1, 0, st>>>(active);
+    k_mg_update<<<ntiles, RSB_BLOCK, 0, st>>>(a, mpad, p, w, x, r, Wb, Pb, diag0, sig[0],
+                                               H.lv[0].sa, H.lv[0].u);
     fin(FIN_CONV, GATE_PCG, 1);
     RSB_LAUNCH_CHECK();
     return 0;
   };
   auto part_b = [&]() -> int {
-    k_mg_copy<<<ntiles, RSB_BLOCK, 0, st>>>(a, z, z0);
-    // down
-    for (int l = 0; l + 1 < nlev; l++) {
-      mg_level_dev &F = H.lv[l];
-      // the residual ends in F.r0 (level 0 starts from the CG residual r)
-      if (l == 0) {
-        k_mg_jac0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, sig[0], r, F.sa, F.u);
-        k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, r, F.r0, F.sa, sig[1], F.sb, F.u);
-        k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, F.r0, F.r0, F.sb, sig[2], F.sa, F.u);
-        k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, F.r0, F.r0, F.sa, 0.0, nullptr, F.u);
-      } else {
-        const mg_csr M{F.m, F.rseg, F.soff, F.rlen, F.sci, F.sw, F.diag, F.spk};
-        const unsigned nb = nblocks(F.m, RSB_BLOCK);
-        k_mg_jac_c<<<nb, RSB_BLOCK, 0, st>>>(a, M, sig[0], F.r0, F.sa, F.u);
-        k_mg_res_c<<<nb, RSB_BLOCK, 0, st>>>(a, M, F.r0, F.sa, sig[1], F.sb, F.u);
-        k_mg_res_c<<<nb, RSB_BLOCK, 0, st>>>(a, M, F.r0, F.sb, sig[2], F.sa, F.u);
-        k_mg_res_c<<<nb, RSB_BLOCK, 0, st>>>(a, M, F.r0, F.sa, 0.0, nullptr, F.u);
-      }
-      mg_level_dev &C = H.lv[l + 1];
-      k_mg_restrict<<<nblocks(C.m, RSB_BLOCK), RSB_BLOCK, 0, st>>>(
-          a, C.m, C.rseg, mg_lvl{F.off, F.n}, mg_lvl{C.off, C.n}, factor, F.r0, C.r0);
+    mg_level_dev &F0 = H.lv[0];
+    // down to l0: the residual ends in F.r0 (level 0 starts from the CG residual r)
+    k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, r, F0.r0, F0.sa, sig[1], F0.sb, F0.u);
+    k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, F0.r0, F0.r0, F0.sb, sig[2], F0.sa, F0.u);
+    k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, F0.r0, F0.r0, F0.sa, 0.0, nullptr, F0.u);
+    for (int l = 1; l < l0; l++) {
+      mg_level_dev &F = H.lv[l], &D = H.lv[l - 1];
+      const mg_csr M{F.m, F.rseg, F.soff, F.rlen, F.sci, F.sw, F.diag, F.spk};
+      const unsigned nb = nblocks(F.m, RSB_BLOCK);
+      k_mg_down<<<nb, RSB_BLOCK, 0, st>>>(a, M, mg_lvl{D.off, D.n}, mg_lvl{F.off, F.n}, factor,
+                                          D.r0, sig[0], F.r0, F.sa, F.u);
+      k_mg_res_c<<<nb, RSB_BLOCK, 0, st>>>(a, M, F.r0, F.sa, sig[1], F.sb, F.u);
+      k_mg_res_c<<<nb, RSB_BLOCK, 0, st>>>(a, M, F.r0, F.sb, sig[2], F.sa, F.u);
+      k_mg_res_c<<<nb, RSB_BLOCK, 0, st>>>(a, M, F.r0, F.sa, 0.0, nullptr, F.u);
     }
-    // up: each coarse level's result goes to its r0
-    for (int l = nlev - 2; l >= 1; l--) {
-      mg_level_dev &F = H.lv[l], &C = H.lv[l + 1];
+    if (l0 < nlev - 1) {
+      mg_level_dev &D = H.lv[l0 - 1];
+      k_mg_low<<<nseg, low_threads, low_lds, st>>>(a, low, mg_lvl{D.off, D.n}, factor, D.r0,
+                                                   sig[0], sig[1], sig[2], H.lv[l0].r0);
+    }
+    // up: each coarse level's result goes to its r0; the last MG_CHAIN levels
+    // above the result of the deepest one are evaluated row by row in k_mg_up0
+    int lu = l0;
+    for (; lu > MG_CHAIN + 1; lu--) {
+      mg_level_dev &F = H.lv[lu - 1], &C = H.lv[lu];
       k_mg_prolong_c<<<nblocks(F.m, RSB_BLOCK), RSB_BLOCK, 0, st>>>(
           a, F.m, F.rseg, mg_lvl{F.off, F.n}, mg_lvl{C.off, C.n}, factor, 1.5, C.r0, F.u, F.r0);
     }
-    mg_level_dev &F0 = H.lv[0], &C1 = H.lv[1];
-    k_mg_prolong0<<<ntiles, RSB_BLOCK, 0, st>>>(a, mg_lvl{C1.off, C1.n}, factor, 1.33333, C1.r0,
-                                                 F0.u, z);
-    k_mg_sum<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_PCG, z);
+    mg_chain ch;
+    ch.depth = lu - 1;
+    for (int l = 1; l <= lu; l++)
+      ch.lv[l - 1] = mg_lvl{H.lv[l].off, H.lv[l].n}, ch.v[l - 1] = l == lu ? H.lv[l].r0 : H.lv[l].u;
+    k_mg_up0<<<ntiles, RSB_BLOCK, 0, st>>>(a, ch, factor, 1.5, 1.33333, F0.u, z, z0);
     fin(FIN_MEAN, GATE_PCG, 1);
     k_mg_zdots<<<ntiles, RSB_BLOCK, 0, st>>>(a, r, z, z0);
     fin(FIN_BETA, GATE_PCG, 2);
     k_mg_pnew<<<ntiles, RSB_BLOCK, 0, st>>>(a, mpad, z, p, Wb);
-    k_mg_coef<<<nseg, RSB_BLOCK, 0, st>>>(a, coef);
+    k_mg_coef<<<dim3(nseg, (max_iter + 3) / 4), RSB_BLOCK, 0, st>>>(a, coef);
     k_mg_pcorr<<<ntiles, RSB_BLOCK, 0, st>>>(a, mpad, p, Pb, coef);
     RSB_LAUNCH_CHECK();
     return 0;
