@@ -536,6 +536,15 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_pcorr(mg_args a, int64_t mpad,
 
 __global__ void k_mg_zero(int *c) { *c = 0; }
 
+// The count of running segments goes to the host's ring of MG_RING slots:
+// c[0] is the count, c[1] the number of reports so far.
+#define MG_RING 4
+__global__ void k_mg_report(int *c, int *ring) {
+  const int q = c[1];
+  c[1] = q + 1;
+  __hip_atomic_store(ring + q % MG_RING, c[0], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // fiedler[cstart + i] = x * ni (fiedler.c:606-616)
 __global__ void __launch_bounds__(RSB_BLOCK) k_mg_out(mg_args a, const double *x, double *fied) {
   mg_tile t;
@@ -1411,6 +1420,8 @@ struct mg_scope {
   std::vector<void *> bufs;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  int *ring = nullptr;  // pinned: the counts that k_mg_report writes
   bool capturing = false;
   explicit mg_scope(hipStream_t s) : st(s) {}
   template <typename T>
@@ -1429,6 +1440,9 @@ struct mg_scope {
     (void)hipStreamSynchronize(st);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (ring) (void)hipHostFree(ring);
     for (void *q : bufs) rsb_dev_release(q);
   }
 };
@@ -1636,7 +1650,10 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   RSB_TRY(own.alloc(stt, sizeof(int) * MI_NI * (size_t)nseg));
   RSB_TRY(own.alloc(partial, sizeof(double) * MG_NP * (size_t)std::max(ntiles, 1)));
   RSB_TRY(own.alloc(coef, sizeof(double) * MG_NP * (size_t)nseg));
-  RSB_TRY(own.alloc(active, sizeof(int)));
+  RSB_TRY(own.alloc(active, 2 * sizeof(int)));
+  RSB_TRY(hipMemsetAsync(active, 0, 2 * sizeof(int), st));
+  RSB_TRY(hipHostMalloc((void **)&own.ring, MG_RING * sizeof(int), hipHostMallocDefault));
+  for (hipEvent_t &e : own.ev) RSB_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   // Gram basis: at most one vector per pass that another pass follows
   mg_gram G{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, max_passes - 1};
   const bool gram = grammian && G.cap >= 1;
@@ -1704,8 +1721,8 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   low.stride = low_rows;
   // One CG iteration is part_a (w = L p, alpha, the update of x and r, the
   // stop test) and part_b (z = V-cycle(r), beta, the new direction made
-  // L-orthogonal to the earlier ones).  The host reads the count of running
-  // segments after each part_a; part_b + part_a of the next iteration run as
+  // L-orthogonal to the earlier ones).  The count of running segments goes to
+  // the host after each part_a; part_b + part_a of the next iteration run as
   // one captured graph (no memset nodes: counters are cleared by a kernel).
   auto part_a = [&]() -> int {
     k_mg_apply<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_PCG, S, p, w);
@@ -1713,6 +1730,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
     k_mg_update<<<ntiles, RSB_BLOCK, 0, st>>>(a, mpad, p, w, x, r, Wb, Pb, diag0, sig[0],
                                                H.lv[0].sa, H.lv[0].u);
     fin(FIN_CONV, GATE_PCG, 1);
+    k_mg_report<<<1, 1, 0, st>>>(active, own.ring);
     RSB_LAUNCH_CHECK();
     return 0;
   };
@@ -1772,6 +1790,21 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
     }
   }
   hipGraphExec_t exec = own.exec;
+  // The host reads the count of iteration q while iteration q + 1, queued
+  // before, runs: reading it before queueing left the device idle for about
+  // 20 us of every 190.  The iteration queued after the last one finds no
+  // running segment, and every one of its launches returns at its gate.
+  int reports = 0;
+  auto queued = [&]() -> int {
+    RSB_TRY(hipEventRecord(own.ev[reports & 1], st));
+    reports++;
+    return 0;
+  };
+  auto count_of = [&](int q, int &n) -> int {
+    RSB_TRY(hipEventSynchronize(own.ev[q & 1]));
+    n = __atomic_load_n(own.ring + q % MG_RING, __ATOMIC_ACQUIRE);
+    return 0;
+  };
   for (int pass = 0; pass < max_passes; pass++) {
     // projection (fiedler.c:94-187)
     k_mg_pass0<<<ntiles, RSB_BLOCK, 0, st>>>(a, b, x, r);
@@ -1780,16 +1813,18 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
     fin(FIN_RZ1, GATE_PCG, 1);
     RSB_LAUNCH_CHECK();
     MG_TRY(part_a());
-    int nact = 0;
-    MG_TRY(count_active(nact));
-    for (int it = 1; it < max_iter && nact > 0; it++) {
+    MG_TRY(queued());
+    for (int it = 1; it < max_iter; it++) {
       if (exec) {
         RSB_TRY(hipGraphLaunch(exec, st));
       } else {
         MG_TRY(part_b());
         MG_TRY(part_a());
       }
-      MG_TRY(count_active(nact));
+      MG_TRY(queued());
+      int nact = 0;
+      MG_TRY(count_of(reports - 2, nact));
+      if (nact == 0) break;
     }
     // end of pass (fiedler.c:231-247): y orthogonalised, z = y / |y|, z orthogonalised
     k_mg_sum<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_INV, x);
