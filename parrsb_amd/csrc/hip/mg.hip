@@ -48,7 +48,7 @@ struct mg_args {
   double *sc;            // MS_NSC per segment
   int *st;               // MI_NI per segment
   double *partial;       // MG_NP per tile
-  int *active;           // count written by finishing kernels
+  int *active;           // running segments: [0] in the CG iteration, [1] reports, [2] passes
   double tol;
   int miter, mpass;
   int ntiles;            // partial is slot-major: slot k of tile t at k * ntiles + t
@@ -75,12 +75,15 @@ struct mg_tile {
 __device__ inline bool mg_tile_of(const mg_args &a, int gate, mg_tile &t) {
   t.ti = blockIdx.x;
   t.s = a.tile[3 * t.ti];
-  if (!mg_gate(a, t.s, gate)) return false;
   t.row0 = a.tile[3 * t.ti + 1];
   t.row1 = a.tile[3 * t.ti + 2];
   t.n = a.seg[a.nseg + t.s];
   t.pstart = a.seg[4 * a.nseg + t.s];
-  return true;
+  const bool go = mg_gate(a, t.s, gate);
+  // (the compiler moves loads that only the rows need behind the branch on
+  // the gate, one more wait in a row)
+  asm volatile("" ::"s"(t.row0), "s"(t.row1), "s"(t.n), "s"(t.pstart));
+  return go;
 }
 #define MG_ROWS(t, row) \
   for (int row = (t).row0 + (int)threadIdx.x; row < (t).row1 && row - (t).pstart < (t).n; row += RSB_BLOCK)
@@ -114,46 +117,69 @@ typedef unsigned mg_u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned mg_u32x2 __attribute__((ext_vector_type(2)));
 #define MG_TB_LOCAL 4096
 
-// Stage x over the tile's rows and halo rows into LDS; returns false (and
-// stages nothing) if the tile has no LDS form.
-__device__ inline bool mg_stage(const mg_sell &L, const mg_tile &t, const double *x, double *xl) {
+// The kernels that multiply by L run one row per thread (MG_RT threads): a
+// tile's 1,024 rows one after another in 256 threads put four rounds of
+// dependent loads in a row, and a level of a few dozen tiles is bound by
+// those.  What a row reads besides x is loaded before x is staged.
+#define MG_RT RSB_TILE
+
+// Where the tile's halo list is (nhalo < 0: the tile has no LDS form)
+__device__ inline bool mg_halo_of(const mg_sell &L, int ti, int &nh, int64_t &ho) {
   if (!L.nhalo) return false;
-  const int nh = L.nhalo[t.ti];
-  if (nh < 0) return false;
+  nh = L.nhalo[ti], ho = L.halo_off[ti];
+  return nh >= 0;
+}
+
+// x over the tile's rows and halo rows into LDS
+__device__ inline void mg_stage(const mg_sell &L, const mg_tile &t, int nh, int64_t ho,
+                                const double *x, double *xl) {
   const int nrows = t.row1 - t.row0, tot = nrows + nh;
-  const int64_t ho = L.halo_off[t.ti];
-  for (int i = threadIdx.x; i < tot; i += blockDim.x)
+  for (int i = threadIdx.x; i < tot; i += MG_RT)
     xl[i] = x[i < nrows ? t.row0 + i : L.halo[ho + i - nrows]];
   __syncthreads();
-  return true;
+}
+
+// A row's 16-bit entries: where they are and the first eight
+struct mg_row16 {
+  const uint16_t *sbase;
+  int w16;
+  mg_u32x4 v;
+};
+__device__ inline void mg_row16_of(const mg_sell &L, int row, mg_row16 &e) {
+  const int sl = __builtin_amdgcn_readfirstlane(row >> 6);  // a wave's rows are one slice
+  e.sbase = L.e16 + L.off16[sl];
+  e.w16 = L.w16[sl];
+  e.v = mg_u32x4{0, 0, 0, 0};
+  if (e.w16 >= 8) e.v = *(const mg_u32x4 *)(e.sbase + (row & 63) * 8);
 }
 
 // sum_j w_ij x_j over the row's 16-bit entries (the same entries in the same
 // order as the 32-bit form, then weight-0 padding, which adds exact zeros)
-__device__ inline double tile_offsum(const mg_sell &L, int row, const double *xl) {
-  const int sl = row >> 6;
-  const uint16_t *sbase = L.e16 + L.off16[sl];
+__device__ inline double tile_offsum(const mg_row16 &r, int row, const double *xl) {
+  const uint16_t *sbase = r.sbase;
   const mg_u32x4 *ep = (const mg_u32x4 *)(sbase + (row & 63) * 8);
-  const int w16 = L.w16[sl], nb = w16 >> 3;
+  const int w16 = r.w16, nb = w16 >> 3;
   double s = 0.0;
+  mg_u32x4 v = r.v;
   for (int jb = 0; jb < nb; jb++) {
-    const mg_u32x4 v = ep[(size_t)jb * RSB_WAVE];
-    const unsigned e[8] = {v.x & 0xffffu, v.x >> 16, v.y & 0xffffu, v.y >> 16,
-                           v.z & 0xffffu, v.z >> 16, v.w & 0xffffu, v.w >> 16};
+    const mg_u32x4 c = v;
+    if (jb + 1 < nb) v = ep[(size_t)(jb + 1) * RSB_WAVE];
+    const unsigned e[8] = {c.x & 0xffffu, c.x >> 16, c.y & 0xffffu, c.y >> 16,
+                           c.z & 0xffffu, c.z >> 16, c.w & 0xffffu, c.w >> 16};
 #pragma unroll
-    for (int k = 0; k < 8; k++) s += (double)(e[k] >> 12) * xl[e[k] & 0xfffu];
+    for (int k = 0; k < 8; k++) s = fma((double)(e[k] >> 12), xl[e[k] & 0xfffu], s);
   }
   if (w16 & 4) {
-    const mg_u32x2 v = *(const mg_u32x2 *)(sbase + nb * 512 + (row & 63) * 4);
-    const unsigned e[4] = {v.x & 0xffffu, v.x >> 16, v.y & 0xffffu, v.y >> 16};
+    const mg_u32x2 c = *(const mg_u32x2 *)(sbase + nb * 512 + (row & 63) * 4);
+    const unsigned e[4] = {c.x & 0xffffu, c.x >> 16, c.y & 0xffffu, c.y >> 16};
 #pragma unroll
-    for (int k = 0; k < 4; k++) s += (double)(e[k] >> 12) * xl[e[k] & 0xfffu];
+    for (int k = 0; k < 4; k++) s = fma((double)(e[k] >> 12), xl[e[k] & 0xfffu], s);
   }
   if (w16 & 2) {
-    const unsigned v = *(const unsigned *)(sbase + nb * 512 + (w16 & 4) * 64 + (row & 63) * 2);
-    const unsigned e[2] = {v & 0xffffu, v >> 16};
+    const unsigned c = *(const unsigned *)(sbase + nb * 512 + (w16 & 4) * 64 + (row & 63) * 2);
+    const unsigned e[2] = {c & 0xffffu, c >> 16};
 #pragma unroll
-    for (int k = 0; k < 2; k++) s += (double)(e[k] >> 12) * xl[e[k] & 0xfffu];
+    for (int k = 0; k < 2; k++) s = fma((double)(e[k] >> 12), xl[e[k] & 0xfffu], s);
   }
   return s;
 }
@@ -275,7 +301,7 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_fin(mg_args a, int op, int gat
     MST(s, MI_ITERS) += ppfi;
     MST(s, MI_NPASS) += 1;
     if (ppfi == 1 || MST(s, MI_NPASS) == a.mpass) MST(s, MI_INV) = 0;
-    else atomicAdd(a.active, 1);
+    else atomicAdd(a.active + 2, 1);
     break;
   }
   case FIN_RAYLEIGH: {  // tot: f.Lf, Lf.Lf, f.f
@@ -400,30 +426,48 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_pass1(mg_args a, const double 
   mg_publish<1>(a, t, acc);
 }
 
-// w = L p; partial p.w.  The first workgroup clears the count of running
-// segments that this iteration's stop test forms two launches later.
-__global__ void __launch_bounds__(RSB_BLOCK) k_mg_apply(mg_args a, int gate, mg_sell L,
-                                                       const double *p, double *w) {
-  __shared__ double xl[MG_TB_LOCAL];
+// w = L p; partial p.w (thread t < RSB_BLOCK sums rows t, t + RSB_BLOCK, ...,
+// as every other kernel's partials)
+__global__ void __launch_bounds__(MG_RT) k_mg_apply(mg_args a, int gate, mg_sell L,
+                                                   const double *p, double *w) {
+  __shared__ double xl[MG_TB_LOCAL], wl[MG_RT], red[RSB_BLOCK / RSB_WAVE];
   mg_tile t;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && gate == GATE_PCG) *a.active = 0;
+  int nh = -1;
+  int64_t ho = 0;
+  const bool tiled = mg_halo_of(L, blockIdx.x, nh, ho);
   if (!mg_tile_of(a, gate, t)) return;
-  double acc[1] = {0.0};
-  if (mg_stage(L, t, p, xl)) {
-    MG_ROWS(t, row) {
-      const double pi = xl[row - t.row0];
-      const double v = L.diag[row] * pi - tile_offsum(L, row, xl);
-      w[row] = v;
-      acc[0] += pi * v;
-    }
+  const int tid = threadIdx.x, row = t.row0 + tid;
+  const bool on = row < t.row1 && row - t.pstart < t.n;
+  const double d = on ? L.diag[row] : 0.0;
+  double v = 0.0;
+  if (tiled) {
+    mg_row16 e{};
+    if (on) mg_row16_of(L, row, e);
+    mg_stage(L, t, nh, ho, p, xl);
+    if (on) v = fma(d, xl[tid], -tile_offsum(e, row, xl));
   } else {
-    MG_ROWS(t, row) {
-      const double v = L.diag[row] * p[row] - sell_offsum(L, row, p);
-      w[row] = v;
-      acc[0] += p[row] * v;
-    }
+    const double pi = on ? p[row] : 0.0;
+    if (on) v = fma(d, pi, -sell_offsum(L, row, p));
+    xl[tid] = pi;
   }
-  mg_publish<1>(a, t, acc);
+  if (on) w[row] = v;
+  wl[tid] = v;
+  __syncthreads();
+  double acc = 0.0;
+  if (tid < RSB_BLOCK) {
+#pragma unroll
+    for (int k = 0; k < MG_RT; k += RSB_BLOCK) {
+      const int r = row + k;
+      if (r < t.row1 && r - t.pstart < t.n) acc = fma(xl[tid + k], wl[tid + k], acc);
+    }
+    acc = wave_sum(acc);
+    if ((tid & (RSB_WAVE - 1)) == 0) red[tid / RSB_WAVE] = acc;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int k = 1; k < RSB_BLOCK / RSB_WAVE; k++) acc += red[k];
+    a.partial[t.ti] = acc;
+  }
 }
 
 // W[i] = pwinv w, P[i] = pwinv p, x += alpha p, r -= alpha w; partial r.r.
@@ -439,17 +483,26 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_update(mg_args a, int64_t mpad
   if (!mg_tile_of(a, GATE_PCG, t)) return;
   const int i = MST(t.s, MI_IT);
   const double alpha = MSC(t.s, MS_ALPHA), pwinv = MSC(t.s, MS_PWINV);
+  constexpr int NR = RSB_TILE / RSB_BLOCK;
+  double pv[NR], wv[NR], xv[NR], rv[NR], d[NR];
+#pragma unroll
+  for (int k = 0; k < NR; k++) {
+    const int row = t.row0 + (int)threadIdx.x + k * RSB_BLOCK;
+    if (row < t.row1 && row - t.pstart < t.n)
+      pv[k] = p[row], wv[k] = w[row], xv[k] = x[row], rv[k] = r[row], d[k] = diag[row];
+  }
   double acc[1] = {0.0};
-  MG_ROWS(t, row) {
-    const double pv = p[row], wv = w[row];
-    Wb[(size_t)i * mpad + row] = pwinv * wv;
-    Pb[(size_t)i * mpad + row] = pwinv * pv;
-    x[row] += alpha * pv;
-    const double rv = r[row] - alpha * wv;
-    r[row] = rv;
-    acc[0] += rv * rv;
-    const double d = diag[row];
-    const double s = d != 0.0 ? sigma * rv / d : 0.0;
+#pragma unroll
+  for (int k = 0; k < NR; k++) {
+    const int row = t.row0 + (int)threadIdx.x + k * RSB_BLOCK;
+    if (!(row < t.row1 && row - t.pstart < t.n)) continue;
+    Wb[(size_t)i * mpad + row] = pwinv * wv[k];
+    Pb[(size_t)i * mpad + row] = pwinv * pv[k];
+    x[row] = fma(alpha, pv[k], xv[k]);
+    const double rn = fma(-alpha, wv[k], rv[k]);
+    r[row] = rn;
+    acc[0] = fma(rn, rn, acc[0]);
+    const double s = d[k] != 0.0 ? sigma * rn / d[k] : 0.0;
     sv[row] = s, u[row] = s;
   }
   mg_publish<1>(a, t, acc);
@@ -461,12 +514,22 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_zdots(mg_args a, const double 
   mg_tile t;
   if (!mg_tile_of(a, GATE_PCG, t)) return;
   const double m = MSC(t.s, MS_MEAN);
+  constexpr int NR = RSB_TILE / RSB_BLOCK;
+  double zv[NR], rv[NR], z0v[NR];
+#pragma unroll
+  for (int k = 0; k < NR; k++) {
+    const int row = t.row0 + (int)threadIdx.x + k * RSB_BLOCK;
+    if (row < t.row1 && row - t.pstart < t.n) zv[k] = z[row], rv[k] = r[row], z0v[k] = z0[row];
+  }
   double acc[2] = {0.0, 0.0};
-  MG_ROWS(t, row) {
-    const double zv = z[row] - m;
-    z[row] = zv;
-    acc[0] += r[row] * zv;
-    acc[1] += r[row] * (zv - z0[row]);
+#pragma unroll
+  for (int k = 0; k < NR; k++) {
+    const int row = t.row0 + (int)threadIdx.x + k * RSB_BLOCK;
+    if (!(row < t.row1 && row - t.pstart < t.n)) continue;
+    const double v = zv[k] - m;
+    z[row] = v;
+    acc[0] = fma(rv[k], v, acc[0]);
+    acc[1] = fma(rv[k], v - z0v[k], acc[1]);
   }
   mg_publish<2>(a, t, acc);
 }
@@ -537,12 +600,14 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_pcorr(mg_args a, int64_t mpad,
 __global__ void k_mg_zero(int *c) { *c = 0; }
 
 // The count of running segments goes to the host's ring of MG_RING slots:
-// c[0] is the count, c[1] the number of reports so far.
+// c[0] is the count (cleared for the next iteration), c[1] the number of
+// reports so far.
 #define MG_RING 4
 __global__ void k_mg_report(int *c, int *ring) {
   const int q = c[1];
   c[1] = q + 1;
   __hip_atomic_store(ring + q % MG_RING, c[0], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  c[0] = 0;
 }
 
 // fiedler[cstart + i] = x * ni (fiedler.c:606-616)
@@ -831,23 +896,34 @@ __global__ void __launch_bounds__(RSB_WAVE) k_gjac_test(int n, const double *Ain
 // above in one launch per step.
 
 // rout = rin - (D s - A s); then, if sigma_next > 0, the next step's s
-__global__ void __launch_bounds__(RSB_BLOCK) k_mg_res0(mg_args a, mg_sell L, const double *rin,
-                                                      double *rout, const double *sv,
-                                                      double sigma_next, double *snext,
-                                                      double *u) {
+__global__ void __launch_bounds__(MG_RT) k_mg_res0(mg_args a, mg_sell L, const double *rin,
+                                                  double *rout, const double *sv,
+                                                  double sigma_next, double *snext, double *u) {
   __shared__ double xl[MG_TB_LOCAL];
   mg_tile t;
+  int nh = -1;
+  int64_t ho = 0;
+  const bool tiled = mg_halo_of(L, blockIdx.x, nh, ho);
   if (!mg_tile_of(a, GATE_PCG, t)) return;
-  const bool tiled = mg_stage(L, t, sv, xl);
-  MG_ROWS(t, row) {
-    const double d = L.diag[row];
-    const double r = tiled ? rin[row] - (d * xl[row - t.row0] - tile_offsum(L, row, xl))
-                           : rin[row] - (d * sv[row] - sell_offsum(L, row, sv));
-    rout[row] = r;
-    if (sigma_next > 0.0) {
-      const double v = d != 0.0 ? sigma_next * r / d : 0.0;
-      snext[row] = v, u[row] += v;
-    }
+  const int row = t.row0 + (int)threadIdx.x;
+  const bool on = row < t.row1 && row - t.pstart < t.n;
+  const double d = on ? L.diag[row] : 0.0, r0 = on ? rin[row] : 0.0;
+  const double u0 = on && sigma_next > 0.0 ? u[row] : 0.0;
+  double ls = 0.0;  // D s - A s
+  if (tiled) {
+    mg_row16 e{};
+    if (on) mg_row16_of(L, row, e);
+    mg_stage(L, t, nh, ho, sv, xl);
+    if (on) ls = fma(d, xl[threadIdx.x], -tile_offsum(e, row, xl));
+  } else if (on) {
+    ls = fma(d, sv[row], -sell_offsum(L, row, sv));
+  }
+  if (!on) return;
+  const double r = r0 - ls;
+  rout[row] = r;
+  if (sigma_next > 0.0) {
+    const double v = d != 0.0 ? sigma_next * r / d : 0.0;
+    snext[row] = v, u[row] = u0 + v;
   }
 }
 
@@ -992,7 +1068,8 @@ __global__ void __launch_bounds__(RSB_BLOCK) k_mg_up0(mg_args a, mg_chain c, int
 // k_mg_prolong_c in their order, so the results are theirs bit for bit.
 // With the first Jacobi step in k_mg_update / k_mg_down and the way up in
 // k_mg_up0 an iteration on 24,576 hexes takes 28 launches instead of 95:
-// 24 parts of that pipe in 118 ms, 189 before.  MG_LOW_ROWS is what two rows
+// 24 parts of that pipe in 118 ms, 189 before, and in
+// 99 with the entries below kept and the rest batched.  MG_LOW_ROWS is what two rows
 // per thread and 98 KB of LDS hold; a level above it fills several CUs.
 #define MG_LOW_THREADS 1024
 #define MG_LOW_ROWS (2 * MG_LOW_THREADS)
@@ -1021,16 +1098,40 @@ __device__ inline void mg_low_sync() {
   }
 }
 
+// entries j0 .. j0 + 7 of a row, j0 < len (past the end: its last entry again)
+__device__ inline void mg_low_entries(const mg_low_level &L, int64_t base, int j0, int len,
+                                      int (&c)[8], int (&w)[8]) {
+  if (L.spk) {
+    const uint32_t *p = L.spk + base;
+    uint32_t e[8];
+#pragma unroll
+    for (int b = 0; b < 8; b++) e[b] = p[min(j0 + b, len - 1) * RSB_WAVE];
+#pragma unroll
+    for (int b = 0; b < 8; b++) c[b] = (int)(e[b] & 0xffffffu), w[b] = (int)(e[b] >> 24);
+  } else {
+    const int *pc = L.sci + base, *pw = L.sw + base;
+#pragma unroll
+    for (int b = 0; b < 8; b++) {
+      const int k = min(j0 + b, len - 1) * RSB_WAVE;
+      c[b] = pc[k], w[b] = pw[k];
+    }
+  }
+}
+
 // three Jacobi steps on one level's n rows (rows tid and tid + nt): r comes in
-// registers and goes to R, u goes to U
+// registers and goes to R, u goes to U.  A row's first ENT entries are kept as
+// local column | weight << 11 where its weights fit (kept = 0 otherwise); the
+// rest is read again by each step, eight entries in flight.
 template <int NR, bool WAVE>
 __device__ inline void mg_low_smooth(const mg_low_level &L, int off, int n, int nt,
                                      double (&r)[NR], double sig0, double sig1, double sig2,
                                      double *R, double *U, double *S0, double *S1) {
-  constexpr int ENT = NR == 1 ? 12 : 6;  // entries of a row kept in registers
+  constexpr int ENT = NR == 1 ? 32 : 8;
+  static_assert(MG_LOW_ROWS <= 1 << 11, "local columns have 11 bits");
   const int tid = threadIdx.x;
   double u[NR], d[NR], s[NR];
-  int len[NR], c[NR][ENT], w[NR][ENT];
+  int len[NR], kept[NR];
+  uint32_t e[NR][ENT];
   int64_t base[NR];
 #pragma unroll
   for (int q = 0; q < NR; q++) {
@@ -1048,50 +1149,59 @@ __device__ inline void mg_low_smooth(const mg_low_level &L, int off, int n, int 
     u[q] = s[q];
     if (tid + q * nt < n) S0[tid + q * nt] = s[q];
   }
-  if (L.spk) {
 #pragma unroll
-    for (int q = 0; q < NR; q++)
+  for (int q = 0; q < NR; q++) {
+    int big = 0;
 #pragma unroll
-      for (int j = 0; j < ENT; j++) {
-        const uint32_t e = j < len[q] ? L.spk[base[q] + (int64_t)j * RSB_WAVE] : (uint32_t)off;
-        c[q][j] = (int)(e & 0xffffffu) - off, w[q][j] = (int)(e >> 24);
+    for (int j0 = 0; j0 < ENT; j0 += 8) {
+      if (j0 >= len[q]) continue;
+      int c[8], w[8];
+      mg_low_entries(L, base[q], j0, len[q], c, w);
+#pragma unroll
+      for (int b = 0; b < 8; b++) {
+        e[q][j0 + b] = (uint32_t)(c[b] - off) | (uint32_t)w[b] << 11;
+        big |= w[b] >> 21;
       }
-  } else {
-#pragma unroll
-    for (int q = 0; q < NR; q++)
-#pragma unroll
-      for (int j = 0; j < ENT; j++) {
-        const int64_t k = base[q] + (int64_t)j * RSB_WAVE;
-        c[q][j] = (j < len[q] ? L.sci[k] : off) - off;
-        w[q][j] = j < len[q] ? L.sw[k] : 0;
-      }
+    }
+    kept[q] = big ? 0 : min(len[q], ENT);
   }
   mg_low_sync<WAVE>();
   double *sc = S0, *sn = S1;
-#pragma unroll
+#pragma unroll 1
   for (int step = 0; step < 3; step++) {
-    const double sigma = step == 0 ? sig1 : step == 1 ? sig2 : 0.0;
+    const double sigma = step == 0 ? sig1 : sig2;
+    // (the unpacked entries are formed again by each step: kept over the
+    // steps they would take three times the registers)
+#pragma unroll
+    for (int q = 0; q < NR; q++)
+#pragma unroll
+      for (int j = 0; j < ENT; j++) asm volatile("" : "+v"(e[q][j]));
 #pragma unroll
     for (int q = 0; q < NR; q++) {
       double as = 0.0;
-      double v[ENT];
 #pragma unroll
-      for (int j = 0; j < ENT; j++) v[j] = sc[c[q][j]];
+      for (int j0 = 0; j0 < ENT; j0 += 8) {
+        if (j0 >= kept[q]) continue;
+        double v[8];
 #pragma unroll
-      for (int j = 0; j < ENT; j++) {
-        const double x = fma((double)w[q][j], v[j], as);
-        as = j < len[q] ? x : as;
-      }
-      for (int j = ENT; j < len[q]; j++) {
-        const int64_t k = base[q] + (int64_t)j * RSB_WAVE;
-        int ci, wi;
-        if (L.spk) {
-          const uint32_t e = L.spk[k];
-          ci = (int)(e & 0xffffffu), wi = (int)(e >> 24);
-        } else {
-          ci = L.sci[k], wi = L.sw[k];
+        for (int b = 0; b < 8; b++) v[b] = sc[e[q][j0 + b] & 0x7ffu];
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+          const double x = fma((double)(int)(e[q][j0 + b] >> 11), v[b], as);
+          as = j0 + b < kept[q] ? x : as;
         }
-        as = fma((double)wi, sc[ci - off], as);
+      }
+      for (int j0 = kept[q]; j0 < len[q]; j0 += 8) {
+        int c[8], w[8];
+        double v[8];
+        mg_low_entries(L, base[q], j0, len[q], c, w);
+#pragma unroll
+        for (int b = 0; b < 8; b++) v[b] = sc[c[b] - off];
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+          const double x = fma((double)w[b], v[b], as);
+          as = j0 + b < len[q] ? x : as;
+        }
       }
       const double rv = r[q] - fma(d[q], s[q], -as);
       r[q] = rv;
@@ -1650,8 +1760,8 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   RSB_TRY(own.alloc(stt, sizeof(int) * MI_NI * (size_t)nseg));
   RSB_TRY(own.alloc(partial, sizeof(double) * MG_NP * (size_t)std::max(ntiles, 1)));
   RSB_TRY(own.alloc(coef, sizeof(double) * MG_NP * (size_t)nseg));
-  RSB_TRY(own.alloc(active, 2 * sizeof(int)));
-  RSB_TRY(hipMemsetAsync(active, 0, 2 * sizeof(int), st));
+  RSB_TRY(own.alloc(active, 3 * sizeof(int)));
+  RSB_TRY(hipMemsetAsync(active, 0, 3 * sizeof(int), st));
   RSB_TRY(hipHostMalloc((void **)&own.ring, MG_RING * sizeof(int), hipHostMallocDefault));
   for (hipEvent_t &e : own.ev) RSB_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   // Gram basis: at most one vector per pass that another pass follows
@@ -1684,7 +1794,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
     k_mg_fin<<<nseg, RSB_BLOCK, 0, st>>>(a, op, gate, nslots);
   };
   auto count_active = [&](int &n) -> int {
-    RSB_TRY(hipMemcpyAsync(&n, active, sizeof(int), hipMemcpyDeviceToHost, st));
+    RSB_TRY(hipMemcpyAsync(&n, active + 2, sizeof(int), hipMemcpyDeviceToHost, st));
     RSB_TRY(hipStreamSynchronize(st));
     return 0;
   };
@@ -1725,7 +1835,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   // the host after each part_a; part_b + part_a of the next iteration run as
   // one captured graph (no memset nodes: counters are cleared by a kernel).
   auto part_a = [&]() -> int {
-    k_mg_apply<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_PCG, S, p, w);
+    k_mg_apply<<<ntiles, MG_RT, 0, st>>>(a, GATE_PCG, S, p, w);
     fin(FIN_ALPHA, GATE_PCG, 1);
     k_mg_update<<<ntiles, RSB_BLOCK, 0, st>>>(a, mpad, p, w, x, r, Wb, Pb, diag0, sig[0],
                                                H.lv[0].sa, H.lv[0].u);
@@ -1737,9 +1847,9 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   auto part_b = [&]() -> int {
     mg_level_dev &F0 = H.lv[0];
     // down to l0: the residual ends in F.r0 (level 0 starts from the CG residual r)
-    k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, r, F0.r0, F0.sa, sig[1], F0.sb, F0.u);
-    k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, F0.r0, F0.r0, F0.sb, sig[2], F0.sa, F0.u);
-    k_mg_res0<<<ntiles, RSB_BLOCK, 0, st>>>(a, S, F0.r0, F0.r0, F0.sa, 0.0, nullptr, F0.u);
+    k_mg_res0<<<ntiles, MG_RT, 0, st>>>(a, S, r, F0.r0, F0.sa, sig[1], F0.sb, F0.u);
+    k_mg_res0<<<ntiles, MG_RT, 0, st>>>(a, S, F0.r0, F0.r0, F0.sb, sig[2], F0.sa, F0.u);
+    k_mg_res0<<<ntiles, MG_RT, 0, st>>>(a, S, F0.r0, F0.r0, F0.sa, 0.0, nullptr, F0.u);
     for (int l = 1; l < l0; l++) {
       mg_level_dev &F = H.lv[l], &D = H.lv[l - 1];
       const mg_csr M{F.m, F.rseg, F.soff, F.rlen, F.sci, F.sw, F.diag, F.spk};
@@ -1832,7 +1942,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
     k_mg_center_dot<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_INV, x);
     fin(FIN_NORM, GATE_INV, 1);
     k_mg_scale_sum<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_INV, x, b);
-    k_mg_zero<<<1, 1, 0, st>>>(active);
+    k_mg_zero<<<1, 1, 0, st>>>(active + 2);
     fin(FIN_PASSEND, GATE_INV, 1);
     k_mg_center<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_INV, b);
     RSB_LAUNCH_CHECK();
@@ -1850,7 +1960,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
       gfin(GF_NORM);
       k_mg_gnew<<<ntiles, RSB_BLOCK, 0, st>>>(a, G, mpad, r, b, p);
       gfin(GF_CNEW);
-      k_mg_apply<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_GRAM, S, p, w);
+      k_mg_apply<<<ntiles, MG_RT, 0, st>>>(a, GATE_GRAM, S, p, w);
       k_mg_gdots<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_GRAM, mpad, G.GZ, w, G.GZ, 1, p);
       gfin(GF_MROW);
       k_mg_gdots<<<ntiles, RSB_BLOCK, 0, st>>>(a, GATE_GRAM, mpad, G.Z, nullptr, nullptr, 0, w);
