@@ -1944,7 +1944,6 @@ __global__ void __launch_bounds__(NT) k_lz_fin(lz_args a, int op) {
       }
       if (k == a.miter[s] && np < a.mpass && !stalled) {
         a.status[s] = LZ_SETUP;
-        atomicAdd(&a.running[1], 1);
       } else {
         a.status[s] = LZ_FINISHED;
       }
@@ -1982,6 +1981,9 @@ struct lz_fuse {
   const double *pa_in;  // partials of the launch before; those of this one go to lz_args.partial
 };
 #define LZ_FUSE_TILES 1024  // most tiles of a segment (see run_lanczos)
+// iterations queued between a compaction and the look at its lengths: two of
+// 5 to 10 us cover the host's look and its next launches
+#define LZ_AHEAD 2
 
 // Scalars after the apply's sums: mean of p, pap, alpha (FIN_APPLY).
 __device__ inline void step_apply(lz_it &x, double n, double sq, double swq, double sw) {
@@ -2342,6 +2344,16 @@ __global__ void k_lz_compact(lz_args a, int ntiles, int want, int *__restrict__ 
   if (i < a.nseg && a.status[i] == want) segs[atomicAdd(&counts[1], 1)] = i;
 }
 
+// The lists' lengths to the host's pinned ring (ring[2] = 1 once they are
+// there), cleared for the next compaction.
+__global__ void k_lz_report(int *counts, int *ring) {
+  const int n0 = counts[0], n1 = counts[1];
+  counts[0] = 0, counts[1] = 0;
+  __hip_atomic_store(ring, n0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(ring + 1, n1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(ring + 2, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void k_lz_init_state(lz_args a, int miter_opt) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= a.nseg) return;
@@ -2464,8 +2476,10 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   } while (0)
   // compacted lists of running tiles / segments for the iteration launches
   int *act = nullptr;
-  RSB_TRY(RSB_SCRATCH(act, sizeof(int) * ((size_t)ntiles + nseg + 2)));
-  int *act_t = act, *act_s = act + ntiles, *act_n = act + ntiles + nseg;
+  const size_t act_len = (size_t)ntiles + nseg;  // two copies, see compact_start
+  RSB_TRY(RSB_SCRATCH(act, sizeof(int) * (2 * act_len + 2)));
+  int *act_t = act, *act_s = act + ntiles, *act_n = act + 2 * act_len;
+  RSB_TRY(hipMemsetAsync(act_n, 0, sizeof(int) * 2, st));
   int nact[2] = {ntiles, nseg};
   // segments of at most LZ_FUSE_TILES tiles take the fused iterations: every
   // workgroup sums its segment's partials by itself
@@ -2481,7 +2495,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   lz_desc *desc = nullptr, *act_d = nullptr;
   lz_it *stt = nullptr;
   if (fuse && ntiles > 0) {
-    RSB_TRY(RSB_SCRATCH(desc, sizeof(lz_desc) * 2 * (size_t)ntiles));
+    RSB_TRY(RSB_SCRATCH(desc, sizeof(lz_desc) * 3 * (size_t)ntiles));
     act_d = desc + ntiles;
     RSB_TRY(RSB_SCRATCH(stt, sizeof(lz_it) * 2 * (size_t)nseg));
     a.st0 = stt + nseg;  // the copy the first launch of a pass reads
@@ -2489,17 +2503,44 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
     RSB_LAUNCH_CHECK();
   }
   double *const PA[2] = {L.partial, L.partial + (size_t)6 * std::max(g->lz_tile_cap, 1)};
-  auto compact = [&](int want) -> int {
-    RSB_TRY(hipMemsetAsync(act_n, 0, sizeof(int) * 2, st));
-    k_lz_compact<<<nblocks(std::max(ntiles, nseg), 256), 256, 0, st>>>(a, ntiles, want, act_t,
-                                                                        act_s, act_n, desc,
-                                                                        act_d);
+  lz_args ai = a;  // iteration launches over the running lists
+  // A compaction is queued by compact_start, into the copy of the lists that
+  // no launch reads, and taken up by compact_take once its lengths have
+  // arrived in pinned memory.  What is queued in between runs on the lists
+  // before (a finished segment's workgroups return at once) and keeps the
+  // device busy while the host looks: a copy and a wait after each left it
+  // idle for 20 to 45 us, three times a pass.  The graph replays hold the
+  // lists' addresses, so they keep one copy and wait.
+  int cur = 0;
+  auto compact_start = [&](int want) -> int {
+    const int to = use_graph ? cur : cur ^ 1;
+    __atomic_store_n(g->ring + 2, 0, __ATOMIC_RELEASE);
+    k_lz_compact<<<nblocks(std::max(ntiles, nseg), 256), 256, 0, st>>>(
+        a, ntiles, want, act + to * act_len, act + to * act_len + ntiles, act_n, desc,
+        desc ? desc + (size_t)(to + 1) * ntiles : nullptr);
+    k_lz_report<<<1, 1, 0, st>>>(act_n, g->ring);
     RSB_LAUNCH_CHECK();
-    RSB_TRY(hipMemcpyAsync(nact, act_n, sizeof(int) * 2, hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipStreamSynchronize(st));
     return 0;
   };
-  lz_args ai = a;  // iteration launches over the running lists
+  auto compact_take = [&]() -> int {
+    for (unsigned q = 1; !__atomic_load_n(g->ring + 2, __ATOMIC_ACQUIRE); q++)
+      if ((q & 0xffff) == 0) {
+        // a failed launch or a fault never reports: ask the stream
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) {
+          (void)hipGetLastError();
+          continue;
+        }
+        RSB_TRY(e);
+        if (!__atomic_load_n(g->ring + 2, __ATOMIC_ACQUIRE)) RSB_FAIL(2, "running lists not reported");
+      }
+    if (!use_graph) cur ^= 1;
+    nact[0] = g->ring[0], nact[1] = g->ring[1];
+    act_t = act + cur * act_len, act_s = act_t + ntiles;
+    if (desc) act_d = desc + (size_t)(cur + 1) * ntiles;
+    ai.act_tiles = act_t, ai.act_segs = act_s;
+    return 0;
+  };
   auto xgrid = [](int n) { return (unsigned)((n + LZ_XCDS - 1) / LZ_XCDS * LZ_XCDS); };
   ai.act_tiles = act_t, ai.act_segs = act_s;
   // The FP64 apply reads the 16-bit entries: with the 12-bit form it took
@@ -2614,19 +2655,21 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
       sizeof(double) * (2 * miter_max + miter_max * ((miter_max + RSB_WAVE - 1) / RSB_WAVE * RSB_WAVE));
   auto passes = [&](int np_max) -> int {
     a.mpass = ai.mpass = np_max;
-    // the running lists of a pass: compacted at the end of the pass before
-    // (the segments that restart are LZ_SETUP there and RUNNING once set up,
-    // which saves a device wait per pass), at its start for the first
-    bool lists_ok = false;
-    for (int pass = 0; pass < np_max; pass++) {
-      // r_0 into basis slot 0
+    // r_0 into basis slot 0
+    auto setup = [&]() -> int {
       k_lz_setup<T><<<ntiles, RSB_BLOCK, 0, st>>>(a, 0, f, basis, p);
       RSB_LAUNCH_CHECK();
       FIN(FIN_SETUP0);
       k_lz_setup<T><<<ntiles, RSB_BLOCK, 0, st>>>(a, 1, f, basis, p);
       RSB_LAUNCH_CHECK();
       FIN(FIN_SETUP1);
-      if (!lists_ok && compact(LZ_RUNNING)) return 2;
+      return 0;
+    };
+    // a pass's lists are those of the segments in LZ_SETUP before its setup,
+    // which is queued before their lengths are looked at (with no segment
+    // left to restart its launches return at the status)
+    if (compact_start(LZ_SETUP) || setup() || compact_take()) return 2;
+    for (int pass = 0; pass < np_max; pass++) {
       fold = nact[0] <= fold_tiles;
       RSB_TRY(hipEventRecord(g->lz_ev0, st));
       int it, nrec = 0;
@@ -2638,10 +2681,10 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
         for (size_t q = old; q < g->spmv_ev.size(); q++) RSB_TRY(hipEventCreate(&g->spmv_ev[q]));
       }
       // the running lists are compacted 8 iterations into the pass and then
-      // at intervals that double (up to 32) while no segment has finished:
-      // each compaction waits on the device, and a finished segment's tiles
-      // only cost launches whose workgroups return at once
-      int next_c = 7, step = 8;
+      // at intervals that double (up to 32) while no segment has finished (a
+      // finished segment's tiles only cost launches whose workgroups return
+      // at once), and taken up LZ_AHEAD iterations later
+      int next_c = 7, step = 8, take_at = -1;
       for (it = 0; it < miter_max; it++) {
         if (nact[0] == 0) break;
         if (use_graph && (it & 7) == 0 && it + 8 < miter_max) {
@@ -2667,7 +2710,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
           g->lz_launches += 8;
           it += 7;
           if (it + 1 < miter_max) {
-            if (compact(LZ_RUNNING)) return 2;
+            if (compact_start(LZ_RUNNING) || compact_take()) return 2;
             if (nact[1] == 0) break;
           }
           continue;
@@ -2685,13 +2728,17 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
         after_apply(it);
         RSB_LAUNCH_CHECK();
         g->lz_launches++;
-        if (it == next_c && it + 1 < miter_max) {
+        if (it == next_c && it + 1 + LZ_AHEAD < miter_max) {
           // drop segments that finished their pass from the launch lists
+          if (compact_start(LZ_RUNNING)) return 2;
+          take_at = it + LZ_AHEAD;
+        }
+        if (it == take_at) {
           const int before = nact[1];
-          if (compact(LZ_RUNNING)) return 2;
+          if (compact_take()) return 2;
           if (nact[1] == 0) break;
           step = nact[1] == before ? std::min(2 * step, 32) : 8;
-          next_c = it + step;
+          next_c += step;
         }
       }
       if (fuse && nact[1] > 0) {
@@ -2703,7 +2750,6 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
         RSB_LAUNCH_CHECK();
       }
       RSB_TRY(hipEventRecord(g->lz_ev1, st));
-      RSB_TRY(hipMemsetAsync(L.running + 1, 0, sizeof(int), st));
       if (long_pass) {
         // segments in chunks whose matrices take at most 1 GiB together
         const size_t zb = sizeof(double) * (size_t)miter_max * miter_max;
@@ -2724,14 +2770,13 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
       k_lz_ritz<T><<<ntiles, RSB_BLOCK, 0, st>>>(a, basis, mpad, f);
       RSB_LAUNCH_CHECK();
       FIN(FIN_RITZ);
-      if (compact(LZ_SETUP)) return 2;  // waits on the device
-      lists_ok = true;
-      int again = 0;
-      RSB_TRY(hipMemcpyAsync(&again, L.running + 1, sizeof(int), hipMemcpyDeviceToHost, st));
-      RSB_TRY(hipStreamSynchronize(st));
+      if (compact_start(LZ_SETUP)) return 2;
+      if (pass + 1 < np_max && setup()) return 2;
+      if (compact_take()) return 2;
       // the pass's events are complete now (one wait per pass end)
       if (gexec) RSB_TRY(hipGraphExecDestroy(gexec));
       float ms = 0.f;
+      RSB_TRY(hipEventSynchronize(g->lz_ev1));
       RSB_TRY(hipEventElapsedTime(&ms, g->lz_ev0, g->lz_ev1));
       g->lz_ms += ms;
       for (int q = 0; q < nrec; q++) {
@@ -2739,7 +2784,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
         g->spmv_ms += ms;
       }
       g->spmv_launches += nrec;
-      if (again == 0) break;
+      if (nact[1] == 0) break;
     }
     return 0;
   };

@@ -49,7 +49,7 @@ extern "C" int rsbgpu_open(rsbgpu **out, int device) {
   rsbgpu *g = new rsbgpu();
   g->device = device;
   hipEvent_t ev[4];
-  if (rsb_arena_stream(device, &g->stream, ev)) {
+  if (rsb_arena_stream(device, &g->stream, ev, &g->ring)) {
     // allocation-free call: the stream and events set up for this device
     g->ev0 = ev[0], g->ev1 = ev[1], g->lz_ev0 = ev[2], g->lz_ev1 = ev[3];
     g->borrowed = true;
@@ -58,14 +58,15 @@ extern "C" int rsbgpu_open(rsbgpu **out, int device) {
   }
   rsb_stream_set ss;
   if (rsb_pool_take_streams(device, &ss)) {
-    g->stream = ss.stream;
+    g->stream = ss.stream, g->ring = ss.ring;
     g->ev0 = ss.ev[0], g->ev1 = ss.ev[1], g->lz_ev0 = ss.ev[2], g->lz_ev1 = ss.ev[3];
     *out = g;
     return 0;
   }
   if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess ||
-      hipEventCreate(&g->lz_ev0) != hipSuccess || hipEventCreate(&g->lz_ev1) != hipSuccess) {
+      hipEventCreate(&g->lz_ev0) != hipSuccess || hipEventCreate(&g->lz_ev1) != hipSuccess ||
+      hipHostMalloc((void **)&g->ring, RSB_RING * sizeof(int), hipHostMallocCoherent) != hipSuccess) {
     delete g;
     return 2;
   }
@@ -149,12 +150,13 @@ extern "C" void rsbgpu_close(rsbgpu *g) {
   g->retired.clear();
   if (!g->borrowed) rsb_pool_tick(g->device);
   if (!g->borrowed &&
-      !(drained && rsb_pool_give_streams(g->device, {g->stream, {g->ev0, g->ev1, g->lz_ev0, g->lz_ev1}}))) {
+      !(drained && rsb_pool_give_streams(g->device, {g->stream, {g->ev0, g->ev1, g->lz_ev0, g->lz_ev1}, g->ring}))) {
     if (g->ev0) hipEventDestroy(g->ev0);
     if (g->ev1) hipEventDestroy(g->ev1);
     if (g->lz_ev0) hipEventDestroy(g->lz_ev0);
     if (g->lz_ev1) hipEventDestroy(g->lz_ev1);
     if (g->stream) hipStreamDestroy(g->stream);
+    if (g->ring) hipHostFree(g->ring);
   }
   delete g;
 }

@@ -1531,7 +1531,6 @@ struct mg_scope {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipEvent_t ev[2] = {nullptr, nullptr};
-  int *ring = nullptr;  // pinned: the counts that k_mg_report writes
   bool capturing = false;
   explicit mg_scope(hipStream_t s) : st(s) {}
   template <typename T>
@@ -1552,7 +1551,6 @@ struct mg_scope {
     if (graph) (void)hipGraphDestroy(graph);
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
-    if (ring) (void)hipHostFree(ring);
     for (void *q : bufs) rsb_dev_release(q);
   }
 };
@@ -1762,7 +1760,6 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   RSB_TRY(own.alloc(coef, sizeof(double) * MG_NP * (size_t)nseg));
   RSB_TRY(own.alloc(active, 3 * sizeof(int)));
   RSB_TRY(hipMemsetAsync(active, 0, 3 * sizeof(int), st));
-  RSB_TRY(hipHostMalloc((void **)&own.ring, MG_RING * sizeof(int), hipHostMallocDefault));
   for (hipEvent_t &e : own.ev) RSB_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   // Gram basis: at most one vector per pass that another pass follows
   mg_gram G{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, max_passes - 1};
@@ -1829,6 +1826,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   }
   while (low_threads < low_rows && low_threads < MG_LOW_THREADS) low_threads *= 2;
   low.stride = low_rows;
+  int *const ring = g->ring + 4;  // pinned: the counts that k_mg_report writes
   // One CG iteration is part_a (w = L p, alpha, the update of x and r, the
   // stop test) and part_b (z = V-cycle(r), beta, the new direction made
   // L-orthogonal to the earlier ones).  The count of running segments goes to
@@ -1840,7 +1838,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
     k_mg_update<<<ntiles, RSB_BLOCK, 0, st>>>(a, mpad, p, w, x, r, Wb, Pb, diag0, sig[0],
                                                H.lv[0].sa, H.lv[0].u);
     fin(FIN_CONV, GATE_PCG, 1);
-    k_mg_report<<<1, 1, 0, st>>>(active, own.ring);
+    k_mg_report<<<1, 1, 0, st>>>(active, ring);
     RSB_LAUNCH_CHECK();
     return 0;
   };
@@ -1912,7 +1910,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   };
   auto count_of = [&](int q, int &n) -> int {
     RSB_TRY(hipEventSynchronize(own.ev[q & 1]));
-    n = __atomic_load_n(own.ring + q % MG_RING, __ATOMIC_ACQUIRE);
+    n = __atomic_load_n(ring + q % MG_RING, __ATOMIC_ACQUIRE);
     return 0;
   };
   for (int pass = 0; pass < max_passes; pass++) {

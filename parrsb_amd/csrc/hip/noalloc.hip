@@ -39,12 +39,13 @@ constexpr int kMaxDevices = 64;
 
 // Set up once per device, with that device current: the device address of
 // `scratch` (host code never uses the array's name for device memory), and
-// the stream and four timing events every allocation-free call borrows.
+// the stream, four timing events and the ring every allocation-free call borrows.
 struct dev_setup {
   bool ready = false;
   unsigned char *ptr = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  int *ring = nullptr;
 };
 dev_setup setups[kMaxDevices];
 std::mutex setup_mu;
@@ -279,11 +280,12 @@ hipError_t rsb_dev_free(const void *p) {
   return hipFree((void *)p);
 }
 
-bool rsb_arena_stream(int device, hipStream_t *stream, hipEvent_t *ev) {
+bool rsb_arena_stream(int device, hipStream_t *stream, hipEvent_t *ev, int **ring) {
   if (!cur_active || cur_arena.device != device) return false;
   const dev_setup &d = setups[device];
   *stream = d.stream;
   for (int i = 0; i < 4; i++) ev[i] = d.ev[i];
+  *ring = d.ring;
   return true;
 }
 
@@ -312,6 +314,9 @@ extern "C" int rsbgpu_noalloc_begin(int device, char *msg, int msglen) {
       return fail(2, "hipStreamCreateWithFlags", e);
     for (int i = 0; i < 4; i++)
       if ((e = hipEventCreate(&d.ev[i])) != hipSuccess) return fail(2, "hipEventCreate", e);
+    if ((e = hipHostMalloc((void **)&d.ring, RSB_RING * sizeof(int), hipHostMallocCoherent)) !=
+        hipSuccess)
+      return fail(2, "hipHostMalloc", e);
     d.ptr = (unsigned char *)ptr;
     d.ready = true;
   }

@@ -30,13 +30,15 @@ void rsb_dev_release(const void *p);
 struct rsb_stream_set {
   hipStream_t stream;
   hipEvent_t ev[4];
+  int *ring;  // pinned: the counts a solve's kernels report to the host
 };
+#define RSB_RING 16  // ints of it
 bool rsb_pool_take_streams(int device, rsb_stream_set *out);
 bool rsb_pool_give_streams(int device, const rsb_stream_set &in);
 void rsb_pool_tick(int device);
-// Inside an allocation-free call on `device`: the stream and the four timing
-// events set up once for that device (returns false otherwise).
-bool rsb_arena_stream(int device, hipStream_t *stream, hipEvent_t *ev);
+// Inside an allocation-free call on `device`: the stream, the four timing
+// events and the ring set up once for that device (returns false otherwise).
+bool rsb_arena_stream(int device, hipStream_t *stream, hipEvent_t *ev, int **ring);
 
 #define RSB_TILE 1024   // Lanczos rows per block (4 rows per thread)
 #define RSB_BLOCK 256
@@ -176,6 +178,7 @@ struct rsbgpu {
   int prof_spmv = 0;                   // bracket every LZ_PROF_EVERY-th SpMV launch with events
   std::vector<hipEvent_t> spmv_ev;
   hipEvent_t lz_ev0 = nullptr, lz_ev1 = nullptr;
+  int *ring = nullptr;  // RSB_RING ints of pinned memory ([0..2] Lanczos lists, [4..7] MG counts)
   std::unordered_map<const void *, size_t> cap;  // bytes held by each dev_alloc slot
   // per-call scratch buffers, one per call site (file, line), kept across
   // calls while large enough and freed with the handle (rsb_scratch)
