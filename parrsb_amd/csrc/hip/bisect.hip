@@ -445,14 +445,8 @@ extern "C" int rsbgpu_bisect(rsbgpu *g, int *nlower, const int *sender, const in
   RSB_TRY(hipMemcpyAsync(g->d_fied, fied2, sizeof(double) * nel, hipMemcpyDeviceToDevice,
                          g->stream));
   std::vector<int> nlo(nseg), nif(nseg);
-  RSB_TRY(hipMemcpyAsync(nlo.data(), d_nlo, sizeof(int) * nseg, hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipMemcpyAsync(nif.data(), d_nif, sizeof(int) * nseg, hipMemcpyDeviceToHost,
-                         g->stream));
-  if (ncomp)
-    RSB_TRY(hipMemcpyAsync(ncomp, d_ncomp, sizeof(int) * 2 * nseg, hipMemcpyDeviceToHost,
-                           g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {nlo.data(), d_nlo, sizeof(int) * nseg}, {nif.data(), d_nif, sizeof(int) * nseg},
+           {ncomp, d_ncomp, ncomp ? sizeof(int) * 2 * nseg : 0});
   rsb_phase_end(g, PH_BAL);
   for (int s = 0; s < nseg; s++) {
     int mv = 0;
@@ -482,8 +476,7 @@ extern "C" int rsbgpu_write_part(rsbgpu *g, int *part, int part_is_device) {
   k_write_part<<<nblocks(nel, 256), 256, 0, g->stream>>>(g->d_segof, g->d_seg, g->nseg, nel, dp);
   RSB_LAUNCH_CHECK();
   if (!part_is_device) {
-    RSB_TRY(hipMemcpyAsync(part, dp, sizeof(int) * nel, hipMemcpyDeviceToHost, g->stream));
-    RSB_TRY(hipStreamSynchronize(g->stream));
+    RSB_READ(g, {part, dp, sizeof(int) * nel});
     rsb_dev_release(dp);
   } else {
     RSB_TRY(hipStreamSynchronize(g->stream));
@@ -510,8 +503,7 @@ extern "C" int rsbgpu_write_seq(rsbgpu *g, int *seq, int seq_is_device) {
   k_write_seq<<<nblocks(nel, 256), 256, 0, g->stream>>>(g->d_order, g->d_segof, g->d_seg, nel, dp);
   RSB_LAUNCH_CHECK();
   if (!seq_is_device) {
-    RSB_TRY(hipMemcpyAsync(seq, dp, sizeof(int) * nel, hipMemcpyDeviceToHost, g->stream));
-    RSB_TRY(hipStreamSynchronize(g->stream));
+    RSB_READ(g, {seq, dp, sizeof(int) * nel});
     rsb_dev_release(dp);
   } else {
     RSB_TRY(hipStreamSynchronize(g->stream));
@@ -568,8 +560,7 @@ extern "C" int rsbgpu_group_by_tag(rsbgpu *g, const int *tag, int tag_is_device,
   k_tag_heads<<<nblocks(nel, 256), 256, 0, st>>>(nel, key, max_groups, nh, heads);
   RSB_LAUNCH_CHECK();
   int n = 0;
-  RSB_TRY(hipMemcpyAsync(&n, nh, sizeof(int), hipMemcpyDeviceToHost, st));
-  RSB_TRY(hipStreamSynchronize(st));
+  RSB_READ(g, {&n, nh, sizeof(int)});
   *ngroups = n;
   if (n <= max_groups) {
     std::vector<int> h((size_t)n);
@@ -734,8 +725,7 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
     RSB_TRY(hipMemsetAsync(bad, 0, sizeof(int), g->stream));
     k_q_check<<<nblocks(nel, 256), 256, 0, g->stream>>>(nel, d_part, nparts, bad);
     RSB_LAUNCH_CHECK();
-    RSB_TRY(hipMemcpyAsync(&hb, bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-    RSB_TRY(hipStreamSynchronize(g->stream));
+    RSB_READ(g, {&hb, bad, sizeof(int)});
     rsb_dev_release(bad);
     if (hb) RSB_FAIL(3, "part ids outside [0, %d)", nparts);
   }
@@ -777,10 +767,7 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
   RSB_LAUNCH_CHECK();
   std::vector<int> hs(2 * (size_t)nparts);
   unsigned long long ha[4];
-  RSB_TRY(hipMemcpyAsync(hs.data(), size, sizeof(int) * 2 * nparts, hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipMemcpyAsync(ha, acc, sizeof(ha), hipMemcpyDeviceToHost, g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {hs.data(), size, sizeof(int) * 2 * nparts}, {ha, acc, sizeof(ha)});
   int64_t mx = 0, mn = INT64_MAX, tot = 0, cmx = 0, empty = 0;
   for (int q = 0; q < nparts; q++) {
     mx = std::max<int64_t>(mx, hs[q]);

@@ -2523,17 +2523,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
     return 0;
   };
   auto compact_take = [&]() -> int {
-    for (unsigned q = 1; !__atomic_load_n(g->ring + 2, __ATOMIC_ACQUIRE); q++)
-      if ((q & 0xffff) == 0) {
-        // a failed launch or a fault never reports: ask the stream
-        const hipError_t e = hipStreamQuery(st);
-        if (e == hipErrorNotReady) {
-          (void)hipGetLastError();
-          continue;
-        }
-        RSB_TRY(e);
-        if (!__atomic_load_n(g->ring + 2, __ATOMIC_ACQUIRE)) RSB_FAIL(2, "running lists not reported");
-      }
+    if (rsb_wait_flag(g, g->ring + 2)) return 2;
     if (!use_graph) cur ^= 1;
     nact[0] = g->ring[0], nact[1] = g->ring[1];
     act_t = act + cur * act_len, act_s = act_t + ntiles;
@@ -2805,8 +2795,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
     k_lz_fallback<<<nblocks(nseg, 256), 256, 0, st>>>(a, L.running + 1);
     RSB_LAUNCH_CHECK();
     int nfb = 0;
-    RSB_TRY(hipMemcpyAsync(&nfb, L.running + 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipStreamSynchronize(st));
+    RSB_READ(g, {&nfb, L.running + 1, sizeof(int)});
     if (nfb > 0 && ((rc = start(0, nullptr)) || (rc = passes(mpass)))) return rc;
   } else {
     if ((rc = start(init_mode == 2 ? 0 : init_mode, g->d_start)) || (rc = passes(mpass)))
@@ -2828,11 +2817,9 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   // read back per-segment results
   std::vector<int> ni(nseg), np(nseg);
   std::vector<double> sc((size_t)nseg * LZ_NSC);
-  RSB_TRY(hipMemcpyAsync(ni.data(), a.niter, sizeof(int) * nseg, hipMemcpyDeviceToHost, st));
-  RSB_TRY(hipMemcpyAsync(np.data(), a.npass, sizeof(int) * nseg, hipMemcpyDeviceToHost, st));
-  RSB_TRY(hipMemcpyAsync(sc.data(), a.sc, sizeof(double) * nseg * LZ_NSC,
-                         hipMemcpyDeviceToHost, st));
-  RSB_TRY(hipStreamSynchronize(st));
+  RSB_READ(g, {ni.data(), a.niter, sizeof(int) * nseg},
+           {np.data(), a.npass, sizeof(int) * nseg},
+           {sc.data(), a.sc, sizeof(double) * nseg * LZ_NSC});
   // Algorithmic bytes, per iteration and segment of n rows and nnz
   // off-diagonals: 4(n+1) row pointers + 4 nnz packed entries + 7 s n vector
   // streams for the whole iteration; for k_lz_apply alone 4(n+1) + 4 nnz +

@@ -164,12 +164,9 @@ extern "C" int rsbgpu_level_laplacian(rsbgpu *g) {
   RSB_LAUNCH_CHECK();
   int rc = rsb_exclusive_scan_i64(g, bytes, g->d_slice_off, g->nslices + 1);
   if (rc) return rc;
-  RSB_TRY(hipMemcpyAsync(&g->lnnz_pad, g->d_slice_off + g->nslices, sizeof(int64_t),
-                         hipMemcpyDeviceToHost, g->stream));
   g->h_seg_nnz.assign(g->nseg, 0);
-  RSB_TRY(hipMemcpyAsync(g->h_seg_nnz.data(), g->d_seg_nnz, sizeof(int64_t) * g->nseg,
-                         hipMemcpyDeviceToHost, g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {&g->lnnz_pad, g->d_slice_off + g->nslices, sizeof(int64_t)},
+           {g->h_seg_nnz.data(), g->d_seg_nnz, sizeof(int64_t) * g->nseg});
   g->lnnz = 0;
   for (int64_t v : g->h_seg_nnz) g->lnnz += v;
   RSB_TRY(dev_alloc(g, g->d_ell, (size_t)g->lnnz_pad));

@@ -4,6 +4,7 @@
 
 #include <algorithm>
 
+#include <cstring>
 #include "state.hpp"
 
 // ---------------------------------------------------------------------------
@@ -159,6 +160,70 @@ extern "C" void rsbgpu_close(rsbgpu *g) {
     if (g->ring) hipHostFree(g->ring);
   }
   delete g;
+}
+
+// ---------------------------------------------------------------------------
+// Small results to the host.  A copy into ordinary memory is staged by the
+// runtime and waited for twice (about 20 us with the stream's own wait, twenty
+// or thirty times a level); one workgroup writes the words into pinned memory
+// instead and the host looks for its flag.  Above RSB_RING_WORDS words the
+// copies are the faster way.
+struct read_args {
+  const int *src[4];
+  int words[4];
+};
+__global__ void __launch_bounds__(1024) k_read_back(read_args a, int *flag, int *out) {
+  int o = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    for (int i = threadIdx.x; i < a.words[k]; i += blockDim.x) out[o + i] = a.src[k][i];
+    o += a.words[k];
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+int rsb_wait_flag(rsbgpu *g, const int *flag) {
+  for (unsigned q = 1; !__atomic_load_n(flag, __ATOMIC_ACQUIRE); q++)
+    if ((q & 0xffff) == 0) {
+      // a failed launch or a fault never sets it: ask the stream
+      const hipError_t e = hipStreamQuery(g->stream);
+      if (e == hipErrorNotReady) {
+        (void)hipGetLastError();
+        continue;
+      }
+      RSB_TRY(e);
+      if (!__atomic_load_n(flag, __ATOMIC_ACQUIRE)) RSB_FAIL(2, "no report from the device");
+    }
+  return 0;
+}
+
+int rsb_read_back(rsbgpu *g, std::initializer_list<rsb_read> r) {
+  size_t bytes = 0;
+  bool ok = r.size() <= 4;
+  for (const rsb_read &x : r) bytes += x.bytes, ok &= x.bytes % sizeof(int) == 0;
+  if (!ok || bytes > sizeof(int) * RSB_RING_WORDS) {
+    for (const rsb_read &x : r)
+      if (x.bytes)
+        RSB_TRY(hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyDeviceToHost, g->stream));
+    RSB_TRY(hipStreamSynchronize(g->stream));
+    return 0;
+  }
+  read_args a{};
+  int k = 0;
+  for (const rsb_read &x : r) a.src[k] = (const int *)x.src, a.words[k++] = (int)(x.bytes / sizeof(int));
+  __atomic_store_n(g->ring + 8, 0, __ATOMIC_RELEASE);
+  k_read_back<<<1, bytes > 4096 ? 1024 : RSB_WAVE, 0, g->stream>>>(a, g->ring + 8, g->ring + 16);
+  RSB_LAUNCH_CHECK();
+  int rc = rsb_wait_flag(g, g->ring + 8);
+  if (rc) return rc;
+  const char *p = (const char *)(g->ring + 16);
+  for (const rsb_read &x : r) {
+    if (x.bytes) memcpy(x.dst, p, x.bytes);
+    p += x.bytes;
+  }
+  return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -338,11 +403,7 @@ static int build_ranks(rsbgpu *g) {
                                                           g->d_rank + (size_t)d * n);
     RSB_LAUNCH_CHECK();
     int last[2] = {0, 0};
-    RSB_TRY(hipMemcpyAsync(&last[0], excl + n - 1, sizeof(int), hipMemcpyDeviceToHost,
-                           g->stream));
-    RSB_TRY(hipMemcpyAsync(&last[1], flag + n - 1, sizeof(int), hipMemcpyDeviceToHost,
-                           g->stream));
-    RSB_TRY(hipStreamSynchronize(g->stream));
+    RSB_READ(g, {&last[0], excl + n - 1, sizeof(int)}, {&last[1], flag + n - 1, sizeof(int)});
     uint32_t mr = (uint32_t)(last[0] + last[1]);
     maxrank = std::max(maxrank, mr);
   }
@@ -372,8 +433,7 @@ static int build_graph(rsbgpu *g) {
       g->d_vtx, ns, key, val, vmax);
   RSB_LAUNCH_CHECK();
   unsigned long long hmax = 0;
-  RSB_TRY(hipMemcpyAsync(&hmax, vmax, sizeof(hmax), hipMemcpyDeviceToHost, g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {&hmax, vmax, sizeof(hmax)});
   g->vmax = hmax;
   int bits = 1;
   while (bits < 64 && (1ull << bits) <= hmax) bits++;
@@ -384,11 +444,8 @@ static int build_graph(rsbgpu *g) {
   rc = rsb_exclusive_scan_i32(g, flag, excl, ns);
   if (rc) return rc;
   int ng_parts[2];
-  RSB_TRY(hipMemcpyAsync(&ng_parts[0], excl + ns - 1, sizeof(int), hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipMemcpyAsync(&ng_parts[1], flag + ns - 1, sizeof(int), hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {&ng_parts[0], excl + ns - 1, sizeof(int)},
+           {&ng_parts[1], flag + ns - 1, sizeof(int)});
   int ng = ng_parts[0] + ng_parts[1];
   RSB_TRY(rsb_dev_malloc((void **)&slot_group, sizeof(int) * (ns + 1)));
   RSB_TRY(rsb_dev_malloc((void **)&gstart, sizeof(int) * (ng + 1)));
@@ -412,9 +469,7 @@ static int build_graph(rsbgpu *g) {
   RSB_LAUNCH_CHECK();
   rc = rsb_exclusive_scan_i64(g, rowlen, g->d_growptr, (int64_t)n + 1);
   if (rc) return rc;
-  RSB_TRY(hipMemcpyAsync(&g->gnnz, g->d_growptr + n, sizeof(int64_t), hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {&g->gnnz, g->d_growptr + n, sizeof(int64_t)});
   RSB_TRY(dev_alloc(g, g->d_gadj, (size_t)g->gnnz));
   k_dual_rows<true><<<nblocks(n, 128), 128, 0, g->stream>>>(
       n, g->nv, slot_group, gstart, val, nullptr, g->d_growptr, g->d_gadj, ovf);
@@ -426,9 +481,7 @@ static int build_graph(rsbgpu *g) {
   }
   int hovf = 0;
   unsigned long long ws = 0;
-  RSB_TRY(hipMemcpyAsync(&hovf, ovf, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-  RSB_TRY(hipMemcpyAsync(&ws, vmax, sizeof(ws), hipMemcpyDeviceToHost, g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {&hovf, ovf, sizeof(int)}, {&ws, vmax, sizeof(ws)});
   g->gwsum = (int64_t)ws;
   for (const void *p : {(const void *)key, (const void *)flag, (const void *)excl,
                         (const void *)val, (const void *)slot_group, (const void *)gstart,
@@ -518,9 +571,7 @@ extern "C" int rsbgpu_get_graph(rsbgpu *g, int64_t *rowptr, int *col, int *wgt) 
     RSB_TRY(rsb_dev_malloc((void **)&dw, sizeof(int) * g->gnnz));
     k_unpack_adj<<<nblocks(g->gnnz, 256), 256, 0, g->stream>>>(g->d_gadj, g->gnnz, dc, dw);
     RSB_LAUNCH_CHECK();
-    RSB_TRY(hipMemcpyAsync(col, dc, sizeof(int) * g->gnnz, hipMemcpyDeviceToHost, g->stream));
-    RSB_TRY(hipMemcpyAsync(wgt, dw, sizeof(int) * g->gnnz, hipMemcpyDeviceToHost, g->stream));
-    RSB_TRY(hipStreamSynchronize(g->stream));
+    RSB_READ(g, {col, dc, sizeof(int) * g->gnnz}, {wgt, dw, sizeof(int) * g->gnnz});
     rsb_dev_free(dc), rsb_dev_free(dw);
   }
   RSB_TRY(hipStreamSynchronize(g->stream));
@@ -529,25 +580,19 @@ extern "C" int rsbgpu_get_graph(rsbgpu *g, int64_t *rowptr, int *col, int *wgt) 
 
 extern "C" int rsbgpu_get_centroids(rsbgpu *g, double *coord) {
   RSB_TRY(hipSetDevice(g->device));
-  RSB_TRY(hipMemcpyAsync(coord, g->d_coord, sizeof(double) * 3 * (size_t)g->nel,
-                         hipMemcpyDeviceToHost, g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {coord, g->d_coord, sizeof(double) * 3 * (size_t)g->nel});
   return 0;
 }
 
 extern "C" int rsbgpu_get_order(rsbgpu *g, int *order) {
   RSB_TRY(hipSetDevice(g->device));
-  RSB_TRY(hipMemcpyAsync(order, g->d_order, sizeof(int) * (size_t)g->nel, hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {order, g->d_order, sizeof(int) * (size_t)g->nel});
   return 0;
 }
 
 extern "C" int rsbgpu_get_fiedler(rsbgpu *g, double *f) {
   RSB_TRY(hipSetDevice(g->device));
-  RSB_TRY(hipMemcpyAsync(f, g->d_fied, sizeof(double) * (size_t)g->nel, hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {f, g->d_fied, sizeof(double) * (size_t)g->nel});
   return 0;
 }
 

@@ -1621,8 +1621,7 @@ static int mg_build(rsbgpu *g, int factor, mg_hier &H, double *diag0) {
     RSB_LAUNCH_CHECK();
     MG_TRY(rsb_exclusive_scan_i64(g, cnt, roff, mc + 1));
     int64_t nr = 0;
-    RSB_TRY(hipMemcpyAsync(&nr, roff + mc, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipStreamSynchronize(st));
+    RSB_READ(g, {&nr, roff + mc, sizeof(int64_t)});
     if (nr >= (int64_t)1 << 31) RSB_FAIL(2, "MG level has too many entries");
     uint64_t *key = nullptr;
     int *idx = nullptr, *flag = nullptr, *rowcnt = nullptr;
@@ -1654,8 +1653,7 @@ static int mg_build(rsbgpu *g, int factor, mg_hier &H, double *diag0) {
     k_mg_widen<<<nblocks(mc + 1, 256), 256, 0, st>>>(mc + 1, rowcnt, rc64);
     MG_TRY(rsb_exclusive_scan_i64(g, rc64, C.rp, mc + 1));
     int64_t nnz = 0;
-    RSB_TRY(hipMemcpyAsync(&nnz, C.rp + mc, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipStreamSynchronize(st));
+    RSB_READ(g, {&nnz, C.rp + mc, sizeof(int64_t)});
     RSB_TRY(rsb_dev_malloc((void **)&C.ci, sizeof(int) * (size_t)std::max<int64_t>(nnz, 1)));
     RSB_TRY(rsb_dev_malloc((void **)&C.w, sizeof(double) * (size_t)std::max<int64_t>(nnz, 1)));
     if (nr > 0) k_mg_compact<<<nblocks(nr, 256), 256, 0, st>>>(nr, key, flag, pos, wsum, C.ci, C.w);
@@ -1672,8 +1670,6 @@ static int mg_build(rsbgpu *g, int factor, mg_hier &H, double *diag0) {
       RSB_LAUNCH_CHECK();
       MG_TRY(rsb_exclusive_scan_i64(g, sbytes, C.soff, nsl + 1));
       int64_t ns = 0;
-      RSB_TRY(hipMemcpyAsync(&ns, C.soff + nsl, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-      RSB_TRY(hipStreamSynchronize(st));
       // one packed word per entry where the row index fits in 24 bits and
       // the weights in 8 (the large coarse levels), two ints otherwise
       int *dmax = nullptr, hmax = 0;
@@ -1683,8 +1679,7 @@ static int mg_build(rsbgpu *g, int factor, mg_hier &H, double *diag0) {
         k_mg_wmax<<<std::min<int64_t>(nblocks(nnz, 256), 2048), 256, 0, st>>>(nnz, C.w, dmax);
         RSB_LAUNCH_CHECK();
       }
-      RSB_TRY(hipMemcpyAsync(&hmax, dmax, sizeof(int), hipMemcpyDeviceToHost, st));
-      RSB_TRY(hipStreamSynchronize(st));
+      RSB_READ(g, {&ns, C.soff + nsl, sizeof(int64_t)}, {&hmax, dmax, sizeof(int)});
       if (mc <= (1 << 24) && hmax < 256) {
         RSB_TRY(rsb_dev_malloc((void **)&C.spk, sizeof(uint32_t) * (size_t)std::max<int64_t>(ns, 1)));
       } else {
@@ -1791,8 +1786,7 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
     k_mg_fin<<<nseg, RSB_BLOCK, 0, st>>>(a, op, gate, nslots);
   };
   auto count_active = [&](int &n) -> int {
-    RSB_TRY(hipMemcpyAsync(&n, active + 2, sizeof(int), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipStreamSynchronize(st));
+    RSB_READ(g, {&n, active + 2, sizeof(int)});
     return 0;
   };
   // start vector, orthogonalised and normalised (fiedler.c:572-585)
@@ -1981,9 +1975,8 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   RSB_LAUNCH_CHECK();
   std::vector<int> hs((size_t)MI_NI * nseg);
   std::vector<double> hsc((size_t)MS_NSC * nseg);
-  RSB_TRY(hipMemcpyAsync(hs.data(), stt, sizeof(int) * hs.size(), hipMemcpyDeviceToHost, st));
-  RSB_TRY(hipMemcpyAsync(hsc.data(), sc, sizeof(double) * hsc.size(), hipMemcpyDeviceToHost, st));
-  RSB_TRY(hipStreamSynchronize(st));
+  RSB_READ(g, {hs.data(), stt, sizeof(int) * hs.size()},
+           {hsc.data(), sc, sizeof(double) * hsc.size()});
   for (int s = 0; s < nseg; s++) {
     if (!(g->h_p[s] > 1 && g->h_n[s] >= 2)) continue;
     if (out->niter) out->niter[s] = hs[(size_t)s * MI_NI + MI_ITERS];

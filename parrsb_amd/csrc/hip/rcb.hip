@@ -1175,9 +1175,7 @@ static int run_rib(rsbgpu *g) {
     int rc = rsb_exclusive_scan_i32(g, ccnt, cfirst, K);
     if (rc) return rc;
     int tail[2];
-    RSB_TRY(hipMemcpyAsync(&tail[0], cfirst + K - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipMemcpyAsync(&tail[1], ccnt + K - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipStreamSynchronize(st));
+    RSB_READ(g, {&tail[0], cfirst + K - 1, sizeof(int)}, {&tail[1], ccnt + K - 1, sizeof(int)});
     const int C = tail[0] + tail[1];
     if ((size_t)C > ccap) RSB_FAIL(2, "RIB chunk table overflow (%d > %zu)", C, ccap);
     if (C > 0) {
@@ -1207,9 +1205,7 @@ static int run_rib(rsbgpu *g) {
     k_child_count<<<nblocks(K, 256), 256, 0, st>>>(K, A, cnt);
     RSB_LAUNCH_CHECK();
     if ((rc = rsb_exclusive_scan_i32(g, cnt, first, K))) return rc;
-    RSB_TRY(hipMemcpyAsync(&tail[0], first + K - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipMemcpyAsync(&tail[1], cnt + K - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipStreamSynchronize(st));
+    RSB_READ(g, {&tail[0], first + K - 1, sizeof(int)}, {&tail[1], cnt + K - 1, sizeof(int)});
     const int K2 = tail[0] + tail[1];
     if ((size_t)K2 > cap) RSB_FAIL(2, "RIB node table overflow (%d > %zu)", K2, cap);
     k_children<<<nblocks(K, 256), 256, 0, st>>>(K, A, first, B, split, nullptr);

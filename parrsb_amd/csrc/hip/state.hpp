@@ -5,6 +5,7 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <initializer_list>
 #include <map>
 #include <unordered_map>
 #include <vector>
@@ -32,7 +33,8 @@ struct rsb_stream_set {
   hipEvent_t ev[4];
   int *ring;  // pinned: the counts a solve's kernels report to the host
 };
-#define RSB_RING 16  // ints of it
+#define RSB_RING_WORDS 8192
+#define RSB_RING (16 + RSB_RING_WORDS)  // ints of it
 bool rsb_pool_take_streams(int device, rsb_stream_set *out);
 bool rsb_pool_give_streams(int device, const rsb_stream_set &in);
 void rsb_pool_tick(int device);
@@ -178,7 +180,7 @@ struct rsbgpu {
   int prof_spmv = 0;                   // bracket every LZ_PROF_EVERY-th SpMV launch with events
   std::vector<hipEvent_t> spmv_ev;
   hipEvent_t lz_ev0 = nullptr, lz_ev1 = nullptr;
-  int *ring = nullptr;  // RSB_RING ints of pinned memory ([0..2] Lanczos lists, [4..7] MG counts)
+  int *ring = nullptr;  // RSB_RING ints of pinned memory: [0..2] Lanczos lists, [4..7] MG counts, [8] and [16..] rsb_read_back
   std::unordered_map<const void *, size_t> cap;  // bytes held by each dev_alloc slot
   // per-call scratch buffers, one per call site (file, line), kept across
   // calls while large enough and freed with the handle (rsb_scratch)
@@ -206,6 +208,23 @@ inline size_t rsb_grown(const rsbgpu *g, size_t bytes, size_t old) {
 
 // ---------------------------------------------------------------------------
 // error helpers
+// Results that the host needs before it can go on, at most four arrays of
+// 4-byte multiples: waits for the stream's work so far.
+struct rsb_read {
+  void *dst;
+  const void *src;
+  size_t bytes;
+};
+int rsb_read_back(rsbgpu *g, std::initializer_list<rsb_read> r);
+#define RSB_READ(g, ...)                          \
+  do {                                            \
+    int rc_ = rsb_read_back((g), {__VA_ARGS__});  \
+    if (rc_) return rc_;                          \
+  } while (0)
+// Wait until a kernel on the stream has set *flag (pinned); 2 if the stream
+// ended or failed without doing so.
+int rsb_wait_flag(rsbgpu *g, const int *flag);
+
 #define RSB_TRY(expr)                                                           \
   do {                                                                          \
     hipError_t e_ = (expr);                                                     \

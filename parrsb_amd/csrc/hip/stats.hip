@@ -102,8 +102,7 @@ extern "C" int rsbgpu_neighbors(rsbgpu *g, int *nbrs) {
                                                   g->d_segof, table, (unsigned)(slots - 1), nb,
                                                   nb + nseg);
     RSB_LAUNCH_CHECK();
-    RSB_TRY(hipMemcpyAsync(h.data(), nb, sizeof(int) * h.size(), hipMemcpyDeviceToHost, st));
-    RSB_TRY(hipStreamSynchronize(st));
+    RSB_READ(g, {h.data(), nb, sizeof(int) * h.size()});
     if (!h[nseg]) break;
     if (slots >= ((int64_t)1 << 31)) RSB_FAIL(2, "too many neighbour pairs");
   }

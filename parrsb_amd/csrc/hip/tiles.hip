@@ -446,10 +446,7 @@ int rsb_level_e12(rsbgpu *g) {
   if (rc) return rc;
   int64_t n12 = 0;
   int bad = 1;
-  RSB_TRY(hipMemcpyAsync(&n12, g->d_off12 + ns, sizeof(int64_t), hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipMemcpyAsync(&bad, g->d_e12_bad, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {&n12, g->d_off12 + ns, sizeof(int64_t)}, {&bad, g->d_e12_bad, sizeof(int)});
   if (bad) return 0;  // a weight other than 1, 2 or 4, or a slice of too many slots
   RSB_TRY(dev_alloc(g, g->d_e12, (size_t)n12 + 8));
   k_tile_e12<<<nt, RSB_BLOCK, 0, g->stream>>>(g->d_tile, g->d_off16, g->d_w16, g->d_e16,
@@ -463,9 +460,7 @@ int rsb_level_e12(rsbgpu *g) {
 static int level_nwide(rsbgpu *g) {
   if (g->nwide >= 0) return 0;
   std::vector<int> nh((size_t)g->ntiles);
-  RSB_TRY(hipMemcpyAsync(nh.data(), g->d_tnhalo, sizeof(int) * nh.size(), hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {nh.data(), g->d_tnhalo, sizeof(int) * nh.size()});
   g->nwide = 0;
   for (int v : nh) g->nwide += v < 0;
   return 0;
@@ -689,9 +684,7 @@ int rsb_build_vtiles(rsbgpu *g) {
   int rc = rsb_exclusive_scan_i64(g, nl, g->d_vt_loff, nt + 1);
   if (rc) return rc;
   int64_t tl = 0;
-  RSB_TRY(hipMemcpyAsync(&tl, g->d_vt_loff + nt, sizeof(int64_t), hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {&tl, g->d_vt_loff + nt, sizeof(int64_t)});
   RSB_TRY(dev_alloc(g, g->d_vt_list, (size_t)tl + 8));
   RSB_TRY(dev_alloc(g, g->d_vt_rowv, (size_t)g->mpad * 8 + 8));
   k_vt_fill<<<nt, RSB_BLOCK, 0, g->stream>>>(in, g->d_vt_n, g->d_vt_loff, g->d_vt_list,
@@ -709,9 +702,7 @@ extern "C" int rsbgpu_level_form(rsbgpu *g, int *wide_tiles, int *vertex_tiles) 
   *vertex_tiles = 0;
   if (!g->vt_ok || g->ntiles == 0) return 0;
   std::vector<int> vn(g->ntiles);
-  RSB_TRY(hipMemcpyAsync(vn.data(), g->d_vt_n, sizeof(int) * g->ntiles, hipMemcpyDeviceToHost,
-                         g->stream));
-  RSB_TRY(hipStreamSynchronize(g->stream));
+  RSB_READ(g, {vn.data(), g->d_vt_n, sizeof(int) * g->ntiles});
   for (int v : vn) *vertex_tiles += v >= 0;
   return 0;
 }
