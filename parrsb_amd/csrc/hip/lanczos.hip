@@ -4,11 +4,12 @@
 // Rows of the level are grouped in tiles of RSB_TILE rows that never cross a
 // segment, one workgroup per tile.  Each workgroup writes the partial sums of
 // its tile (fixed reduction tree), so results do not depend on block
-// scheduling.  The segment totals and scalar updates are done by a small
-// k_lz_fin launch after each reduction (one workgroup per segment), so no
-// workgroup ever waits on another inside a launch.  One CG-Lanczos
-// iteration is two launches over all rows of the level, each followed by
-// its k_lz_fin:
+// scheduling.  The segment totals and scalar updates are formed by the launch
+// that needs them (segments of at most LZ_FUSE_TILES tiles, "Fused
+// iterations" below) or by a small k_lz_fin launch after each reduction (one
+// workgroup per segment), so no workgroup ever waits on another inside a
+// launch.  One CG-Lanczos iteration is two launches over all rows of the
+// level:
 //   k_lz_apply    p = beta (p_old - mean) + r formed on the fly for each row
 //                 and its neighbours (staged in LDS per tile), w = L p from the
 //                 tile's 12- or 16-bit entries (the SELL-64 global form where a
@@ -1980,7 +1981,11 @@ struct lz_fuse {
   lz_it *st_out;
   const double *pa_in;  // partials of the launch before; those of this one go to lz_args.partial
 };
-#define LZ_FUSE_TILES 1024  // most tiles of a segment (see run_lanczos)
+// most tiles of a segment: one round of four loads per thread covers the
+// partials.  Whole calls at 1,024 / 512 / 256 / 0 (separate launches): 1M
+// hexes FP64 78.7 / 80.3 / 82.1 / 86.2 ms, FP32 60.9 / 61.3 / 62.4 / 64.6, 2M
+// pipe 702 / 704 / 707 / 739, 260k quads 239 / 239 / 239 / 302
+#define LZ_FUSE_TILES 1024
 // iterations queued between a compaction and the look at its lengths: two of
 // 5 to 10 us cover the host's look and its next launches
 #define LZ_AHEAD 2
