@@ -44,7 +44,6 @@ struct lz_args {
   int *status, *iter, *k, *npass, *niter, *miter;
   double *sc, *T, *y, *partial;
   double *rn;  // (miter_max + 1) per segment: 1 / |r_j|
-  int *running;
   int mpass;
   int mode;  // start vector: 0 reference, 1 caller per element, 2 learned per row
   int max_n; // mode 2: segments with more rows take the reference start
@@ -1822,7 +1821,6 @@ __device__ inline void rupdate_step(const lz_args &a, int s, double rtr) {
   if (rnorm < SC(s, SC_RTOL) || it + 1 == mi) {
     a.k[s] = it + 1;
     a.status[s] = LZ_PASSDONE;
-    atomicSub(&a.running[0], 1);
   } else {
     a.iter[s] = it + 1;
     SC(s, SC_RTZ2) = rtz1;
@@ -1892,7 +1890,6 @@ __global__ void __launch_bounds__(NT) k_lz_fin(lz_args a, int op) {
       if (a.st0) a.st0[s] = lz_it{rtr, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, rn * a.tol, -1, a.miter[s]};
       a.iter[s] = 0;
       a.status[s] = LZ_RUNNING;
-      atomicAdd(&a.running[0], 1);
       break;
     }
     case FIN_APPLY: {  // mean of p, pap = w.(p - mean), alpha (fiedler.c:470-478)
@@ -2027,7 +2024,6 @@ __device__ inline bool step_update(const lz_args &a, int s, lz_it &x, double rtr
       a.iter[s] = it;
       a.k[s] = it + 1;
       a.status[s] = LZ_PASSDONE;
-      atomicSub(&a.running[0], 1);
     }
   }
   if (stop) return false;
@@ -2450,7 +2446,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
     RSB_TRY(rsb_dev_malloc((void **)&L.partial, sizeof(double) * 12 * cap));
     g->lz_tile_cap = cap;
   }
-  if (!L.running) RSB_TRY(rsb_dev_malloc((void **)&L.running, sizeof(int) * 2));
+  if (!L.count) RSB_TRY(rsb_dev_malloc((void **)&L.count, sizeof(int)));
   lz_args a;
   a.st0 = nullptr;
   a.act_tiles = nullptr, a.act_segs = nullptr;
@@ -2458,8 +2454,7 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   a.nseg = nseg;
   a.status = L.status, a.iter = L.iter, a.k = L.k, a.npass = L.npass, a.niter = L.niter;
   a.miter = L.status + 5 * std::max(g->lz_nseg_cap, 1);
-  a.sc = L.sc, a.T = L.T, a.y = L.y, a.partial = L.partial, a.rn = L.rn,
-  a.running = L.running;
+  a.sc = L.sc, a.T = L.T, a.y = L.y, a.partial = L.partial, a.rn = L.rn;
   a.mpass = mpass, a.mode = init_mode, a.tol = tol, a.miter_max = miter_max;
   {
     const char *sv = getenv("PARRSB_AMD_LZ_STALL"), *sm = getenv("PARRSB_AMD_LZ_STALL_MIN");
@@ -2626,7 +2621,6 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
     }
   };
 
-  RSB_TRY(hipMemsetAsync(L.running, 0, sizeof(int) * 2, st));
   k_lz_init_state<<<nblocks(nseg, 256), 256, 0, st>>>(a, miter_opt);
   RSB_LAUNCH_CHECK();
   k_lz_zero_small<<<nblocks(nseg, 256), 256, 0, st>>>(a, g->d_fied);
@@ -2796,11 +2790,11 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
     float *srow = (float *)w;
     if ((rc = rsb_lws_predict(g, g->lws_params, g->lws_level, srow))) return rc;
     if ((rc = start(2, srow)) || (rc = passes(std::min(g->lws_passes, mpass)))) return rc;
-    RSB_TRY(hipMemsetAsync(L.running + 1, 0, sizeof(int), st));
-    k_lz_fallback<<<nblocks(nseg, 256), 256, 0, st>>>(a, L.running + 1);
+    RSB_TRY(hipMemsetAsync(L.count, 0, sizeof(int), st));
+    k_lz_fallback<<<nblocks(nseg, 256), 256, 0, st>>>(a, L.count);
     RSB_LAUNCH_CHECK();
     int nfb = 0;
-    RSB_READ(g, {&nfb, L.running + 1, sizeof(int)});
+    RSB_READ(g, {&nfb, L.count, sizeof(int)});
     if (nfb > 0 && ((rc = start(0, nullptr)) || (rc = passes(mpass)))) return rc;
   } else {
     if ((rc = start(init_mode == 2 ? 0 : init_mode, g->d_start)) || (rc = passes(mpass)))

@@ -138,7 +138,7 @@ extern "C" void rsbgpu_close(rsbgpu *g) {
   FREE(g->lz.y);
   FREE(g->lz.partial);
   FREE(g->lz.rn);
-  FREE(g->lz.running);
+  FREE(g->lz.count);
   FREE(g->d_sort_tmp);
   FREE(g->d_k0);
   FREE(g->d_k1);

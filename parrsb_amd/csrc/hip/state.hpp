@@ -60,7 +60,7 @@ struct lz_state {
   double *y;       // miter per segment: Ritz coefficients
   double *partial; // 6 per tile
   double *rn;      // miter + 1 per segment: 1 / |r_j| of the pass's residuals
-  int *running;    // count of RUNNING segments
+  int *count;      // segments that the learned start's fallback solves again
 };
 enum { LZ_IDLE = 0, LZ_SETUP = 1, LZ_RUNNING = 2, LZ_PASSDONE = 3, LZ_FINISHED = 4 };
 // scalar slots
