@@ -1,5 +1,7 @@
 """Level kernels at the sizes where their forms change: LDS sorts, LDS sets of
 neighbouring segments, 32- and 64-bit quality keys."""
+import time
+
 import numpy as np
 import pytest
 
@@ -33,6 +35,39 @@ def test_fiedler_sort_is_the_stable_sort(n):
         o, g = d.order(), d.fiedler_values()
     want = np.r_[np.argsort(f[:n], kind="stable"), np.arange(n, n + 50)]
     assert np.array_equal(o, want) and np.array_equal(g, f[want])
+
+
+@pytest.mark.parametrize("size", [1, 2, 25, 26, 40])
+def test_fiedler_sort_of_many_small_segments(size):
+    """Segments so small that a workgroup each takes longer than device-wide
+    sorts: the stable order on both sides of the rule (65,536 elements: LDS
+    from 26 elements a segment on), and no more than a few times one large
+    segment's time for segments of one element, where a workgroup each took
+    2.3 ms of device time against 0.1."""
+    print("fsort small", size, flush=True)
+    vtx, xyz, nv = M.box_hex(32, 32, 64, jitter=0.0)
+    rng = np.random.default_rng(size)
+    f = rng.integers(-3, 3, vtx.shape[0]) * 0.25
+    took = {}
+    with _dev() as d:
+        d.set_mesh(vtx, xyz, nv)
+        n = vtx.shape[0]
+        for ln in (size, n):
+            start = np.arange(0, n, ln)
+            cnt = np.minimum(ln, n - start)
+            for _ in range(4):
+                d.set_segments(start, cnt, np.full(start.size, 2), 2 * np.arange(start.size))
+                d.set_fiedler_values(f)
+                at = d.order()  # the elements' own order; also waits
+                t0 = time.perf_counter()
+                d.fiedler_sort()
+                got = d.order()
+                took[ln] = min(took.get(ln, 1.0), time.perf_counter() - t0)
+            want = np.concatenate([b + np.argsort(f[b:b + c], kind="stable")
+                                   for b, c in zip(start, cnt)])
+            assert np.array_equal(got, at[want])
+    if size == 1:
+        assert took[size] < 6 * took[n], took
 
 
 @pytest.mark.parametrize("size", [1, 3, 40, 700])
