@@ -27,25 +27,37 @@ static int ensure_kv(rsbgpu *g, size_t n) {
   return 0;
 }
 
-// Above SORT_MERGE_MAX items the radix sort's single-pass (onesweep) form,
-// below it the merge sort: a merge sort makes a launch per doubling from its
-// block size up.
-#define SORT_MERGE_MAX 65536
-typedef rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
-                                   rocprim::default_config, SORT_MERGE_MAX>
-    sort_cfg;
+// The radix sort's single-pass (onesweep) form costs about 22 us per 8 key
+// bits whatever the size, the merge sort about one launch per doubling.  Pairs,
+// merge / onesweep in us: 200,000 keys of 64 bits 75 / 207, of 32 bits 60 / 120,
+// of 12 bits 59 / 63; 300,000 keys of 64 bits 130 / 215, of 32 bits 120 / 121,
+// of 20 bits 118 / 92; 1M keys of 64 bits 199 / 242, of 44 bits 194 / 183, of
+// 32 bits 164 / 135; 1.5M keys of 64 bits 234 / 262, of 44 bits 227 / 199.
+static bool sort_by_merging(int64_t n, int bits) {
+  return n <= (bits > 32 ? 1 << 20 : 1 << 18);
+}
+template <unsigned MERGE_MAX>
+using sort_cfg = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
+                                            rocprim::default_config, MERGE_MAX>;
+#define SORT_MERGE (1u << 20)  // every size that the rule merges
+#define SORT_ONESWEEP 1u
 
+template <unsigned M, typename K>
+static hipError_t pairs(rsbgpu *g, void *tmp, size_t &bytes, const K *keys, K *kout,
+                        const int *vals, int *vout, int64_t n, int bb, int eb) {
+  return rocprim::radix_sort_pairs<sort_cfg<M>>(tmp, bytes, keys, kout, vals, vout, (size_t)n, bb,
+                                                eb, g->stream);
+}
 template <typename K>
 static int sort_into(rsbgpu *g, const K *keys, K *kout, const int *vals, int *vout, int64_t n,
                      int bb, int eb) {
+  auto *sort = sort_by_merging(n, eb - bb) ? pairs<SORT_MERGE, K> : pairs<SORT_ONESWEEP, K>;
   size_t bytes = 0;
-  RSB_TRY(rocprim::radix_sort_pairs<sort_cfg>(nullptr, bytes, keys, kout, vals, vout, (size_t)n,
-                                              bb, eb, g->stream));
+  RSB_TRY(sort(g, nullptr, bytes, keys, kout, vals, vout, n, bb, eb));
   int rc = ensure_tmp(g, bytes);
   if (rc) return rc;
   bytes = g->sort_tmp_bytes;
-  RSB_TRY(rocprim::radix_sort_pairs<sort_cfg>(g->d_sort_tmp, bytes, keys, kout, vals, vout,
-                                              (size_t)n, bb, eb, g->stream));
+  RSB_TRY(sort(g, g->d_sort_tmp, bytes, keys, kout, vals, vout, n, bb, eb));
   return 0;
 }
 
@@ -88,16 +100,20 @@ int rsb_sort_vals_u32(rsbgpu *g, const uint32_t *keys, const int *vals, int *out
 }
 
 // Keys alone, into another array.
+template <unsigned M, typename K>
+static hipError_t only_keys(rsbgpu *g, void *tmp, size_t &bytes, const K *keys, K *out, int64_t n,
+                            int eb) {
+  return rocprim::radix_sort_keys<sort_cfg<M>>(tmp, bytes, keys, out, (size_t)n, 0, eb, g->stream);
+}
 template <typename K>
 static int sort_keys(rsbgpu *g, const K *keys, K *out, int64_t n, int eb) {
+  auto *sort = sort_by_merging(n, eb) ? only_keys<SORT_MERGE, K> : only_keys<SORT_ONESWEEP, K>;
   size_t bytes = 0;
-  RSB_TRY(rocprim::radix_sort_keys<sort_cfg>(nullptr, bytes, keys, out, (size_t)n, 0, eb,
-                                             g->stream));
+  RSB_TRY(sort(g, nullptr, bytes, keys, out, n, eb));
   int rc = ensure_tmp(g, bytes);
   if (rc) return rc;
   bytes = g->sort_tmp_bytes;
-  RSB_TRY(rocprim::radix_sort_keys<sort_cfg>(g->d_sort_tmp, bytes, keys, out, (size_t)n, 0, eb,
-                                             g->stream));
+  RSB_TRY(sort(g, g->d_sort_tmp, bytes, keys, out, n, eb));
   return 0;
 }
 int rsb_sort_keys_u32(rsbgpu *g, const uint32_t *keys, uint32_t *out, int64_t n, int eb) {

@@ -70,6 +70,43 @@ def test_fiedler_sort_of_many_small_segments(size):
         assert took[size] < 6 * took[n], took
 
 
+def _sort_large(n, cuts):
+    """Fiedler sort of n elements in segments too large for LDS: checks the
+    stable order, returns the least time of four."""
+    vtx, xyz, nv = M.box_hex(128, 64, n // 8192 + 1, jitter=0.0)
+    vtx, xyz = vtx[:n], xyz[:n]
+    f = np.random.default_rng(n).integers(-20000, 20000, n) * 0.125
+    cnt, took = np.diff(cuts + [n]), 1.0
+    with _dev() as d:
+        d.set_mesh(vtx, xyz, nv)
+        for _ in range(4):
+            d.set_segments(cuts, cnt, [2] * len(cuts), 2 * np.arange(len(cuts)))
+            d.set_fiedler_values(f)
+            at = d.order()
+            t0 = time.perf_counter()
+            d.fiedler_sort()  # waits
+            took = min(took, time.perf_counter() - t0)
+        want = np.concatenate([b + np.argsort(f[b:b + c], kind="stable")
+                               for b, c in zip(cuts, cnt)])
+        assert np.array_equal(d.order(), at[want])
+    return took
+
+
+@pytest.mark.parametrize("n", [262144, 262145, 1048576, 1048577])
+def test_device_wide_sorts_either_side_of_their_forms(n):
+    """64-bit values merge up to 2^20 elements, segment numbers up to 2^18."""
+    print("fsort large", n, flush=True)
+    _sort_large(n, [0, n // 3, n // 2])
+
+
+def test_device_wide_sort_times_do_not_jump():
+    """100,000 elements against 65,000: the onesweep form takes 235 us there,
+    the merge sort 90 (85 for 65,000)."""
+    print("fsort times", flush=True)
+    took = {n: _sort_large(n, [0]) for n in (65000, 100000)}
+    assert took[100000] < 1.8 * took[65000], took
+
+
 @pytest.mark.parametrize("size", [1, 3, 40, 700])
 def test_neighbour_counts_of_small_segments(size):
     """Segments of one to a few elements: a workgroup's set of pairs overflows
