@@ -142,6 +142,18 @@ int parrsb_amd_partition_quality(const int *part, const long long *vtx, int nel,
 int parrsb_amd_partition_quality_dev(const int *d_part, const long long *d_vtx, int nel,
                                      int nv, int nparts, int64_t *out);
 
+/* Device memory after a call.  The buffers of a finished call (and its stream
+ * and a little pinned host memory) stay with the process for the next one,
+ * at most PARRSB_AMD_POOL_MB MiB per GPU (environment, default 4096; 0 keeps
+ * nothing): mapping them anew takes 3 ms of a 4,096-element call and 25 ms of
+ * a 1M-element one.  What 16 later calls do not ask for, and everything when a
+ * call here runs short of memory, goes back by itself; other allocators in the
+ * process cannot take it.  parrsb_amd_release_memory gives all of it back at
+ * once, for a program that partitions and then fills the GPU itself, and
+ * before hipDeviceReset; it returns the bytes of device memory given back.
+ * Calls running on other threads are not disturbed. */
+long long parrsb_amd_release_memory(void);
+
 /* free() for the arrays parrsb_read_mesh allocates, for callers that cannot
  * reach the C library's free (bindings from other languages). */
 void parrsb_amd_free(void *p);

@@ -37,6 +37,15 @@ typedef struct {
                        above the size limit and took the reference start */
 } rsbgpu_fiedler_out;
 
+/* Device blocks, streams and pinned memory of closed handles stay in a pool
+ * for the next one (at most PARRSB_AMD_POOL_MB MiB of blocks per device,
+ * default 4096, 0 keeps nothing).  rsbgpu_release_memory gives all of it back
+ * and returns the bytes of device memory; rsbgpu_memory reports the bytes
+ * that open handles hold (out[0]), that the pool holds (out[1]) and the most
+ * of both since the last release (out[2]). */
+long long rsbgpu_release_memory(void);
+int rsbgpu_memory(int device, int64_t *out);
+
 int rsbgpu_open(rsbgpu **g, int device);
 void rsbgpu_close(rsbgpu *g);
 const char *rsbgpu_error(const rsbgpu *g);

@@ -124,7 +124,10 @@ SIGNATURES = {
     "parrsb_parse_cmd_opts": (C.POINTER(CmdOpts), [I, C.POINTER(C.c_char_p)]),
     "parrsb_cmd_opts_free": (None, [C.POINTER(CmdOpts)]),
     "parrsb_amd_free": (None, [P]),
+    "parrsb_amd_release_memory": (C.c_longlong, []),
     # rsbgpu.h
+    "rsbgpu_release_memory": (C.c_longlong, []),
+    "rsbgpu_memory": (I, [I, P]),
     "rsbgpu_open": (I, [C.POINTER(P), I]),
     "rsbgpu_close": (None, [P]),
     "rsbgpu_error": (C.c_char_p, [P]),
@@ -214,6 +217,22 @@ def last_report() -> dict:
 
 def last_error() -> str:
     return (lib().parrsb_amd_last_error() or b"").decode()
+
+
+def release_memory() -> int:
+    """Give the device memory that finished calls left with the process back
+    to the GPU; returns its bytes."""
+    return lib().parrsb_amd_release_memory()
+
+
+def device_memory(device: int = 0):
+    """Bytes in open handles, bytes idle in the pool, the most of both since
+    the last release_memory()."""
+    out = np.zeros(3, dtype=np.int64)
+    rc = lib().rsbgpu_memory(device, _p(out))
+    if rc:
+        raise ParrsbError(rc, "no such device")
+    return tuple(int(x) for x in out)
 
 
 def set_precision(bits: int):

@@ -149,15 +149,10 @@ extern "C" void rsbgpu_close(rsbgpu *g) {
   g->scratch.clear();
   for (void *p : g->retired) FREE(p);
   g->retired.clear();
-  if (!g->borrowed) rsb_pool_tick(g->device);
-  if (!g->borrowed &&
-      !(drained && rsb_pool_give_streams(g->device, {g->stream, {g->ev0, g->ev1, g->lz_ev0, g->lz_ev1}, g->ring}))) {
-    if (g->ev0) hipEventDestroy(g->ev0);
-    if (g->ev1) hipEventDestroy(g->ev1);
-    if (g->lz_ev0) hipEventDestroy(g->lz_ev0);
-    if (g->lz_ev1) hipEventDestroy(g->lz_ev1);
-    if (g->stream) hipStreamDestroy(g->stream);
-    if (g->ring) hipHostFree(g->ring);
+  if (!g->borrowed) {
+    rsb_pool_tick(g->device);
+    const rsb_stream_set ss{g->stream, {g->ev0, g->ev1, g->lz_ev0, g->lz_ev1}, g->ring};
+    if (!drained || !rsb_pool_give_streams(g->device, ss)) rsb_destroy_streams(ss);
   }
   delete g;
 }

@@ -7,7 +7,7 @@
 //
 // rsb_dev_malloc / rsb_dev_free are the library's only device allocator:
 // outside such a call they are hipMalloc / hipFree behind a pool of closed
-// handles' blocks (below).  Inside one, blocks come
+// handles' blocks (runtime.hip).  Inside one, blocks come
 // first-fit (lowest address) from a free list over the array.  A freed block
 // is not reused at once: work queued on the call's stream may still read it,
 // and some copies of the library are synchronous on the null stream, which a
@@ -99,146 +99,15 @@ struct arena {
 thread_local arena cur_arena;
 thread_local bool cur_active = false;
 
-// Blocks of closed handles, kept for the next call.  A call allocates ~80
-// buffers (several hundred with the MG solver), and mapping and unmapping
-// them took about 3 ms of a 4,096-element call and 25 ms of a 1M-element one.
-// A block enters the pool only when the work that used it has finished
-// (rsb_dev_release), so it may go to any thread and stream; the pool holds at
-// most kPoolBytes per device, gives back blocks that kPoolIdle closes have
-// not asked for, and empties itself when the device runs out of memory.
-constexpr size_t kPoolBytes = 4ull << 30;
-constexpr unsigned long long kPoolIdle = 16;
-constexpr size_t kPoolStreams = 8;
-
-struct pool_block {
-  void *p;
-  unsigned long long tick;  // close count when it came in
-};
-struct dev_pool {
-  std::multimap<size_t, pool_block> idle;  // by size
-  size_t held = 0;
-  unsigned long long tick = 0;
-  std::vector<rsb_stream_set> streams;
-};
-struct pool_state {
-  std::mutex mu;
-  std::unordered_map<const void *, std::pair<size_t, int>> live;  // size, device
-  dev_pool dev[kMaxDevices];
-};
-pool_state &pool() {
-  static pool_state *s = new pool_state();  // never destroyed: threads may outlive main
-  return *s;
-}
-
-// Sizes in steps of an eighth of their power of two (at least 4 KiB), so
-// that buffers of nearly equal sizes can take each other's place.
-size_t pool_size(size_t bytes) {
-  size_t step = 4096;
-  while (step * 16 <= bytes) step *= 2;
-  return (std::max<size_t>(bytes, 1) + step - 1) / step * step;
-}
-
-// Blocks idle since before `before` leave the pool (mu held).
-void pool_trim(dev_pool &d, unsigned long long before) {
-  for (auto it = d.idle.begin(); it != d.idle.end();) {
-    if (it->second.tick < before) {
-      d.held -= it->first;
-      (void)hipFree(it->second.p);
-      it = d.idle.erase(it);
-    } else {
-      ++it;
-    }
-  }
-}
-
-hipError_t pool_malloc(void **p, size_t bytes) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= kMaxDevices) return hipMalloc(p, bytes);
-  const size_t need = pool_size(bytes);
-  pool_state &s = pool();
-  {
-    std::lock_guard<std::mutex> lock(s.mu);
-    dev_pool &d = s.dev[dev];
-    auto it = d.idle.lower_bound(need);
-    if (it != d.idle.end() && it->first <= 2 * need) {
-      *p = it->second.p;
-      s.live[*p] = {it->first, dev};
-      d.held -= it->first;
-      d.idle.erase(it);
-      return hipSuccess;
-    }
-  }
-  e = hipMalloc(p, need);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    std::lock_guard<std::mutex> lock(s.mu);
-    pool_trim(s.dev[dev], ~0ull);
-    if ((e = hipMalloc(p, need)) != hipSuccess) return e;
-  }
-  std::lock_guard<std::mutex> lock(s.mu);
-  s.live[*p] = {need, dev};
-  return hipSuccess;
-}
-
 }  // namespace
 
 void rsb_dev_release(const void *p) {
-  if (!p) return;
-  if (cur_active) {
-    (void)rsb_dev_free(p);
-    return;
-  }
-  pool_state &s = pool();
-  {
-    std::lock_guard<std::mutex> lock(s.mu);
-    auto it = s.live.find(p);
-    if (it != s.live.end()) {
-      const size_t size = it->second.first;
-      dev_pool &d = s.dev[it->second.second];
-      s.live.erase(it);
-      if (d.held + size <= kPoolBytes) {
-        d.idle.emplace(size, pool_block{(void *)p, d.tick});
-        d.held += size;
-        return;
-      }
-    }
-  }
-  (void)hipFree((void *)p);
-}
-
-bool rsb_pool_take_streams(int device, rsb_stream_set *out) {
-  if (device < 0 || device >= kMaxDevices) return false;
-  pool_state &s = pool();
-  std::lock_guard<std::mutex> lock(s.mu);
-  auto &v = s.dev[device].streams;
-  if (v.empty()) return false;
-  *out = v.back();
-  v.pop_back();
-  return true;
-}
-
-bool rsb_pool_give_streams(int device, const rsb_stream_set &in) {
-  if (device < 0 || device >= kMaxDevices) return false;
-  pool_state &s = pool();
-  std::lock_guard<std::mutex> lock(s.mu);
-  auto &v = s.dev[device].streams;
-  if (v.size() >= kPoolStreams) return false;
-  v.push_back(in);
-  return true;
-}
-
-void rsb_pool_tick(int device) {
-  if (device < 0 || device >= kMaxDevices) return;
-  pool_state &s = pool();
-  std::lock_guard<std::mutex> lock(s.mu);
-  dev_pool &d = s.dev[device];
-  if (++d.tick > kPoolIdle) pool_trim(d, d.tick - kPoolIdle);
+  if (cur_active) (void)rsb_dev_free(p);
+  else rsb_pool_release(p);
 }
 
 hipError_t rsb_dev_malloc(void **p, size_t bytes) {
-  if (!cur_active) return pool_malloc(p, bytes);
+  if (!cur_active) return rsb_pool_malloc(p, bytes);
   arena &a = cur_arena;
   const size_t need = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
   size_t off = 0;
@@ -272,12 +141,7 @@ hipError_t rsb_dev_free(const void *p) {
       return hipSuccess;
     }
   }
-  {
-    pool_state &s = pool();
-    std::lock_guard<std::mutex> lock(s.mu);
-    s.live.erase(p);
-  }
-  return hipFree((void *)p);
+  return rsb_pool_free(p);
 }
 
 bool rsb_arena_stream(int device, hipStream_t *stream, hipEvent_t *ev, int **ring) {

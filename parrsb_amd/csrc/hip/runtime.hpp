@@ -1,0 +1,27 @@
+// Host side of the device layer: the pool of idle device blocks and streams.
+// No kernels and no header of theirs, so it compiles with any C++ compiler
+// and its rules are tested without a GPU (tests/test_pool.py).
+#pragma once
+
+#include <hip/hip_runtime_api.h>
+#include <stddef.h>
+#include <stdint.h>
+
+// A block of device memory, from the pool where one fits, else hipMalloc.
+hipError_t rsb_pool_malloc(void **p, size_t bytes);
+// Back to the device now (hipFree waits for it).
+hipError_t rsb_pool_free(const void *p);
+// To the pool: only a block that no queued work uses any more.
+void rsb_pool_release(const void *p);
+
+// The stream, events and pinned ring of closed handles, likewise.
+struct rsb_stream_set {
+  hipStream_t stream;
+  hipEvent_t ev[4];
+  int *ring;  // pinned: the counts a solve's kernels report to the host
+};
+bool rsb_pool_take_streams(int device, rsb_stream_set *out);
+bool rsb_pool_give_streams(int device, const rsb_stream_set &in);
+void rsb_destroy_streams(const rsb_stream_set &s);
+// One more handle of the device has closed.
+void rsb_pool_tick(int device);

@@ -12,6 +12,7 @@
 
 #include "rsbgpu.h"
 #include "common.hpp"
+#include "runtime.hpp"
 
 // ---------------------------------------------------------------------------
 // Device memory of the library.  Every device allocation goes through these
@@ -27,17 +28,8 @@ inline hipError_t rsb_dev_malloc(T **p, size_t bytes) {
 // Give back a block that no queued work uses any more: it goes to the pool
 // of idle blocks (rsb_dev_free returns it to the device, waiting for it).
 void rsb_dev_release(const void *p);
-// The stream and events of closed handles, likewise.
-struct rsb_stream_set {
-  hipStream_t stream;
-  hipEvent_t ev[4];
-  int *ring;  // pinned: the counts a solve's kernels report to the host
-};
 #define RSB_RING_WORDS 8192
-#define RSB_RING (16 + RSB_RING_WORDS)  // ints of it
-bool rsb_pool_take_streams(int device, rsb_stream_set *out);
-bool rsb_pool_give_streams(int device, const rsb_stream_set &in);
-void rsb_pool_tick(int device);
+#define RSB_RING (16 + RSB_RING_WORDS)  // ints of a handle's pinned ring
 // Inside an allocation-free call on `device`: the stream, the four timing
 // events and the ring set up once for that device (returns false otherwise).
 bool rsb_arena_stream(int device, hipStream_t *stream, hipEvent_t *ev, int **ring);

@@ -553,6 +553,8 @@ int parrsb_amd_conn_mesh_dev(long long *d_vtx, const double *d_coord, int nel, i
   return rc;
 }
 
+long long parrsb_amd_release_memory(void) { return rsbgpu_release_memory(); }
+
 static int quality(const int *part, const long long *vtx, int nel, int nv, int nparts,
                    int64_t *out, int on_device) {
   rsbgpu *g = NULL;

@@ -55,3 +55,20 @@ def test_threads_share_the_pool():
     for t in ts:
         t.join(100)
     assert not bad and not any(t.is_alive() for t in ts)
+
+
+def test_memory_left_by_a_call_goes_back(monkeypatch):
+    """After the last close the device gets everything back on request, and
+    with a bound of 0 at once."""
+    import parrsb_amd as pa
+    mesh = MESHES[1]()
+    before = pa.device_memory()[0]
+    first = _part(mesh, 4)
+    live, idle, peak = pa.device_memory()
+    assert live == before and 0 < idle <= 4 << 30 and peak >= live + idle
+    assert pa.release_memory() == idle
+    assert pa.device_memory() == (live, 0, live) and pa.release_memory() == 0
+    monkeypatch.setenv("PARRSB_AMD_POOL_MB", "0")
+    o, lam = _part(mesh, 4)
+    assert np.array_equal(o, first[0]) and np.array_equal(lam, first[1])
+    assert pa.device_memory()[:2] == (live, 0)
