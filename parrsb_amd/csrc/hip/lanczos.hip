@@ -2405,32 +2405,41 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   // buffers
   size_t vb = (size_t)mpad * sizeof(T);
   if (vb > g->vec_bytes) {
-    const size_t nb = rsb_grown(g, vb, g->vec_bytes);
+    const size_t old = g->vec_bytes;
+    size_t got = ~(size_t)0;
+    g->vec_bytes = 0;
     for (void **q : {&g->d_p, &g->d_p2, &g->d_w, &g->d_f, &g->d_w2}) {
-      RSB_TRY(rsb_retire(g, *q, g->vec_bytes));
-      *q = nullptr;
-      RSB_TRY(rsb_dev_malloc(q, nb + 256));
+      size_t one = 0;
+      RSB_TRY(rsb_retire(g, *q, old));
+      RSB_TRY(rsb_dev_malloc_grown(g, q, vb + 256, old, &one));
+      got = std::min(got, one);
     }
-    g->vec_bytes = nb;
+    g->vec_bytes = got - 256;
   }
   // the pass's residuals r_0 .. r_miter (the last one written, not used)
   size_t bb = vb * ((size_t)miter_max + 1);
   if (bb > g->basis_bytes) {
-    const size_t nb = rsb_grown(g, bb, g->basis_bytes);
-    RSB_TRY(rsb_retire(g, g->d_basis, g->basis_bytes));
-    g->d_basis = nullptr;
-    RSB_TRY(rsb_dev_malloc(&g->d_basis, nb + 256));
-    g->basis_bytes = nb;
+    const size_t old = g->basis_bytes;
+    size_t got = 0;
+    g->basis_bytes = 0;
+    RSB_TRY(rsb_retire(g, g->d_basis, old));
+    RSB_TRY(rsb_dev_malloc_grown(g, &g->d_basis, bb + 256, old, &got));
+    g->basis_bytes = got - 256;
   }
   double *xrow = nullptr;
   RSB_TRY(RSB_SCRATCH(xrow, sizeof(double) * (mpad + 1)));
   lz_state &L = g->lz;
   if (nseg > g->lz_nseg_cap || miter_max > g->lz_miter_cap) {
     // iter, k, npass, niter and miter are carved from the status block
-    for (void *q : {(void *)L.status, (void *)L.sc, (void *)L.T, (void *)L.y, (void *)L.rn})
-      RSB_TRY(rsb_retire(g, q, 1));
+    const size_t os = (size_t)g->lz_nseg_cap, om = (size_t)g->lz_miter_cap;
+    g->lz_nseg_cap = g->lz_miter_cap = 0;
+    RSB_TRY(rsb_retire(g, L.status, sizeof(int) * os * 6));
+    RSB_TRY(rsb_retire(g, L.sc, sizeof(double) * os * LZ_NSC));
+    RSB_TRY(rsb_retire(g, L.T, sizeof(double) * os * 2 * om));
+    RSB_TRY(rsb_retire(g, L.y, sizeof(double) * os * om));
+    RSB_TRY(rsb_retire(g, L.rn, sizeof(double) * os * (om + 1)));
     // the segment count doubles every level
-    const int cap = nseg <= 4096 && !g->borrowed ? std::max(64, (g->lz_nseg_cap ? 4 : 1) * nseg) : nseg;
+    const size_t cap = nseg <= 4096 && !g->borrowed ? std::max(64, (os ? 4 : 1) * nseg) : nseg;
     RSB_TRY(rsb_dev_malloc((void **)&L.status, sizeof(int) * cap * 6));
     L.iter = L.status + cap, L.k = L.status + 2 * cap, L.npass = L.status + 3 * cap;
     L.niter = L.status + 4 * cap;
@@ -2438,13 +2447,15 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
     RSB_TRY(rsb_dev_malloc((void **)&L.T, sizeof(double) * cap * 2 * miter_max));
     RSB_TRY(rsb_dev_malloc((void **)&L.y, sizeof(double) * cap * miter_max));
     RSB_TRY(rsb_dev_malloc((void **)&L.rn, sizeof(double) * cap * ((size_t)miter_max + 1)));
-    g->lz_nseg_cap = cap, g->lz_miter_cap = miter_max;
+    g->lz_nseg_cap = (int)cap, g->lz_miter_cap = miter_max;
   }
   if (ntiles > g->lz_tile_cap) {
-    RSB_TRY(rsb_retire(g, L.partial, 1));
-    const int cap = (int)rsb_grown(g, std::max(ntiles, 1), g->lz_tile_cap);
-    RSB_TRY(rsb_dev_malloc((void **)&L.partial, sizeof(double) * 12 * cap));
-    g->lz_tile_cap = cap;
+    const size_t old = sizeof(double) * 12 * (size_t)g->lz_tile_cap;
+    size_t got = 0;
+    g->lz_tile_cap = 0;
+    RSB_TRY(rsb_retire(g, L.partial, old));
+    RSB_TRY(rsb_dev_malloc_grown(g, (void **)&L.partial, sizeof(double) * 12 * ntiles, old, &got));
+    g->lz_tile_cap = (int)(got / (sizeof(double) * 12));
   }
   if (!L.count) RSB_TRY(rsb_dev_malloc((void **)&L.count, sizeof(int)));
   lz_args a;

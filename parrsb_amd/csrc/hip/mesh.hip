@@ -47,6 +47,7 @@ extern "C" int rsbgpu_open(rsbgpu **out, int device) {
   if (device < 0 || device >= ndev) return 2;
   if (hipSetDevice(device) != hipSuccess) return 2;
   (void)hipGetLastError();  // start from a clean error state
+  rsb_pool_settings();
   rsbgpu *g = new rsbgpu();
   g->device = device;
   hipEvent_t ev[4];

@@ -3,7 +3,7 @@
 // them took about 3 ms of a 4,096-element call and 25 ms of a 1M-element one.
 // A block enters the pool only when the work that used it has finished
 // (rsb_pool_release), so it may go to any thread and stream; the pool holds
-// at most pool_limit() bytes per device, gives back blocks that kPoolIdle
+// at most most_idle bytes per device, gives back blocks that kPoolIdle
 // closes have not asked for, empties itself when the device runs out of
 // memory, and gives everything back when the caller asks
 // (rsbgpu_release_memory).
@@ -24,14 +24,6 @@ constexpr int kMaxDevices = 64;
 constexpr unsigned long long kPoolIdle = 16;
 constexpr size_t kPoolStreams = 8;
 
-// PARRSB_AMD_POOL_MB (default 4096; 0: keep nothing).  4 GiB hold a call of
-// 1M elements whole and all but the largest buffers of a 16.7M-element one.
-size_t pool_limit() {
-  const char *v = getenv("PARRSB_AMD_POOL_MB");
-  const long long mb = v && *v ? atoll(v) : 4096;
-  return mb > 0 ? (size_t)mb << 20 : 0;
-}
-
 struct pool_block {
   void *p;
   unsigned long long tick;  // close count when it came in
@@ -43,8 +35,12 @@ struct dev_pool {
   std::vector<rsb_stream_set> streams;
   void in_use(size_t size) { live += size, peak = std::max(peak, live + held); }
 };
+// 4 GiB hold a call of 1M elements whole and all but the largest buffers of
+// a 16.7M-element one.
+constexpr size_t kPoolBytes = 4ull << 30, kNoLimit = ~(size_t)0;
 struct pool_state {
   std::mutex mu;
+  size_t most_idle = kPoolBytes, most = kNoLimit;  // bytes per device (rsb_pool_settings)
   std::unordered_map<const void *, std::pair<size_t, int>> live;  // size, device
   dev_pool dev[kMaxDevices];
 };
@@ -59,6 +55,22 @@ size_t pool_size(size_t bytes) {
   size_t step = 4096;
   while (step * 16 <= bytes) step *= 2;
   return (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+}
+
+// hipMalloc within the limit on bytes in use and idle.  A failure leaves no
+// error behind for a later launch check to find.
+hipError_t device_malloc(const dev_pool &d, void **p, size_t bytes) {
+  {
+    std::lock_guard<std::mutex> lock(pool().mu);
+    const size_t most = pool().most, used = d.live + d.held;
+    if (used > most || bytes > most - used) return hipErrorOutOfMemory;
+  }
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
+  }
+  return e;
 }
 
 // Blocks idle since before `before` leave the pool (mu held); the caller
@@ -82,6 +94,18 @@ void free_all(const std::vector<void *> &v) {
 
 }  // namespace
 
+void rsb_pool_settings(void) {
+  auto mib = [](const char *name, size_t unset) {
+    const char *v = getenv(name);
+    return v && *v ? (size_t)std::max(0ll, atoll(v)) << 20 : unset;
+  };
+  const size_t idle = mib("PARRSB_AMD_POOL_MB", kPoolBytes);
+  const size_t most = mib("PARRSB_AMD_MEM_LIMIT_MB", kNoLimit);
+  pool_state &s = pool();
+  std::lock_guard<std::mutex> lock(s.mu);
+  s.most_idle = idle, s.most = most;
+}
+
 hipError_t rsb_pool_malloc(void **p, size_t bytes) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -102,20 +126,23 @@ hipError_t rsb_pool_malloc(void **p, size_t bytes) {
       return hipSuccess;
     }
   }
-  e = hipMalloc(p, need);
+  // the rounded size; with the pool emptied; the exact size
+  size_t size = need;
+  e = device_malloc(d, p, size);
   if (e != hipSuccess) {
-    (void)hipGetLastError();
     std::vector<void *> idle;
     {
       std::lock_guard<std::mutex> lock(s.mu);
       idle = pool_trim(d, ~0ull);
     }
     free_all(idle);
-    if ((e = hipMalloc(p, need)) != hipSuccess) return e;
+    e = device_malloc(d, p, size);
+    if (e != hipSuccess) e = device_malloc(d, p, size = bytes);
+    if (e != hipSuccess) return e;
   }
   std::lock_guard<std::mutex> lock(s.mu);
-  s.live[*p] = {need, dev};
-  d.in_use(need);
+  s.live[*p] = {size, dev};
+  d.in_use(size);
   return hipSuccess;
 }
 
@@ -135,7 +162,6 @@ hipError_t rsb_pool_free(const void *p) {
 
 void rsb_pool_release(const void *p) {
   if (!p) return;
-  const size_t limit = pool_limit();
   pool_state &s = pool();
   {
     std::lock_guard<std::mutex> lock(s.mu);
@@ -145,7 +171,7 @@ void rsb_pool_release(const void *p) {
       dev_pool &d = s.dev[it->second.second];
       s.live.erase(it);
       d.live -= size;
-      if (d.held + size <= limit) {
+      if (d.held + size <= s.most_idle) {
         d.idle.emplace(size, pool_block{(void *)p, d.tick});
         d.held += size;
         return;
@@ -167,11 +193,11 @@ bool rsb_pool_take_streams(int device, rsb_stream_set *out) {
 }
 
 bool rsb_pool_give_streams(int device, const rsb_stream_set &in) {
-  if (device < 0 || device >= kMaxDevices || pool_limit() == 0) return false;
+  if (device < 0 || device >= kMaxDevices) return false;
   pool_state &s = pool();
   std::lock_guard<std::mutex> lock(s.mu);
   auto &v = s.dev[device].streams;
-  if (v.size() >= kPoolStreams) return false;
+  if (v.size() >= kPoolStreams || s.most_idle == 0) return false;
   v.push_back(in);
   return true;
 }

@@ -7,6 +7,10 @@
 #include <stddef.h>
 #include <stdint.h>
 
+// Reads the bounds of this process's device memory from the environment, once
+// per handle: PARRSB_AMD_POOL_MB (idle blocks per device, default 4096; 0:
+// keep nothing) and PARRSB_AMD_MEM_LIMIT_MB (all blocks; unset: no limit).
+void rsb_pool_settings(void);
 // A block of device memory, from the pool where one fits, else hipMalloc.
 hipError_t rsb_pool_malloc(void **p, size_t bytes);
 // Back to the device now (hipFree waits for it).

@@ -8,19 +8,21 @@
 
 static int ensure_tmp(rsbgpu *g, size_t bytes) {
   if (bytes <= g->sort_tmp_bytes && g->d_sort_tmp) return 0;
-  RSB_TRY(rsb_retire(g, g->d_sort_tmp, g->sort_tmp_bytes));
-  bytes = rsb_grown(g, bytes, g->d_sort_tmp ? g->sort_tmp_bytes : 0);
-  g->d_sort_tmp = nullptr;
-  RSB_TRY(rsb_dev_malloc(&g->d_sort_tmp, bytes + 256));
-  g->sort_tmp_bytes = bytes + 256;
+  const size_t old = g->d_sort_tmp ? g->sort_tmp_bytes : 0;
+  g->sort_tmp_bytes = 0;
+  RSB_TRY(rsb_retire(g, g->d_sort_tmp, old));
+  size_t got = 0;
+  RSB_TRY(rsb_dev_malloc_grown(g, &g->d_sort_tmp, bytes + 256, old, &got));
+  g->sort_tmp_bytes = got;
   return 0;
 }
 
 static int ensure_kv(rsbgpu *g, size_t n) {
   if (n <= g->sort_cap && g->d_k1) return 0;
-  RSB_TRY(rsb_retire(g, g->d_k1, g->sort_cap * sizeof(uint64_t)));
-  RSB_TRY(rsb_retire(g, g->d_v1, g->sort_cap * sizeof(int)));
-  g->d_k1 = nullptr, g->d_v1 = nullptr;
+  const size_t old = g->sort_cap;
+  g->sort_cap = 0;
+  RSB_TRY(rsb_retire(g, g->d_k1, old * sizeof(uint64_t)));
+  RSB_TRY(rsb_retire(g, g->d_v1, old * sizeof(int)));
   RSB_TRY(rsb_dev_malloc((void **)&g->d_k1, n * sizeof(uint64_t)));
   RSB_TRY(rsb_dev_malloc((void **)&g->d_v1, n * sizeof(int)));
   g->sort_cap = n;

@@ -180,22 +180,39 @@ struct rsbgpu {
   // buffers replaced by larger ones while queued work may still use them,
   // released when the handle closes
   std::vector<void *> retired;
+  size_t retired_bytes = 0;
 };
 
-// Replaces a buffer: small ones wait for the handle's close instead of making
-// the device wait now (a free does), large ones are freed at once, and so
-// are those of an allocation-free call, whose frees never wait.
-inline hipError_t rsb_retire(rsbgpu *g, void *p, size_t bytes) {
-  if (!p) return hipSuccess;
-  if (g->borrowed || bytes > ((size_t)64 << 20)) return rsb_dev_free(p);
-  g->retired.push_back(p);
+// Gives up a buffer that a larger one replaces (p becomes nullptr).  Small
+// ones wait for the handle's close instead of making the device wait now (a
+// free does), at most RSB_RETIRED_MAX bytes of them; large ones are freed at
+// once, and so are those of an allocation-free call, whose frees never wait.
+#define RSB_RETIRE_MAX ((size_t)64 << 20)
+#define RSB_RETIRED_MAX ((size_t)256 << 20)
+template <typename T>
+inline hipError_t rsb_retire(rsbgpu *g, T *&p, size_t bytes) {
+  void *q = (void *)p;
+  p = nullptr;
+  if (!q) return hipSuccess;
+  if (g->borrowed || bytes > RSB_RETIRE_MAX || g->retired_bytes + bytes > RSB_RETIRED_MAX)
+    return rsb_dev_free(q);
+  g->retired.push_back(q);
+  g->retired_bytes += bytes;
   return hipSuccess;
 }
-// size of a buffer that takes a smaller one's place: the level loop asks for
-// slightly more every level (padding, segment counts); not in the fixed
-// array of an allocation-free call
-inline size_t rsb_grown(const rsbgpu *g, size_t bytes, size_t old) {
-  return old && !g->borrowed ? bytes + bytes / 8 : bytes;
+// A buffer of `need` bytes, in place of one of `old` bytes if that is not 0:
+// then an eighth larger, because the level loop asks for slightly more every
+// level (padding, segment counts), but not in the fixed array of an
+// allocation-free call, and not where the memory for it is not there.  Where
+// it runs short the retired buffers go back first.  *got: its size.
+inline hipError_t rsb_dev_malloc_grown(rsbgpu *g, void **p, size_t need, size_t old, size_t *got) {
+  *got = old && !g->borrowed ? need + need / 8 : need;
+  hipError_t e = rsb_dev_malloc(p, *got);
+  if (e == hipSuccess || g->borrowed) return e;
+  for (void *q : g->retired) (void)rsb_dev_free(q);  // (waits for the device)
+  g->retired.clear(), g->retired_bytes = 0;
+  *got = need;
+  return rsb_dev_malloc(p, need);
 }
 
 // ---------------------------------------------------------------------------
@@ -256,19 +273,14 @@ inline hipError_t dev_alloc(rsbgpu *g, T *&p, size_t n) {
   // enough: the level loop re-sizes the same slots every level, and freeing
   // and mapping the multi-GB level matrices again each time cost ~10 ms a
   // level at 16.7M elements (contents are never assumed to be fresh)
-  size_t bytes = (n ? n : 1) * sizeof(T);
-  auto it = g->cap.find((const void *)&p);
-  const size_t old = p && it != g->cap.end() ? it->second : 0;
-  if (p && old >= bytes) return hipSuccess;
-  if (p) {
-    hipError_t e = rsb_retire(g, (void *)p, old);
-    if (e != hipSuccess) return e;
-    p = nullptr;
-    bytes = rsb_grown(g, bytes, old);
-  }
-  hipError_t e = rsb_dev_malloc((void **)&p, bytes);
-  if (e == hipSuccess) g->cap[(const void *)&p] = bytes;
-  return e;
+  const size_t bytes = (n ? n : 1) * sizeof(T);
+  size_t &held = g->cap[(const void *)&p];
+  const size_t old = p ? held : 0;
+  if (old >= bytes) return hipSuccess;
+  hipError_t e = rsb_retire(g, p, old);
+  held = 0;
+  if (e != hipSuccess) return e;
+  return rsb_dev_malloc_grown(g, (void **)&p, bytes, old, &held);
 }
 
 // Scratch buffer of one call site: the level loop used to hipMalloc and
@@ -282,18 +294,15 @@ inline hipError_t rsb_scratch(rsbgpu *g, const void *file, int line, size_t byte
     *out = s.first;
     return hipSuccess;
   }
-  if (s.first) {
-    hipError_t e = rsb_retire(g, s.first, s.second);
-    bytes = rsb_grown(g, bytes, s.second);
-    s.first = nullptr, s.second = 0;
-    if (e != hipSuccess) return e;
-  }
-  hipError_t e = rsb_dev_malloc(&s.first, bytes ? bytes : 1);
+  const size_t old = s.first ? s.second : 0;
+  hipError_t e = rsb_retire(g, s.first, old);
+  s.second = 0;
+  if (e != hipSuccess) return e;
+  e = rsb_dev_malloc_grown(g, &s.first, bytes ? bytes : 1, old, &s.second);
   if (e != hipSuccess) {
-    s.first = nullptr;
+    s.first = nullptr, s.second = 0;
     return e;
   }
-  s.second = bytes;
   *out = s.first;
   return hipSuccess;
 }

@@ -45,6 +45,7 @@ hipError_t hipHostFree(void *) { objects--; return hipSuccess; }
 void *t_malloc(size_t n) { void *p = nullptr; return rsb_pool_malloc(&p, n) == hipSuccess ? p : nullptr; }
 void t_free(void *p) { (void)rsb_pool_free(p); }
 void t_release(void *p) { rsb_pool_release(p); }
+void t_settings(void) { rsb_pool_settings(); }
 void t_tick(void) { rsb_pool_tick(0); }
 void t_capacity(size_t n) { capacity = n; }
 size_t t_used(void) { return used; }
@@ -120,6 +121,7 @@ def test_idle_blocks_serve_again_and_go_back_on_request(pool):
 def test_bound(pool, mb, monkeypatch):
     if mb is not None:
         monkeypatch.setenv("PARRSB_AMD_POOL_MB", str(mb))
+    pool.t_settings()
     limit = (4096 if mb is None else mb) * MB
     unit = MB if mb is not None else 512 * MB
     for p in [pool.t_malloc(unit) for _ in range(12)]:
@@ -144,6 +146,21 @@ def test_memory_running_out_empties_the_pool(pool):
     p = pool.t_malloc(60 * MB)
     assert p and pool.t_used() == 60 * MB and _stats(pool)[1] == 0
     assert not pool.t_malloc(60 * MB)
+
+
+def test_a_block_that_fits_only_at_its_own_size(pool, monkeypatch):
+    """Sizes are rounded up to an eighth of their power of two, unless only
+    the exact size fits."""
+    n = 8 * MB + 5
+    pool.t_capacity(9 * MB - 1)
+    p = pool.t_malloc(n)
+    assert p and pool.t_used() == n and _stats(pool)[0] == n
+    pool.t_release(p)
+    assert pool.t_malloc(n - 3 * MB) == p and pool.t_used() == n  # up to twice the size serves
+    pool.t_capacity(1 << 40)
+    monkeypatch.setenv("PARRSB_AMD_MEM_LIMIT_MB", "10")
+    pool.t_settings()
+    assert not pool.t_malloc(2 * MB) and pool.t_malloc(MB)
 
 
 def test_threads(pool):
