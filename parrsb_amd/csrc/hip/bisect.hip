@@ -753,9 +753,8 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
   k_q_roots<<<nblocks(nel, 256), 256, 0, g->stream>>>(nel, d_part, par, ncomp);
   RSB_LAUNCH_CHECK();
   int64_t ns = (int64_t)nel * g->nv;
-  uint64_t *key = nullptr, *sorted = nullptr;
+  uint64_t *key = nullptr;
   RSB_TRY(rsb_dev_malloc((void **)&key, sizeof(uint64_t) * ns));
-  RSB_TRY(rsb_dev_malloc((void **)&sorted, sizeof(uint64_t) * ns));
   // as few key bits as the ids and parts take, in 32 bits if they fit
   int vbits = 1, pbits = 1;
   while (vbits < 64 && (g->vmax >> vbits) != 0) vbits++;
@@ -763,16 +762,18 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
   const unsigned vb = (unsigned)std::min<int64_t>(nblocks(ns, 256), 2048);
   int rc;
   if (vbits + pbits <= 32) {
-    uint32_t *k4 = (uint32_t *)key, *s4 = (uint32_t *)sorted;
+    uint32_t *k4 = (uint32_t *)key;
+    const uint32_t *s4 = nullptr;
     k_q_vkeys<<<nblocks(ns, 256), 256, 0, g->stream>>>(g->d_vtx, d_part, ns, g->nv, pbits, k4);
     RSB_LAUNCH_CHECK();
-    if ((rc = rsb_sort_keys_u32(g, k4, s4, ns, vbits + pbits))) return rc;
+    if ((rc = rsb_sort_keys_u32(g, k4, &s4, ns, vbits + pbits))) return rc;
     k_q_volume<<<vb, 256, 0, g->stream>>>(s4, ns, pbits, acc + 2);
   } else {
     k_q_vkeys<<<nblocks(ns, 256), 256, 0, g->stream>>>(g->d_vtx, d_part, ns, g->nv, pbits, key);
     RSB_LAUNCH_CHECK();
-    if ((rc = rsb_sort_keys_u64(g, key, sorted, ns, std::min(64, vbits + pbits)))) return rc;
-    k_q_volume<<<vb, 256, 0, g->stream>>>(sorted, ns, pbits, acc + 2);
+    const uint64_t *s8 = nullptr;
+    if ((rc = rsb_sort_keys_u64(g, key, &s8, ns, std::min(64, vbits + pbits)))) return rc;
+    k_q_volume<<<vb, 256, 0, g->stream>>>(s8, ns, pbits, acc + 2);
   }
   RSB_LAUNCH_CHECK();
   std::vector<int> hs(2 * (size_t)nparts);
@@ -788,7 +789,6 @@ extern "C" int rsbgpu_quality(rsbgpu *g, const int *d_part, int nparts, int64_t 
   }
   out[0] = (int64_t)ha[0], out[1] = (int64_t)ha[1], out[2] = mx, out[3] = mn, out[4] = tot;
   out[5] = cmx, out[6] = (int64_t)ha[2], out[7] = empty;
-  rsb_dev_release(acc), rsb_dev_release(par), rsb_dev_release(size), rsb_dev_release(key),
-      rsb_dev_release(sorted);
+  rsb_dev_release(acc), rsb_dev_release(par), rsb_dev_release(size), rsb_dev_release(key);
   return 0;
 }

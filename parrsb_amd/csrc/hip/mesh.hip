@@ -466,6 +466,11 @@ static int build_graph(rsbgpu *g) {
   rc = rsb_exclusive_scan_i64(g, rowlen, g->d_growptr, (int64_t)n + 1);
   if (rc) return rc;
   RSB_READ(g, {&g->gnnz, g->d_growptr + n, sizeof(int64_t)});
+  // the sort's arrays (2.1 GB for 16.7M hexes) serve the call's next buffers:
+  // what used them has finished
+  for (const void *p : {(const void *)key, (const void *)flag, (const void *)excl,
+                        (const void *)rowlen})
+    rsb_dev_release(p);
   RSB_TRY(dev_alloc(g, g->d_gadj, (size_t)g->gnnz));
   k_dual_rows<true><<<nblocks(n, 128), 128, 0, g->stream>>>(
       n, g->nv, slot_group, gstart, val, nullptr, g->d_growptr, g->d_gadj, ovf);
@@ -479,9 +484,8 @@ static int build_graph(rsbgpu *g) {
   unsigned long long ws = 0;
   RSB_READ(g, {&hovf, ovf, sizeof(int)}, {&ws, vmax, sizeof(ws)});
   g->gwsum = (int64_t)ws;
-  for (const void *p : {(const void *)key, (const void *)flag, (const void *)excl,
-                        (const void *)val, (const void *)slot_group, (const void *)gstart,
-                        (const void *)rowlen, (const void *)ovf, (const void *)vmax})
+  for (const void *p : {(const void *)val, (const void *)slot_group, (const void *)gstart,
+                        (const void *)ovf, (const void *)vmax})
     rsb_dev_release(p);
   if (hovf) RSB_FAIL(3, "two elements share more than 15 vertex ids");
   return 0;

@@ -101,27 +101,30 @@ int rsb_sort_vals_u32(rsbgpu *g, const uint32_t *keys, const int *vals, int *out
   return sort_into(g, keys, (uint32_t *)g->d_k1, vals, out, n, bb, eb);
 }
 
-// Keys alone, into another array.
+// Keys alone, into the handle's own array: *out, valid until its next sort.
 template <unsigned M, typename K>
 static hipError_t only_keys(rsbgpu *g, void *tmp, size_t &bytes, const K *keys, K *out, int64_t n,
                             int eb) {
   return rocprim::radix_sort_keys<sort_cfg<M>>(tmp, bytes, keys, out, (size_t)n, 0, eb, g->stream);
 }
 template <typename K>
-static int sort_keys(rsbgpu *g, const K *keys, K *out, int64_t n, int eb) {
+static int sort_keys(rsbgpu *g, const K *keys, const K **out, int64_t n, int eb) {
   auto *sort = sort_by_merging(n, eb) ? only_keys<SORT_MERGE, K> : only_keys<SORT_ONESWEEP, K>;
-  size_t bytes = 0;
-  RSB_TRY(sort(g, nullptr, bytes, keys, out, n, eb));
-  int rc = ensure_tmp(g, bytes);
+  int rc = ensure_kv(g, (size_t)n);
   if (rc) return rc;
+  K *sorted = (K *)g->d_k1;
+  size_t bytes = 0;
+  RSB_TRY(sort(g, nullptr, bytes, keys, sorted, n, eb));
+  if ((rc = ensure_tmp(g, bytes))) return rc;
   bytes = g->sort_tmp_bytes;
-  RSB_TRY(sort(g, g->d_sort_tmp, bytes, keys, out, n, eb));
+  RSB_TRY(sort(g, g->d_sort_tmp, bytes, keys, sorted, n, eb));
+  *out = sorted;
   return 0;
 }
-int rsb_sort_keys_u32(rsbgpu *g, const uint32_t *keys, uint32_t *out, int64_t n, int eb) {
+int rsb_sort_keys_u32(rsbgpu *g, const uint32_t *keys, const uint32_t **out, int64_t n, int eb) {
   return sort_keys(g, keys, out, n, eb);
 }
-int rsb_sort_keys_u64(rsbgpu *g, const uint64_t *keys, uint64_t *out, int64_t n, int eb) {
+int rsb_sort_keys_u64(rsbgpu *g, const uint64_t *keys, const uint64_t **out, int64_t n, int eb) {
   return sort_keys(g, keys, out, n, eb);
 }
 

@@ -330,8 +330,10 @@ int rsb_sort_vals_u64(rsbgpu *g, const uint64_t *keys, const int *vals, int *out
                       int begin_bit, int end_bit);
 int rsb_sort_vals_u32(rsbgpu *g, const uint32_t *keys, const int *vals, int *out, int64_t n,
                       int begin_bit, int end_bit);
-int rsb_sort_keys_u32(rsbgpu *g, const uint32_t *keys, uint32_t *out, int64_t n, int end_bit);
-int rsb_sort_keys_u64(rsbgpu *g, const uint64_t *keys, uint64_t *out, int64_t n, int end_bit);
+int rsb_sort_keys_u32(rsbgpu *g, const uint32_t *keys, const uint32_t **out, int64_t n,
+                      int end_bit);
+int rsb_sort_keys_u64(rsbgpu *g, const uint64_t *keys, const uint64_t **out, int64_t n,
+                      int end_bit);
 int rsb_exclusive_scan_i64(rsbgpu *g, const int64_t *in, int64_t *out, int64_t n);
 int rsb_exclusive_scan_i32(rsbgpu *g, const int *in, int *out, int64_t n);
 

@@ -74,3 +74,23 @@ def test_room_to_grow_is_not_needed(monkeypatch):
     live = pa.device_memory()[0] >> 20
     monkeypatch.setenv("PARRSB_AMD_MEM_LIMIT_MB", str(limit + live))
     assert call(True) == two
+
+
+def test_graph_build_gives_its_sort_arrays_back_before_the_graph(monkeypatch):
+    """Most bytes per corner of a quality report, when the rows are counted:
+    keys, slots, flags and offsets of the sort 20, its output and scratch 24,
+    groups 5, row lengths and offsets 2, centroids and ranks 4.5, in blocks up
+    to an eighth larger: at most 62.5.  The graph's entries (13) come after
+    the first 16 of them have gone; beside them it would be 68.5 at least."""
+    import parrsb_amd as pa
+    vtx, _, nv = M.box_hex(64, 64, 64, jitter=0.0)
+    n = vtx.shape[0]
+    monkeypatch.setenv("PARRSB_AMD_POOL_MB", "0")
+    with pa.Device() as d:
+        dv = d.upload(np.ascontiguousarray(vtx))
+        dp = d.upload(np.arange(n, dtype=np.int32) * 8 // n)
+    q, peak = _peak(lambda: pa.quality_dev(dp, dv, n, nv, 8))
+    pa.Device.free(dv), pa.Device.free(dp)
+    print("bytes per corner", peak / vtx.size, flush=True)
+    assert q["components"] == 8
+    assert peak < 64 * vtx.size
