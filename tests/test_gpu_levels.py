@@ -127,6 +127,33 @@ def test_neighbour_counts_of_small_segments(size):
     assert np.array_equal(got, np.bincount(pairs[:, 0], minlength=start.size))
 
 
+@pytest.mark.parametrize("mesh", ["apart", "box"])
+def test_neighbour_counts_of_a_segment_per_element(mesh):
+    """300,000 elements that share nothing, and a box whose 8.7M pairs do not
+    fit the set's first size: a set of at most 64 MiB to begin with, doubled
+    once for the box."""
+    import parrsb_amd as pa
+    print("neighbours", mesh, flush=True)
+    if mesh == "apart":
+        n, nv = 300000, 4
+        vtx = np.arange(1, 4 * n + 1, dtype=np.int64).reshape(n, nv)
+        xyz = np.zeros((n, nv, 2))
+    else:
+        vtx, xyz, nv = M.box_hex(70, 70, 70, jitter=0.0)
+        n = vtx.shape[0]
+    pa.release_memory()
+    with _dev() as d:
+        d.set_mesh(vtx, xyz, nv)
+        e = np.arange(n)
+        d.set_segments(e, np.ones_like(e), np.ones_like(e), e)
+        live = pa.device_memory()[0]
+        got = d.neighbors(n)
+        took = pa.device_memory()[0] - live
+        rowptr = d.graph()[0]
+    assert np.array_equal(got, np.diff(rowptr))
+    assert took <= (72 << 20 if mesh == "apart" else 300 << 20), took
+
+
 @pytest.mark.parametrize("shift", [0, 1 << 20, 1 << 40])
 @pytest.mark.parametrize("parts", [1, 2, 37, 1000])
 @pytest.mark.parametrize("mesh", ["hex", "quads"])
