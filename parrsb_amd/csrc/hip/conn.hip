@@ -508,14 +508,11 @@ extern "C" int rsbgpu_conn_mesh(int device, long long *vtx_out, const double *co
   }
 done:
 #undef CON_TRY
-  if (hipStreamSynchronize(st) != hipSuccess && rc == 0) rc = 2;
   if (on_device) dcoord = nullptr, dvtx = nullptr;  // the caller's
-  for (const void *p :
-       {(const void *)dcoord, (const void *)dvtx, (const void *)x, (const void *)dx,
-        (const void *)lay, (const void *)val, (const void *)segp, (const void *)flag,
-        (const void *)excl, (const void *)key, (const void *)err, (const void *)pdev,
-        (const void *)pfid, (const void *)pgone, (const void *)pfx})
-    rsb_dev_release(p);
+  if (!rsb_drain_release(st, {dcoord, dvtx, x, dx, lay, val, segp, flag, excl, key, err, pdev,
+                              pfid, pgone, pfx}) &&
+      rc == 0)
+    rc = 2;
   if (rc == 2 && msg && msg_len > 0) snprintf(msg, (size_t)msg_len, "device failure in connectivity");
   rsbgpu_close(g);
   return rc;

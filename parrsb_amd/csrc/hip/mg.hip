@@ -1486,15 +1486,12 @@ struct mg_level_dev {
 struct mg_hier {
   std::vector<mg_level_dev> lv;
   std::vector<std::vector<int>> h_off, h_n;
-  // (rsb_mg_free has waited for the stream)
-  ~mg_hier() {
-    for (auto &l : lv)
-      for (const void *p :
-           {(const void *)l.off, (const void *)l.n, (const void *)l.rseg, (const void *)l.rp,
-            (const void *)l.ci, (const void *)l.w, (const void *)l.diag, (const void *)l.r0,
-            (const void *)l.sa, (const void *)l.sb, (const void *)l.u, (const void *)l.soff,
-            (const void *)l.rlen, (const void *)l.sci, (const void *)l.sw, (const void *)l.spk})
-        rsb_dev_release(p);
+  std::vector<const void *> blocks() const {
+    std::vector<const void *> v;
+    for (const auto &l : lv)
+      v.insert(v.end(), {l.off, l.n, l.rseg, l.rp, l.ci, l.w, l.diag, l.r0, l.sa, l.sb, l.u,
+                         l.soff, l.rlen, l.sci, l.sw, l.spk});
+    return v;
   }
 };
 
@@ -1509,7 +1506,8 @@ double sigma_cheb(int k, int n, double lmin, double lmax) {
 // The hierarchy of the last rsbgpu_fiedler_mg call stays with the handle
 // (for the parity hook rsbgpu_mg_level_csr) until the next call or close.
 void rsb_mg_free(rsbgpu *g) {
-  if (g->mg && g->stream) (void)hipStreamSynchronize(g->stream);
+  if (!g->mg) return;
+  (void)rsb_drain_release(g->stream, ((mg_hier *)g->mg)->blocks());
   delete (mg_hier *)g->mg;
   g->mg = nullptr;
 }
@@ -1527,7 +1525,7 @@ void rsb_mg_free(rsbgpu *g) {
 // stream has drained (an early return may leave launches queued).
 struct mg_scope {
   hipStream_t st;
-  std::vector<void *> bufs;
+  std::vector<const void *> bufs;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipEvent_t ev[2] = {nullptr, nullptr};
@@ -1536,7 +1534,7 @@ struct mg_scope {
   template <typename T>
   hipError_t alloc(T *&ptr, size_t bytes) {
     hipError_t e = rsb_dev_malloc((void **)&ptr, bytes);
-    if (e == hipSuccess) bufs.push_back((void *)ptr);
+    if (e == hipSuccess) bufs.push_back(ptr);
     else ptr = nullptr;
     return e;
   }
@@ -1546,12 +1544,11 @@ struct mg_scope {
       (void)hipStreamEndCapture(st, &left);
       if (left) (void)hipGraphDestroy(left);
     }
-    (void)hipStreamSynchronize(st);
+    (void)rsb_drain_release(st, bufs);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
-    for (void *q : bufs) rsb_dev_release(q);
   }
 };
 

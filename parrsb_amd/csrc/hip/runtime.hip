@@ -181,6 +181,15 @@ void rsb_pool_release(const void *p) {
   (void)hipFree((void *)p);
 }
 
+bool rsb_drain_release(hipStream_t st, const std::vector<const void *> &blocks) {
+  const bool drained = st && hipStreamSynchronize(st) == hipSuccess;
+  for (const void *p : blocks) {
+    if (drained) rsb_dev_release(p);
+    else (void)rsb_dev_free(p);
+  }
+  return drained;
+}
+
 bool rsb_pool_take_streams(int device, rsb_stream_set *out) {
   if (device < 0 || device >= kMaxDevices) return false;
   pool_state &s = pool();

@@ -7,6 +7,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <vector>
+
 // Reads the bounds of this process's device memory from the environment, once
 // per handle: PARRSB_AMD_POOL_MB (idle blocks per device, default 4096; 0:
 // keep nothing) and PARRSB_AMD_MEM_LIMIT_MB (all blocks; unset: no limit).
@@ -29,3 +31,13 @@ bool rsb_pool_give_streams(int device, const rsb_stream_set &in);
 void rsb_destroy_streams(const rsb_stream_set &s);
 // One more handle of the device has closed.
 void rsb_pool_tick(int device);
+
+// The library's allocator (noalloc.hip): rsb_pool_malloc and its counterparts,
+// or the fixed array inside an allocation-free call.
+hipError_t rsb_dev_malloc(void **p, size_t bytes);
+hipError_t rsb_dev_free(const void *p);
+void rsb_dev_release(const void *p);
+// Gives back the blocks that a stream's work has used: released once the
+// stream has drained; freed if it cannot be shown to have, since a block of
+// the pool may go to any thread and stream.  Returns whether it has.
+bool rsb_drain_release(hipStream_t st, const std::vector<const void *> &blocks);

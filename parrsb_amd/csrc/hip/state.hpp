@@ -15,19 +15,14 @@
 #include "runtime.hpp"
 
 // ---------------------------------------------------------------------------
-// Device memory of the library.  Every device allocation goes through these
-// two functions: hipMalloc / hipFree normally; inside an allocation-free call
+// Device memory of the library.  Every device allocation goes through
+// rsb_dev_malloc and rsb_dev_free or rsb_dev_release (runtime.hpp): hipMalloc / hipFree normally; inside an allocation-free call
 // (noalloc.hip) a bump allocator over a fixed device array, whose frees are
 // no-ops until the call ends.
-hipError_t rsb_dev_malloc(void **p, size_t bytes);
-hipError_t rsb_dev_free(const void *p);
 template <typename T>
 inline hipError_t rsb_dev_malloc(T **p, size_t bytes) {
   return rsb_dev_malloc((void **)p, bytes);
 }
-// Give back a block that no queued work uses any more: it goes to the pool
-// of idle blocks (rsb_dev_free returns it to the device, waiting for it).
-void rsb_dev_release(const void *p);
 #define RSB_RING_WORDS 8192
 #define RSB_RING (16 + RSB_RING_WORDS)  // ints of a handle's pinned ring
 // Inside an allocation-free call on `device`: the stream, the four timing

@@ -42,6 +42,12 @@ hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { objects--; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { objects--; return hipSuccess; }
 hipError_t hipHostFree(void *) { objects--; return hipSuccess; }
+static hipError_t drain = hipSuccess;
+hipError_t hipStreamSynchronize(hipStream_t) { return drain; }
+int t_drain(int ok, int n, void **p) {
+  drain = ok ? hipSuccess : hipErrorUnknown;
+  return rsb_drain_release((hipStream_t)8, std::vector<const void *>(p, p + n));
+}
 void *t_malloc(size_t n) { void *p = nullptr; return rsb_pool_malloc(&p, n) == hipSuccess ? p : nullptr; }
 void t_free(void *p) { (void)rsb_pool_free(p); }
 void t_release(void *p) { rsb_pool_release(p); }
@@ -59,6 +65,8 @@ int t_give_streams(void) {
 }
 int t_objects(void) { return objects; }
 }
+hipError_t rsb_dev_free(const void *p) { return rsb_pool_free(p); }
+void rsb_dev_release(const void *p) { rsb_pool_release(p); }
 """
 
 
@@ -161,6 +169,13 @@ def test_a_block_that_fits_only_at_its_own_size(pool, monkeypatch):
     monkeypatch.setenv("PARRSB_AMD_MEM_LIMIT_MB", "10")
     pool.t_settings()
     assert not pool.t_malloc(2 * MB) and pool.t_malloc(MB)
+
+
+@pytest.mark.parametrize("ok", [0, 1])
+def test_blocks_of_a_stream_that_did_not_drain_stay_out(pool, ok):
+    p = (C.c_void_p * 4)(pool.t_malloc(MB), None, pool.t_malloc(2 * MB), pool.t_malloc(MB))
+    assert pool.t_drain(ok, 4, p) == ok
+    assert _stats(pool)[:2] == [0, 4 * MB * ok] and pool.t_used() == 4 * MB * ok
 
 
 def test_threads(pool):
