@@ -50,6 +50,7 @@ extern "C" int rsbgpu_open(rsbgpu **out, int device) {
   rsb_pool_settings();
   rsbgpu *g = new rsbgpu();
   g->device = device;
+  g->schedule = rsb_schedule();
   hipEvent_t ev[4];
   if (rsb_arena_stream(device, &g->stream, ev, &g->ring)) {
     // allocation-free call: the stream and events set up for this device
@@ -181,17 +182,9 @@ __global__ void __launch_bounds__(1024) k_read_back(read_args a, int *flag, int 
 }
 
 int rsb_wait_flag(rsbgpu *g, const int *flag) {
-  for (unsigned q = 1; !__atomic_load_n(flag, __ATOMIC_ACQUIRE); q++)
-    if ((q & 0xffff) == 0) {
-      // a failed launch or a fault never sets it: ask the stream
-      const hipError_t e = hipStreamQuery(g->stream);
-      if (e == hipErrorNotReady) {
-        (void)hipGetLastError();
-        continue;
-      }
-      RSB_TRY(e);
-      if (!__atomic_load_n(flag, __ATOMIC_ACQUIRE)) RSB_FAIL(2, "no report from the device");
-    }
+  const hipError_t e = rsb_await(g->stream, flag, g->schedule);
+  if (e == hipErrorNotReady) RSB_FAIL(2, "no report from the device");
+  RSB_TRY(e);
   return 0;
 }
 

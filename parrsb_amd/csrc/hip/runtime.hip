@@ -9,6 +9,8 @@
 // (rsbgpu_release_memory).
 #include "runtime.hpp"
 
+#include <sched.h>
+
 #include <algorithm>
 #include <cstdlib>
 #include <map>
@@ -258,4 +260,40 @@ extern "C" int rsbgpu_memory(int device, int64_t *out) {
   const dev_pool &d = s.dev[device];
   out[0] = (int64_t)d.live, out[1] = (int64_t)d.held, out[2] = (int64_t)d.peak;
   return 0;
+}
+
+unsigned rsb_schedule(void) {
+  unsigned f = 0;
+  if (hipGetDeviceFlags(&f) != hipSuccess) {
+    (void)hipGetLastError();
+    f = hipDeviceScheduleAuto;
+  }
+  return f & hipDeviceScheduleMask;
+}
+
+// Most reports arrive within microseconds of the look, so a thread that wants
+// to sleep looks for about as long first (kLooks) before it does.
+hipError_t rsb_await(hipStream_t st, const int *flag, unsigned schedule) {
+  constexpr unsigned kLooks = 1u << 10, kQuery = 1u << 16;
+  const bool yields = schedule == hipDeviceScheduleYield;
+  for (unsigned q = 1;; q++) {
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE)) return hipSuccess;
+    if (schedule == hipDeviceScheduleBlockingSync && q == kLooks) {
+      const hipError_t e = hipStreamSynchronize(st);
+      if (e != hipSuccess) return e;
+      return __atomic_load_n(flag, __ATOMIC_ACQUIRE) ? hipSuccess : hipErrorNotReady;
+    }
+    if (yields) sched_yield();
+    else __builtin_ia32_pause();
+    if (q % (yields ? kLooks : kQuery) == 0) {
+      // a failed launch or a fault never sets it: ask the stream
+      const hipError_t e = hipStreamQuery(st);
+      if (e == hipErrorNotReady) {
+        (void)hipGetLastError();
+        continue;
+      }
+      if (e != hipSuccess) return e;
+      return __atomic_load_n(flag, __ATOMIC_ACQUIRE) ? hipSuccess : hipErrorNotReady;
+    }
+  }
 }

@@ -1,4 +1,5 @@
-// Host side of the device layer: the pool of idle device blocks and streams.
+// Host side of the device layer: the pool of idle device blocks and streams,
+// and the wait for a kernel's report.
 // No kernels and no header of theirs, so it compiles with any C++ compiler
 // and its rules are tested without a GPU (tests/test_pool.py).
 #pragma once
@@ -41,3 +42,12 @@ void rsb_dev_release(const void *p);
 // stream has drained; freed if it cannot be shown to have, since a block of
 // the pool may go to any thread and stream.  Returns whether it has.
 bool rsb_drain_release(hipStream_t st, const std::vector<const void *> &blocks);
+
+// The schedule flags (hipDeviceSchedule*) of the current device.
+unsigned rsb_schedule(void);
+// Waits until a kernel on the stream has set *flag (pinned memory), as the
+// schedule flags ask: looking all the time (Auto, Spin), with the rest of the
+// time slice given away after each look (Yield), or asleep in the runtime
+// until the stream has drained (BlockingSync).  hipErrorNotReady: the stream
+// has ended without setting it.
+hipError_t rsb_await(hipStream_t st, const int *flag, unsigned schedule);

@@ -167,6 +167,7 @@ struct rsbgpu {
   int prof_spmv = 0;                   // bracket every LZ_PROF_EVERY-th SpMV launch with events
   std::vector<hipEvent_t> spmv_ev;
   hipEvent_t lz_ev0 = nullptr, lz_ev1 = nullptr;
+  unsigned schedule = 0;  // the device's schedule flags: how the host waits
   int *ring = nullptr;  // RSB_RING ints of pinned memory: [0..2] Lanczos lists, [4..7] MG counts, [8] and [16..] rsb_read_back
   std::unordered_map<const void *, size_t> cap;  // bytes held by each dev_alloc slot
   // per-call scratch buffers, one per call site (file, line), kept across

@@ -42,8 +42,24 @@ hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { objects--; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { objects--; return hipSuccess; }
 hipError_t hipHostFree(void *) { objects--; return hipSuccess; }
-static hipError_t drain = hipSuccess;
-hipError_t hipStreamSynchronize(hipStream_t) { return drain; }
+static hipError_t drain = hipSuccess, query = hipErrorNotReady;
+static int flag, sets_after, queries, syncs, yields;
+static unsigned device_flags;
+hipError_t hipStreamSynchronize(hipStream_t) { syncs++, flag = sets_after > 0; return drain; }
+hipError_t hipStreamQuery(hipStream_t) {
+  if (++queries == sets_after) flag = 1;
+  return query;
+}
+hipError_t hipGetDeviceFlags(unsigned *f) { *f = device_flags; return hipSuccess; }
+int sched_yield(void) { yields++; return 0; }
+// waits for a flag set at the n-th query or by the synchronisation (0: never)
+int t_await(unsigned flags, int n, int drains, int ended, int *out) {
+  flag = queries = syncs = yields = 0, sets_after = n, device_flags = flags | hipDeviceMapHost;
+  drain = drains ? hipSuccess : hipErrorUnknown, query = ended ? hipSuccess : hipErrorNotReady;
+  const hipError_t e = rsb_await((hipStream_t)8, &flag, rsb_schedule());
+  out[0] = queries, out[1] = syncs, out[2] = yields;
+  return e;
+}
 int t_drain(int ok, int n, void **p) {
   drain = ok ? hipSuccess : hipErrorUnknown;
   return rsb_drain_release((hipStream_t)8, std::vector<const void *>(p, p + n));
@@ -176,6 +192,25 @@ def test_blocks_of_a_stream_that_did_not_drain_stay_out(pool, ok):
     p = (C.c_void_p * 4)(pool.t_malloc(MB), None, pool.t_malloc(2 * MB), pool.t_malloc(MB))
     assert pool.t_drain(ok, 4, p) == ok
     assert _stats(pool)[:2] == [0, 4 * MB * ok] and pool.t_used() == 4 * MB * ok
+
+
+AUTO, SPIN, YIELD, BLOCKING = 0, 1, 2, 4
+NOT_READY, UNKNOWN = 600, 999
+
+
+@pytest.mark.parametrize("flags", [AUTO, SPIN, YIELD, BLOCKING])
+def test_the_host_waits_as_the_schedule_flags_ask(pool, flags):
+    out = (C.c_int * 3)()
+    assert pool.t_await(flags, 3, 1, 0, out) == 0
+    queries, syncs, yields = out
+    if flags == BLOCKING:  # asleep in the runtime, not looking
+        assert (queries, syncs, yields) == (0, 1, 0)
+        assert pool.t_await(flags, 0, 1, 0, out) == NOT_READY
+        assert pool.t_await(flags, 3, 0, 0, out) == UNKNOWN
+    else:
+        assert queries == 3 and syncs == 0 and (yields > 1000) == (flags == YIELD)
+        # a stream that ends without setting the flag
+        assert pool.t_await(flags, 0, 1, 1, out) == NOT_READY and out[0] == 1
 
 
 def test_threads(pool):
