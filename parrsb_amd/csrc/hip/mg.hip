@@ -1528,7 +1528,6 @@ struct mg_scope {
   std::vector<const void *> bufs;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  hipEvent_t ev[2] = {nullptr, nullptr};
   bool capturing = false;
   explicit mg_scope(hipStream_t s) : st(s) {}
   template <typename T>
@@ -1547,8 +1546,6 @@ struct mg_scope {
     (void)rsb_drain_release(st, bufs);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
-    for (hipEvent_t e : ev)
-      if (e) (void)hipEventDestroy(e);
   }
 };
 
@@ -1752,7 +1749,6 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   RSB_TRY(own.alloc(coef, sizeof(double) * MG_NP * (size_t)nseg));
   RSB_TRY(own.alloc(active, 3 * sizeof(int)));
   RSB_TRY(hipMemsetAsync(active, 0, 3 * sizeof(int), st));
-  for (hipEvent_t &e : own.ev) RSB_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   // Gram basis: at most one vector per pass that another pass follows
   mg_gram G{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, max_passes - 1};
   const bool gram = grammian && G.cap >= 1;
@@ -1893,14 +1889,17 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
   // before, runs: reading it before queueing left the device idle for about
   // 20 us of every 190.  The iteration queued after the last one finds no
   // running segment, and every one of its launches returns at its gate.
+  // (the events of the handle's set that time the Lanczos passes: a call
+  // makes none of its own)
+  const hipEvent_t ev[2] = {g->lz_ev0, g->lz_ev1};
   int reports = 0;
   auto queued = [&]() -> int {
-    RSB_TRY(hipEventRecord(own.ev[reports & 1], st));
+    RSB_TRY(hipEventRecord(ev[reports & 1], st));
     reports++;
     return 0;
   };
   auto count_of = [&](int q, int &n) -> int {
-    RSB_TRY(hipEventSynchronize(own.ev[q & 1]));
+    RSB_TRY(hipEventSynchronize(ev[q & 1]));
     n = __atomic_load_n(ring + q % MG_RING, __ATOMIC_ACQUIRE);
     return 0;
   };

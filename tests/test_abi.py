@@ -117,6 +117,17 @@ def test_input_errors_before_device(monkeypatch):
     assert "at most 64 passes" in pa.last_error()
 
 
+def test_calls_make_no_streams_or_events_of_their_own():
+    """They come with the handle (made once per GPU for allocation-free calls,
+    as the header says); only profiling and the bandwidth test add events."""
+    hip = os.path.join(ROOT, "parrsb_amd", "csrc", "hip")
+    makers = {f for f in os.listdir(hip)
+              if re.search(r"hip(Event|Stream)Create", open(os.path.join(hip, f)).read())}
+    assert makers == {"mesh.hip", "noalloc.hip", "lanczos.hip", "stream.hip"}
+    lz = open(os.path.join(hip, "lanczos.hip")).read()
+    assert re.findall(r"hip\w+Create\w*\([^)]*\)", lz) == ["hipEventCreate(&g->spmv_ev[q])"]
+
+
 def test_oracle_is_not_linked_by_the_product():
     nm = subprocess.run(["nm", "-D", pa.LIB_PATH], capture_output=True, text=True).stdout
     assert "oracle_" not in nm
