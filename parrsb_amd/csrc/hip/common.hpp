@@ -104,52 +104,3 @@ __device__ inline void block_sum(double (&v)[NV], double *red) {
   __syncthreads();
 }
 
-// Error-free transformation a + b = s + e (Knuth two-sum), for compensated
-// FP32 accumulation.
-__device__ inline void two_sum(float a, float b, float &s, float &e) {
-  s = a + b;
-  float bb = s - a;
-  e = (a - (s - bb)) + (b - bb);
-}
-
-// Compensated accumulator: value = hi + lo.
-struct fsum {
-  float hi, lo;
-  __device__ fsum() : hi(0.f), lo(0.f) {}
-  __device__ inline void add(float x) {
-    float s, e;
-    two_sum(hi, x, s, e);
-    hi = s;
-    lo += e;
-  }
-  __device__ inline double value() const { return (double)hi + (double)lo; }
-};
-
-// Agent-scope load that bypasses the non-coherent per-CU cache; used when a
-// block reads values that other blocks published in the same launch.
-template <typename T>
-__device__ inline T load_acquire(const T *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// "Last block of a group" handshake: every block of a group of `count`
-// blocks calls this once after publishing its partial results; it returns
-// true in exactly one block (the last to arrive), after which that block may
-// read every partial of the group.  The counter is re-armed for the next
-// use.  Must be called by all threads of the block.
-__device__ inline bool last_block_of(unsigned *counter, unsigned count) {
-  __shared__ bool is_last;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();
-    unsigned prev = atomicAdd(counter, 1u);
-    is_last = (prev == count - 1);
-    if (is_last) {
-      __threadfence();
-      __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  __syncthreads();
-  if (is_last) __threadfence();
-  return is_last;
-}

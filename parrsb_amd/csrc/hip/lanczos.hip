@@ -2589,27 +2589,35 @@ static int run_lanczos(rsbgpu *g, int miter_opt, int mpass, double tol, int init
   auto apply_launch = [&](int it) {
     T *pold = (it & 1) ? p2 : p, *pnew = (it & 1) ? p : p2;
     const unsigned grid = xgrid(nact[0]);
-    if (fuse) {
-      lz_args af;
-      if (fold) {
+    if constexpr (sizeof(T) == 4) {  // FP64 passes are never folded
+      if (fold && fuse) {
+        lz_args af;
         const lz_fuse fu = fused(it, (it + 1) & 1, af);
         k_lz_apply_f<T, true><<<grid, RSB_BLOCK, 0, st>>>(af, fu, pold, pnew, W[it & 1], basis,
                                                           mpad, ta, W[(it + 1) & 1]);
-      } else {
-        const lz_fuse fu = fused(it, 1, af);
-        k_lz_apply_f<T, false><<<grid, RSB_BLOCK, 0, st>>>(af, fu, pold, pnew, w, basis, mpad, ta,
-                                                           nullptr);
+        return;
       }
-    } else if (fold)
-      k_lz_apply<T, true><<<grid, RSB_BLOCK, 0, st>>>(ai, pold, pnew, W[it & 1], basis, mpad, ta,
-                                                      nact[0], W[(it + 1) & 1]);
-    else if (vform)
-      k_lz_apply_v<float><<<grid, RSB_BLOCK, 0, st>>>(ai, (const float *)pold, (float *)pnew,
-                                                      (float *)w, (const float *)basis, mpad, va,
-                                                      ta, nact[0]);
-    else
+      if (fold) {
+        k_lz_apply<T, true><<<grid, RSB_BLOCK, 0, st>>>(ai, pold, pnew, W[it & 1], basis, mpad, ta,
+                                                        nact[0], W[(it + 1) & 1]);
+        return;
+      }
+      if (vform) {
+        k_lz_apply_v<float><<<grid, RSB_BLOCK, 0, st>>>(ai, (const float *)pold, (float *)pnew,
+                                                        (float *)w, (const float *)basis, mpad, va,
+                                                        ta, nact[0]);
+        return;
+      }
+    }
+    if (fuse) {
+      lz_args af;
+      const lz_fuse fu = fused(it, 1, af);
+      k_lz_apply_f<T, false><<<grid, RSB_BLOCK, 0, st>>>(af, fu, pold, pnew, w, basis, mpad, ta,
+                                                         nullptr);
+    } else {
       k_lz_apply<T, false><<<grid, RSB_BLOCK, 0, st>>>(ai, pold, pnew, w, basis, mpad, ta,
                                                        nact[0], nullptr);
+    }
   };
   // the iteration sums: wide workgroups where the segments are big
   const bool wide_fin = max_seg_tiles > LZ_FIN_WIDE;

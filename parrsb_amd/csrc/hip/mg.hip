@@ -1083,8 +1083,7 @@ struct mg_low_level {
   const uint32_t *spk;
 };
 struct mg_low {
-  int nlev;    // levels that have a coarser one below
-  int stride;  // rows of the largest segment on the first of them
+  int nlev;  // levels that have a coarser one below
   mg_low_level lv[MG_LOW_LEVELS];
 };
 
@@ -1812,7 +1811,6 @@ extern "C" int rsbgpu_fiedler_mg(rsbgpu *g, int max_iter, int max_passes, double
     low_lds = std::max(low_lds, sizeof(double) * 2 * (tot + (size_t)H.h_n[l0][s]));
   }
   while (low_threads < low_rows && low_threads < MG_LOW_THREADS) low_threads *= 2;
-  low.stride = low_rows;
   int *const ring = g->ring + 4;  // pinned: the counts that k_mg_report writes
   // One CG iteration is part_a (w = L p, alpha, the update of x and r, the
   // stop test) and part_b (z = V-cycle(r), beta, the new direction made

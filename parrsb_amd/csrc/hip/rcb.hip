@@ -269,7 +269,7 @@ __global__ void k_child_count(int K, const nodes_t nd, int *__restrict__ cnt) {
 }
 
 __global__ void k_children(int K, const nodes_t nd, const int *__restrict__ first, nodes_t ch,
-                           int *__restrict__ split, int *__restrict__ stat) {
+                           int *__restrict__ split) {
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= K) return;
   int c = first[k];
@@ -286,18 +286,6 @@ __global__ void k_children(int K, const nodes_t nd, const int *__restrict__ firs
   ch.start[c + 1] = nd.start[k] + nl, ch.len[c + 1] = n - nl, ch.p[c + 1] = pu;
   ch.frozen[c + 1] = (n - nl) <= 1;
   split[k] = nd.start[k] + nl;
-  // stat[0]: longest child that still splits; stat[1]: some such child has
-  // more ranks than elements (then empty nodes can appear below it)
-  if (stat) {
-    if (nl > 1) {
-      atomicMax(&stat[0], nl);
-      if (pl > nl) atomicOr(&stat[1], 1);
-    }
-    if (n - nl > 1) {
-      atomicMax(&stat[0], n - nl);
-      if (pu > n - nl) atomicOr(&stat[1], 1);
-    }
-  }
 }
 
 __global__ void k_nodeof_next(int nel, const int *__restrict__ first,
@@ -1208,7 +1196,7 @@ static int run_rib(rsbgpu *g) {
     RSB_READ(g, {&tail[0], first + K - 1, sizeof(int)}, {&tail[1], cnt + K - 1, sizeof(int)});
     const int K2 = tail[0] + tail[1];
     if ((size_t)K2 > cap) RSB_FAIL(2, "RIB node table overflow (%d > %zu)", K2, cap);
-    k_children<<<nblocks(K, 256), 256, 0, st>>>(K, A, first, B, split, nullptr);
+    k_children<<<nblocks(K, 256), 256, 0, st>>>(K, A, first, B, split);
     RSB_LAUNCH_CHECK();
     k_nodeof_next<<<nblocks(nel, 256), 256, 0, st>>>(nel, first, split, nodeof);
     RSB_LAUNCH_CHECK();

@@ -248,21 +248,6 @@ int rsb_wait_flag(rsbgpu *g, const int *flag);
     return (code);                                                              \
   } while (0)
 
-// grow-only device allocation
-template <typename T>
-inline hipError_t dev_ensure(T *&p, size_t &cap_elems, size_t need) {
-  if (need <= cap_elems && p) return hipSuccess;
-  if (p) {
-    hipError_t e = rsb_dev_free(p);
-    if (e != hipSuccess) return e;
-    p = nullptr;
-  }
-  size_t n = need ? need : 1;
-  hipError_t e = rsb_dev_malloc((void **)&p, n * sizeof(T));
-  if (e == hipSuccess) cap_elems = n;
-  return e;
-}
-
 template <typename T>
 inline hipError_t dev_alloc(rsbgpu *g, T *&p, size_t n) {
   // a buffer slot of the handle keeps its allocation while it is large

@@ -119,15 +119,6 @@ __device__ inline int tb_scan(int v, int *total) {
   return incl - v;
 }
 
-// Position of entry j of lane `lane` in its slice's 16-bit entries: groups
-// of 8 (row-interleaved 16-byte words), then a group of 4 (8-byte words)
-// and a group of 2 (4-byte words) where the width w8 has them.
-__device__ inline int e16_pos(int j, int lane, int w8) {
-  const int full = w8 & ~7, k = j - full, t4 = (w8 - full) & 4;
-  return j < full ? (j >> 3) * 512 + lane * 8 + (j & 7)
-                  : (k < t4 ? full * 64 + lane * 4 + k : full * 64 + t4 * 64 + lane * 2 + (k - t4));
-}
-
 // 21 slots (stride RSB_BLOCK in LDS) into the eight words of a block:
 // index k at bit 12 k.  Unrolled, so the words stay in registers.
 __device__ inline void pack21(const uint16_t *my, uint32_t (&pw)[8]) {
@@ -161,8 +152,10 @@ __device__ inline void lds_bitonic(int *a, int n) {
 // tile t's list has room for every row it can hold (halo_off, from the host),
 // so no count has to come first.  A tile's halo rows are listed in ascending
 // row order (local index nrows + rank), so the apply's staging gathers them
-// at increasing addresses and neighbouring lanes share cache lines.  Entries
-// are written a whole group (16, 8 or 4 bytes a lane) at a time.
+// at increasing addresses and neighbouring lanes share cache lines.  A slice's
+// entries lie in groups of 8 (row-interleaved 16-byte words), then a group of
+// 4 (8-byte words) and a group of 2 (4-byte words) where its width has them,
+// written and read a whole group at a time.
 __global__ void __launch_bounds__(RSB_BLOCK) k_tile_build(
     const int *__restrict__ tile, const int64_t *__restrict__ slice_off,
     const int *__restrict__ slice_w, const uint32_t *__restrict__ ell, int all_wide,
