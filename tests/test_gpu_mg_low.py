@@ -2,7 +2,9 @@
 oracle, at the sizes where its form changes: a level of 64 / 65 rows (one
 wave or the workgroup), of 1024 / 1025 rows (one or two rows per thread) and
 of 2048 / 2050 rows (the workgroup or a launch per step), and factors that
-are no powers of two."""
+are no powers of two.  With four and five levels above k_mg_low (33,920 and
+67,200 elements) the way up takes k_mg_prolong_c first and evaluates the last
+three in k_mg_up0."""
 import numpy as np
 import pytest
 
@@ -14,7 +16,8 @@ from parrsb_amd import meshgen as M
 @pytest.mark.parametrize("dims,factor", [((4, 4, 8), 2), ((2, 5, 13), 2), ((8, 8, 32), 2),
                                          ((5, 10, 41), 2), ((8, 16, 32), 2), ((10, 10, 41), 2),
                                          ((1, 1, 2), 2), ((1, 1, 3), 7), ((6, 7, 20), 3),
-                                         ((16, 20, 30), 5)])
+                                         ((16, 20, 30), 5), ((16, 20, 106), 2), ((10, 24, 280), 2),
+                                         ((16, 24, 170), 3)])
 def test_low_levels_match_oracle(oracle, dims, factor):
     print("mg low", dims, factor, flush=True)
     vtx, xyz, nv = M.box_hex(*dims)
