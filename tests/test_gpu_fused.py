@@ -55,6 +55,34 @@ def test_fused_iterations_equal_separate_launches(name, prec, fold, tiles, monke
     assert np.array_equal(ff, fu)
 
 
+@pytest.mark.parametrize("prec,fold", [(64, "0"), (32, "0"), (32, "4096")])
+@pytest.mark.parametrize("dims", [(64, 64, 128), (128, 64, 127), (128, 64, 128)])
+def test_fused_iterations_of_large_segments(dims, prec, fold, monkeypatch):
+    """Segments of 512, 1,016 and 1,024 tiles, the last the fused form's limit,
+    and the same cut at 513 tiles (at one for the first): the sums of a
+    segment take one round of a workgroup's loads, folded two above 512."""
+    print("fused large", dims, prec, fold, flush=True)
+    (vtx, xyz, nv), n = M.box_hex(*dims, jitter=0.1, seed=1), int(np.prod(dims))
+    res = {}
+    monkeypatch.setenv("PARRSB_AMD_LZ_FOLD_TILES", fold)
+    for fuse in ("1024", "0"):
+        monkeypatch.setenv("PARRSB_AMD_LZ_FUSE_TILES", fuse)
+        import parrsb_amd as pa
+        with pa.Device() as d:
+            d.set_mesh(vtx, xyz, nv)
+            for b in ([0, n], [0, 513 * 1024 - 100, n] if n > 513 * 1024 else [0, 1000, n]):
+                nseg = len(b) - 1
+                d.set_segments(b[:-1], np.diff(b), [2] * nseg, 2 * np.arange(nseg))
+                d.prepartition(1)
+                d.level_laplacian()
+                out = d.fiedler(nseg, precision=prec, max_iter=12, max_passes=2)
+                res.setdefault(fuse, []).append((out, d.fiedler_values()))
+    for (of, ff), (ou, fu) in zip(res["1024"], res["0"]):
+        for k in ("niter", "npass", "lambda", "rnorm", "resid"):
+            assert np.array_equal(of[k], ou[k], equal_nan=True), k
+        assert np.array_equal(ff, fu)
+
+
 @pytest.mark.parametrize("n", [1, 2, 50, 63, 64, 65, 128])
 def test_tridiagonal_solves_over_wide_ranges(n, oracle):
     """Entries over 300 decades, zero off-diagonals and a zero diagonal leave
