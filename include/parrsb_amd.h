@@ -112,7 +112,8 @@ int parrsb_amd_last_report(parrsb_amd_report *rep);
 const char *parrsb_amd_last_error(void);
 
 /* Lanczos vector precision for later calls: 64 (reference, default) or 32
- * (FP32 vectors, compensated dot products, FP64 scalars and eigen-solve).
+ * (FP32 vectors, dot products within 2^-24 of the sum of their terms'
+ * magnitudes, FP64 scalars and eigen-solve).
  * Overridden by PARRSB_AMD_PRECISION. */
 int parrsb_amd_set_precision(int bits);
 

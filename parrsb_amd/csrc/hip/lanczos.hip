@@ -25,9 +25,10 @@
 // first instruction.
 //
 // Precision: vectors are T (double, or float); every scalar and the
-// tridiagonal eigen-solve are FP64.  With T = float, dot products are
-// compensated (Dot2: exact products and error-free sums in FP32) and their
-// block partials are combined in FP64.
+// tridiagonal eigen-solve are FP64.  With T = float, the dot products of a
+// thread's rows are summed in FP32 with a running correction, to within
+// 2^-24 of the sum of the products' magnitudes (acc_t), and block partials
+// are combined in FP64.
 #include <algorithm>
 #include <vector>
 
@@ -115,7 +116,16 @@ struct acc_t<double> {
 template <>
 struct acc_t<float> {
   float s = 0.f, c = 0.f;
-  // s + xy rounded once; c takes that sum's error and the product's
+  // s + xy rounded once (et: that rounding's error).  ep, the rounding error
+  // of the product alone, belongs to the sum of rounded products (dot2); here
+  // it is counted although the product was never rounded, so a sum is off by
+  // up to 2^-24 sum |x y| (at most 5e-8, 1.3e-8 and 4e-9 of it in 20,000 sums
+  // of 4, 64 and 1,024 terms of one sign; 1e-14, 1e-13 and 2e-12 without ep).
+  // It stays because it decides bits: this is what the two-sum of x * y has
+  // always compiled to under contraction, and c + et moves 2.3% of the
+  // elements of 250k holed quads in 256 parts and 0.2% of a 2M-hex pipe's to
+  // other parts, at the same cut (+0.002% on the pipe) and 0.4% and 0.2% more
+  // iterations; the parts of four other meshes stay the same.
   __device__ inline void dot(float x, float y) {
 #pragma clang fp contract(off)
     const float ep = fmat(x, y, -(x * y));
@@ -1790,10 +1800,13 @@ __device__ inline void fin_sums(const double *__restrict__ partial, int stride, 
 }
 
 // |r - af w|^2 from the folded apply's sums r.r, r.w, w.w, af = alpha as the
-// next launch rounds it: FP64 sums of exact FP32 products, from this
-// iteration's stored r and w, so the value does not drift over the
-// iterations; it differs from the sum of squares of the rounded new r by at
-// most 2^-23 relative.
+// next launch rounds it, from this iteration's stored r and w, so the value
+// does not drift over the iterations.  With rho = |r| / |r - af w| it is off by
+// at most 2^-24 (2 rho + 1)^2 relative from the sums (each within 2^-24 of its
+// magnitude, |af w| <= |r| + |r - af w|), and by 2^-23 from the rounding of
+// the new r: 1e-6 or less where an iteration leaves the residual about as it
+// was, as nearly all do.  Errors of the sums' terms cancel mostly: 3e-7 was
+// measured at rho = 10, 3e-5 at 100 (1,170 rows; 2e-6 from the stored new r).
 __device__ inline double fold_rtr(double alpha, double rr, double rw, double ww) {
   const double af = (double)(float)alpha;
   const double rtr = fmat(af * af, ww, fmat(-2.0 * af, rw, rr));
@@ -1972,16 +1985,18 @@ __global__ void __launch_bounds__(NT) k_lz_fin(lz_args a, int op) {
 // hexes in FP64 from 13.5 + 4.0 + 2 x 3.75 to 11.6 + 4.1 us.
 struct lz_fuse {
   const lz_desc *list;  // tiles of the launch, split over the XCDs as in list_index
-  int nlist, per, it;   // per: grid / LZ_XCDS
-        // it: iteration of the pass (the same for every running segment)
+  int nlist, per;       // per: grid / LZ_XCDS
+  int it;               // iteration of the pass (the same for every running segment)
   const lz_it *st_in;
   lz_it *st_out;
   const double *pa_in;  // partials of the launch before; those of this one go to lz_args.partial
 };
 // most tiles of a segment: one round of four loads per thread covers the
-// partials.  Whole calls at 1,024 / 512 / 256 / 0 (separate launches): 1M
-// hexes FP64 78.7 / 80.3 / 82.1 / 86.2 ms, FP32 60.9 / 61.3 / 62.4 / 64.6, 2M
-// pipe 702 / 704 / 707 / 739, 260k quads 239 / 239 / 239 / 302
+// partials of an unfolded launch, two rounds of two (of each of six slots)
+// those of a folded one from 513 tiles on.  Whole calls at 1,024 / 512 / 256 /
+// 0 (separate launches): 1M hexes FP64 78.7 / 80.3 / 82.1 / 86.2 ms, FP32
+// 60.9 / 61.3 / 62.4 / 64.6, 2M pipe 702 / 704 / 707 / 739, 260k quads 239 /
+// 239 / 239 / 302
 #define LZ_FUSE_TILES 1024
 // iterations queued between a compaction and the look at its lengths: two of
 // 5 to 10 us cover the host's look and its next launches
