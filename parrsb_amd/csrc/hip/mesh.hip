@@ -149,7 +149,7 @@ extern "C" void rsbgpu_close(rsbgpu *g) {
   for (auto &kv : g->scratch)
     FREE(kv.second.first);
   g->scratch.clear();
-  for (void *p : g->retired) FREE(p);
+  for (const void *p : g->retired) FREE(p);
   g->retired.clear();
   if (!g->borrowed) {
     rsb_pool_tick(g->device);

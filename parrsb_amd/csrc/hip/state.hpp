@@ -175,14 +175,15 @@ struct rsbgpu {
   std::map<std::pair<const void *, int>, std::pair<void *, size_t>> scratch;
   // buffers replaced by larger ones while queued work may still use them,
   // released when the handle closes
-  std::vector<void *> retired;
+  std::vector<const void *> retired;
   size_t retired_bytes = 0;
 };
 
 // Gives up a buffer that a larger one replaces (p becomes nullptr).  Small
 // ones wait for the handle's close instead of making the device wait now (a
-// free does), at most RSB_RETIRED_MAX bytes of them; large ones are freed at
-// once, and so are those of an allocation-free call, whose frees never wait.
+// free does); once RSB_RETIRED_MAX bytes of them have come together they go
+// to the pool, for one wait.  Large ones are freed at once, and so are those of
+// an allocation-free call, whose frees never wait.
 #define RSB_RETIRE_MAX ((size_t)64 << 20)
 #define RSB_RETIRED_MAX ((size_t)256 << 20)
 template <typename T>
@@ -190,10 +191,13 @@ inline hipError_t rsb_retire(rsbgpu *g, T *&p, size_t bytes) {
   void *q = (void *)p;
   p = nullptr;
   if (!q) return hipSuccess;
-  if (g->borrowed || bytes > RSB_RETIRE_MAX || g->retired_bytes + bytes > RSB_RETIRED_MAX)
-    return rsb_dev_free(q);
+  if (g->borrowed || bytes > RSB_RETIRE_MAX) return rsb_dev_free(q);
   g->retired.push_back(q);
   g->retired_bytes += bytes;
+  if (g->retired_bytes > RSB_RETIRED_MAX) {
+    (void)rsb_drain_release(g->stream, g->retired);
+    g->retired.clear(), g->retired_bytes = 0;
+  }
   return hipSuccess;
 }
 // A buffer of `need` bytes, in place of one of `old` bytes if that is not 0:
@@ -205,7 +209,7 @@ inline hipError_t rsb_dev_malloc_grown(rsbgpu *g, void **p, size_t need, size_t 
   *got = old && !g->borrowed ? need + need / 8 : need;
   hipError_t e = rsb_dev_malloc(p, *got);
   if (e == hipSuccess || g->borrowed) return e;
-  for (void *q : g->retired) (void)rsb_dev_free(q);  // (waits for the device)
+  for (const void *q : g->retired) (void)rsb_dev_free(q);  // (waits for the device)
   g->retired.clear(), g->retired_bytes = 0;
   *got = need;
   return rsb_dev_malloc(p, need);
