@@ -124,8 +124,9 @@ struct acc_t<float> {
   // It stays because it decides bits: this is what the two-sum of x * y has
   // always compiled to under contraction, and c + et moves 2.3% of the
   // elements of 250k holed quads in 256 parts and 0.2% of a 2M-hex pipe's to
-  // other parts, at the same cut (+0.002% on the pipe) and 0.4% and 0.2% more
-  // iterations; the parts of four other meshes stay the same.
+  // other parts, at the same cut (-0.002% on the pipe) and 0.4% and 0.2% fewer
+  // iterations, as many as without the folded update; the parts of four other
+  // meshes stay the same.
   __device__ inline void dot(float x, float y) {
 #pragma clang fp contract(off)
     const float ep = fmat(x, y, -(x * y));
@@ -163,7 +164,11 @@ struct tile_t {
 // eight contiguous parts, one per XCD, so a tile's halo rows are mostly rows
 // its XCD has just read (grid: nlist rounded up to a multiple of 8).
 #define LZ_XCDS 8
-// running tiles up to which an FP32 pass folds its r-update into the apply
+// running tiles up to which an FP32 pass folds its r-update into the apply.
+// Whole calls at 0 / 1,024 / 2,048 / 4,096, fused launches: 250k holed quads
+// 311 / 256 / 254 / 254 ms, 2M-hex pipe 693 / 690 / 670 / 671, 1M hexes with the
+// learned start 63.3 / 61.9 / 61.1 / 61.4; 256^3 hexes in 65,536 parts at 2,048
+// / 4,096 / 8,192: 4,796 / 4,792 / 4,798
 #define LZ_FOLD_TILES 4096
 // segments of more tiles than this take 512-thread finishing workgroups
 #define LZ_FIN_WIDE 1024
