@@ -26,7 +26,7 @@ typedef struct {
                                  TQLI+Ritz, sort, components, balance */
   double lanczos_bytes;       /* algorithmic bytes of all CG-Lanczos iterations */
   double lanczos_ms;          /* time of the iteration loops */
-  double lanczos_iters;       /* iterations launched (3 kernels each) */
+  double lanczos_iters;       /* iterations launched */
   double spmv_bytes;          /* algorithmic bytes of the SpMV kernel */
   double spmv_ms;             /* time inside SpMV launches (profiling on: every
                                  11th launch is timed, the mean times all) */
@@ -75,9 +75,12 @@ typedef struct {
  * search directions take the most memory per element), or more parts than
  * PARRSB_AMD_NOALLOC_MAX_NEL, are rejected with 3, and so are tagged mode
  * and rsb_mg_grammian = 1 with rsb_algo = 1 (its Gram matrices take
- * rsb_max_passes^2 doubles per segment); at
- * these limits a call holds at most about a third (Lanczos) or half (MG) of
- * the array.  The array keeps the last call's contents and is shared
+ * rsb_max_passes^2 doubles per segment).  At
+ * these limits a call into up to about a thousand parts holds at most a third
+ * (Lanczos) or two fifths (MG) of the array; parts of a few elements take
+ * more, as every segment's rows are padded to 64 (16,384 parts of four
+ * elements hold half of it), and a call that does not fit returns 2.  The
+ * array keeps the last call's contents and is shared
  * by every allocation-free call on that GPU: calls that overlap on one GPU
  * (two host threads) race.  Host bookkeeping still uses the C heap. */
 #define PARRSB_AMD_NOALLOC_BYTES (256ull << 20)

@@ -70,6 +70,8 @@ extern "C" int rsbgpu_open(rsbgpu **out, int device) {
       hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess ||
       hipEventCreate(&g->lz_ev0) != hipSuccess || hipEventCreate(&g->lz_ev1) != hipSuccess ||
       hipHostMalloc((void **)&g->ring, RSB_RING * sizeof(int), hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();
+    rsb_destroy_streams({g->stream, {g->ev0, g->ev1, g->lz_ev0, g->lz_ev1}, g->ring});
     delete g;
     return 2;
   }
